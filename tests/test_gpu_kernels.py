@@ -248,6 +248,25 @@ def test_linear_float32_does_not_depend_on_the_row_count(ops, n, k):
         assert torch.equal(small[:m], big[:m]) and torch.all(small[m] == 7.0), f"{m} rows"
 
 
+@pytest.mark.parametrize("n,k", [(63, 252), (64, 256), (65, 260), (8192, 36), (129, 2052), (20000, 64), (130, 4500)])
+def test_linear_float32_at_the_edges_of_its_tiles(ops, n, k):
+    """Row counts around the tiles of 16 and 64 tokens, columns around those of 64 and 128, K around the segments of 256:
+    every count gives the bits a single row gives, nothing is written past the end, and the error against 64 bits is that of
+    chains of at most 64 terms and what is added of them: k / 64 sums, 2^-24 each, at random."""
+    x, w = rnd(1100, k, seed=1), rnd(n, k, seed=2)
+    single = torch.cat([torch.empty(1, n, device=DEV) for _ in range(6)])
+    picks = (0, 15, 16, 63, 64, 1099)
+    for i, row in enumerate(picks):
+        ops.linear(x[row:row + 1], w, single[i:i + 1])
+    assert rel(single, x[list(picks)].double() @ w.double().T) < 6e-8 * (64 + k / 64) ** 0.5
+    for m in (16, 17, 32, 33, 48, 49, 64, 65, 128, 1100):
+        out = torch.full((m + 1, n), 7.0, device=DEV)
+        ops.linear(x[:m], w, out[:m])
+        assert torch.all(out[m] == 7.0)
+        for i, row in enumerate(picks):
+            assert row >= m or torch.equal(out[row], single[i]), f"{m} rows: row {row}"
+
+
 @pytest.mark.parametrize("m", [1, 2, 7, 16, 17, 33, 64])
 @pytest.mark.parametrize("n,k", [(48, 64), (1000, 96), (129, 2048), (16, 8), (250, 72)])
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
