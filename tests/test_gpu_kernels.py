@@ -650,6 +650,41 @@ def test_paged_attention_mixed_batch(ops, act, hq, hkv, d):
     assert rel(got, want) < (2e-5 if act == torch.float32 else 2e-2)
 
 
+@pytest.mark.parametrize("hq,hkv,d,window", [(8, 2, 64, None), (16, 1, 16, None), (8, 4, 32, 130), (4, 4, 128, 33), (8, 1, 64, 16)])
+def test_float32_attention_does_not_depend_on_the_step(ops, hq, hkv, d, window):
+    """Tiles of 16 queries and heads, runs of 128 keys: positions one before, at and behind a run's, a page's and a tile's
+    edge, each once in the whole prompt, once as a single token and once inside a portion, bit for bit the same, and the
+    whole prompt's error is that of weighted sums in runs of 128 (2^-24 a term)."""
+    n, blocks = 600, 40
+    perm = np.random.default_rng(d).permutation(blocks).tolist()
+    table = perm[: -(-n // 16)]
+    pk = StepPacker(torch.device(DEV), [GroupMeta(blocks, window)], 10, 100000, 8, ops.PREFILL_TILE_Q, skew_rule=ops.decode_is_skewed)
+    kv = torch.full((blocks, 2, hkv, 16 * d), float("nan"), device=DEV)
+    qkv = rnd(n, (hq + 2 * hkv) * d, seed=d)
+    k, v = (qkv[:, c * d: (c + hkv) * d].reshape(n, hkv, d) for c in (hq, hq + hkv))
+    pages, off = torch.tensor(table, device=DEV)[torch.arange(n, device=DEV) // 16], torch.arange(n, device=DEV) % 16
+    kv[:, 0].view(blocks, hkv, 16, d)[pages, :, off, :] = k
+    kv[:, 1].view(blocks, hkv, d, 16)[pages, :, :, off] = v
+
+    def run(first, count):
+        out = torch.empty(count, hq * d, device=DEV)
+        ctx = pk.pack([StepItem(0, [1] * count, first, [table])])
+        ops.paged_attention(qkv[first: first + count].contiguous(), out, kv, ctx, 0, hq, hkv, d, d ** -0.5, window)
+        return out
+
+    whole = run(0, n)
+    back = torch.arange(n, device=DEV)[:, None] - torch.arange(n, device=DEV)[None]
+    q = qkv[:, : hq * d].view(n, hq, d).double().transpose(0, 1)
+    s = (q @ k.double().repeat_interleave(hq // hkv, 1).permute(1, 2, 0)) * d ** -0.5
+    p = torch.softmax(s.masked_fill((back < 0) | (back >= (window or n)), float("-inf")), -1)
+    want = (p @ v.double().repeat_interleave(hq // hkv, 1).transpose(0, 1)).transpose(0, 1).reshape(n, hq * d)
+    assert rel(whole, want) < 2e-6
+    for pos in (0, 1, 15, 16, 31, 127, 128, 129, 255, 256, 511, 513, 599):
+        assert torch.equal(run(pos, 1)[0], whole[pos]), f"position {pos} alone"
+        first = max(pos - 5, 0)
+        assert torch.equal(run(first, pos - first + 1), whole[first: pos + 1]), f"portion up to {pos}"
+
+
 @pytest.mark.parametrize("hq,hkv,d,longest,window", [
     (32, 8, 64, 700, None),        # 40 requests x 8 kv heads: keys not split over workgroups
     (32, 8, 64, 700, 150),         # the same with a window whose first pages were given back
