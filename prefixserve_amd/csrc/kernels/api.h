@@ -148,7 +148,7 @@ int psamd_moe_experts_rows(void* stream, const void* x, const int32_t* chosen, c
 
 // The same for bfloat16 with the pairs sorted by expert and every expert's pairs run through its
 // matrices in tiles on the matrix cores. ints: scratch of pairs + 3 * psamd_moe_grouped_max_tiles(pairs,
-// experts) integers (pairs = tokens * top). K and F multiples of 8.
+// experts) + 1 integers (pairs = tokens * top). K and F multiples of 8.
 int psamd_moe_grouped_tile_rows(int64_t pairs, int experts);
 int psamd_moe_grouped_max_tiles(int64_t pairs, int experts);
 int psamd_moe_experts_grouped(void* stream, const void* x, const int32_t* chosen, const float* weight,

@@ -391,14 +391,14 @@ __global__ __launch_bounds__(256) void moe_down_rows_kernel(
 
 // One workgroup sorts the step's pairs by expert and lists the tiles of `tile_rows` pairs the
 // products run over. ints: sorted[pairs] (pair indices, expert by expert), then per tile slot
-// tile_expert, tile_first (index into sorted), tile_count; slots past the last tile hold -1.
+// tile_expert, tile_first (index into sorted), tile_count; slots past the last tile hold -1; then the number of tiles.
 // The order of an expert's pairs among themselves is whatever the atomics gave: every pair's
 // result is computed from its own row alone, so it does not matter which rows share a tile.
 // `count`, `start`, `tstart`, `cursor` are LDS arrays of `experts` integers each.
 __device__ __forceinline__ void group_pairs(const int32_t* __restrict__ chosen, int pairs, int experts, int tile_rows,
                                             int max_tiles, int32_t* __restrict__ sorted, int32_t* __restrict__ tile_expert,
                                             int32_t* __restrict__ tile_first, int32_t* __restrict__ tile_count,
-                                            int32_t* count, int32_t* start, int32_t* tstart, int32_t* cursor,
+                                            int32_t* tiles_out, int32_t* count, int32_t* start, int32_t* tstart, int32_t* cursor,
                                             int32_t* n_tiles) {
   for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = cursor[e] = 0;
   __syncthreads();
@@ -437,6 +437,7 @@ __device__ __forceinline__ void group_pairs(const int32_t* __restrict__ chosen, 
       tile_count[nt] = min(tile_rows, count[e] - r0);
     }
   }
+  if (threadIdx.x == 0) *tiles_out = *n_tiles;
   for (int nt = *n_tiles + threadIdx.x; nt < max_tiles; nt += blockDim.x) tile_expert[nt] = -1;
   for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
     const int e = min(max(chosen[p], 0), experts - 1);
@@ -449,7 +450,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t* __restri
                                                          int32_t* __restrict__ tile_expert, int32_t* __restrict__ tile_first,
                                                          int32_t* __restrict__ tile_count) {
   extern __shared__ int32_t group_smem[];      // count, start, tstart, cursor [experts] each, n_tiles
-  group_pairs(chosen, pairs, experts, tile_rows, max_tiles, sorted, tile_expert, tile_first, tile_count, group_smem,
+  group_pairs(chosen, pairs, experts, tile_rows, max_tiles, sorted, tile_expert, tile_first, tile_count, tile_count + max_tiles, group_smem,
               group_smem + experts, group_smem + 2 * experts, group_smem + 3 * experts, group_smem + 4 * experts);
 }
 
@@ -472,7 +473,7 @@ __global__ __launch_bounds__(1024) void moe_topk_group_kernel(const float* __res
   }
   __threadfence_block();
   __syncthreads();                             // the workgroup's own writes of `chosen` are read below
-  group_pairs(chosen, tokens * top, buckets, tile_rows, max_tiles, sorted, tile_expert, tile_first, tile_count, group_smem,
+  group_pairs(chosen, tokens * top, buckets, tile_rows, max_tiles, sorted, tile_expert, tile_first, tile_count, tile_count + max_tiles, group_smem,
               group_smem + experts, group_smem + 2 * experts, group_smem + 3 * experts, group_smem + 4 * experts);
 }
 
@@ -673,6 +674,173 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
   }
 }
 
+// ------------------------------------------------------------------ experts, many pairs each
+
+// A tile of TM pairs by TN rows of the expert's matrix per workgroup of WM x WN waves, both operands through LDS 64 k at a
+// time. The matrices of all experts are read at the rate the matrix cores use them only if a workgroup multiplies each byte
+// often: 256 x 256 asks for half the bytes per product of the kernel above, whose rows of the matrix go from memory to
+// registers for one tile of 128 pairs (14 TB/s out of the L2s at 16,384 pairs over 32 experts of 1,024 x 2,048: 250 us for
+// the first product, 143 for the second; here 187 and 123). What it does about each bound:
+//  * memory to LDS without registers (global_load_lds, 16 bytes a lane), the step after next always under way;
+//  * LDS rows of 128 bytes with the 16-byte pieces exchanged by row / 2, so that the 16 rows a read touches lie on all
+//    banks (the exchange is done by which piece a lane fetches: the copy itself writes lanes side by side);
+//  * the operands of half a step are read from LDS between the matrix instructions of the half before, and the one
+//    barrier of a step stands between its halves, where the matrix cores still have work;
+//  * an expert's tiles run on one die (its L2 then holds the expert's rows): die d takes the d-th eighth of the tiles;
+//  * the waves for pairs that a tile does not have skip the arithmetic, so an expert's last tile costs what it holds to
+//    half a tile.
+// GATED: a wave's 64 rows are 32 gate rows and the 32 up rows of the same columns.
+typedef __attribute__((address_space(1))) const void* global_ptr;
+typedef __attribute__((address_space(3))) void* lds_ptr;
+
+template <int TM, int TN, int WM, int WN, int FORM>
+__global__ __launch_bounds__(64 * WM * WN, 2) void moe_tile_kernel(
+    const bf16_t* __restrict__ a, const float* __restrict__ pair_weight, const bf16_t* __restrict__ w,
+    const int32_t* __restrict__ sorted, const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_first,
+    const int32_t* __restrict__ tile_count, const int32_t* __restrict__ n_tiles, bf16_t* __restrict__ out_act,
+    float* __restrict__ out_f32, int64_t tokens, int K, int N, int top, float gate_alpha, float limit, float up_shift,
+    int into_stream, const float* __restrict__ col_scale, int experts, const bf16_t* __restrict__ x,
+    const float* __restrict__ weight, int column_tiles) {
+  constexpr bool GATED = FORM == kFormGated;
+  constexpr int WV = WM * WN, BK = 64, RM = TM / WM / 16, RN = TN / WN / 16, WROWS = TN / WN;
+  constexpr int COLS = GATED ? TN / 2 : TN, WCOLS = GATED ? WROWS / 2 : WROWS;   // columns of the workgroup, of a wave
+  constexpr int LA = TM / 8 / WV, LB = TN / 8 / WV;                              // copies of 8 rows per wave and step
+  __shared__ __align__(16) bf16_t a0[TM * BK], a1[TM * BK], b0[TN * BK], b1[TN * BK];
+  __shared__ int32_t pair_s[TM];
+  const int tiles = *n_tiles, per_die = (tiles + 7) / 8;
+  const int at = static_cast<int>(blockIdx.x >> 3), slot = static_cast<int>(blockIdx.x & 7) * per_die + at / column_tiles;
+  if (at / column_tiles >= per_die || slot >= tiles) return;                     // uniform for the workgroup
+  const int n0 = at % column_tiles * COLS;
+  const int e = tile_expert[slot], first = tile_first[slot], count = tile_count[slot];
+  if (e >= experts) {                           // a tile of identity pairs: the tokens themselves times their weights
+    if (FORM != kFormDown) return;
+    for (int idx = threadIdx.x; idx < count * COLS; idx += 64 * WV) {
+      const int pair = sorted[first + idx / COLS], n = n0 + idx % COLS;
+      if (n >= N) continue;
+      const int64_t t = pair / top;
+      const float y = weight[pair] * bf16_to_float(x[t * N + n]);
+      if (into_stream) add_float(out_f32 + t * N + n, col_scale != nullptr ? col_scale[n] * y : y);
+      else out_f32[(static_cast<int64_t>(pair % top) * tokens + t) * N + n] = y;
+    }
+    return;
+  }
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int r = lane & 15, g = lane >> 4;
+  const int wm = wave / WN * (TM / WM), wn = wave % WN;                          // waves of a SIMD share no rows of pairs
+  for (int i = threadIdx.x; i < TM; i += 64 * WV) pair_s[i] = i < count ? sorted[first + i] : -1;
+  // What this lane copies: piece p of row 8 j + lane / 8 of an operand lies at place lane % 8 of that row.
+  const char* a_base = reinterpret_cast<const char*>(a);
+  const char* w_base = reinterpret_cast<const char*>(w + static_cast<int64_t>(e) * (GATED ? 2 : 1) * N * K);
+  uint32_t a_off[LA], b_off[LB];
+#pragma unroll
+  for (int i = 0; i < LA; ++i) {
+    const int row = (wave * LA + i) * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+    const int pair = sorted[first + min(row, count - 1)];
+    a_off[i] = static_cast<uint32_t>(FORM != kFormDown ? pair / top : pair) * (2u * K) + 16u * piece;
+  }
+#pragma unroll
+  for (int i = 0; i < LB; ++i) {
+    const int row = (wave * LB + i) * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+    const int col = min(n0 + (row / WROWS) * WCOLS + row % WCOLS, N - 1);
+    b_off[i] = static_cast<uint32_t>(GATED && row % WROWS >= WCOLS ? N + col : col) * (2u * K) + 16u * piece;
+  }
+  auto copy = [&](int k0, bf16_t* as, bf16_t* bs) {
+#pragma unroll
+    for (int i = 0; i < LA; ++i)
+      __builtin_amdgcn_global_load_lds((global_ptr)(a_base + a_off[i] + 2 * k0), (lds_ptr)(as + (wave * LA + i) * 8 * BK), 16, 0, 0);
+#pragma unroll
+    for (int i = 0; i < LB; ++i)
+      __builtin_amdgcn_global_load_lds((global_ptr)(w_base + b_off[i] + 2 * k0), (lds_ptr)(bs + (wave * LB + i) * 8 * BK), 16, 0, 0);
+  };
+  f32x4 acc[RN][RM];
+#pragma unroll
+  for (int i = 0; i < RN; ++i)
+#pragma unroll
+    for (int j = 0; j < RM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const bool works = wm < count;
+  const int swap = (r >> 1) & 7;
+  bf16x8 fa[2][RM], fb[2][RN];
+  auto operands = [&](const bf16_t* as, const bf16_t* bs, int half) {
+    const int c = ((half * 4 + g) ^ swap) * 8;
+#pragma unroll
+    for (int i = 0; i < RN; ++i) fb[half][i] = *reinterpret_cast<const bf16x8*>(bs + (wn * WROWS + i * 16 + r) * BK + c);
+#pragma unroll
+    for (int j = 0; j < RM; ++j) fa[half][j] = *reinterpret_cast<const bf16x8*>(as + (wm + j * 16 + r) * BK + c);
+  };
+  auto multiply = [&](int half) {
+#pragma unroll
+    for (int i = 0; i < RN; ++i)
+#pragma unroll
+      for (int j = 0; j < RM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[half][i], fa[half][j], acc[i][j], 0, 0, 0);
+#pragma unroll
+    for (int q = 0; q < RM + RN; ++q) {                                          // one read of the other half's operands, then
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                         // the matrix instructions it hides behind
+      __builtin_amdgcn_sched_group_barrier(0x008, RM * RN / (RM + RN), 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, RM * RN, 0);
+  };
+  const int steps = K / BK;
+  auto step = [&](bf16_t* ca, bf16_t* cb, bf16_t* na, bf16_t* nb, int t) {
+    if (works) {
+      operands(ca, cb, 1);
+      multiply(0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();                            // step t + 1 has arrived, and everybody has read step t
+    if (t + 2 < steps) copy((t + 2) * BK, ca, cb);
+    __builtin_amdgcn_sched_barrier(0);
+    if (works) {
+      operands(na, nb, 0);                      // behind the last step: what lies there, not used
+      multiply(1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  copy(0, a0, b0);
+  __syncthreads();
+  if (steps > 1) copy(BK, a1, b1);
+  __builtin_amdgcn_sched_barrier(0);
+  if (works) operands(a0, b0, 0);
+  for (int t = 0; t < steps; t += 2) {
+    step(a0, b0, a1, b1, t);
+    if (t + 1 < steps) step(a1, b1, a0, b0, t + 1);
+  }
+  if (!works) return;
+  // Lane (r, g) holds, for the pair in row wm + 16 j + r, columns 4 g .. + 3 of every 16 of the wave's.
+#pragma unroll
+  for (int j = 0; j < RM; ++j) {
+    const int pair = pair_s[wm + j * 16 + r];
+    if (pair < 0) continue;
+    const float pw = pair_weight != nullptr ? pair_weight[pair] : 1.f;           // on the input's sums (GATED) or on the output's
+#pragma unroll
+    for (int i = 0; i < WCOLS / 16; ++i) {
+      const int nc = n0 + wn * WCOLS + i * 16 + 4 * g;
+      if (nc >= N) continue;                                                     // N is a multiple of 8
+      if (FORM != kFormDown) {
+        bf16_t res[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          if (!GATED) {
+            const float p = fmaxf(pw * acc[i][j][v], 0.f);
+            res[v] = float_to_bf16(p * p);
+            continue;
+          }
+          const float gg = fminf(pw * acc[i][j][v], limit);
+          const float uu = fminf(fmaxf(pw * acc[(i + RN / 2) % RN][j][v], -limit), limit);
+          res[v] = float_to_bf16(gg / (1.f + __expf(-gate_alpha * gg)) * (uu + up_shift));
+        }
+        *reinterpret_cast<ushort4*>(out_act + static_cast<int64_t>(pair) * N + nc) = ushort4{res[0], res[1], res[2], res[3]};
+      } else if (into_stream) {
+        float* o = out_f32 + static_cast<int64_t>(pair / top) * N + nc;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) add_float(o + v, (col_scale != nullptr ? col_scale[nc + v] : 1.f) * (pw * acc[i][j][v]));
+      } else {
+        float* o = out_f32 + (static_cast<int64_t>(pair % top) * tokens + pair / top) * N + nc;
+        *reinterpret_cast<float4*>(o) = float4{pw * acc[i][j][0], pw * acc[i][j][1], pw * acc[i][j][2], pw * acc[i][j][3]};
+      }
+    }
+  }
+}
+
 // What the experts' two products have in common.
 struct ExpertCall {
   const void* x;
@@ -713,6 +881,45 @@ static int launch_grouped(hipStream_t s, const ExpertCall& c, const int32_t* int
   run_grouped<MT, RT, kFormDown>(s, c, ints, max_tiles);
   return check_launch("psamd_moe_experts_grouped (down)");
 }
+
+template <int TM, int TN, int WM, int WN, int FORM>
+static void run_tiles(hipStream_t s, const ExpertCall& c, const int32_t* ints, int max_tiles) {
+  const int32_t* sorted = ints;
+  const int32_t* t_e = ints + c.tokens * c.top;
+  const int32_t* t_f = t_e + max_tiles;
+  const int32_t* t_c = t_f + max_tiles;
+  constexpr bool down = FORM == kFormDown;
+  const int N = down ? c.K : c.F, K = down ? c.F : c.K;
+  const int column_tiles = static_cast<int>(ceil_div(N, FORM == kFormGated ? TN / 2 : TN));
+  const dim3 grid(static_cast<unsigned>(8 * ceil_div(max_tiles, 8) * column_tiles));
+  moe_tile_kernel<TM, TN, WM, WN, FORM><<<grid, dim3(64 * WM * WN), 0, s>>>(
+      static_cast<const bf16_t*>(down ? c.act : c.x), (c.weight_on_output != 0) == down ? c.weight : nullptr,
+      static_cast<const bf16_t*>(down ? c.w_down : c.w_in), sorted, t_e, t_f, t_c, t_c + max_tiles,
+      down ? nullptr : static_cast<bf16_t*>(c.act), down ? c.out : nullptr, c.tokens, K, N, c.top, c.gate_alpha, c.limit,
+      c.up_shift, c.into_stream, c.col_scale, c.experts, static_cast<const bf16_t*>(c.x), c.weight, column_tiles);
+}
+
+template <int TM, int TN, int WM, int WN>
+static int launch_tiles(hipStream_t s, const ExpertCall& c, const int32_t* ints, int max_tiles) {
+  if (c.kind == kExpertGated) run_tiles<TM, TN, WM, WN, kFormGated>(s, c, ints, max_tiles);
+  else run_tiles<TM, TN, WM, WN, kFormSquaredRelu>(s, c, ints, max_tiles);
+  if (check_launch("psamd_moe_experts_grouped (in)")) return 1;
+  run_tiles<TM, TN, WM, WN, kFormDown>(s, c, ints, max_tiles);
+  return check_launch("psamd_moe_experts_grouped (down)");
+}
+
+// Whether the tiles of the kernel for many pairs take these experts: whole steps of 64 k in both products, and offsets inside
+// an operand that fit 32 bits.
+static bool tiles_take(int64_t tokens, int64_t pairs, int K, int F) {
+  const int64_t most = (1LL << 32) - 1;
+  return K % 64 == 0 && F % 64 == 0 && 2 * tokens * K <= most && 2 * pairs * F <= most && 4LL * K * F <= most;
+}
+
+// ... and their rows: 0 where the kernel above takes the step. Both products and the sorting, 32 experts of 1,024 x 2,048,
+// us in tiles of 256 x 256 / 128 x 128 / the kernel above: 512 pairs an expert 323 / 374 / 428, 448 pairs 307 / 299 / 366,
+// 340 pairs 322 / 246 / 302, 150 pairs - / 157 / 240, 50 pairs - / 114 / 153, 25 pairs - / 145 / 130. The large tile wants
+// half the bytes per product, but one workgroup fills a compute unit and few rounds of them leave the last one half empty.
+static int wide_tile_rows(int64_t pairs, int experts) { return pairs >= 480LL * experts ? 256 : (pairs >= 48LL * experts ? 128 : 0); }
 
 template <typename A>
 static int launch_experts_rows(hipStream_t s, const ExpertCall& c) {
@@ -863,8 +1070,10 @@ int psamd_moe_experts_grouped(void* stream, const void* x, const int32_t* chosen
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t pairs = tokens * top;
   const int buckets = experts + (identity > 0 ? 1 : 0);      // all identity pairs lie in one, behind the experts'
-  const int rows = psamd_moe_grouped_tile_rows(pairs, buckets);
-  const int max_tiles = psamd_moe_grouped_max_tiles(pairs, buckets);
+  // Pairs that the router's kernel has sorted lie in the tiles of a small step.
+  const int wide = grouped_already == 0 && tiles_take(tokens, pairs, K, F) ? wide_tile_rows(pairs, buckets) : 0;
+  const int rows = wide != 0 ? wide : psamd_moe_grouped_tile_rows(pairs, buckets);
+  const int max_tiles = static_cast<int>(std::min<int64_t>(ceil_div(pairs, rows) + buckets, pairs));
   PSAMD_REQUIRE(max_tiles <= 65535, "too many tiles for one launch");
   if (grouped_already == 0) {
     moe_group_kernel<<<dim3(1), dim3(1024), sizeof(int32_t) * (4 * buckets + 1), s>>>(
@@ -874,6 +1083,8 @@ int psamd_moe_experts_grouped(void* stream, const void* x, const int32_t* chosen
   }
   const ExpertCall c{x, chosen, weight, w_in, w_down, act, out, tokens, K, F, experts, top, kind,
                      gate_alpha, limit, up_shift, weight_on_output, into_stream, col_scale};
+  if (wide == 256) return launch_tiles<256, 256, 2, 4>(s, c, ints, max_tiles);
+  if (wide == 128) return launch_tiles<128, 128, 2, 2>(s, c, ints, max_tiles);
   if (rows == 128) return launch_grouped<8, 2>(s, c, ints, max_tiles);
   if (rows == 64) return launch_grouped<4, 2>(s, c, ints, max_tiles);
   return launch_grouped<1, 1>(s, c, ints, max_tiles);

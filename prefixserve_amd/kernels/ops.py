@@ -851,7 +851,7 @@ class HipOps:
 
     def _group_ints(self, t: int, top: int, e: int) -> torch.Tensor:
         tiles = int(self.lib.psamd_moe_grouped_max_tiles(t * top, e))
-        return self.ws.get("moe.group", (t * top + 3 * tiles,), torch.int32)
+        return self.ws.get("moe.group", (t * top + 3 * tiles + 1,), torch.int32)
 
     def moe_experts(self, x, chosen, weight, w_in, w_down, act, out, gate_alpha: float, limit: float,
                     up_shift: float, weight_on_output: bool = False, kind: str = "gated", residual=None, col_scale=None,

@@ -1111,3 +1111,43 @@ def test_kernels_refuse_what_they_do_not_take(ops):
     x = rnd(2, 8).to(torch.float16)
     with pytest.raises(KernelError):
         ops.swiglu(x, torch.empty(2, 4, dtype=torch.float16, device=DEV))
+
+
+@pytest.mark.parametrize("counts,k,f", [
+    ((0, 127, 128, 129, 255, 256, 257, 512, 1900, 1500), 192, 320),  # tiles of 256 pairs: empty experts, edges, halves without pairs
+    ((1700, 0, 3, 511), 64, 64),                                    # one step of k, fewer columns than a tile
+    ((0, 1, 63, 64, 65, 127, 128, 129, 10), 128, 192),              # tiles of 128 pairs
+    ((200, 130, 97, 0, 90), 320, 128),
+])
+@pytest.mark.parametrize("kind,on_output,identity", [("gated", False, 0), ("gated", True, 2), ("squared_relu", True, 0)])
+def test_experts_with_many_pairs_each(ops, counts, k, f, kind, on_output, identity):
+    """Experts whose pairs fill, just miss or just pass the tiles of the kernels for many pairs, in random order of the
+    tokens, against float64 with the activations rounded to bfloat16 where the engine holds them: what is left is the
+    product's rounding of its inputs' sums (2^-9 of the activation, at random over f of them)."""
+    gen = torch.Generator().manual_seed(sum(counts) + k)
+    e = len(counts)
+    choice = torch.cat([torch.full((c,), i) for i, c in enumerate(counts)] + [torch.full((40,), e + i) for i in range(identity)])
+    t = len(choice)
+    chosen = choice[torch.randperm(t, generator=gen)].to(torch.int32).view(t, 1).to(DEV)
+    weight = (0.4 + 0.6 * torch.rand(t, 1, generator=gen)).to(DEV)
+    x = rnd(t, k, dtype=torch.bfloat16, seed=1)
+    w_in = rnd(e, (2 if kind == "gated" else 1) * f, k, dtype=torch.bfloat16, seed=2, scale=0.15)
+    down = rnd(e, k, f, dtype=torch.bfloat16, seed=3, scale=0.15)
+    want = torch.empty(t, k, dtype=torch.float64, device=DEV)
+    for i in range(e + identity):
+        rows = (chosen[:, 0] == i).nonzero()[:, 0]
+        h, w = x[rows].double(), weight[rows].double()
+        if i >= e:
+            want[rows] = w * h
+            continue
+        z = (h if on_output else w * h) @ w_in[i].double().T
+        if kind == "gated":
+            g, u = z[:, :f].clamp(max=5.0), z[:, f:].clamp(-5.0, 5.0)
+            a = g * torch.sigmoid(1.702 * g) * (u + 1.0)
+        else:
+            a = torch.relu(z).square()
+        want[rows] = (w if on_output else 1.0) * (a.to(torch.bfloat16).double() @ down[i].double().T)
+    act = torch.empty(t, f, dtype=torch.bfloat16, device=DEV)
+    out = torch.full((1, t + 1, k), 7.0, device=DEV)
+    ops.moe_experts(x, chosen, weight, w_in, down, act, out[:, :t], 1.702, 5.0, 1.0, weight_on_output=on_output, kind=kind, identity=identity)
+    assert rel(out[0, :t], want) < 3e-3 and torch.all(out[0, t] == 7.0)
