@@ -295,7 +295,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(
     const float* __restrict__ rvec, int64_t key_row, int heads_per_group, const float* __restrict__ dvec, int64_t dvec_row,
     const float* __restrict__ dscal, const float* __restrict__ pscal, const float* __restrict__ xscal, int64_t scal_row,
     const float* __restrict__ x, int64_t x_row, float* __restrict__ out, int64_t out_row, float* __restrict__ state,
-    int64_t state_row, const int32_t* __restrict__ item_start, const int32_t* __restrict__ slots, int dim, int vdim) {
+    int64_t state_row, const int32_t* __restrict__ item_start, const int32_t* __restrict__ slots, int dim, int vdim, int most) {
   constexpr int DP = E * kLPC;                          // the column's length, padded
   constexpr int TT = kScanRun<E>;                       // tokens per run
   constexpr int VPT = TT * DP / 256;                    // vector entries a thread carries per run
@@ -308,6 +308,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(
   const int col = threadIdx.x / kLPC, l = threadIdx.x % kLPC;
   const int j0 = blockIdx.z * kCols, j = j0 + col;
   const int64_t s0 = item_start[item], s1 = item_start[item + 1];
+  if (most > 0 && s1 - s0 > most) return;                // uniform for the workgroup; another kernel walks this item
   float* st = state + static_cast<int64_t>(slots[item]) * state_row + (static_cast<int64_t>(h) * vdim + j) * dim + l * E;
   float s[E];
 #pragma unroll
@@ -430,10 +431,10 @@ static int launch_delta_scan(hipStream_t s, dim3 grid, const float* kvec, const 
                              const float* rvec, int64_t key_row, int heads_per_group, const float* dvec, int64_t dvec_row,
                              const float* dscal, const float* pscal, const float* xscal, int64_t scal_row, const float* x,
                              int64_t x_row, float* out, int64_t out_row, float* state, int64_t state_row,
-                             const int32_t* item_start, const int32_t* slots, int dim, int vdim) {
+                             const int32_t* item_start, const int32_t* slots, int dim, int vdim, int most) {
   delta_scan_kernel<E, SAME, RD, NR><<<grid, dim3(256), 0, s>>>(kvec, cvec, pvec, rvec, key_row, heads_per_group, dvec, dvec_row,
                                                            dscal, pscal, xscal, scal_row, x, x_row, out, out_row, state,
-                                                           state_row, item_start, slots, dim, vdim);
+                                                           state_row, item_start, slots, dim, vdim, most);
   return check_launch("psamd_delta_scan");
 }
 
@@ -517,7 +518,7 @@ int psamd_delta_scan(void* stream, const float* kvec, const float* cvec, const f
                      int key_groups, const float* dvec, int64_t dvec_row, const float* dscal, const float* pscal,
                      const float* xscal, int64_t scal_row, const float* x, int64_t x_row, float* out, int64_t out_row,
                      float* state, int64_t state_row, const int32_t* item_start, const int32_t* slots, int items, int heads,
-                     int dim, int vdim, int reads_decayed) {
+                     int dim, int vdim, int reads_decayed, int most) {
   PSAMD_REQUIRE(items >= 0 && heads > 0 && key_groups > 0 && heads % key_groups == 0 && dim > 0 && vdim > 0, "bad sizes");
   PSAMD_REQUIRE(dim <= 16 * kLPC, "key size at most 256");
   PSAMD_REQUIRE(state_row >= static_cast<int64_t>(heads) * dim * vdim, "state rows too short");
@@ -535,7 +536,7 @@ int psamd_delta_scan(void* stream, const float* kvec, const float* cvec, const f
   PSAMD_REQUIRE(reads_decayed != 2 || same, "a recurrence without removal comes in the gated rule's form");
 #define PSAMD_SCAN_ARGS                                                                                                   \
   s, grid, kvec, cvec, pvec, rvec, key_row, hpg, dvec, dvec_row, dscal, pscal, xscal, scal_row, x, x_row, out, out_row, state, \
-      state_row, item_start, slots, dim, vdim
+      state_row, item_start, slots, dim, vdim, most
 #define PSAMD_SCAN(E)                                                                                   \
   return same ? (reads_decayed == 2 ? launch_delta_scan<E, true, true, true>(PSAMD_SCAN_ARGS)           \
                                     : launch_delta_scan<E, true, true>(PSAMD_SCAN_ARGS))                \

@@ -1,0 +1,557 @@
+// The recurrences of delta.hip over prompts, run by run on the matrix cores (float32: v_mfma_f32_16x16x4_f32).
+//
+// Token by token (delta_scan_kernel) a head's 2,048 tokens are 2,048 sums that wait for each other, 0.19 us each, on half
+// the compute units: 385 us for 16 heads of 128 x 128, 394 for 32 of 64 x 64. In a run of kRunTokens tokens the state S0 in
+// front of the run enters linearly. With D_t the product of the decays up to token t of the run (a number per head, or a
+// vector over the key channels), in the gated form (p = ps k, c = k, both with the decayed state)
+//     w_t = ps_t k_t^T (D_t S0) + sum_{s<t} L_ts w_s + xs_t x_t,     L_ts = ps_t (D_t / D_s) (k_t . k_s)
+//     o_t = (D_t q_t)^T S0 + sum_{s<=t} (D_t / D_s) (q_t . k_s) w_s
+//     S   = D_n S0 + sum_s (D_n / D_s) k_s w_s^T
+// so with T = (1 - L)^-1 (unit lower triangular) the run is W = Wx + Kt S0 with Wx = T diag(xs) X and Kt = T diag(ps D) K,
+// known without S0. The general form (a decay per channel, the removal reads the state before the decay) has the same shape with
+//     L_ts = (c_t D_{t-1}) . (p_s / D_s), W = U (what is taken out), Wx = T (M X), M_ts = (c_t D_{t-1}) . (k_s / D_s),
+//     Kt = T (c D_{-1}), and what the values alone leave in the output (Y) and the state (Z).
+// Three launches: runs_prepare (all runs side by side: everything that does not need S0), runs_chain (an item's runs in turn:
+// two small products each), runs_output (all runs side by side). 2,048 tokens as above: 66 + 94 + 30 us (gated), 126 + 59 + 25
+// (general). The chain is what bounds a long prompt: 64 matrix instructions and two barriers a run, 2.9 us of 32 runs in turn.
+//
+// Numerics: everything is float32. T is built by substitution, 16 x 16 on the diagonal and block by block below it (a product
+// of powers of L is shorter and loses everything where keys repeat). The gated form's ratios D_t / D_s are products of the
+// decays between the two tokens, so a decay may be 0; the general form divides by D_s and is only taken where the decays'
+// floor keeps D_s far from underflow.
+//
+// Operand layout of a 16 x 16 x 4 instruction: lane (r = l % 16, g = l / 16) gives k = 4 g + i, i = 0..3, of row r and of column
+// r, and receives rows 4 g .. 4 g + 3 of column r: what it receives is the column operand of a product over those rows.
+
+#include "api.h"
+#include "common.h"
+
+namespace psamd {
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+constexpr int kRunTokens = 64, kRunTiles = kRunTokens / 16;
+constexpr int kLd = kRunTokens + 4;                      // LDS row stride of [.][run] arrays, in floats
+
+struct DeltaRuns {
+  const float* kvec;
+  const float* cvec;
+  const float* pvec;
+  const float* rvec;
+  int64_t key_row;
+  int heads_per_group;
+  const float* dvec;
+  int64_t dvec_row;
+  const float* dscal;
+  const float* pscal;
+  const float* xscal;
+  int64_t scal_row;
+  const float* x;
+  int64_t x_row;
+  float* out;
+  int64_t out_row;
+  float* state;
+  int64_t state_row;
+  const int32_t* item_start;
+  const int32_t* slots;
+  const int32_t* pf_tiles;     // (item, first token within the item) of the step's tiles of 32
+  const int32_t* pf_blocks;    // the first tile of each four of one item
+  int n_blocks, heads, vdim;
+  float* scratch;              // [2 n_blocks][heads][run_floats]
+};
+
+// Where a run's arrays lie in its scratch.
+struct RunLayout {
+  int kt, kd, qd, w, p, s0, z, dc, total;
+};
+__host__ __device__ constexpr RunLayout run_layout(int dim, int vdim, bool general) {
+  RunLayout l{};
+  int at = 0;
+  l.kt = at, at += kRunTokens * dim;                     // [t][dim]
+  l.kd = at, at += kRunTokens * dim;                     // [dim][t]
+  l.qd = at, at += kRunTokens * dim;                     // [t][dim]
+  l.w = at, at += kRunTokens * vdim;                     // [vdim][t]: Wx, then W
+  l.p = at, at += kRunTokens * kRunTokens;               // [t][s]
+  l.s0 = at, at += dim * vdim;                           // [vdim][dim]
+  l.z = at, at += general ? dim * vdim : 0;              // [vdim][dim]
+  l.dc = at, at += dim;
+  l.total = at;
+  return l;
+}
+
+// acc + 16 products. The products are summed on their own first: chains of 64 left the outputs 1.7 times as far from 64 bits
+// as the token-by-token walk, whose sums over the key channels are sums of 8 added in a tree.
+__device__ __forceinline__ f32x4 mma(f32x4 a, f32x4 b, f32x4 acc) {
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], sum, 0, 0, 0);
+  return acc + sum;
+}
+
+// A barrier for what passes through LDS alone: loads from memory stay under way across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+constexpr int kGatedForm = 0, kPlainForm = 1, kGeneralForm = 2;   // plain: the gated form with nothing taken out
+
+// Run `blockIdx.x`'s item, first token and length (0: the block has no such run).
+__device__ __forceinline__ int run_of(const DeltaRuns& c, int64_t& t0) {
+  const int tile = c.pf_blocks[blockIdx.x >> 1], item = c.pf_tiles[2 * tile];
+  const int q0 = c.pf_tiles[2 * tile + 1] + (blockIdx.x & 1) * kRunTokens;
+  t0 = c.item_start[item] + static_cast<int64_t>(q0);
+  return min(kRunTokens, c.item_start[item + 1] - c.item_start[item] - q0);
+}
+
+// grid (2 blocks, heads), four waves: wave w makes the rows of tokens 16 w .. 16 w + 15.
+template <int DT, int FORM>
+__global__ __launch_bounds__(256) void runs_prepare_kernel(DeltaRuns c) {
+  constexpr int D = DT * 16, LD = D + 4;
+  constexpr bool GENERAL = FORM == kGeneralForm, SOLVES = FORM != kPlainForm;
+  extern __shared__ __align__(16) float run_smem[];
+  float* tm = run_smem;                                  // [t][s]: the ratios D_t / D_s, later T
+  float* lm = tm + kRunTokens * kLd;                     // [t][s]: L
+  float* ds = lm + kRunTokens * kLd;                     // general: D [t][dim]
+  float* mx = ds + (GENERAL ? kRunTokens * LD : 0);      // general: M X, [vdim][t]
+  __shared__ float num[5][kRunTokens];                   // per token: decay, D_t, D_n / D_t, ps, xs
+  int64_t t0;
+  const int n = run_of(c, t0);
+  if (n <= 0) return;                                    // uniform for the workgroup
+  const int h = blockIdx.y, grp = h / c.heads_per_group;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const RunLayout lay = run_layout(D, c.vdim, GENERAL);
+  float* sc = c.scratch + (static_cast<int64_t>(blockIdx.x) * c.heads + h) * lay.total;
+  const int64_t key0 = t0 * c.key_row + static_cast<int64_t>(grp) * D;
+  const int64_t x0 = t0 * c.x_row + static_cast<int64_t>(h) * c.vdim;
+
+  if (threadIdx.x < kRunTokens) {
+    const int t = threadIdx.x;
+    const int64_t at = (t0 + t) * c.scal_row + h;
+    num[0][t] = !GENERAL && t < n && c.dscal != nullptr ? c.dscal[at] : 1.f;
+    num[3][t] = t >= n ? 0.f : c.pscal != nullptr ? c.pscal[at] : 1.f;
+    num[4][t] = t >= n ? 0.f : c.xscal != nullptr ? c.xscal[at] : 1.f;
+  }
+  if constexpr (GENERAL) {
+    for (int idx = threadIdx.x; idx < kRunTokens * D; idx += 256) {
+      const int t = idx / D, i = idx % D;
+      ds[t * LD + i] = t < n ? c.dvec[(t0 + t) * c.dvec_row + static_cast<int64_t>(h) * D + i] : 1.f;
+    }
+    __syncthreads();
+    if (threadIdx.x < D) {
+      float d = 1.f;
+#pragma unroll 8
+      for (int t = 0; t < kRunTokens; ++t) {
+        d *= ds[t * LD + threadIdx.x];
+        ds[t * LD + threadIdx.x] = d;
+      }
+    }
+  }
+  __syncthreads();
+  if constexpr (!GENERAL) {
+    if (threadIdx.x < kRunTokens) {
+      const int s = threadIdx.x;
+      float ratio = 1.f;
+      for (int t = s; t < kRunTokens; ++t) {
+        if (t > s) ratio *= num[0][t];
+        tm[t * kLd + s] = ratio;
+      }
+      num[2][s] = ratio;
+    }
+    __syncthreads();
+    if (threadIdx.x < kRunTokens) num[1][threadIdx.x] = tm[threadIdx.x * kLd] * num[0][0];
+    __syncthreads();
+  }
+
+  // The run's products over the key channels, a lane's rows and columns read 16 bytes at a time.
+  const int t = 16 * wave + r;
+  const bool has = t < n;
+  auto row4 = [&](const float* v, int tok, int d) {      // dimensions 16 d + 4 g .. of a token's vector, zeros behind the run
+    return tok < n ? *reinterpret_cast<const f32x4*>(v + key0 + tok * c.key_row + 16 * d + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  f32x4 ct[DT], qt[DT];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) {
+    ct[d] = row4(GENERAL ? c.cvec : c.kvec, t, d);
+    qt[d] = row4(c.rvec, t, d);
+    if constexpr (GENERAL) {
+      if (t > 0) ct[d] *= *reinterpret_cast<const f32x4*>(ds + (t - 1) * LD + 16 * d + 4 * g);
+      qt[d] *= *reinterpret_cast<const f32x4*>(ds + t * LD + 16 * d + 4 * g);
+    }
+    *reinterpret_cast<f32x4*>(sc + lay.qd + t * D + 16 * d + 4 * g) = GENERAL ? qt[d] : qt[d] * num[1][t];
+  }
+  f32x4 m_reg[kRunTiles], pk_reg[kRunTiles];             // general: M and (D_t r_t) . (k_s / D_s), rows s, column t
+#pragma unroll
+  for (int st = 0; st < kRunTiles; ++st) {
+    m_reg[st] = pk_reg[st] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (st > wave) continue;
+    const int sr = 16 * st + r;                          // the row this lane supplies
+    f32x4 cc = {0.f, 0.f, 0.f, 0.f}, qc = cc, ck = cc, qk = cc;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      f32x4 first = row4(GENERAL ? c.pvec : c.kvec, sr, d);
+      if constexpr (GENERAL) {
+        const f32x4 dd = *reinterpret_cast<const f32x4*>(ds + sr * LD + 16 * d + 4 * g);
+        f32x4 second = row4(c.kvec, sr, d);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          first[i] /= dd[i];
+          second[i] /= dd[i];
+        }
+        ck = mma(second, ct[d], ck);
+        qk = mma(second, qt[d], qk);
+      }
+      if constexpr (SOLVES) cc = mma(first, ct[d], cc);
+      qc = mma(first, qt[d], qc);
+    }
+    f32x4 l, p;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int s = 16 * st + 4 * g + v;
+      const float ratio = GENERAL ? 1.f : (s <= t ? tm[t * kLd + s] : 0.f);
+      l[v] = s < t ? (GENERAL ? cc[v] : num[3][t] * (ratio * cc[v])) : 0.f;
+      p[v] = s <= t ? (GENERAL ? qc[v] : ratio * qc[v]) : 0.f;
+      if constexpr (GENERAL) {
+        m_reg[st][v] = s < t ? ck[v] : 0.f;
+        pk_reg[st][v] = s <= t ? qk[v] : 0.f;
+      }
+    }
+    if constexpr (SOLVES) *reinterpret_cast<f32x4*>(lm + t * kLd + 16 * st + 4 * g) = l;
+    *reinterpret_cast<f32x4*>(sc + lay.p + t * kRunTokens + 16 * st + 4 * g) = p;
+  }
+  // A lane's four tokens s of column j of the values (k = 4 g + i of the operand of either kind).
+  auto x4 = [&](int st, int j) {
+    f32x4 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int s = 16 * st + 4 * g + i;
+      v[i] = s < n ? c.x[x0 + s * c.x_row + j] : 0.f;
+    }
+    return v;
+  };
+  if constexpr (GENERAL) {
+    for (int j0 = 0; j0 < c.vdim; j0 += 16) {
+      f32x4 y = {0.f, 0.f, 0.f, 0.f}, m = y;
+#pragma unroll
+      for (int st = 0; st < kRunTiles; ++st) {
+        if (st > wave) continue;
+        const f32x4 xv = x4(st, j0 + r);
+        y = mma(xv, pk_reg[st], y);
+        m = mma(xv, m_reg[st], m);
+      }
+      if (has) *reinterpret_cast<f32x4*>(c.out + (t0 + t) * c.out_row + static_cast<int64_t>(h) * c.vdim + j0 + 4 * g) = y;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) mx[(j0 + 4 * g + v) * kLd + t] = m[v];
+    }
+  }
+  __syncthreads();                                       // L is whole, the ratios have been read
+  if constexpr (SOLVES) {
+    // T = (1 - L)^-1: the blocks on the diagonal by substitution, a column per lane, ...
+    float col[16];
+    const float* lb = lm + 16 * wave * kLd + 16 * wave;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float v = i == r ? 1.f : 0.f;
+#pragma unroll
+      for (int s = 0; s < i; ++s) v = fmaf(lb[i * kLd + s], col[s], v);
+      col[i] = v;
+    }
+    if (g == 0) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) tm[(16 * wave + i) * kLd + 16 * wave + r] = col[i];
+    }
+    __syncthreads();
+    // ... and T_ij = T_ii sum_k L_ik T_kj below it, by distance from the diagonal.
+#pragma unroll
+    for (int off = 1; off < kRunTiles; ++off) {
+      if (wave >= off) {
+        const int bj = wave - off;
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+        for (int bk = bj; bk < wave; ++bk) {
+          f32x4 b;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) b[i] = tm[(16 * bk + 4 * g + i) * kLd + 16 * bj + r];
+          sum = mma(*reinterpret_cast<const f32x4*>(lm + (16 * wave + r) * kLd + 16 * bk + 4 * g), b, sum);
+        }
+        const f32x4 res = mma(*reinterpret_cast<const f32x4*>(tm + (16 * wave + r) * kLd + 16 * wave + 4 * g), sum, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int v = 0; v < 4; ++v) tm[(16 * wave + 4 * g + v) * kLd + 16 * bj + r] = res[v];
+      }
+      __syncthreads();
+    }
+  }
+  f32x4 tr[kRunTiles];                                   // row t of T
+#pragma unroll
+  for (int st = 0; st < kRunTiles; ++st)
+    tr[st] = SOLVES && st <= wave ? *reinterpret_cast<const f32x4*>(tm + t * kLd + 16 * st + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int j0 = 0; j0 < c.vdim; j0 += 16) {              // Wx, rows t, column j
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int st = 0; st < kRunTiles; ++st) {
+      if (SOLVES ? st > wave : st != wave) continue;
+      f32x4 b;
+      if constexpr (GENERAL) {
+        b = *reinterpret_cast<const f32x4*>(mx + (j0 + r) * kLd + 16 * st + 4 * g);
+      } else {
+        b = x4(st, j0 + r);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) b[i] *= num[4][16 * st + 4 * g + i];
+      }
+      acc = SOLVES ? mma(tr[st], b, acc) : b;
+    }
+    *reinterpret_cast<f32x4*>(sc + lay.w + (j0 + r) * kRunTokens + 16 * wave + 4 * g) = acc;
+  }
+  for (int i0 = 0; i0 < D; i0 += 16) {                   // Kt, rows i, column t; Kd of this wave's tokens
+    const int i = i0 + r;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int st = 0; st < kRunTiles; ++st) {
+      if (st > wave) continue;
+      f32x4 a, kd;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int s = 16 * st + 4 * g + v;
+        const float k = s < n ? (GENERAL ? c.cvec : c.kvec)[key0 + s * c.key_row + i] : 0.f;
+        a[v] = GENERAL ? (s > 0 ? k * ds[(s - 1) * LD + i] : k) : num[3][s] * num[1][s] * k;
+        if (st == wave) {
+          if constexpr (GENERAL) kd[v] = s < n ? c.pvec[key0 + s * c.key_row + i] * (ds[(kRunTokens - 1) * LD + i] / ds[s * LD + i]) : 0.f;
+          else kd[v] = num[2][s] * k;
+        }
+      }
+      if constexpr (SOLVES) acc = mma(a, tr[st], acc);
+      if (st == wave) *reinterpret_cast<f32x4*>(sc + lay.kd + i * kRunTokens + 16 * st + 4 * g) = kd;
+    }
+    if constexpr (SOLVES) *reinterpret_cast<f32x4*>(sc + lay.kt + t * D + i0 + 4 * g) = acc;
+  }
+  if constexpr (GENERAL) {
+    for (int it = wave; it < DT; it += 4) {              // Z, rows i, column j
+      f32x4 kk[kRunTiles];
+      const int i = 16 * it + r;
+#pragma unroll
+      for (int st = 0; st < kRunTiles; ++st)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int s = 16 * st + 4 * g + v;
+          kk[st][v] = s < n ? c.kvec[key0 + s * c.key_row + i] * (ds[(kRunTokens - 1) * LD + i] / ds[s * LD + i]) : 0.f;
+        }
+      for (int j0 = 0; j0 < c.vdim; j0 += 16) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int st = 0; st < kRunTiles; ++st) acc = mma(kk[st], x4(st, j0 + r), acc);
+        *reinterpret_cast<f32x4*>(sc + lay.z + (j0 + r) * D + 16 * it + 4 * g) = acc;
+      }
+    }
+  }
+  for (int i = threadIdx.x; i < D; i += 256) sc[lay.dc + i] = GENERAL ? ds[(kRunTokens - 1) * LD + i] : num[1][kRunTokens - 1];
+}
+
+// grid (items, heads, vdim / 16), four waves: an item's runs in turn for 16 value channels. Wave w makes the rows of tokens
+// 16 w .. of W and keeps the state's key channels 16 (w + 4 o) .. in registers.
+template <int DT, int FORM>
+__global__ __launch_bounds__(256, 1) void runs_chain_kernel(DeltaRuns c) {
+  constexpr int D = DT * 16, LD = D + 4, OWN = (DT + 3) / 4;
+  constexpr bool GENERAL = FORM == kGeneralForm, SOLVES = FORM != kPlainForm;
+  __shared__ __align__(16) float st_s[16 * LD];          // the state, [value channel][key channel]
+  __shared__ f32x4 w_s[kRunTiles][64];
+  __shared__ int first_s;
+  const int item = blockIdx.x, h = blockIdx.y, j0 = blockIdx.z * 16;
+  const int n = c.item_start[item + 1] - c.item_start[item];
+  if (n < 2) return;                                     // single tokens are not in the list of tiles
+  if (threadIdx.x == 0) first_s = c.n_blocks;
+  __syncthreads();
+  for (int b = threadIdx.x; b < c.n_blocks; b += 256)
+    if (c.pf_tiles[2 * c.pf_blocks[b]] == item) atomicMin(&first_s, b);
+  __syncthreads();
+  const int first = first_s, runs = (n + kRunTokens - 1) / kRunTokens;
+  if (first >= c.n_blocks) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const RunLayout lay = run_layout(D, c.vdim, GENERAL);
+  const int64_t run_stride = static_cast<int64_t>(c.heads) * lay.total;
+  float* sc = c.scratch + (static_cast<int64_t>(2 * first) * c.heads + h) * lay.total;
+  float* st = c.state + static_cast<int64_t>(c.slots[item]) * c.state_row + (static_cast<int64_t>(h) * c.vdim + j0 + r) * D + 4 * g;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 s[OWN];
+#pragma unroll
+  for (int o = 0; o < OWN; ++o) {
+    const int it = wave + 4 * o;
+    s[o] = it < DT ? *reinterpret_cast<const f32x4*>(st + 16 * it) : zero;
+  }
+  // What a run needs from memory. Two runs' operands are held: a run's are asked for as soon as those of the run two in
+  // front of it have been used, more than a run's time ahead.
+  struct Operands {
+    f32x4 kt[DT], wx, kd[OWN][kRunTiles], dc[OWN], z[OWN];
+  };
+  Operands even, odd;
+  auto ask_front = [&](Operands& a, int run) {           // what the first product takes
+    const float* q = sc + min(run, runs - 1) * run_stride;             // no branch: what is asked for behind the last is not used
+    if constexpr (SOLVES) {
+#pragma unroll
+      for (int d = 0; d < DT; ++d) a.kt[d] = *reinterpret_cast<const f32x4*>(q + lay.kt + (16 * wave + r) * D + 16 * d + 4 * g);
+    }
+    a.wx = *reinterpret_cast<const f32x4*>(q + lay.w + (j0 + r) * kRunTokens + 16 * wave + 4 * g);
+  };
+  auto ask_back = [&](Operands& a, int run) {            // what the second takes
+    const float* q = sc + min(run, runs - 1) * run_stride;
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) {
+      const int it = min(wave + 4 * o, DT - 1);
+#pragma unroll
+      for (int t = 0; t < kRunTiles; ++t) a.kd[o][t] = *reinterpret_cast<const f32x4*>(q + lay.kd + (16 * it + r) * kRunTokens + 16 * t + 4 * g);
+      a.dc[o] = *reinterpret_cast<const f32x4*>(q + lay.dc + 16 * it + 4 * g);
+      if constexpr (GENERAL) a.z[o] = *reinterpret_cast<const f32x4*>(q + lay.z + (j0 + r) * D + 16 * it + 4 * g);
+    }
+  };
+  auto walk = [&](Operands& a, int run) {
+    float* q = sc + run * run_stride;
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) {
+      const int it = wave + 4 * o;
+      if (it >= DT) break;
+      *reinterpret_cast<f32x4*>(q + lay.s0 + (j0 + r) * D + 16 * it + 4 * g) = s[o];
+      if constexpr (SOLVES) *reinterpret_cast<f32x4*>(st_s + r * LD + 16 * it + 4 * g) = s[o];
+    }
+    lds_barrier();                                       // the state is whole; the run before's W has been read
+    f32x4 w = a.wx;
+    if constexpr (SOLVES) {
+      f32x4 from_state = zero;
+#pragma unroll
+      for (int d = 0; d < DT; ++d) from_state = mma(a.kt[d], *reinterpret_cast<const f32x4*>(st_s + r * LD + 16 * d + 4 * g), from_state);
+      w += from_state;
+      *reinterpret_cast<f32x4*>(q + lay.w + (j0 + r) * kRunTokens + 16 * wave + 4 * g) = w;
+    }
+    w_s[wave][lane] = w;
+    ask_front(a, run + 2);
+    lds_barrier();
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) {
+      f32x4 sum = zero;
+#pragma unroll
+      for (int t = 0; t < kRunTiles; ++t) sum = mma(a.kd[o][t], w_s[t][lane], sum);
+      if constexpr (GENERAL) sum += a.z[o];
+      s[o] = s[o] * a.dc[o] + sum;
+    }
+    ask_back(a, run + 2);
+  };
+  ask_front(even, 0);
+  ask_back(even, 0);
+  ask_front(odd, 1);
+  ask_back(odd, 1);
+  for (int run = 0; run < runs; run += 2) {
+    walk(even, run);
+    if (run + 1 < runs) walk(odd, run + 1);
+  }
+#pragma unroll
+  for (int o = 0; o < OWN; ++o) {
+    const int it = wave + 4 * o;
+    if (it < DT) *reinterpret_cast<f32x4*>(st + 16 * it) = s[o];
+  }
+}
+
+// grid (2 blocks, heads), four waves: out = Qd S0 + P W (+ Y), rows of values, column t.
+template <int DT, int FORM>
+__global__ __launch_bounds__(256) void runs_output_kernel(DeltaRuns c) {
+  constexpr int D = DT * 16;
+  constexpr bool GENERAL = FORM == kGeneralForm;
+  int64_t t0;
+  const int n = run_of(c, t0);
+  const int h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4, t = 16 * wave + r;
+  if (16 * wave >= n) return;                            // no barrier below
+  const RunLayout lay = run_layout(D, c.vdim, GENERAL);
+  const float* sc = c.scratch + (static_cast<int64_t>(blockIdx.x) * c.heads + h) * lay.total;
+  f32x4 q[DT], p[kRunTiles];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) q[d] = *reinterpret_cast<const f32x4*>(sc + lay.qd + t * D + 16 * d + 4 * g);
+#pragma unroll
+  for (int st = 0; st < kRunTiles; ++st)
+    p[st] = st <= wave ? *reinterpret_cast<const f32x4*>(sc + lay.p + t * kRunTokens + 16 * st + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
+  float* o = c.out + (t0 + t) * c.out_row + static_cast<int64_t>(h) * c.vdim + 4 * g;
+  for (int j0 = 0; j0 < c.vdim; j0 += 16) {
+    f32x4 a[DT], w[kRunTiles];
+#pragma unroll
+    for (int d = 0; d < DT; ++d) a[d] = *reinterpret_cast<const f32x4*>(sc + lay.s0 + (j0 + r) * D + 16 * d + 4 * g);
+#pragma unroll
+    for (int st = 0; st < kRunTiles; ++st)
+      if (st <= wave) w[st] = *reinterpret_cast<const f32x4*>(sc + lay.w + (j0 + r) * kRunTokens + 16 * st + 4 * g);
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    if (GENERAL && t < n) sum = *reinterpret_cast<const f32x4*>(o + j0);
+#pragma unroll
+    for (int d = 0; d < DT; ++d) sum = mma(a[d], q[d], sum);
+#pragma unroll
+    for (int st = 0; st < kRunTiles; ++st)
+      if (st <= wave) sum = mma(w[st], p[st], sum);
+    if (t < n) *reinterpret_cast<f32x4*>(o + j0) = sum;
+  }
+}
+
+template <int DT, int FORM>
+static int launch_runs(hipStream_t s, const DeltaRuns& c, int items) {
+  constexpr int D = DT * 16;
+  constexpr bool GENERAL = FORM == kGeneralForm;
+  const dim3 all(static_cast<unsigned>(2 * c.n_blocks), static_cast<unsigned>(c.heads));
+  const size_t smem = sizeof(float) * (2 * kRunTokens * kLd + (GENERAL ? kRunTokens * (D + 4) + c.vdim * kLd : 0));
+  auto prepare = runs_prepare_kernel<DT, FORM>;
+  if (smem > 60 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(prepare), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              static_cast<int>(smem)) != hipSuccess)
+    return fail("psamd_delta_runs: " + std::to_string(smem) + " bytes of LDS were refused");
+  prepare<<<all, dim3(256), smem, s>>>(c);
+  if (check_launch("psamd_delta_runs (prepare)")) return 1;
+  runs_chain_kernel<DT, FORM><<<dim3(static_cast<unsigned>(items), static_cast<unsigned>(c.heads), static_cast<unsigned>(c.vdim / 16)),
+                                dim3(256), 0, s>>>(c);
+  if (check_launch("psamd_delta_runs (chain)")) return 1;
+  runs_output_kernel<DT, FORM><<<all, dim3(256), 0, s>>>(c);
+  return check_launch("psamd_delta_runs (output)");
+}
+
+}  // namespace psamd
+
+using namespace psamd;
+
+extern "C" {
+
+// Whether psamd_delta_runs takes a recurrence of this shape: 1, or 0. general: a decay per key channel, of which decay_least
+// is the least a token can have (the run's decays are divided by).
+int psamd_delta_runs_supports(int dim, int vdim, int64_t key_row, int64_t x_row, int64_t out_row, int64_t dvec_row, int64_t state_row,
+                              int general, float decay_least) {
+  if ((dim != 64 && dim != 128) || vdim % 16 != 0 || vdim < 16 || vdim > 256) return 0;
+  if (key_row % 4 != 0 || out_row % 4 != 0 || x_row < 1 || dvec_row < 0 || state_row % 4 != 0) return 0;
+  // e^-40: D_s and its reciprocal, times operands of any ordinary size, stay far inside float32.
+  if (general && !(decay_least > 0.f && kRunTokens * -logf(decay_least) <= 40.f)) return 0;
+  return 1;
+}
+
+// Scratch floats for a step of n_blocks blocks of 128 tokens.
+int64_t psamd_delta_runs_floats(int n_blocks, int heads, int dim, int vdim, int general) {
+  return static_cast<int64_t>(2) * n_blocks * heads * run_layout(dim, vdim, general != 0).total;
+}
+
+int psamd_delta_runs(void* stream, const float* kvec, const float* cvec, const float* pvec, const float* rvec, int64_t key_row,
+                     int key_groups, const float* dvec, int64_t dvec_row, const float* dscal, const float* pscal, const float* xscal,
+                     int64_t scal_row, const float* x, int64_t x_row, float* out, int64_t out_row, float* state, int64_t state_row,
+                     const int32_t* item_start, const int32_t* slots, const int32_t* pf_tiles, const int32_t* pf_blocks, int n_blocks,
+                     int items, int heads, int dim, int vdim, int form, float decay_least, float* scratch) {
+  PSAMD_REQUIRE(form == kGatedForm || form == kPlainForm || form == kGeneralForm, "form: gated, plain or general");
+  PSAMD_REQUIRE(items >= 0 && n_blocks >= 0 && heads > 0 && key_groups > 0 && heads % key_groups == 0, "bad sizes");
+  const bool general = form == kGeneralForm;
+  PSAMD_REQUIRE(psamd_delta_runs_supports(dim, vdim, key_row, x_row, out_row, dvec_row, state_row, general ? 1 : 0, decay_least), "unsupported shape");
+  PSAMD_REQUIRE(general ? (dvec != nullptr && dscal == nullptr && pscal == nullptr && xscal == nullptr && key_groups == heads)
+                        : (cvec == kvec && pvec == kvec && dvec == nullptr), "operands of another form");
+  PSAMD_REQUIRE(kvec && cvec && pvec && rvec && x && out && state && scratch, "missing operands");
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(kvec) | reinterpret_cast<uintptr_t>(cvec) | reinterpret_cast<uintptr_t>(pvec) |
+                         reinterpret_cast<uintptr_t>(rvec) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(state) |
+                         reinterpret_cast<uintptr_t>(scratch);
+  PSAMD_REQUIRE(bits % 16 == 0, "operands must lie on 16 bytes");
+  PSAMD_REQUIRE(state_row >= static_cast<int64_t>(heads) * dim * vdim && heads <= 65535, "state rows too short, or too many heads");
+  if (n_blocks == 0 || items == 0) return 0;
+  const DeltaRuns c{kvec, cvec, pvec, rvec, key_row, heads / key_groups, dvec, dvec_row, dscal, pscal, xscal, scal_row, x, x_row, out,
+                    out_row, state, state_row, item_start, slots, pf_tiles, pf_blocks, n_blocks, heads, vdim, scratch};
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (form == kGatedForm) return dim == 64 ? launch_runs<4, kGatedForm>(s, c, items) : launch_runs<8, kGatedForm>(s, c, items);
+  if (form == kPlainForm) return dim == 64 ? launch_runs<4, kPlainForm>(s, c, items) : launch_runs<8, kPlainForm>(s, c, items);
+  return dim == 64 ? launch_runs<4, kGeneralForm>(s, c, items) : launch_runs<8, kGeneralForm>(s, c, items);
+}
+
+}  // extern "C"

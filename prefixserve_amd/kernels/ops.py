@@ -16,6 +16,7 @@ import logging
 import os
 from typing import Any, Sequence
 
+import numpy as np
 import torch
 
 from prefixserve_amd.build import ensure_kernels
@@ -107,7 +108,10 @@ _SIGNATURES = {
     "psamd_general_delta_prepare": [_vp, _vp, _i32, _i64, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _i32, _i32,
                                     _i32, _f32, _f32],
     "psamd_delta_scan": [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64,
-                         _vp, _vp, _i32, _i32, _i32, _i32, _i32],
+                         _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32],
+    "psamd_delta_runs_supports": [_i32, _i32, _i64, _i64, _i64, _i64, _i64, _i32, _f32],
+    "psamd_delta_runs": [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64,
+                         _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _vp],
     "psamd_heads_norm_gate": [_vp, _vp, _i64, _i32, _i32, _vp, _i32, _f32, _vp, _i32, _i64, _i32, _vp],
     "psamd_short_conv_to": [_vp, _vp, _i32, _i64, _vp, _vp, _vp, _i32, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32],
     "psamd_stream_rms_norm": [_vp, _vp, _vp, _f32, _i64, _i32],
@@ -151,6 +155,8 @@ class HipOps:
     MOE_ROUTE_FUSED_MAX_TOKENS = 0   # up to here one kernel computes router logits and choice; above, product + choice
     MOE_CHOICE_SORTS_MAX_TOKENS = 16 # up to here the workgroup that chooses a step's experts also sorts the pairs
     MOE_PAIRWISE_MAX_TOKENS = 2     # up to here a bfloat16 step's experts run pair by pair; above, grouped by expert
+    DELTA_RUNS_MIN_TOKENS = 48      # from this prompt length on a recurrence runs in runs of 64 tokens (where the caller allows it)
+    DELTA_RUNS_MAX_BYTES = 2 << 30  # scratch that the runs of one step may take; a step with more is walked token by token
     MFMA_ATTENTION_EXTRAS = True    # whether the matrix-core attention takes a sink and a bias by distance
     name = "hip"
 
@@ -165,6 +171,8 @@ class HipOps:
             fn.argtypes = argtypes
             fn.restype = ctypes.c_int
         self.lib.psamd_last_error.restype = ctypes.c_char_p
+        self.lib.psamd_delta_runs_floats.argtypes = [_i32] * 5
+        self.lib.psamd_delta_runs_floats.restype = ctypes.c_int64
         self.lib.psamd_sample_scratch_floats.argtypes = [ctypes.c_int]
         self.lib.psamd_sample_scratch_floats.restype = ctypes.c_int64
         self.ws = workspace
@@ -1202,7 +1210,7 @@ class HipOps:
 
     def delta_scan(self, keys, directions, removals, queries, key_groups: int, decay_vectors, decay, removal_scale,
                    value_scale, values, out, state, state_offset: int, ctx, heads: int, dim: int, vdim: int,
-                   reads_decayed: bool, no_removal: bool = False) -> None:
+                   reads_decayed: bool, no_removal: bool = False, in_runs: bool = False, decay_least: float = 0.0) -> None:
         """The delta-rule recurrence over each item's tokens from its state slot. Every operand is a pair
         (float32 tensor [T, row], first column) or None. Per head h (its key group g = h // (heads / key_groups))
         and token: S' = d S with d = decay_vectors[h, :] (per key channel) times decay[h] (a number), either may
@@ -1212,7 +1220,9 @@ class HipOps:
         ``value_scale``. The state of head h is ``state[slot, state_offset + (h vdim + j) dim + i]``; out is
         float32 [T, heads vdim]. ``no_removal``: the caller says that ``removal_scale`` is zero throughout (a linear
         recurrence S = d S + k (xs x)^T in the gated rule's form: keys, directions and removals one vector, a decay per
-        head); the kernel then skips the removal and the sum it waits for."""
+        head); the kernel then skips the removal and the sum it waits for. ``in_runs``: the items of a step with a long one may
+        be computed run by run (the sums in another order, all in float32); ``decay_least``: what no entry of
+        ``decay_vectors`` is under."""
         t = out.shape[0]
         self._need(t == ctx.num_tokens and out.dtype == torch.float32 and out.shape == (t, heads * vdim) and out.is_contiguous(),
                    "delta_scan: out is float32 [T, heads vdim]")
@@ -1243,12 +1253,31 @@ class HipOps:
         def at(pair):
             return None if pair is None else pair[0].data_ptr() + 4 * pair[1]
 
-        self._ok(self.lib.psamd_delta_scan(
+        operands = (
             self._stream(), at(keys), at(directions), at(removals), at(queries), base.shape[1], key_groups,
             at(decay_vectors), 0 if decay_vectors is None else decay_vectors[0].shape[1], at(decay), at(removal_scale),
             at(value_scale), 0 if sbase is None else sbase.shape[1], at(values), xv.shape[1], out.data_ptr(), out.shape[1],
-            state.data_ptr() + 4 * state_offset, state.shape[1], ctx.item_start.data_ptr(), ctx.slots.data_ptr(),
-            ctx.num_items, heads, dim, vdim, 2 if no_removal else int(reads_decayed)))
+            state.data_ptr() + 4 * state_offset, state.shape[1], ctx.item_start.data_ptr(), ctx.slots.data_ptr())
+        most = 0
+        if in_runs and ctx.num_prefill_blocks:
+            # A prompt of under DELTA_RUNS_MIN_TOKENS is walked in the time the three launches of the runs take.
+            longest = int(np.diff(ctx.host["item_start"]).max())
+            same = keys[1] == directions[1] == removals[1] and decay_vectors is None and reads_decayed
+            form = (1 if no_removal else 0) if same else 2
+            fits = same or (not reads_decayed and decay_vectors is not None and decay is None and removal_scale is None
+                            and value_scale is None and key_groups == heads)
+            floats = int(self.lib.psamd_delta_runs_floats(ctx.num_prefill_blocks, heads, dim, vdim, int(form == 2)))
+            if (longest >= self.DELTA_RUNS_MIN_TOKENS and fits and 4 * floats <= self.DELTA_RUNS_MAX_BYTES
+                    and all(p % 16 == 0 for p in (at(keys), at(directions), at(removals), at(queries), out.data_ptr(), operands[17]))
+                    and self.lib.psamd_delta_runs_supports(dim, vdim, base.shape[1], xv.shape[1], out.shape[1], operands[8],
+                                                           state.shape[1], int(form == 2), float(decay_least))):
+                scratch = self.ws.get("delta.runs", (floats,), torch.float32)
+                self._ok(self.lib.psamd_delta_runs(*operands, ctx.pf_tiles.data_ptr(), ctx.pf_blocks.data_ptr(), ctx.num_prefill_blocks,
+                                                   ctx.num_items, heads, dim, vdim, form, float(decay_least), scratch.data_ptr()))
+                if ctx.num_decode == 0:
+                    return
+                most = 1                       # the single tokens are left
+        self._ok(self.lib.psamd_delta_scan(*operands, ctx.num_items, heads, dim, vdim, 2 if no_removal else int(reads_decayed), most))
 
     def heads_norm_gate(self, o, heads: int, vdim: int, weight, weight_per_head: bool, eps: float, gate_rows, gate_col: int,
                         activation: str, out) -> None:

@@ -21,6 +21,14 @@ if TYPE_CHECKING:
 UNIT_EPS = 1e-6          # inside the root when a key or query is made a unit vector
 
 
+def in_runs(rt: Runtime, decay_least: float = 0.0) -> dict[str, Any]:
+    """What a mixer adds to its ``delta_scan`` call: a serving step may sum a prompt run by run; the exact mode sums token by
+    token, so that a position's bits do not depend on how its sequence was cut."""
+    if rt.dtype != torch.bfloat16 or not hasattr(rt.ops, "DELTA_RUNS_MIN_TOKENS"):
+        return {}
+    return {"in_runs": True, "decay_least": decay_least}
+
+
 class GatedDeltaRule(Mixer):
     """The gated delta rule. q and k (``num_kv_heads`` x ``head_dim``; head h uses vector
     h // (heads / kv_heads)) and v (``num_heads`` x ``value_dim``) each pass a causal convolution per
@@ -107,7 +115,7 @@ class GatedDeltaRule(Mixer):
         ops.delta_scan(keys=(u, k_col), directions=(u, k_col), removals=(u, k_col), queries=(u, 0),
                        key_groups=self.num_kv_heads, decay_vectors=None, decay=(coef, 0), removal_scale=(coef, hd),
                        value_scale=(coef, 2 * hd), values=(u, v_col), out=o, state=state, state_offset=self.state_base + self.tail, ctx=ctx,
-                       heads=hd, dim=self.head_dim, vdim=self.value_dim, reads_decayed=True)
+                       heads=hd, dim=self.head_dim, vdim=self.value_dim, reads_decayed=True, **in_runs(rt))
         out = ws.get("delta.out", (t, self.value_size), rt.dtype)
         ops.heads_norm_gate(o, hd, self.value_dim, self.norm_w, False, self.norm_eps, rows, self.channels, "silu", out)
         return ops.linear_to_residual(out, self.w_o, "delta.delta", getattr(ctx, "residual", None))
@@ -179,7 +187,7 @@ class GeneralizedDeltaRule(Mixer):
         ops.delta_scan(keys=(operands, s), directions=(operands, 5 * s), removals=(operands, 4 * s), queries=(operands, 0),
                        key_groups=hd, decay_vectors=(operands, 3 * s), decay=None, removal_scale=None, value_scale=None,
                        values=(operands, 2 * s), out=o, state=state, state_offset=self.state_base, ctx=ctx, heads=hd, dim=self.head_dim,
-                       vdim=self.head_dim, reads_decayed=False)
+                       vdim=self.head_dim, reads_decayed=False, **in_runs(rt, math.exp(-self.decay_floor)))
         out = ws.get("gdelta.out", (t, s), rt.dtype)
         ops.heads_norm_gate(o, hd, self.head_dim, self.norm_w, True, self.norm_eps, rows, 3 * s, "sigmoid", out)
         return ops.linear_to_residual(out, self.w_o, "gdelta.delta", getattr(ctx, "residual", None))

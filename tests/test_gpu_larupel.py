@@ -538,3 +538,71 @@ def test_random_configurations_in_both_dtypes(seed, tmp_path):
             assert max(errors) < F32_TOL, (cfg, max(errors))
         else:
             check_rows(errors, dtype, bf16_bars(folder, truth, reqs))
+
+
+@pytest.mark.parametrize("form,heads,groups,dim,vdim", [("gated", 4, 2, 128, 128), ("gated", 2, 2, 64, 48), ("plain", 6, 1, 128, 64),
+                                                        ("plain", 2, 2, 64, 16), ("general", 3, 3, 64, 64), ("general", 2, 2, 128, 32)])
+def test_recurrences_in_runs_of_64_tokens(ops, form, heads, groups, dim, vdim):
+    """Items shorter than, as long as and longer than one and two runs, single tokens among them (they are walked), each from
+    a state of its own, run by run and token by token against float64. Keys that repeat (the systems to solve are then full),
+    decays of zero (gated, plain) and decays at their floor (general) included. The sums differ in order alone: the runs may be as
+    far off as the walk, twice for the chance of it."""
+    from prefixserve_amd.engine.batch import GroupMeta, StepItem, StepPacker
+
+    lengths = [1, 2, 63, 64, 65, 128, 1, 200, 17]
+    t = sum(lengths)
+    pages = [-(-n // 16) for n in lengths]
+    pk = StepPacker(torch.device(DEV), [GroupMeta(sum(pages))], 10, 4096, 16, ops.PREFILL_TILE_Q, skew_rule=ops.decode_is_skewed)
+    first = np.cumsum([0] + pages)
+    ctx = pk.pack([StepItem(i, [1] * n, 0, [list(range(first[i], first[i + 1]))], slot=15 - i) for i, n in enumerate(lengths)])
+    unit = lambda x: x / x.norm(dim=-1, keepdim=True)
+    k = unit(rnd(t, groups, dim, seed=1))
+    k[200:300] = k[200]                                     # a hundred times the same key
+    r, x = rnd(t, groups, dim, seed=2, scale=dim ** -0.5), rnd(t, heads, vdim, seed=3)
+    state = rnd(16, heads * vdim * dim + 4, seed=4)
+    args = dict(key_groups=groups, ctx=ctx, heads=heads, dim=dim, vdim=vdim, state_offset=4)
+    if form == "general":
+        c, p = k, -torch.sigmoid(rnd(t, heads, dim, seed=5)) * k
+        k = k * (0.5 + rnd(t, heads, 1, seed=6).abs())
+        d = torch.exp(-math.exp(-0.5) * torch.sigmoid(2.0 * rnd(t, heads, dim, seed=7)))
+        d[250:400] = math.exp(-math.exp(-0.5))
+        rows = torch.cat([v.reshape(t, -1) for v in (r, k, c, p, d)], 1).contiguous()
+        s = heads * dim
+        args.update(keys=(rows, s), queries=(rows, 0), directions=(rows, 2 * s), removals=(rows, 3 * s), decay_vectors=(rows, 4 * s),
+                    decay=None, removal_scale=None, value_scale=None, reads_decayed=False, decay_least=math.exp(-math.exp(-0.5)))
+        per, ps, xs = 1, torch.ones(t, heads, device=DEV), torch.ones(t, heads, device=DEV)
+    else:
+        rows = torch.cat([r.reshape(t, -1), k.reshape(t, -1)], 1).contiguous()
+        c = p = k
+        g = torch.exp(-0.2 * rnd(t, heads, seed=5).abs())
+        g[150:153] = 0.0
+        xs = torch.sigmoid(rnd(t, heads, seed=6) + 1.0)
+        ps = -xs if form == "gated" else torch.zeros_like(xs)
+        coef = torch.cat([g, ps, xs], 1).contiguous()
+        kc = (rows, groups * dim)
+        args.update(keys=kc, directions=kc, removals=kc, queries=(rows, 0), decay_vectors=None, decay=(coef, 0),
+                    removal_scale=(coef, heads), value_scale=(coef, 2 * heads), reads_decayed=True, no_removal=form == "plain")
+        per, d = heads // groups, g[:, :, None].expand(t, heads, dim)
+    xflat = x.reshape(t, heads * vdim).contiguous()
+    want, want_state, at = torch.empty(t, heads, vdim, dtype=torch.float64, device=DEV), state.double().clone(), 0
+    wide = lambda v, i: v[i].double().repeat_interleave(per, 0)
+    for i, n in enumerate(lengths):
+        s = state[15 - i, 4:].double().view(heads, vdim, dim).clone()
+        for j in range(at, at + n):
+            seen = s if form == "general" else s * d[j].double()[:, None]
+            taken = (seen * wide(c, j)[:, None]).sum(-1)
+            s = s * d[j].double()[:, None] + (ps[j].double()[:, None] * taken)[:, :, None] * wide(p, j)[:, None]
+            s = s + (xs[j].double()[:, None] * x[j].double())[:, :, None] * wide(k, j)[:, None]
+            want[j] = (s * wide(r, j)[:, None]).sum(-1)
+        want_state[15 - i, 4:] = s.reshape(-1)
+        at += n
+    off = {}
+    for runs in (False, True):
+        st, out = state.clone(), torch.full((t + 1, heads * vdim), 7.0, device=DEV)
+        ops.delta_scan(values=(xflat, 0), out=out[:t], state=st, in_runs=runs, **args)
+        assert torch.all(out[t] == 7.0) and torch.equal(st[:7], state[:7]) and torch.equal(st[:, :4], state[:, :4])
+        gap = lambda a, b: float((a.double() - b).norm() / b.norm())
+        off[runs] = (gap(out[:t].view(t, heads, vdim), want), gap(st[:, 4:], want_state[:, 4:]))
+        print(form, dim, runs, off[runs])
+    assert off[True] != off[False]                          # the sums were made in another order
+    assert all(b < max(2.0 * a, 3e-7) for a, b in zip(off[False], off[True])), off
