@@ -372,7 +372,7 @@ int psamd_attention_decode_plan(int n_dec, int kv_len, int skewed, int hkv, int 
 int psamd_attention_decode_max_parts(int max_requests);
 
 int psamd_attention_decode(void* stream, const void* qkv, int q_stride, void* out, const void* kv, float* part_o,
-                           float* part_ml, const int32_t* dec_items, int n_dec, const int32_t* item_start,
+                           float* part_ml, int32_t* arrived, const int32_t* dec_items, int n_dec, const int32_t* item_start,
                            const int32_t* item_end, const int32_t* table_off, const int32_t* block_ids, int hq,
                            int hkv, int head_dim, int nsplit, float scale, int window, int min_split_keys,
                            int exact_weights);
@@ -387,7 +387,7 @@ int psamd_attention_prefill_extras(void* stream, const void* qkv, int q_stride, 
                                    const float* sink, const float* dist_bias, int n_dist,
                             const void* gate, int64_t gate_row);
 int psamd_attention_decode_extras(void* stream, const void* qkv, int q_stride, void* out, const void* kv, float* part_o,
-                                  float* part_ml, const int32_t* dec_items, int n_dec, const int32_t* item_start,
+                                  float* part_ml, int32_t* arrived, const int32_t* dec_items, int n_dec, const int32_t* item_start,
                                   const int32_t* item_end, const int32_t* table_off, const int32_t* block_ids, int hq,
                                   int hkv, int head_dim, int nsplit, float scale, int window, int min_split_keys,
                                   int exact_weights, const float* sink, const float* dist_bias, int n_dist,

@@ -1147,12 +1147,17 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(
 
 // ------------------------------------------------------------------ decode (split keys)
 
+// A float that workgroups on different dies pass to each other inside a launch: past the caches that they do not share.
+__device__ __forceinline__ void shared_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float shared_load(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
 // NS = D / 16, CT = ceil(group / 16) column tiles of query heads.
-// part_o[dec][head][split][D], part_ml[dec][head][split][2] = (max, sum).
-template <int NS, int CT, bool P3 = false>
+// part_o[dec][head][split][D], part_ml[dec][head][split][2] = (max, sum); arrived[dec][kv head]: how many of a request's
+// workgroups have written their runs, zero between launches.
+template <int NS, int CT, bool P3 = false, bool MERGE = false>
 __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
     const bf16_t* __restrict__ qkv, int q_stride, const bf16_t* __restrict__ kv, bf16_t* __restrict__ out,
-    float* __restrict__ part_o, float* __restrict__ part_ml, const int32_t* __restrict__ dec_items,
+    float* part_o, float* part_ml, int32_t* arrived, const int32_t* __restrict__ dec_items,
     const int32_t* __restrict__ item_start,
     const int32_t* __restrict__ item_end, const int32_t* __restrict__ table_off,
     const int32_t* __restrict__ block_ids, int hq, int hkv, int nsplit, float scale, int window, int min_tiles,
@@ -1194,12 +1199,12 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
   const int my_lo = tile_lo + split * tps;
   const int my_hi = min(my_lo + tps, tile_hi + 1);
   if (my_lo >= my_hi) {
-    // No keys left for this split (only with nsplit > 1): an empty sum and an output of zeros,
-    // which the merge kernel multiplies by a weight of zero (what lay there before might be NaN).
+    // No keys left for this split (only with nsplit > 1): an empty sum and, for the merge kernel, an output of zeros, which it
+    // multiplies by a weight of zero (what lay there before might be NaN). The merge in this kernel does not read it.
     for (int idx = threadIdx.x; idx < group * D; idx += blockDim.x) {
       const int hh = idx / D, d = idx - hh * D;
       const int64_t slot = (static_cast<int64_t>(di) * hq + kvh * group + hh) * nsplit + split;
-      part_o[slot * D + d] = 0.f;
+      if (!MERGE) part_o[slot * D + d] = 0.f;
       if (d == 0) {
         part_ml[slot * 2 + 0] = -INFINITY;
         part_ml[slot * 2 + 1] = 0.f;
@@ -1345,6 +1350,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
     }
   }
   __syncthreads();
+  const int runs = MERGE ? (tile_hi - tile_lo + tps) / tps : 1;        // of this request that have keys
   for (int idx = threadIdx.x; idx < group * D; idx += blockDim.x) {
     const int hh = idx / D, d = idx - hh * D;
     float mm = -INFINITY;
@@ -1358,7 +1364,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
       acc += wgt * sm_o[(static_cast<int64_t>(w) * group + hh) * D + d];
       ll += wgt * sm_l[w * group + hh];
     }
-    if (nsplit == 1) {   // nothing to merge with: this is the result
+    if (MERGE ? runs == 1 : nsplit == 1) {     // nothing to merge with: this is the result
       if (ex.sink != nullptr) ll += __expf(ex.sink[kvh * group + hh] - mm);
       const int64_t at = static_cast<int64_t>(kvh * group + hh) * D + d;
       if (ex.gate != nullptr) acc *= 1.f / (1.f + __expf(-bf16_to_float(ex.gate[t * ex.gate_row + at])));
@@ -1366,11 +1372,58 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
       continue;
     }
     const int64_t slot = (static_cast<int64_t>(di) * hq + kvh * group + hh) * nsplit + split;
-    part_o[slot * D + d] = acc;
-    if (d == 0) {
-      part_ml[slot * 2 + 0] = mm;
-      part_ml[slot * 2 + 1] = ll;
+    if constexpr (!MERGE) {                               // a kernel behind this one merges
+      part_o[slot * D + d] = acc;
+      if (d == 0) {
+        part_ml[slot * 2 + 0] = mm;
+        part_ml[slot * 2 + 1] = ll;
+      }
+      continue;
     }
+    shared_store(part_o + slot * D + d, acc);
+    if (d == 0) {
+      shared_store(part_ml + slot * 2 + 0, mm);
+      shared_store(part_ml + slot * 2 + 1, ll);
+    }
+  }
+  if (!MERGE || runs == 1) return;
+  __shared__ int last_s;
+  // The last of a request's workgroups to get here merges the runs. The partial results pass between dies: they are written and read past the dies' caches,
+  // the writes have arrived before the workgroup counts itself, and whoever counts last reads all of them.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  int32_t* counter = arrived + static_cast<int64_t>(di) * hkv + kvh;
+  if (threadIdx.x == 0) last_s = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == runs - 1;
+  __syncthreads();
+  if (!last_s) return;
+  if (threadIdx.x == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
+  const int64_t base = (static_cast<int64_t>(di) * hq + kvh * group) * nsplit;
+  float* run_m = smem;                                    // [group][runs], then the sums
+  float* run_l = smem + group * runs;
+  for (int idx = threadIdx.x; idx < group * runs; idx += blockDim.x) {
+    const int64_t slot = base + static_cast<int64_t>(idx / runs) * nsplit + idx % runs;
+    run_m[idx] = shared_load(part_ml + slot * 2);
+    run_l[idx] = shared_load(part_ml + slot * 2 + 1);
+  }
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < group * D; idx += blockDim.x) {
+    const int hh = idx / D, d = idx - hh * D;
+    const float* ms = run_m + hh * runs;
+    const float* ls = run_l + hh * runs;
+    const float* po = part_o + (base + static_cast<int64_t>(hh) * nsplit) * D + d;
+    float mm = -INFINITY;
+    for (int s = 0; s < runs; ++s) mm = fmaxf(mm, ms[s]);
+    float acc = 0.f, ll = 0.f;
+#pragma unroll 8
+    for (int s = 0; s < runs; ++s) {
+      const float wgt = __expf(ms[s] - mm);
+      acc += wgt * shared_load(po + static_cast<int64_t>(s) * D);
+      ll += wgt * ls[s];
+    }
+    if (ex.sink != nullptr) ll += __expf(ex.sink[kvh * group + hh] - mm);
+    const int64_t at = static_cast<int64_t>(kvh * group + hh) * D + d;
+    if (ex.gate != nullptr) acc *= 1.f / (1.f + __expf(-bf16_to_float(ex.gate[t * ex.gate_row + at])));
+    out[t * (static_cast<int64_t>(hq) * D) + at] = float_to_bf16(acc / ll);
   }
 }
 
@@ -1583,28 +1636,34 @@ static int launch_prefill(hipStream_t s, const void* qkv, int q_stride, void* ou
 
 template <int NS, int CT, bool P3>
 static int launch_decode(hipStream_t s, const void* qkv, int q_stride, const void* kv, void* out, float* part_o,
-                         float* part_ml, const int32_t* dec_items, int n_dec, const int32_t* item_start, const int32_t* item_end,
+                         float* part_ml, int32_t* arrived, const int32_t* dec_items, int n_dec, const int32_t* item_start, const int32_t* item_end,
                          const int32_t* table_off, const int32_t* block_ids, int hq, int hkv, int nsplit, float scale,
                          int window, int min_tiles) {
   const int group = hq / hkv;
-  const size_t smem = sizeof(float) * (8 * group + 4 * static_cast<size_t>(group) * 16 * NS);
+  // The waves' results, and for the merge two numbers per head and run.
+  const size_t smem = sizeof(float) * std::max<size_t>(8 * group + 4 * static_cast<size_t>(group) * 16 * NS, 2 * static_cast<size_t>(group) * nsplit);
   const int64_t groups_of_8 = ceil_div(static_cast<int64_t>(n_dec) * nsplit, 8);
-  if (!lds_allowed(attn_decode_mfma_kernel<NS, CT, P3>, smem))
-    return fail("psamd_attention_decode: " + std::to_string(smem) + " bytes of LDS were refused");
-  attn_decode_mfma_kernel<NS, CT, P3><<<dim3(8 * hkv, static_cast<unsigned>(groups_of_8)), dim3(256), smem, s>>>(
-      static_cast<const bf16_t*>(qkv), q_stride, static_cast<const bf16_t*>(kv), static_cast<bf16_t*>(out), part_o,
-      part_ml, dec_items, item_start, item_end, table_off, block_ids, hq, hkv, nsplit, scale, window, min_tiles, n_dec,
-      g_extras);
-  return check_launch("psamd_attention_decode");
+  auto run = [&](auto kernel) {
+    if (!lds_allowed(kernel, smem)) return fail("psamd_attention_decode: " + std::to_string(smem) + " bytes of LDS were refused");
+    kernel<<<dim3(8 * hkv, static_cast<unsigned>(groups_of_8)), dim3(256), smem, s>>>(
+        static_cast<const bf16_t*>(qkv), q_stride, static_cast<const bf16_t*>(kv), static_cast<bf16_t*>(out), part_o,
+        part_ml, arrived, dec_items, item_start, item_end, table_off, block_ids, hq, hkv, nsplit, scale, window, min_tiles, n_dec,
+        g_extras);
+    return check_launch("psamd_attention_decode");
+  };
+  if constexpr (CT == 1) {
+    if (arrived != nullptr) return run(attn_decode_mfma_kernel<NS, CT, P3, true>);
+  }
+  return run(attn_decode_mfma_kernel<NS, CT, P3>);
 }
 
 template <int NS, bool P3>
 static int dispatch_decode_ct(int ct, hipStream_t s, const void* qkv, int q_stride, const void* kv, void* out,
-                              float* part_o, float* part_ml, const int32_t* dec_items, int n_dec, const int32_t* item_start,
+                              float* part_o, float* part_ml, int32_t* arrived, const int32_t* dec_items, int n_dec, const int32_t* item_start,
                               const int32_t* item_end, const int32_t* table_off, const int32_t* block_ids, int hq,
                               int hkv, int nsplit, float scale, int window, int min_tiles) {
 #define PSAMD_DEC(CT_)                                                                                             \
-  return launch_decode<NS, CT_, P3>(s, qkv, q_stride, kv, out, part_o, part_ml, dec_items, n_dec, item_start, item_end, \
+  return launch_decode<NS, CT_, P3>(s, qkv, q_stride, kv, out, part_o, part_ml, arrived, dec_items, n_dec, item_start, item_end, \
                                 table_off, block_ids, hq, hkv, nsplit, scale, window, min_tiles)
   switch (ct) {
     case 1: PSAMD_DEC(1);
@@ -1791,17 +1850,19 @@ int psamd_attention_decode_plan(int n_dec, int kv_len, int skewed, int hkv, int 
 // results of every decode step, so that the buffers never grow.
 int psamd_attention_decode_max_parts(int max_requests) { return std::max({4096, 512, max_requests}); }
 
-// part_o needs n_dec * hq * nsplit * head_dim floats, part_ml n_dec * hq * nsplit * 2.
+// part_o needs n_dec * hq * nsplit * head_dim floats, part_ml n_dec * hq * nsplit * 2, arrived n_dec * hkv integers that are
+// zero and are left zero. Launches that share them follow each other on one stream.
 // min_split_keys: a request's keys are cut into runs no shorter than this (a multiple of 32), so
 // that nsplit can follow the longest request of a step without cutting the short ones to pieces.
 int psamd_attention_decode(void* stream, const void* qkv, int q_stride, void* out, const void* kv, float* part_o,
-                           float* part_ml, const int32_t* dec_items, int n_dec, const int32_t* item_start,
+                           float* part_ml, int32_t* arrived, const int32_t* dec_items, int n_dec, const int32_t* item_start,
                            const int32_t* item_end, const int32_t* table_off, const int32_t* block_ids, int hq,
                            int hkv, int head_dim, int nsplit, float scale, int window, int min_split_keys,
                            int exact_weights) {
   PSAMD_REQUIRE(psamd_attention_mfma_supports(hq, hkv, head_dim), "shape not supported by the matrix-core kernels");
   PSAMD_REQUIRE(q_stride % 8 == 0, "query row stride must be a multiple of 8 elements");
   PSAMD_REQUIRE(nsplit >= 1 && nsplit <= 64, "nsplit must be in [1, 64]");
+  PSAMD_REQUIRE(nsplit == 1 || (part_o != nullptr && part_ml != nullptr && arrived != nullptr), "runs need their buffers");
   PSAMD_REQUIRE(min_split_keys >= 32 && min_split_keys % 32 == 0, "min_split_keys must be a positive multiple of 32");
   const int min_tiles = min_split_keys / 32;
   PSAMD_REQUIRE(static_cast<int64_t>(n_dec) * nsplit <= 8 * 65535, "too many (request, split) pairs for one launch");
@@ -1809,12 +1870,16 @@ int psamd_attention_decode(void* stream, const void* qkv, int q_stride, void* ou
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int group = hq / hkv;
   const int ct = group <= 16 ? 1 : (group <= 32 ? 2 : 4);
+  // Where a kv head's runs are few numbers, the last of its workgroups merges them: attention + merge of one request behind 300
+  // tokens 9.5 -> 7.3 us, of eight behind 2,048 15.6 -> 13.5 (4 heads of 64 a kv head). 16 heads of 256 in 32 runs would be half
+  // a megabyte past the caches for one workgroup: 24.6 -> 47 us, and a merge kernel with a block per head stays.
+  if (nsplit == 1 || ct > 1 || static_cast<int64_t>(group) * head_dim * nsplit > 16384) arrived = nullptr;
   int rc;
 #define PSAMD_DEC_NS(NS_)                                                                                          \
-  rc = exact_weights ? dispatch_decode_ct<NS_, true>(ct, s, qkv, q_stride, kv, out, part_o, part_ml, dec_items, n_dec,  \
+  rc = exact_weights ? dispatch_decode_ct<NS_, true>(ct, s, qkv, q_stride, kv, out, part_o, part_ml, arrived, dec_items, n_dec, \
                                                      item_start, item_end, table_off, block_ids, hq, hkv, nsplit, scale, \
                                                      window, min_tiles)                                          \
-                     : dispatch_decode_ct<NS_, false>(ct, s, qkv, q_stride, kv, out, part_o, part_ml, dec_items, n_dec, \
+                     : dispatch_decode_ct<NS_, false>(ct, s, qkv, q_stride, kv, out, part_o, part_ml, arrived, dec_items, n_dec, \
                                                       item_start, item_end, table_off, block_ids, hq, hkv, nsplit, scale, \
                                                       window, min_tiles);                                        \
   break
@@ -1832,7 +1897,7 @@ int psamd_attention_decode(void* stream, const void* qkv, int q_stride, void* ou
     default: PSAMD_DEC_NS(16);
   }
 #undef PSAMD_DEC_NS
-  if (rc != 0 || nsplit == 1) return rc;
+  if (rc != 0 || nsplit == 1 || arrived != nullptr) return rc;
   attn_decode_merge_kernel<<<dim3(n_dec, hq), dim3(64), 0, s>>>(part_o, part_ml, static_cast<bf16_t*>(out), dec_items,
                                                                item_start, hq, head_dim, nsplit, g_extras);
   return check_launch("psamd_attention_decode(merge)");
@@ -1859,7 +1924,7 @@ int psamd_attention_prefill_extras(void* stream, const void* qkv, int q_stride, 
 }
 
 int psamd_attention_decode_extras(void* stream, const void* qkv, int q_stride, void* out, const void* kv, float* part_o,
-                                  float* part_ml, const int32_t* dec_items, int n_dec, const int32_t* item_start,
+                                  float* part_ml, int32_t* arrived, const int32_t* dec_items, int n_dec, const int32_t* item_start,
                                   const int32_t* item_end, const int32_t* table_off, const int32_t* block_ids, int hq,
                                   int hkv, int head_dim, int nsplit, float scale, int window, int min_split_keys,
                                   int exact_weights, const float* sink, const float* dist_bias, int n_dist, const void* gate, int64_t gate_row) {
@@ -1867,7 +1932,7 @@ int psamd_attention_decode_extras(void* stream, const void* qkv, int q_stride, v
   PSAMD_REQUIRE(gate == nullptr || (gate_row % 4 == 0 && gate_row >= static_cast<int64_t>(hq) * head_dim &&
                                     reinterpret_cast<uintptr_t>(gate) % 8 == 0), "the gate's rows");
   g_extras = Extras{sink, dist_bias, n_dist, static_cast<const bf16_t*>(gate), gate_row};
-  const int rc = psamd_attention_decode(stream, qkv, q_stride, out, kv, part_o, part_ml, dec_items, n_dec, item_start,
+  const int rc = psamd_attention_decode(stream, qkv, q_stride, out, kv, part_o, part_ml, arrived, dec_items, n_dec, item_start,
                                         item_end, table_off, block_ids, hq, hkv, head_dim, nsplit, scale, window,
                                         min_split_keys, exact_weights);
   g_extras = kNoExtras;

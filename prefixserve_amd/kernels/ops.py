@@ -71,11 +71,11 @@ _SIGNATURES = {
     "psamd_attention_decode_max_parts": [_i32],
     "psamd_attention_prefill": [_vp, _vp, _i32, _vp, _vp, _vp, _i32, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32,
                                 _f32, _i32, _vp, _vp, _i32, _i32],
-    "psamd_attention_decode": [_vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32,
+    "psamd_attention_decode": [_vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32,
                                _i32, _f32, _i32, _i32, _i32],
     "psamd_attention_prefill_extras": [_vp, _vp, _i32, _vp, _vp, _vp, _i32, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32,
                                        _f32, _i32, _vp, _vp, _i32, _i32, _vp, _vp, _i32, _vp, _i64],
-    "psamd_attention_decode_extras": [_vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32,
+    "psamd_attention_decode_extras": [_vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32,
                                       _i32, _f32, _i32, _i32, _i32, _vp, _vp, _i32, _vp, _i64],
     "psamd_sample": [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32],
     "psamd_scaled_add_rmsnorm": [_vp, _vp, _f32, _vp, _i32, _i32, _i64, _vp, _i32, _f32, _vp, _i32, _i64, _i32],
@@ -1422,10 +1422,11 @@ class HipOps:
                 self._need(ctx.num_decode * nsplit <= parts, "attention: more (request, run) pairs than planned for")
                 part_o = self.ws.get("attn.part_o", (parts * hq * d,), torch.float32)
                 part_ml = self.ws.get("attn.part_ml", (parts * hq * 2,), torch.float32)
+                arrived = self.ws.get_zeroed("attn.arrived", (parts * hkv,), torch.int32)      # left zero by every launch
                 tail = (_ptr(sink), _ptr(dist_bias), 0 if dist_bias is None else dist_bias.shape[1], *gate) if extras else ()
                 self._ok((self.lib.psamd_attention_decode_extras if extras else self.lib.psamd_attention_decode)(
                     s, qkv.data_ptr(), stride, out.data_ptr(), kv.data_ptr(), part_o.data_ptr(), part_ml.data_ptr(),
-                    ctx.dec_items.data_ptr(), ctx.num_decode, ctx.item_start.data_ptr(),
+                    arrived.data_ptr(), ctx.dec_items.data_ptr(), ctx.num_decode, ctx.item_start.data_ptr(),
                     ctx.item_end.data_ptr(), g.table_off.data_ptr(), g.block_ids.data_ptr(), hq, hkv, d, nsplit, scale,
                     win, min_run, int(exact_weights), *tail))
             return

@@ -707,6 +707,22 @@ def test_decode_attention_of_many_requests(ops, hq, hkv, d, longest, window):
     assert rel(got, want) < 2e-2
 
 
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 64), (8, 8, 128), (16, 1, 64), (6, 3, 48), (32, 1, 64)])
+@pytest.mark.parametrize("old", [(0,), (127, 128, 129), (2047, 300, 0, 511), (4000,)])
+def test_decode_attention_merges_its_runs_each_time_it_is_launched(ops, hq, hkv, d, old):
+    """Few requests, their keys in runs that the last workgroup of a kv head merges (or, with more numbers than that pays
+    for, a kernel of its own): contexts of one run, of whole runs and of a key more, again and again on the same counters,
+    which are zero after every launch, and the same bits every time."""
+    pages = sum(-(-(o + 1) // 16) for o in old) + 8
+    first = None
+    for _ in range(3):
+        got, want = paged_case(ops, torch.bfloat16, hq, hkv, d, [1] * len(old), old, seed=9, num_blocks=pages, poison=float("nan"))
+        assert rel(got, want) < 2e-2
+        assert int(ops.ws._bufs["attn.arrived"].abs().max()) == 0
+        first = got if first is None else first
+        assert torch.equal(got, first)
+
+
 @pytest.mark.parametrize("hq,hkv,d,short,longest", [
     (32, 8, 64, 31, 9000),         # many workgroups already: the long request alone gets more runs
     (16, 8, 128, 7, 12500),        # few requests: runs of 1,024 keys instead of the usual short ones
