@@ -300,7 +300,9 @@ int psamd_gemm_lt(void* stream, const void* x, const void* w, void* out, int out
                   int use_workspace, int accumulate);
 
 
-// bfloat16 product for M <= 64 on the matrix cores. epilogue 1: w = [gate; up], out = silu(gate) * up;
+// 1 if psamd_linear_skinny (gated: with one of its gated epilogues) and, for out = qkv_out, psamd_qkv_rope_append take M > 64.
+int psamd_linear_skinny_takes(const void* x, const void* w, const void* out, int M, int n_out, int K, int gated);
+// bfloat16 product for M <= 64 (128 where psamd_linear_skinny_takes says so) on the matrix cores. epilogue 1: w = [gate; up], out = silu(gate) * up;
 // 2 and 3: the same with ReLU and with GELU (tanh form) on the gate.
 // ksplit > 1: out receives ksplit float32 partial sums [ksplit][M, n_out] (plain epilogue only).
 int psamd_linear_skinny_ksplit(int M, int n_out, int K);

@@ -13,6 +13,7 @@
 #include "api.h"
 #include "common.h"
 #include "linear_f32.h"
+#include "linear_stream.h"
 
 namespace psamd {
 
@@ -887,7 +888,9 @@ int psamd_linear(void* stream, const void* x, int x_dtype, const void* w, int w_
 // The K-split that fills the chip for a linear product of M <= 64 tokens whose float32 partial
 // sums a consumer adds up: as many workgroups as there are compute units to spare.
 int psamd_linear_skinny_ksplit(int M, int n_out, int K) {
-  if (M < 1 || M > 64 || n_out < 1 || K < 1) return 1;
+  if (n_out < 1 || K < 1) return 1;
+  if (linear_stream_takes(nullptr, nullptr, nullptr, M, n_out, K, false)) return linear_stream_ksplit(n_out, K);
+  if (M < 1 || M > 64) return 1;
   const int mt = static_cast<int>(ceil_div(M, 16));
   const int64_t groups = ceil_div(ceil_div(n_out, 16), skinny_rt(mt, false));
   const int64_t steps = ceil_div(K, 32);
@@ -908,11 +911,16 @@ int psamd_linear_skinny_ksplit(int M, int n_out, int K) {
   return static_cast<int>(std::max<int64_t>(split, 1));
 }
 
+int psamd_linear_skinny_takes(const void* x, const void* w, const void* out, int M, int n_out, int K, int gated) {
+  return linear_stream_takes(x, w, out, M, n_out, K, gated != 0) ? 1 : 0;
+}
+
 // out[ksplit][M, n_out]; epilogue 0: n_out = rows of w; epilogue 1 (SwiGLU): w has 2 * n_out rows.
 // ksplit > 1 splits K over workgroups: out then holds ksplit float32 partial sums to be added.
 int psamd_linear_skinny(void* stream, const void* x, const void* w, void* out, int out_dtype, int M, int n_out, int K,
                         int epilogue, int ksplit) {
-  PSAMD_REQUIRE(M >= 1 && M <= 64, "M must be in [1, 64]");
+  const bool stream_takes = linear_stream_takes(x, w, out, M, n_out, K, epilogue >= 1);
+  PSAMD_REQUIRE(M >= 1 && (M <= 64 || stream_takes), "M must be in [1, 64]");
   PSAMD_REQUIRE(n_out > 0 && K > 0 && K % 8 == 0, "K must be a positive multiple of 8");
   PSAMD_REQUIRE(epilogue >= 0 && epilogue <= 3, "unknown epilogue");
   if (epilogue >= 1) {             // 1, 2, 3: the gated epilogue with SiLU, ReLU or GELU (tanh form) on the gate
@@ -925,6 +933,9 @@ int psamd_linear_skinny(void* stream, const void* x, const void* w, void* out, i
   PSAMD_REQUIRE(ksplit == 1 || (epilogue == 0 && out_dtype == kF32), "partial sums are float32 and linear");
   PSAMD_REQUIRE(ceil_div(n_out, 16) <= 2147483647LL, "too many columns");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (stream_takes && ksplit <= K / 64 && ceil_div(K / 64, ceil_div(K / 64, ksplit)) == ksplit)
+    return launch_linear_stream(s, x, w, out, out_dtype == kF32, M, n_out, K, epilogue == 1 ? g_gate_act : -1, ksplit);
+  PSAMD_REQUIRE(M <= 64, "M must be in [1, 64]");
   const int mt = static_cast<int>(ceil_div(M, 16));
   switch (mt) {
     case 1: return launch_skinny<1>(s, x, w, out, out_dtype, M, n_out, K, epilogue, ksplit);
@@ -940,7 +951,11 @@ int psamd_linear_skinny(void* stream, const void* x, const void* w, void* out, i
 int psamd_qkv_rope_append(void* stream, const void* x, const void* w, void* qkv_out, int M, int K, int hq, int hkv,
                           int head_dim, const int32_t* positions, const float* table, void* kv,
                           const int32_t* write_slot) {
-  PSAMD_REQUIRE(M >= 1 && M <= 64, "M must be in [1, 64]");
+  // From 25 tokens on both operands go through LDS, from 17 on where there are 320 tiles (3,072 x 2,048: 7.7 us here and 8.2
+  // there at 17 tokens, 8.4 and 8.2 at 24, 13.4 and 10.5 at 64; 6,144 x 4,096: 19.5 and 15.8 at 17, 30.6 and 20.4 at 64).
+  const bool stream_takes = hq > 0 && hkv > 0 && (M > 24 || (hq + 2 * hkv) * (head_dim / 16) >= 320) &&
+                            linear_stream_takes(x, w, qkv_out, M, (hq + 2 * hkv) * head_dim, K, false);
+  PSAMD_REQUIRE(M >= 1 && (M <= 64 || stream_takes), "M must be in [1, 64]");
   PSAMD_REQUIRE(K > 0 && K % 8 == 0, "K must be a positive multiple of 8");
   PSAMD_REQUIRE(hq > 0 && hkv > 0 && head_dim >= 16 && head_dim % 16 == 0, "head_dim must be a multiple of 16");
   PSAMD_REQUIRE(positions != nullptr, "positions are needed");
@@ -951,6 +966,7 @@ int psamd_qkv_rope_append(void* stream, const void* x, const void* w, void* qkv_
   bf16_t* op = static_cast<bf16_t*>(qkv_out);
   const float2* tab = reinterpret_cast<const float2*>(table);
   bf16_t* kvp = static_cast<bf16_t*>(kv);
+  if (stream_takes) return launch_qkv_stream(s, x, w, qkv_out, M, K, QkvOut{hq, hkv, head_dim, positions, tab, kvp, write_slot});
   switch (static_cast<int>(ceil_div(M, 16))) {
     case 1: launch_qkv<1>(s, xp, wp, op, M, K, hq, hkv, head_dim, positions, tab, kvp, write_slot); break;
     case 2: launch_qkv<2>(s, xp, wp, op, M, K, hq, hkv, head_dim, positions, tab, kvp, write_slot); break;

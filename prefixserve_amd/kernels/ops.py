@@ -54,6 +54,7 @@ _SIGNATURES = {
     "psamd_linear_skinny": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32],
     "psamd_linear_skinny_ksplit": [_i32, _i32, _i32],
     "psamd_qkv_rope_append": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp],
+    "psamd_linear_skinny_takes": [_vp, _vp, _vp, _i32, _i32, _i32, _i32],
     "psamd_normed_supports": [_i32, _i32],
     "psamd_linear_skinny_add": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp],
     "psamd_linear_normed": [_vp, _vp, _vp, _vp, _i32, _f32, _vp, _vp, _i32, _i32, _i32, _i32, _i32],
@@ -150,6 +151,7 @@ GATE_ACTIVATIONS = {"silu": 0, "relu": 1, "gelu_tanh": 2}
 class HipOps:
     PREFILL_TILE_Q = 32    # queries per workgroup of the prefill attention kernel (its 4 waves split the keys)
     SKINNY_MAX_ROWS = 64
+    STREAM_MAX_ROWS = 128           # whole 64-element steps of K and aligned operands: the products with both operands through LDS
     FUSED_SWIGLU_MAX_ROWS = 32      # above it (to SKINNY_MAX_ROWS) gate/up goes to the library, where there is one
     LIBRARY_ADD_MIN_ROWS = 1024     # from here on a product that feeds the residual stream adds into it in the library
     MOE_ROUTE_FUSED_MAX_TOKENS = 0   # up to here one kernel computes router logits and choice; above, product + choice
@@ -634,7 +636,7 @@ class HipOps:
 
     def qkv_rope_append(self, x, w_qkv, qkv, hq: int, hkv: int, d: int, positions, table, kv, write_slot) -> None:
         """qkv = x @ w_qkv^T, q and k rotated, k and v written to their pages. One kernel for a
-        bfloat16 step of at most 64 tokens; otherwise the product followed by ``rope_kv_append``."""
+        bfloat16 step of at most 64 tokens (128: ``_through_lds``); otherwise the product followed by ``rope_kv_append``."""
         m, k = x.shape
         if isinstance(x, NormedRows):
             if (x.rows is None and d % 16 == 0 and qkv.dtype == torch.bfloat16 and self.fuses_norm(m, k, x.dtype)):
@@ -654,7 +656,8 @@ class HipOps:
                     positions.data_ptr(), _ptr(table), _ptr(kv), None if kv is None else write_slot.data_ptr()))
                 return
             x = self.normed(x)
-        if (x.dtype == torch.bfloat16 and 0 < m <= self.SKINNY_MAX_ROWS and k % 8 == 0 and d % 16 == 0):
+        if (x.dtype == torch.bfloat16 and k % 8 == 0 and d % 16 == 0
+                and (0 < m <= self.SKINNY_MAX_ROWS or self._through_lds(x, w_qkv, qkv, m, qkv.shape[1], k))):
             self._need(w_qkv.shape == ((hq + 2 * hkv) * d, k) and qkv.shape == (m, (hq + 2 * hkv) * d), "qkv: shapes")
             self._need(x.is_contiguous() and w_qkv.is_contiguous() and qkv.is_contiguous(), "qkv: contiguous operands")
             self._need(positions.dtype == torch.int32 and positions.numel() == m, "qkv: positions")
@@ -673,6 +676,14 @@ class HipOps:
         self.rope_kv_append(qkv, hq, hkv, d, positions, table, kv, write_slot)
 
     # ---------------------------------------------------------------- products
+
+    def _through_lds(self, x, w, out, m: int, n: int, k: int, gated: bool = False) -> bool:
+        """Whether the products of 17 to 128 tokens with both operands through LDS take this one. At the 1B shape they
+        take, against the library's product (and the kernels behind it), at 77 tokens: o 5.0 us for 8.5, down 11.4 for 20.8,
+        gate/up with its activation 21.4 for 23.1."""
+        return (self.FUSED_SWIGLU_MAX_ROWS < m <= self.STREAM_MAX_ROWS and x.dtype == torch.bfloat16
+                and w.dtype == torch.bfloat16 and out.dtype == torch.bfloat16
+                and bool(self.lib.psamd_linear_skinny_takes(x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, int(gated))))
 
     def linear(self, x, w, out) -> None:
         m, k = x.shape
@@ -745,13 +756,13 @@ class HipOps:
             if rc != 2:                          # 2: no algorithm for this shape: the ways below
                 self._ok(rc)
                 return None
-        if x.dtype == torch.bfloat16 and k % 8 == 0 and 0 < m <= self.SKINNY_MAX_ROWS:
+        if x.dtype == torch.bfloat16 and k % 8 == 0 and (0 < m <= self.SKINNY_MAX_ROWS or self._through_lds(x, w, x, m, n, k)):
             ksplit = self.lib.psamd_linear_skinny_ksplit(m, n, k)
             if ksplit > 1:
                 self._need(w.shape[1] == k and x.is_contiguous() and w.is_contiguous(), "linear_to_residual: operands")
                 # Room for the most slices of the most rows, so that the buffer never grows.
                 self._need(ksplit <= 8, "linear_to_residual: more slices than there is room for")
-                room = self.ws.get(name + ".slices", (8 * self.SKINNY_MAX_ROWS * n,), torch.float32)
+                room = self.ws.get(name + ".slices", (8 * self.STREAM_MAX_ROWS * n,), torch.float32)
                 kept = self._slice_views.get((name, ksplit, m))
                 if kept is None or kept[0] is not room:
                     kept = self._slice_views[(name, ksplit, m)] = (room, room[:ksplit * m * n].view(ksplit, m, n))
@@ -780,8 +791,9 @@ class HipOps:
                 return
             x = self.normed(x)
         self._need(x.is_contiguous() and w_gate_up.is_contiguous() and out.is_contiguous(), "linear_swiglu: contiguous operands")
-        small = x.dtype == torch.bfloat16 and k % 8 == 0 and m <= self.SKINNY_MAX_ROWS
-        if small and m > self.FUSED_SWIGLU_MAX_ROWS and self._direct_library:
+        lds = self._through_lds(x, w_gate_up, out, m, inter, k, True)
+        small = x.dtype == torch.bfloat16 and k % 8 == 0 and (m <= self.SKINNY_MAX_ROWS or lds)
+        if small and m > self.FUSED_SWIGLU_MAX_ROWS and not lds and self._direct_library:
             # Between these row counts the library's product and the activation kernel behind it
             # take less time than the fused form, which streams the weights with too few rows a wave.
             gu = self.ws.get("mlp.gate_up", (m, 2 * inter), x.dtype)

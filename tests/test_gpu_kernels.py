@@ -567,6 +567,58 @@ def test_linear_swiglu_wide(ops, m, inter):
         assert rel(out[:m], want) < 1e-2 and torch.all(out[m] == 7.0)
 
 
+@pytest.mark.parametrize("m", [17, 32, 33, 64, 65, 79, 128])
+@pytest.mark.parametrize("n,k", [(64, 64), (100, 64 * 3), (1024, 64 * 9), (16 * 200 + 4, 64 * 5), (64 * 193, 64 * 8)])
+def test_products_of_17_to_128_tokens(ops, m, n, k):
+    """Both operands through LDS: one step of K, fewer and more steps than there are buffers, an odd one out; tiles of 16, 32 and
+    64 rows of w with a part of the last; every number of token tiles. Against 64 bits; beside each the general kernels, which an
+    operand off a 16-byte boundary takes. float32 sums of K products: 1e-6 is several times sqrt(K) ulps; bfloat16 rounds at 2^-9."""
+    x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd(2 * n, k, dtype=torch.bfloat16, seed=2, scale=0.2)
+    prod = x.double() @ w.double().T
+    assert ops.lib.psamd_linear_skinny_takes(x.data_ptr(), w.data_ptr(), x.data_ptr(), m, n, k, 1) == 1
+    slices = ops.linear_to_residual(x, w[:n], f"t{n}")
+    assert slices.dtype == (torch.float32 if slices.dim() == 3 else torch.bfloat16)
+    assert rel(slices.double().sum(0) if slices.dim() == 3 else slices, prod[:, :n]) < (1e-6 if slices.dim() == 3 else 1e-2)
+    want = torch.nn.functional.silu(prod[:, :n]) * prod[:, n:]
+    shifted = torch.zeros(m * k + 1, dtype=torch.bfloat16, device=DEV)[1:].view(m, k)
+    shifted.copy_(x)
+    for rows in ((x, shifted) if m <= 64 else (x,)):
+        for dtype in (torch.float32, torch.bfloat16):
+            out = torch.full((m + 1, n), 7.0, dtype=dtype, device=DEV)
+            ops.linear(rows, w[:n], out[:m])
+            assert rel(out[:m], prod[:, :n]) < (1e-6 if dtype == torch.float32 else 1e-2) and torch.all(out[m] == 7.0)
+        out = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+        ops.linear_swiglu(rows, w, out[:m])
+        assert rel(out[:m], want) < 1e-2 and torch.all(out[m] == 7.0)
+
+
+@pytest.mark.parametrize("m", [25, 64, 65, 128])
+@pytest.mark.parametrize("hq,hkv,d,k", [(4, 2, 16, 64), (6, 3, 48, 192), (32, 8, 64, 576), (32, 8, 128, 128)])
+@pytest.mark.parametrize("rotate", [True, False])
+def test_qkv_of_17_to_128_tokens(ops, m, hq, hkv, d, k, rotate):
+    """The q/k/v product with both operands through LDS against the product, the rotation and the pages of 64 bits; bfloat16
+    rounds at 2^-9. Heads whose halves are no multiple of a tile; nothing outside the written slots changes."""
+    n = (hq + 2 * hkv) * d
+    x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2, scale=0.2)
+    pos = torch.randperm(300)[:m].to(torch.int32).to(DEV)
+    table = rnd(300, d // 2, 2, dtype=torch.float32, seed=3)
+    slot = (torch.randperm(20 * 16)[:m]).to(torch.int32).to(DEV)
+    kv = torch.full((20, 2, hkv, 16 * d), 7.0, dtype=torch.bfloat16, device=DEV)
+    out = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.qkv_rope_append(x, w, out[:m], hq, hkv, d, pos, table if rotate else None, kv, slot)
+    want = (x.double() @ w.double().T).view(m, hq + 2 * hkv, 2, d // 2)
+    if rotate:
+        c = table[pos.long()].double()[:, None]
+        a, b = want[:, :hq + hkv, 0].clone(), want[:, :hq + hkv, 1].clone()
+        want[:, :hq + hkv, 0], want[:, :hq + hkv, 1] = a * c[..., 0] - b * c[..., 1], b * c[..., 0] + a * c[..., 1]
+    assert rel(out[:m], want.reshape(m, n)) < 1e-2 and torch.all(out[m] == 7.0)
+    heads, at = out[:m].view(m, hq + 2 * hkv, d), slot.long()
+    expected = torch.full_like(kv, 7.0)
+    expected[:, 0].view(20, hkv, 16, d)[at // 16, :, at % 16] = heads[:, hq:hq + hkv]
+    expected[:, 1].view(20, hkv, d, 16)[at // 16, :, :, at % 16] = heads[:, hq + hkv:]
+    assert torch.equal(kv, expected)
+
+
 # -------------------------------------------------------------------- attention
 
 def paged_case(ops, act, hq, hkv, d, lens_new, lens_old, window=None, seed=0, num_blocks=64, poison=1e30, give_back=False,
