@@ -48,6 +48,30 @@ __device__ __forceinline__ float softplusf_(float z) { return z > 20.f ? z : log
 // replaced by the item's last ones: both are the work of one thread per (item, channel), so that
 // nobody reads a saved input another thread has already replaced.
 template <typename A, typename O>
+__device__ __forceinline__ void short_conv_item(const A* __restrict__ in, int64_t in_row, const float* __restrict__ wc, float b,
+                                                O* __restrict__ out, int64_t out_row, float* __restrict__ saved, int64_t s0, int n,
+                                                int c, int channels, int taps, int act) {
+  const int keep = taps - 1;
+  const int first = min(n, keep);
+  for (int li = 0; li < first; ++li) {
+    float acc = b;
+    for (int j = 0; j < taps; ++j) {
+      const int src = li - keep + j;
+      const float v = src >= 0 ? to_float<A>(in[(s0 + src) * in_row + c]) : saved[static_cast<int64_t>(keep + src) * channels];
+      acc = fmaf(wc[j], v, acc);
+    }
+    out[(s0 + li) * out_row + c] = from_float<O>(act ? acc * sigmoidf_(acc) : acc);
+  }
+  // The new saved inputs, oldest first: entry j is the input n - keep + j of the item, or a saved one
+  // further back. Ascending j reads saved entries at or behind the one it writes.
+  for (int j = 0; j < keep; ++j) {
+    const int src = n - keep + j;
+    saved[static_cast<int64_t>(j) * channels] =
+        src >= 0 ? to_float<A>(in[(s0 + src) * in_row + c]) : saved[static_cast<int64_t>(keep + src) * channels];
+  }
+}
+
+template <typename A, typename O>
 __global__ __launch_bounds__(256) void short_conv_kernel(
     const A* __restrict__ in, int64_t in_row, const float* __restrict__ w, const float* __restrict__ bias, O* __restrict__ out,
     int64_t out_row, float* __restrict__ state, int64_t state_row, const int32_t* __restrict__ tok_item,
@@ -68,24 +92,77 @@ __global__ __launch_bounds__(256) void short_conv_kernel(
   }
   const int item = static_cast<int>(blockIdx.x) - tokens;
   const int64_t s0 = item_start[item];
-  const int n = static_cast<int>(item_start[item + 1] - s0);
-  float* saved = state + static_cast<int64_t>(slots[item]) * state_row + c;      // saved[j * channels]: oldest first
-  const int first = min(n, keep);
-  for (int li = 0; li < first; ++li) {
-    float acc = b;
-    for (int j = 0; j < taps; ++j) {
-      const int src = li - keep + j;
-      const float v = src >= 0 ? to_float<A>(in[(s0 + src) * in_row + c]) : saved[static_cast<int64_t>(keep + src) * channels];
-      acc = fmaf(wc[j], v, acc);
-    }
-    out[(s0 + li) * out_row + c] = from_float<O>(act ? acc * sigmoidf_(acc) : acc);
+  short_conv_item<A, O>(in, in_row, wc, b, out, out_row, state + static_cast<int64_t>(slots[item]) * state_row + c, s0,
+                        static_cast<int>(item_start[item + 1] - s0), c, channels, taps, act);   // saved[j * channels]: oldest first
+}
+
+// The same for four taps and operands that lie on four channels: grid (ceil(tokens / 4) + items, ceil(channels / 256)). A thread
+// makes four channels of four tokens from seven rows, each read once in one load, in the same order of sums. A thread per token and
+// channel read every row four times, two bytes a lane: 2,048 tokens of 4,096 bfloat16 channels to float32 45.9 -> 15.1 us (3.3
+// TB/s), 512 tokens beside 23 requests 15.4 -> 7.3, a token for each of 64 requests 5.5 -> 3.8.
+constexpr int kConvTokens = 4;
+
+template <typename T> struct Four;
+template <> struct Four<float> { typedef float4 type; };
+template <> struct Four<bf16_t> { typedef ushort4 type; };
+
+template <typename A, typename O>
+__global__ __launch_bounds__(256) void short_conv4_kernel(
+    const A* __restrict__ in, int64_t in_row, const float* __restrict__ w, const float* __restrict__ bias, O* __restrict__ out,
+    int64_t out_row, float* __restrict__ state, int64_t state_row, const int32_t* __restrict__ tok_item,
+    const int32_t* __restrict__ item_start, const int32_t* __restrict__ slots, int tokens, int channels, int act) {
+  const int groups = (tokens + kConvTokens - 1) / kConvTokens;
+  if (static_cast<int>(blockIdx.x) >= groups) {
+    const int c = blockIdx.y * 256 + threadIdx.x, item = static_cast<int>(blockIdx.x) - groups;
+    if (c >= channels) return;
+    const int64_t s0 = item_start[item];
+    short_conv_item<A, O>(in, in_row, w + 4LL * c, bias != nullptr ? bias[c] : 0.f, out, out_row,
+                          state + static_cast<int64_t>(slots[item]) * state_row + c, s0, static_cast<int>(item_start[item + 1] - s0),
+                          c, channels, 4, act);
+    return;
   }
-  // The new saved inputs, oldest first: entry j is the input n - keep + j of the item, or a saved one
-  // further back. Ascending j reads saved entries at or behind the one it writes.
-  for (int j = 0; j < keep; ++j) {
-    const int src = n - keep + j;
-    saved[static_cast<int64_t>(j) * channels] =
-        src >= 0 ? to_float<A>(in[(s0 + src) * in_row + c]) : saved[static_cast<int64_t>(keep + src) * channels];
+  const int c = (blockIdx.y * 256 + threadIdx.x) * 4;
+  if (c >= channels) return;                                   // whole blocks from a quarter of the grid on
+  const int t0 = static_cast<int>(blockIdx.x) * kConvTokens;
+  float v[kConvTokens + 3][4];
+#pragma unroll
+  for (int i = 0; i < kConvTokens + 3; ++i) {                  // rows in front of the step or behind it are nobody's to use
+    const int64_t t = min(max(t0 - 3 + i, 0), tokens - 1);
+    const typename Four<A>::type q = *reinterpret_cast<const typename Four<A>::type*>(in + t * in_row + c);
+    v[i][0] = to_float<A>(q.x);
+    v[i][1] = to_float<A>(q.y);
+    v[i][2] = to_float<A>(q.z);
+    v[i][3] = to_float<A>(q.w);
+  }
+  float wc[4][4], b[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float4 q = *reinterpret_cast<const float4*>(w + 4LL * (c + e));
+    wc[e][0] = q.x;
+    wc[e][1] = q.y;
+    wc[e][2] = q.z;
+    wc[e][3] = q.w;
+    b[e] = bias != nullptr ? bias[c + e] : 0.f;
+  }
+#pragma unroll
+  for (int i = 0; i < kConvTokens; ++i) {
+    const int t = t0 + i;
+    if (t >= tokens) return;
+    if (t - item_start[tok_item[t]] < 3) continue;
+    float r[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float acc = b[e];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc = fmaf(wc[e][j], v[i + j][e], acc);
+      r[e] = act ? acc * sigmoidf_(acc) : acc;
+    }
+    typename Four<O>::type q;
+    q.x = from_float<O>(r[0]);
+    q.y = from_float<O>(r[1]);
+    q.z = from_float<O>(r[2]);
+    q.w = from_float<O>(r[3]);
+    *reinterpret_cast<typename Four<O>::type*>(out + static_cast<int64_t>(t) * out_row + c) = q;
   }
 }
 
@@ -456,15 +533,31 @@ int psamd_short_conv_to(void* stream, const void* in, int in_dtype, int64_t in_r
                 "input and output are float32 or bfloat16");
   if (tokens == 0) return 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid(static_cast<unsigned>(tokens + items), static_cast<unsigned>(ceil_div(channels, 256)));
+  const unsigned parts = static_cast<unsigned>(ceil_div(channels, 256));
+  const dim3 grid(static_cast<unsigned>(tokens + items), parts);
+  const int64_t in_size = in_dtype == kBF16 ? 2 : 4, out_size = out_dtype == kBF16 ? 2 : 4;
+  const bool fours = taps == 4 && channels % 4 == 0 && in_row % 4 == 0 && out_row % 4 == 0 &&
+                     reinterpret_cast<uintptr_t>(in) % (4 * in_size) == 0 && reinterpret_cast<uintptr_t>(out) % (4 * out_size) == 0 &&
+                     reinterpret_cast<uintptr_t>(taps_w) % 16 == 0;
+  const dim3 grid4(static_cast<unsigned>(ceil_div(tokens, kConvTokens) + items), parts);
 #define PSAMD_CONV(A_, O_)                                                                                              \
+  if (fours)                                                                                                            \
+    short_conv4_kernel<A_, O_><<<grid4, dim3(256), 0, s>>>(static_cast<const A_*>(in), in_row, taps_w, bias,            \
+                                                           static_cast<O_*>(out), out_row, state, state_row, tok_item,  \
+                                                           item_start, slots, static_cast<int>(tokens), channels, act); \
+  else                                                                                              \
   short_conv_kernel<A_, O_><<<grid, dim3(256), 0, s>>>(static_cast<const A_*>(in), in_row, taps_w, bias,               \
                                                        static_cast<O_*>(out), out_row, state, state_row, tok_item,     \
                                                        item_start, slots, static_cast<int>(tokens), channels, taps, act)
-  if (in_dtype == kBF16 && out_dtype == kF32) PSAMD_CONV(bf16_t, float);
-  else if (in_dtype == kF32 && out_dtype == kF32) PSAMD_CONV(float, float);
-  else if (in_dtype == kF32 && out_dtype == kBF16) PSAMD_CONV(float, bf16_t);
-  else PSAMD_CONV(bf16_t, bf16_t);
+  if (in_dtype == kBF16 && out_dtype == kF32) {
+    PSAMD_CONV(bf16_t, float);
+  } else if (in_dtype == kF32 && out_dtype == kF32) {
+    PSAMD_CONV(float, float);
+  } else if (in_dtype == kF32 && out_dtype == kBF16) {
+    PSAMD_CONV(float, bf16_t);
+  } else {
+    PSAMD_CONV(bf16_t, bf16_t);
+  }
 #undef PSAMD_CONV
   return check_launch("psamd_short_conv");
 }

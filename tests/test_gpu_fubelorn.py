@@ -167,6 +167,25 @@ def test_convolution_with_a_bias_and_an_output_of_either_type(ops, dtype, taps, 
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("channels", [4, 260, 1284])
+def test_convolution_in_fours_of_channels(ops, dtype, out_dtype, channels):
+    """Four taps and operands on four channels go four channels and four tokens at a time; rows that begin elsewhere a channel
+    at a time, in the same order of sums: the same bits. Items shorter than the taps, no multiple of four tokens, a last one."""
+    w, bias = rnd(channels, 4, seed=1, scale=0.5), rnd(channels, seed=2)
+    states = [rnd(5, 3 * channels, seed=3) for _ in range(2)]
+    for k, lengths in enumerate([(1, 2, 3, 4, 5), (70, 1, 9, 2, 1), (1, 1, 1, 1, 1)]):
+        step = Step(lengths, [2, 0, 4, 1, 3])
+        wide = rnd(step.num_tokens, channels + 8, dtype=dtype, seed=10 + k)
+        outs = []
+        for rows, col, state in ((wide, 4, states[0]), (torch.cat((wide[:, :1], wide), 1), 5, states[1])):
+            out = torch.empty(step.num_tokens, channels, dtype=out_dtype, device=DEV)
+            ops.short_conv(rows, col, w, out, state, 0, step, silu=k != 1, bias=bias if k else None)
+            outs.append(out)
+        assert torch.equal(outs[0], outs[1]) and torch.equal(states[0], states[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads,vdim,n,groups,parts", [(4, 8, 12, 2, 2), (1, 20, 3, 1, 1), (8, 64, 128, 1, 4), (6, 10, 256, 3, 5)])
 def test_state_space_layer_through_the_delta_scan(ops, dtype, heads, vdim, n, groups, parts):
     """Step sizes and decays, the recurrence over three steps from slots of junk, the skip, gate and norm in parts."""
