@@ -157,7 +157,7 @@ class HipOps:
     MOE_ROUTE_FUSED_MAX_TOKENS = 0   # up to here one kernel computes router logits and choice; above, product + choice
     MOE_CHOICE_SORTS_MAX_TOKENS = 16 # up to here the workgroup that chooses a step's experts also sorts the pairs
     MOE_PAIRWISE_MAX_TOKENS = 2     # up to here a bfloat16 step's experts run pair by pair; above, grouped by expert
-    DELTA_RUNS_MIN_TOKENS = 48      # from this prompt length on a recurrence runs in runs of 64 tokens (where the caller allows it)
+    DELTA_RUNS_MIN_TOKENS = 425     # from this length on a lone prompt's recurrence goes in runs of 64 tokens (where the caller allows it)
     DELTA_RUNS_MAX_BYTES = 2 << 30  # scratch that the runs of one step may take; a step with more is walked token by token
     MFMA_ATTENTION_EXTRAS = True    # whether the matrix-core attention takes a sink and a bias by distance
     name = "hip"
@@ -1272,14 +1272,17 @@ class HipOps:
             state.data_ptr() + 4 * state_offset, state.shape[1], ctx.item_start.data_ptr(), ctx.slots.data_ptr())
         most = 0
         if in_runs and ctx.num_prefill_blocks:
-            # A prompt of under DELTA_RUNS_MIN_TOKENS is walked in the time the three launches of the runs take.
+            # The walk takes 0.19 us for every token of the longest item, the runs 55 us and 0.06 (general rule: 0.09) for every
+            # token of the step: one item of 256 tokens 54 us against 78 (gated; general 53 and 63), of 512 102 against 91 (101
+            # and 76), of 2,048 391 against 182 (393 and 193); two of 1,024 200 against 140, four of 1,024 253 against 277, four
+            # of 512 133 against 141, one of 1,024 beside sixteen of 64 331 against 218.
             longest = int(np.diff(ctx.host["item_start"]).max())
             same = keys[1] == directions[1] == removals[1] and decay_vectors is None and reads_decayed
             form = (1 if no_removal else 0) if same else 2
             fits = same or (not reads_decayed and decay_vectors is not None and decay is None and removal_scale is None
                             and value_scale is None and key_groups == heads)
             floats = int(self.lib.psamd_delta_runs_floats(ctx.num_prefill_blocks, heads, dim, vdim, int(form == 2)))
-            if (longest >= self.DELTA_RUNS_MIN_TOKENS and fits and 4 * floats <= self.DELTA_RUNS_MAX_BYTES
+            if (3 * longest >= t + 2 * self.DELTA_RUNS_MIN_TOKENS and fits and 4 * floats <= self.DELTA_RUNS_MAX_BYTES
                     and all(p % 16 == 0 for p in (at(keys), at(directions), at(removals), at(queries), out.data_ptr(), operands[17]))
                     and self.lib.psamd_delta_runs_supports(dim, vdim, base.shape[1], xv.shape[1], out.shape[1], operands[8],
                                                            state.shape[1], int(form == 2), float(decay_least))):

@@ -542,7 +542,7 @@ def test_random_configurations_in_both_dtypes(seed, tmp_path):
 
 @pytest.mark.parametrize("form,heads,groups,dim,vdim", [("gated", 4, 2, 128, 128), ("gated", 2, 2, 64, 48), ("plain", 6, 1, 128, 64),
                                                         ("plain", 2, 2, 64, 16), ("general", 3, 3, 64, 64), ("general", 2, 2, 128, 32)])
-def test_recurrences_in_runs_of_64_tokens(ops, form, heads, groups, dim, vdim):
+def test_recurrences_in_runs_of_64_tokens(ops, monkeypatch, form, heads, groups, dim, vdim):
     """Items shorter than, as long as and longer than one and two runs, single tokens among them (they are walked), each from
     a state of its own, run by run and token by token against float64. Keys that repeat (the systems to solve are then full),
     decays of zero (gated, plain) and decays at their floor (general) included. The sums differ in order alone: the runs may be as
@@ -597,6 +597,7 @@ def test_recurrences_in_runs_of_64_tokens(ops, form, heads, groups, dim, vdim):
         want_state[15 - i, 4:] = s.reshape(-1)
         at += n
     off = {}
+    monkeypatch.setattr(ops, "DELTA_RUNS_MIN_TOKENS", -t)   # these items are too short for the runs to pay
     for runs in (False, True):
         st, out = state.clone(), torch.full((t + 1, heads * vdim), 7.0, device=DEV)
         ops.delta_scan(values=(xflat, 0), out=out[:t], state=st, in_runs=runs, **args)
