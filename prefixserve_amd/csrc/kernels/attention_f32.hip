@@ -69,6 +69,7 @@ __global__ __launch_bounds__(64 * kAttnWaves) void attention_f32_kernel(Attentio
   const int64_t t = c.item_start[item] + q0 + qi;
   const int first_pos = c.item_pos0[item] + q0, last_pos = first_pos + nq - 1, pos = first_pos + qi;
   const int lo = c.window > 0 ? pos - c.window + 1 : 0;                // this column's first key (may be negative)
+  const int last_lo = c.window > 0 ? last_pos - c.window + 1 : 0;      // the last column's
   const int32_t* table = c.block_ids + c.table_off[item];
   const int64_t page_elems = 2LL * c.hkv * kPage * D, half_elems = static_cast<int64_t>(c.hkv) * kPage * D;
   const float* kv = c.kv + static_cast<int64_t>(kvh) * kPage * D;
@@ -135,6 +136,7 @@ __global__ __launch_bounds__(64 * kAttnWaves) void attention_f32_kernel(Attentio
       f32x4 acc[DT];
 #pragma unroll
       for (int d = 0; d < DT; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+      unsigned odd = 0;                                                // pages whose values are not all finite (the same in all lanes)
 #pragma unroll
       for (int i0 = 0; i0 < kRunPages; i0 += 4) {
         f32x4 chain[DT];
@@ -144,20 +146,60 @@ __global__ __launch_bounds__(64 * kAttnWaves) void attention_f32_kernel(Attentio
         for (int i = i0; i < i0 + 4; ++i) {
           const int p = run * kRunPages + i;
           if (p < p_begin || p >= p_end) continue;
-          const float* vr = kv + table[p] * page_elems + half_elems + r * kPage + 4 * g;
+          const float* vp = kv + table[p] * page_elems + half_elems;
+          const float* vr = vp + r * kPage + 4 * g;
           const int key0 = p * kPage + 4 * g;
+          f32x4 val[DT];
 #pragma unroll
           for (int d = 0; d < DT; ++d) {
-            f32x4 val = *reinterpret_cast<const f32x4*>(vr + d * 16 * kPage);
+            val[d] = *reinterpret_cast<const f32x4*>(vr + d * 16 * kPage);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const float y = key0 + j <= last_pos ? val[j] : 0.f;     // what lies behind the last position is nobody's
-              chain[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(y, s[i][j], chain[d], 0, 0, 0);
+            for (int j = 0; j < 4; ++j) val[d][j] = key0 + j <= last_pos ? val[d][j] : 0.f;   // what lies behind the last position is nobody's
+          }
+          // Where some column does not see all of the page's keys: a weight of zero does not hide a value that is not finite.
+          if (p * kPage + kPage - 1 > first_pos || p * kPage < last_lo) {
+            float zeros = 0.f;
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) zeros = fmaf(val[d][j], 0.f, zeros);
+            if (__any(zeros != 0.f)) {
+              odd |= 1u << i;
+#pragma unroll
+              for (int d = 0; d < DT; ++d)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) val[d][j] = fabsf(val[d][j]) < INFINITY ? val[d][j] : 0.f;
             }
           }
+#pragma unroll
+          for (int d = 0; d < DT; ++d)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) chain[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(val[d][j], s[i][j], chain[d], 0, 0, 0);
         }
 #pragma unroll
         for (int d = 0; d < DT; ++d) acc[d] += chain[d];
+      }
+      // What was left out is added for the columns that see its key; the others keep their bits.
+      for (; odd != 0; odd &= odd - 1) {
+        const int i = __builtin_ctz(odd), p = run * kRunPages + i;
+        f32x4 weights = s[0];
+#pragma unroll
+        for (int k = 1; k < kRunPages; ++k) weights = i == k ? s[k] : weights;
+        const float* vp = kv + table[p] * page_elems + half_elems + 4 * g * kPage;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          for (int src = 0; src < 4; ++src) {                          // the lanes of group src hold key 4 src + j
+            const float weight = __shfl(weights[j], 16 * src + r, kWave);
+            const int at = 4 * src + j, key = p * kPage + at;
+            if (key > pos || key < lo) continue;
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+              for (int v = 0; v < 4; ++v) {
+                const float y = vp[(16 * d + v) * kPage + at];
+                if (!(fabsf(y) < INFINITY)) acc[d][v] += weight * y;
+              }
+          }
       }
 #pragma unroll
       for (int d = 0; d < DT; ++d) acc_s[wave][d][lane] = acc[d];

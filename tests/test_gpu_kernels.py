@@ -1219,3 +1219,40 @@ def test_experts_with_many_pairs_each(ops, counts, k, f, kind, on_output, identi
     out = torch.full((1, t + 1, k), 7.0, device=DEV)
     ops.moe_experts(x, chosen, weight, w_in, down, act, out[:, :t], 1.702, 5.0, 1.0, weight_on_output=on_output, kind=kind, identity=identity)
     assert rel(out[0, :t], want) < 3e-3 and torch.all(out[0, t] == 7.0)
+
+
+@pytest.mark.parametrize("hq,hkv,d,window", [(8, 2, 64, None), (16, 1, 16, None), (8, 4, 32, 130), (4, 4, 128, 33), (8, 1, 64, 16)])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+def test_float32_attention_of_values_that_are_not_finite(ops, hq, hkv, d, window, bad):
+    """A value that is not finite reaches its own dimension of the queries that see its key, and nothing else: not the queries in
+    front of it in its tile, nor those whose window it has left. Every other output keeps its bits, in a whole prompt and in a
+    portion whose tile begins in front of the key and ends behind it."""
+    n, blocks, kvh, dim = 300, 24, hkv - 1, d - 3
+    table = np.random.default_rng(d).permutation(blocks).tolist()[: -(-n // 16)]
+    pk = StepPacker(torch.device(DEV), [GroupMeta(blocks, window)], 10, 100000, 8, ops.PREFILL_TILE_Q, skew_rule=ops.decode_is_skewed)
+    qkv = rnd(n, (hq + 2 * hkv) * d, seed=d)
+    pages, off = torch.tensor(table, device=DEV)[torch.arange(n, device=DEV) // 16], torch.arange(n, device=DEV) % 16
+    kv = torch.zeros(blocks, 2, hkv, 16 * d, device=DEV)
+    kv[:, 0].view(blocks, hkv, 16, d)[pages, :, off, :] = qkv[:, hq * d: (hq + hkv) * d].reshape(n, hkv, d)
+    values = kv[:, 1].view(blocks, hkv, d, 16)
+    values[pages, :, :, off] = qkv[:, (hq + hkv) * d:].reshape(n, hkv, d)
+
+    def run(first, count):
+        out = torch.empty(count, hq, d, device=DEV)
+        ctx = pk.pack([StepItem(0, [1] * count, first, [table])])
+        ops.paged_attention(qkv[first: first + count].contiguous(), out.view(count, hq * d), kv, ctx, 0, hq, hkv, d, d ** -0.5, window)
+        return out
+
+    clean = run(0, n)
+    heads = slice(kvh * hq // hkv, (kvh + 1) * hq // hkv)
+    for at in (0, 5, 31, 127, 130, 299):
+        kept = values[table[at // 16], kvh, dim, at % 16].clone()
+        values[table[at // 16], kvh, dim, at % 16] = bad
+        hit = torch.zeros(n, hq, d, dtype=torch.bool, device=DEV)
+        hit[at: min(n, at + window) if window else n, heads, dim] = True
+        portion = max(0, at - 5)
+        for first, got in ((0, run(0, n)), (portion, run(portion, min(n - portion, 40)))):
+            h = hit[first: first + len(got)]
+            assert not torch.isfinite(got[h]).any(), f"key {at}: a query that sees it has a finite output"
+            assert torch.equal(got[~h], clean[first: first + len(got)][~h]), f"key {at}: it reached a query that does not see it"
+        values[table[at // 16], kvh, dim, at % 16] = kept
