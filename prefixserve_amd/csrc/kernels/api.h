@@ -339,10 +339,10 @@ int psamd_attention_generic(void* stream, const void* qkv, int q_stride, void* o
                             float scale, int window, const float* sink, const float* dist_bias, int n_dist,
                             const void* gate, int64_t gate_row);
 
-// The same on the float32 matrix instructions, from the step's lists of tiles of 32 queries and of single tokens.
+// The same on the float32 matrix instructions, from the step's lists of tiles of tile_queries queries and of single tokens.
 int psamd_attention_f32_supports(int hq, int hkv, int head_dim, int q_stride);
 int psamd_attention_f32(void* stream, const float* qkv, int q_stride, float* out, const float* kv, const int32_t* pf_tiles,
-                        int n_pf, const int32_t* dec_items, int n_dec, const int32_t* item_start, const int32_t* item_pos0,
+                        int n_pf, int tile_queries, const int32_t* dec_items, int n_dec, const int32_t* item_start, const int32_t* item_pos0,
                         const int32_t* table_off, const int32_t* block_ids, int hq, int hkv, int head_dim, float scale,
                         int window, const float* sink, const float* dist_bias, int n_dist, const float* gate, int64_t gate_row);
 

@@ -5,10 +5,13 @@
 // A tile is 16 columns: 16 / G queries of one request for all G query heads of one kv head, so that a key is read once
 // for the group. Keys are taken in runs of kRun positions counted from position 0; a run gives (maximum, sum, weighted
 // values) on its own, and the runs are merged in ascending order. A run that lies outside a query's keys leaves its sums as they
-// are, so a query's result is the same bit for bit whichever queries share its tile and however its sequence was cut.
+// are, so a query's result is the same bit for bit whichever queries share its tile and however its sequence was cut. So does
+// a value that is not finite behind a query or in front of its window, which a weight of zero would not hide: in pages that some
+// query of the tile does not see whole such values are added on their own.
 //
 // Bound by the matrix instructions (1,024 cycles of them per 16 columns and page at a head size of 64 against 8 KB read).
-// 600 tokens x 32 heads of 64 on 8: 820 us (one wave per token and head, every key read four times over) -> 54.
+// 600 tokens x 32 heads of 64 on 8: 820 us (one wave per token and head, every key read four times over) -> 53, of 128 1,655 -> 99
+// (110 with a page's values asked for 16 dimensions at a time).
 
 #include "api.h"
 #include "common.h"
@@ -19,7 +22,6 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 constexpr int kRunPages = 8, kRun = kRunPages * kPage;   // keys per run
 constexpr int kAttnWaves = 4;
-constexpr int kTileQueries = 32;                         // queries of a tile of the step's list
 
 struct AttentionF32 {
   const float* qkv;
@@ -263,7 +265,7 @@ int psamd_attention_f32_supports(int hq, int hkv, int head_dim, int q_stride) {
 }
 
 int psamd_attention_f32(void* stream, const float* qkv, int q_stride, float* out, const float* kv, const int32_t* pf_tiles,
-                        int n_pf, const int32_t* dec_items, int n_dec, const int32_t* item_start, const int32_t* item_pos0,
+                        int n_pf, int tile_queries, const int32_t* dec_items, int n_dec, const int32_t* item_start, const int32_t* item_pos0,
                         const int32_t* table_off, const int32_t* block_ids, int hq, int hkv, int head_dim, float scale,
                         int window, const float* sink, const float* dist_bias, int n_dist, const float* gate, int64_t gate_row) {
   PSAMD_REQUIRE(psamd_attention_f32_supports(hq, hkv, head_dim, q_stride), "unsupported head counts or head size");
@@ -273,7 +275,9 @@ int psamd_attention_f32(void* stream, const float* qkv, int q_stride, float* out
   PSAMD_REQUIRE(dist_bias == nullptr || n_dist >= 1, "a distance bias needs at least one entry per head");
   PSAMD_REQUIRE(gate == nullptr || gate_row >= static_cast<int64_t>(hq) * head_dim, "the gate's rows");
   if (n_pf + n_dec == 0) return 0;
-  const int subs = kTileQueries / (16 / (hq / hkv));
+  const int per_tile = 16 / (hq / hkv);
+  PSAMD_REQUIRE(tile_queries >= 1 && tile_queries % per_tile == 0, "the list's tiles must be whole tiles of 16 columns");
+  const int subs = tile_queries / per_tile;
   PSAMD_REQUIRE(static_cast<int64_t>(n_pf) * subs + n_dec <= 2147483647LL, "too many tiles for one launch");
   const AttentionF32 c{qkv, q_stride, out, kv, pf_tiles, n_pf, subs, dec_items, item_start, item_pos0, table_off, block_ids,
                        hq, hkv, scale, window, sink, dist_bias, n_dist, gate, gate_row};

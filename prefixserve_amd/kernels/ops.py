@@ -62,7 +62,7 @@ _SIGNATURES = {
     "psamd_attention_generic": [_vp, _vp, _i32, _vp, _vp, _i32, _i64, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _f32, _i32,
                                 _vp, _vp, _i32, _vp, _i64],
     "psamd_attention_f32_supports": [_i32, _i32, _i32, _i32],
-    "psamd_attention_f32": [_vp, _vp, _i32, _vp, _vp, _vp, _i32, _vp, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _f32, _i32,
+    "psamd_attention_f32": [_vp, _vp, _i32, _vp, _vp, _vp, _i32, _i32, _vp, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _f32, _i32,
                             _vp, _vp, _i32, _vp, _i64],
     "psamd_attention_mfma_supports": [_i32, _i32, _i32],
     "psamd_attention_prefill_nsplit": [_i32, _i32, _i32, _i32, _i32],
@@ -1450,7 +1450,7 @@ class HipOps:
                 and self.lib.psamd_attention_f32_supports(hq, hkv, d, stride)):
             self._ok(self.lib.psamd_attention_f32(
                 s, qkv.data_ptr(), stride, out.data_ptr(), kv.data_ptr(), ctx.pf_tiles.data_ptr(), ctx.num_prefill_tiles,
-                ctx.dec_items.data_ptr(), ctx.num_decode, ctx.item_start.data_ptr(), ctx.item_pos0.data_ptr(),
+                self.PREFILL_TILE_Q, ctx.dec_items.data_ptr(), ctx.num_decode, ctx.item_start.data_ptr(), ctx.item_pos0.data_ptr(),
                 g.table_off.data_ptr(), g.block_ids.data_ptr(), hq, hkv, d, scale, win,
                 _ptr(sink), _ptr(dist_bias), 0 if dist_bias is None else dist_bias.shape[1], *gate))
             return

@@ -1256,3 +1256,12 @@ def test_float32_attention_of_values_that_are_not_finite(ops, hq, hkv, d, window
             assert not torch.isfinite(got[h]).any(), f"key {at}: a query that sees it has a finite output"
             assert torch.equal(got[~h], clean[first: first + len(got)][~h]), f"key {at}: it reached a query that does not see it"
         values[table[at // 16], kvh, dim, at % 16] = kept
+
+
+@pytest.mark.parametrize("hq,hkv", [(8, 2), (4, 4), (16, 1)])
+def test_float32_attention_takes_the_tiles_the_step_was_cut_into(ops, monkeypatch, hq, hkv):
+    """A step whose lists cut its prompts into tiles of another size gives the same bits."""
+    want, _ = paged_case(ops, torch.float32, hq, hkv, 32, [100, 1, 37], [0, 50, 70], seed=3)
+    for tile in (16, 64):
+        monkeypatch.setattr(ops, "PREFILL_TILE_Q", tile)
+        assert torch.equal(paged_case(ops, torch.float32, hq, hkv, 32, [100, 1, 37], [0, 50, 70], seed=3)[0], want)
