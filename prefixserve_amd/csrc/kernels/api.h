@@ -211,18 +211,18 @@ int psamd_delta_scan(void* stream, const float* kvec, const float* cvec, const f
                      float* state, int64_t state_row, const int32_t* item_start, const int32_t* slots, int items, int heads,
                      int dim, int vdim, int reads_decayed, int most);
 
-// The same for the items of two tokens or more, in runs of 64 tokens on the float32 matrix instructions (delta_runs.hip), from
-// the step's lists of tiles of 32 tokens and of the first tiles of four. form 0: c = p = k and no dvec, reads_decayed; 1: the
-// same with pscal zero throughout; 2: dvec, no pscal and xscal, a key group per head, the removal reads the state before the
-// decay, and no decay is under decay_least.
+// The same for the items of more than `most` tokens, in runs of 64 tokens on the float32 matrix instructions (delta_runs.hip);
+// starts: item_start on the host. form 0: c = p = k and no dvec, reads_decayed; 1: the same with pscal zero throughout; 2: dvec,
+// no pscal and xscal, a key group per head, the removal reads the state before the decay, and no decay is under decay_least.
 int psamd_delta_runs_supports(int dim, int vdim, int64_t key_row, int64_t x_row, int64_t out_row, int64_t dvec_row, int64_t state_row,
                               int general, float decay_least);
-int64_t psamd_delta_runs_floats(int n_blocks, int heads, int dim, int vdim, int general);
+int psamd_delta_runs_at_once(int heads, int dim, int vdim, int general);
+int64_t psamd_delta_runs_floats(int heads, int dim, int vdim, int general);
 int psamd_delta_runs(void* stream, const float* kvec, const float* cvec, const float* pvec, const float* rvec, int64_t key_row,
                      int key_groups, const float* dvec, int64_t dvec_row, const float* dscal, const float* pscal, const float* xscal,
                      int64_t scal_row, const float* x, int64_t x_row, float* out, int64_t out_row, float* state, int64_t state_row,
-                     const int32_t* item_start, const int32_t* slots, const int32_t* pf_tiles, const int32_t* pf_blocks, int n_blocks,
-                     int items, int heads, int dim, int vdim, int form, float decay_least, float* scratch);
+                     const int32_t* starts, const int32_t* slots, int items, int most, int heads, int dim, int vdim, int form,
+                     float decay_least, float* scratch);
 // out[t, h, :] = o[t, h, :] / sqrt(mean(o^2) + eps) * weight * act(gate[t, h, :]); o float, weight float [vdim]
 // (or [heads * vdim] with weight_per_head), gate rows gate_row apart in act_dtype, act 0 = SiLU, 1 = sigmoid.
 int psamd_heads_norm_gate(void* stream, const float* o, int64_t tokens, int heads, int vdim, const float* weight,

@@ -23,6 +23,8 @@
 // Operand layout of a 16 x 16 x 4 instruction: lane (r = l % 16, g = l / 16) gives k = 4 g + i, i = 0..3, of row r and of column
 // r, and receives rows 4 g .. 4 g + 3 of column r: what it receives is the column operand of a product over those rows.
 
+#include <algorithm>
+
 #include "api.h"
 #include "common.h"
 
@@ -52,12 +54,20 @@ struct DeltaRuns {
   int64_t out_row;
   float* state;
   int64_t state_row;
-  const int32_t* item_start;
   const int32_t* slots;
-  const int32_t* pf_tiles;     // (item, first token within the item) of the step's tiles of 32
-  const int32_t* pf_blocks;    // the first tile of each four of one item
-  int n_blocks, heads, vdim;
-  float* scratch;              // [2 n_blocks][heads][run_floats]
+  int heads, vdim;
+  float* scratch;              // [kMaxRuns at most][heads][run_layout().total]
+};
+
+// The runs that one round of launches makes, in the order of their tokens, and the items that they are of. The host lists them (it
+// has the items' lengths) and hands the list over as a kernel argument.
+constexpr int kMaxRuns = 64;
+struct RunList {
+  int32_t t0[kMaxRuns];        // a run's first token of the step
+  int32_t tokens[kMaxRuns];    // how many it has
+  int32_t item[kMaxRuns];      // parts: an item, its first run of the list, how many follow each other there
+  int32_t first[kMaxRuns];
+  int32_t runs[kMaxRuns];
 };
 
 // Where a run's arrays lie in its scratch.
@@ -97,17 +107,9 @@ __device__ __forceinline__ void lds_barrier() {
 
 constexpr int kGatedForm = 0, kPlainForm = 1, kGeneralForm = 2;   // plain: the gated form with nothing taken out
 
-// Run `blockIdx.x`'s item, first token and length (0: the block has no such run).
-__device__ __forceinline__ int run_of(const DeltaRuns& c, int64_t& t0) {
-  const int tile = c.pf_blocks[blockIdx.x >> 1], item = c.pf_tiles[2 * tile];
-  const int q0 = c.pf_tiles[2 * tile + 1] + (blockIdx.x & 1) * kRunTokens;
-  t0 = c.item_start[item] + static_cast<int64_t>(q0);
-  return min(kRunTokens, c.item_start[item + 1] - c.item_start[item] - q0);
-}
-
-// grid (2 blocks, heads), four waves: wave w makes the rows of tokens 16 w .. 16 w + 15.
+// grid (runs, heads), four waves: wave w makes the rows of tokens 16 w .. 16 w + 15.
 template <int DT, int FORM>
-__global__ __launch_bounds__(256) void runs_prepare_kernel(DeltaRuns c) {
+__global__ __launch_bounds__(256) void runs_prepare_kernel(DeltaRuns c, RunList list) {
   constexpr int D = DT * 16, LD = D + 4;
   constexpr bool GENERAL = FORM == kGeneralForm, SOLVES = FORM != kPlainForm;
   extern __shared__ __align__(16) float run_smem[];
@@ -116,9 +118,8 @@ __global__ __launch_bounds__(256) void runs_prepare_kernel(DeltaRuns c) {
   float* ds = lm + kRunTokens * kLd;                     // general: D [t][dim]
   float* mx = ds + (GENERAL ? kRunTokens * LD : 0);      // general: M X, [vdim][t]
   __shared__ float num[5][kRunTokens];                   // per token: decay, D_t, D_n / D_t, ps, xs
-  int64_t t0;
-  const int n = run_of(c, t0);
-  if (n <= 0) return;                                    // uniform for the workgroup
+  const int64_t t0 = list.t0[blockIdx.x];
+  const int n = list.tokens[blockIdx.x];
   const int h = blockIdx.y, grp = h / c.heads_per_group;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
@@ -347,30 +348,22 @@ __global__ __launch_bounds__(256) void runs_prepare_kernel(DeltaRuns c) {
   for (int i = threadIdx.x; i < D; i += 256) sc[lay.dc + i] = GENERAL ? ds[(kRunTokens - 1) * LD + i] : num[1][kRunTokens - 1];
 }
 
-// grid (items, heads, vdim / 16), four waves: an item's runs in turn for 16 value channels. Wave w makes the rows of tokens
+// grid (parts, heads, vdim / 16), four waves: an item's runs in turn for 16 value channels, from the state in its slot, which is
+// left as it is behind them (the item's next runs, in another round of launches, begin there). Wave w makes the rows of tokens
 // 16 w .. of W and keeps the state's key channels 16 (w + 4 o) .. in registers.
 template <int DT, int FORM>
-__global__ __launch_bounds__(256, 1) void runs_chain_kernel(DeltaRuns c) {
+__global__ __launch_bounds__(256, 1) void runs_chain_kernel(DeltaRuns c, RunList list) {
   constexpr int D = DT * 16, LD = D + 4, OWN = (DT + 3) / 4;
   constexpr bool GENERAL = FORM == kGeneralForm, SOLVES = FORM != kPlainForm;
   __shared__ __align__(16) float st_s[16 * LD];          // the state, [value channel][key channel]
   __shared__ f32x4 w_s[kRunTiles][64];
-  __shared__ int first_s;
-  const int item = blockIdx.x, h = blockIdx.y, j0 = blockIdx.z * 16;
-  const int n = c.item_start[item + 1] - c.item_start[item];
-  if (n < 2) return;                                     // single tokens are not in the list of tiles
-  if (threadIdx.x == 0) first_s = c.n_blocks;
-  __syncthreads();
-  for (int b = threadIdx.x; b < c.n_blocks; b += 256)
-    if (c.pf_tiles[2 * c.pf_blocks[b]] == item) atomicMin(&first_s, b);
-  __syncthreads();
-  const int first = first_s, runs = (n + kRunTokens - 1) / kRunTokens;
-  if (first >= c.n_blocks) return;
+  const int item = list.item[blockIdx.x], first = list.first[blockIdx.x], runs = list.runs[blockIdx.x];
+  const int h = blockIdx.y, j0 = blockIdx.z * 16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
   const RunLayout lay = run_layout(D, c.vdim, GENERAL);
   const int64_t run_stride = static_cast<int64_t>(c.heads) * lay.total;
-  float* sc = c.scratch + (static_cast<int64_t>(2 * first) * c.heads + h) * lay.total;
+  float* sc = c.scratch + (static_cast<int64_t>(first) * c.heads + h) * lay.total;
   float* st = c.state + static_cast<int64_t>(c.slots[item]) * c.state_row + (static_cast<int64_t>(h) * c.vdim + j0 + r) * D + 4 * g;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   f32x4 s[OWN];
@@ -450,13 +443,13 @@ __global__ __launch_bounds__(256, 1) void runs_chain_kernel(DeltaRuns c) {
   }
 }
 
-// grid (2 blocks, heads), four waves: out = Qd S0 + P W (+ Y), rows of values, column t.
+// grid (runs, heads), four waves: out = Qd S0 + P W (+ Y), rows of values, column t.
 template <int DT, int FORM>
-__global__ __launch_bounds__(256) void runs_output_kernel(DeltaRuns c) {
+__global__ __launch_bounds__(256) void runs_output_kernel(DeltaRuns c, RunList list) {
   constexpr int D = DT * 16;
   constexpr bool GENERAL = FORM == kGeneralForm;
-  int64_t t0;
-  const int n = run_of(c, t0);
+  const int64_t t0 = list.t0[blockIdx.x];
+  const int n = list.tokens[blockIdx.x];
   const int h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4, t = 16 * wave + r;
   if (16 * wave >= n) return;                            // no barrier below
@@ -488,22 +481,28 @@ __global__ __launch_bounds__(256) void runs_output_kernel(DeltaRuns c) {
 }
 
 template <int DT, int FORM>
-static int launch_runs(hipStream_t s, const DeltaRuns& c, int items) {
+static int launch_runs(hipStream_t s, const DeltaRuns& c, const RunList& list, int n_runs, int n_parts) {
   constexpr int D = DT * 16;
   constexpr bool GENERAL = FORM == kGeneralForm;
-  const dim3 all(static_cast<unsigned>(2 * c.n_blocks), static_cast<unsigned>(c.heads));
+  const dim3 all(static_cast<unsigned>(n_runs), static_cast<unsigned>(c.heads));
   const size_t smem = sizeof(float) * (2 * kRunTokens * kLd + (GENERAL ? kRunTokens * (D + 4) + c.vdim * kLd : 0));
   auto prepare = runs_prepare_kernel<DT, FORM>;
   if (smem > 60 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(prepare), hipFuncAttributeMaxDynamicSharedMemorySize,
                                               static_cast<int>(smem)) != hipSuccess)
     return fail("psamd_delta_runs: " + std::to_string(smem) + " bytes of LDS were refused");
-  prepare<<<all, dim3(256), smem, s>>>(c);
+  prepare<<<all, dim3(256), smem, s>>>(c, list);
   if (check_launch("psamd_delta_runs (prepare)")) return 1;
-  runs_chain_kernel<DT, FORM><<<dim3(static_cast<unsigned>(items), static_cast<unsigned>(c.heads), static_cast<unsigned>(c.vdim / 16)),
-                                dim3(256), 0, s>>>(c);
+  runs_chain_kernel<DT, FORM><<<dim3(static_cast<unsigned>(n_parts), static_cast<unsigned>(c.heads), static_cast<unsigned>(c.vdim / 16)),
+                                dim3(256), 0, s>>>(c, list);
   if (check_launch("psamd_delta_runs (chain)")) return 1;
-  runs_output_kernel<DT, FORM><<<all, dim3(256), 0, s>>>(c);
+  runs_output_kernel<DT, FORM><<<all, dim3(256), 0, s>>>(c, list);
   return check_launch("psamd_delta_runs (output)");
+}
+
+static int launch_runs_form(hipStream_t s, const DeltaRuns& c, const RunList& list, int n_runs, int n_parts, int dim, int form) {
+  if (form == kGatedForm) return dim == 64 ? launch_runs<4, kGatedForm>(s, c, list, n_runs, n_parts) : launch_runs<8, kGatedForm>(s, c, list, n_runs, n_parts);
+  if (form == kPlainForm) return dim == 64 ? launch_runs<4, kPlainForm>(s, c, list, n_runs, n_parts) : launch_runs<8, kPlainForm>(s, c, list, n_runs, n_parts);
+  return dim == 64 ? launch_runs<4, kGeneralForm>(s, c, list, n_runs, n_parts) : launch_runs<8, kGeneralForm>(s, c, list, n_runs, n_parts);
 }
 
 }  // namespace psamd
@@ -523,35 +522,62 @@ int psamd_delta_runs_supports(int dim, int vdim, int64_t key_row, int64_t x_row,
   return 1;
 }
 
-// Scratch floats for a step of n_blocks blocks of 128 tokens.
-int64_t psamd_delta_runs_floats(int n_blocks, int heads, int dim, int vdim, int general) {
-  return static_cast<int64_t>(2) * n_blocks * heads * run_layout(dim, vdim, general != 0).total;
+// How many runs of a recurrence of this shape the scratch holds at a time, and its floats. Both follow from the shape alone: the
+// scratch is at most 128 MiB whatever a step holds (a step with more runs makes them in several rounds of launches), so that it
+// never grows once a first prompt has been run. 39 runs of 16 heads of 128 x 128, 64 of 32 heads of 64 x 64.
+int psamd_delta_runs_at_once(int heads, int dim, int vdim, int general) {
+  const int64_t run = sizeof(float) * static_cast<int64_t>(heads) * run_layout(dim, vdim, general != 0).total;
+  return static_cast<int>(std::min<int64_t>(kMaxRuns, (128LL << 20) / run));
+}
+int64_t psamd_delta_runs_floats(int heads, int dim, int vdim, int general) {
+  return static_cast<int64_t>(psamd_delta_runs_at_once(heads, dim, vdim, general)) * heads * run_layout(dim, vdim, general != 0).total;
 }
 
+// starts: item_start on the host. Items of `most` tokens or fewer are left out.
 int psamd_delta_runs(void* stream, const float* kvec, const float* cvec, const float* pvec, const float* rvec, int64_t key_row,
                      int key_groups, const float* dvec, int64_t dvec_row, const float* dscal, const float* pscal, const float* xscal,
                      int64_t scal_row, const float* x, int64_t x_row, float* out, int64_t out_row, float* state, int64_t state_row,
-                     const int32_t* item_start, const int32_t* slots, const int32_t* pf_tiles, const int32_t* pf_blocks, int n_blocks,
-                     int items, int heads, int dim, int vdim, int form, float decay_least, float* scratch) {
+                     const int32_t* starts, const int32_t* slots, int items, int most, int heads, int dim, int vdim, int form,
+                     float decay_least, float* scratch) {
   PSAMD_REQUIRE(form == kGatedForm || form == kPlainForm || form == kGeneralForm, "form: gated, plain or general");
-  PSAMD_REQUIRE(items >= 0 && n_blocks >= 0 && heads > 0 && key_groups > 0 && heads % key_groups == 0, "bad sizes");
+  PSAMD_REQUIRE(items >= 0 && most >= 0 && heads > 0 && key_groups > 0 && heads % key_groups == 0, "bad sizes");
   const bool general = form == kGeneralForm;
   PSAMD_REQUIRE(psamd_delta_runs_supports(dim, vdim, key_row, x_row, out_row, dvec_row, state_row, general ? 1 : 0, decay_least), "unsupported shape");
   PSAMD_REQUIRE(general ? (dvec != nullptr && dscal == nullptr && pscal == nullptr && xscal == nullptr && key_groups == heads)
                         : (cvec == kvec && pvec == kvec && dvec == nullptr), "operands of another form");
-  PSAMD_REQUIRE(kvec && cvec && pvec && rvec && x && out && state && scratch, "missing operands");
+  PSAMD_REQUIRE(kvec && cvec && pvec && rvec && x && out && state && starts && slots && scratch, "missing operands");
   const uintptr_t bits = reinterpret_cast<uintptr_t>(kvec) | reinterpret_cast<uintptr_t>(cvec) | reinterpret_cast<uintptr_t>(pvec) |
                          reinterpret_cast<uintptr_t>(rvec) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(state) |
                          reinterpret_cast<uintptr_t>(scratch);
   PSAMD_REQUIRE(bits % 16 == 0, "operands must lie on 16 bytes");
   PSAMD_REQUIRE(state_row >= static_cast<int64_t>(heads) * dim * vdim && heads <= 65535, "state rows too short, or too many heads");
-  if (n_blocks == 0 || items == 0) return 0;
+  const int at_once = psamd_delta_runs_at_once(heads, dim, vdim, general ? 1 : 0);
+  PSAMD_REQUIRE(at_once >= 1, "more heads than the scratch holds a run of");
   const DeltaRuns c{kvec, cvec, pvec, rvec, key_row, heads / key_groups, dvec, dvec_row, dscal, pscal, xscal, scal_row, x, x_row, out,
-                    out_row, state, state_row, item_start, slots, pf_tiles, pf_blocks, n_blocks, heads, vdim, scratch};
+                    out_row, state, state_row, slots, heads, vdim, scratch};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (form == kGatedForm) return dim == 64 ? launch_runs<4, kGatedForm>(s, c, items) : launch_runs<8, kGatedForm>(s, c, items);
-  if (form == kPlainForm) return dim == 64 ? launch_runs<4, kPlainForm>(s, c, items) : launch_runs<8, kPlainForm>(s, c, items);
-  return dim == 64 ? launch_runs<4, kGeneralForm>(s, c, items) : launch_runs<8, kGeneralForm>(s, c, items);
+  RunList list{};
+  int n_runs = 0, n_parts = 0;
+  for (int i = 0; i < items; ++i) {
+    PSAMD_REQUIRE(starts[i] >= 0 && starts[i + 1] >= starts[i], "the items' first tokens must ascend");
+    const int n = starts[i + 1] - starts[i];
+    if (n <= most) continue;
+    for (int q = 0; q < n; q += kRunTokens) {
+      if (n_runs == at_once) {
+        if (launch_runs_form(s, c, list, n_runs, n_parts, dim, form)) return 1;
+        n_runs = n_parts = 0;
+      }
+      if (q == 0 || n_parts == 0) {
+        list.item[n_parts] = i;
+        list.first[n_parts] = n_runs;
+        list.runs[n_parts++] = 0;
+      }
+      ++list.runs[n_parts - 1];
+      list.t0[n_runs] = starts[i] + q;
+      list.tokens[n_runs++] = std::min(kRunTokens, n - q);
+    }
+  }
+  return n_runs == 0 ? 0 : launch_runs_form(s, c, list, n_runs, n_parts, dim, form);
 }
 
 }  // extern "C"

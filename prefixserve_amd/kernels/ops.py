@@ -111,8 +111,9 @@ _SIGNATURES = {
     "psamd_delta_scan": [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64,
                          _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32],
     "psamd_delta_runs_supports": [_i32, _i32, _i64, _i64, _i64, _i64, _i64, _i32, _f32],
+    "psamd_delta_runs_at_once": [_i32, _i32, _i32, _i32],
     "psamd_delta_runs": [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64,
-                         _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _vp],
+                         _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _vp],
     "psamd_heads_norm_gate": [_vp, _vp, _i64, _i32, _i32, _vp, _i32, _f32, _vp, _i32, _i64, _i32, _vp],
     "psamd_short_conv_to": [_vp, _vp, _i32, _i64, _vp, _vp, _vp, _i32, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32],
     "psamd_stream_rms_norm": [_vp, _vp, _vp, _f32, _i64, _i32],
@@ -158,7 +159,7 @@ class HipOps:
     MOE_CHOICE_SORTS_MAX_TOKENS = 16 # up to here the workgroup that chooses a step's experts also sorts the pairs
     MOE_PAIRWISE_MAX_TOKENS = 2     # up to here a bfloat16 step's experts run pair by pair; above, grouped by expert
     DELTA_RUNS_MIN_TOKENS = 425     # from this length on a lone prompt's recurrence goes in runs of 64 tokens (where the caller allows it)
-    DELTA_RUNS_MAX_BYTES = 2 << 30  # scratch that the runs of one step may take; a step with more is walked token by token
+    DELTA_RUNS_SHORT = 64           # items of up to this many tokens beside it are walked: each would cost a whole run
     MFMA_ATTENTION_EXTRAS = True    # whether the matrix-core attention takes a sink and a bias by distance
     name = "hip"
 
@@ -173,7 +174,7 @@ class HipOps:
             fn.argtypes = argtypes
             fn.restype = ctypes.c_int
         self.lib.psamd_last_error.restype = ctypes.c_char_p
-        self.lib.psamd_delta_runs_floats.argtypes = [_i32] * 5
+        self.lib.psamd_delta_runs_floats.argtypes = [_i32] * 4
         self.lib.psamd_delta_runs_floats.restype = ctypes.c_int64
         self.lib.psamd_sample_scratch_floats.argtypes = [ctypes.c_int]
         self.lib.psamd_sample_scratch_floats.restype = ctypes.c_int64
@@ -1272,26 +1273,31 @@ class HipOps:
             state.data_ptr() + 4 * state_offset, state.shape[1], ctx.item_start.data_ptr(), ctx.slots.data_ptr())
         most = 0
         if in_runs and ctx.num_prefill_blocks:
-            # The walk takes 0.19 us for every token of the longest item, the runs 55 us and 0.06 (general rule: 0.09) for every
-            # token of the step: one item of 256 tokens 54 us against 78 (gated; general 53 and 63), of 512 102 against 91 (101
-            # and 76), of 2,048 391 against 182 (393 and 193); two of 1,024 200 against 140, four of 1,024 253 against 277, four
-            # of 512 133 against 141, one of 1,024 beside sixteen of 64 331 against 218.
-            longest = int(np.diff(ctx.host["item_start"]).max())
             same = keys[1] == directions[1] == removals[1] and decay_vectors is None and reads_decayed
             form = (1 if no_removal else 0) if same else 2
             fits = same or (not reads_decayed and decay_vectors is not None and decay is None and removal_scale is None
                             and value_scale is None and key_groups == heads)
-            floats = int(self.lib.psamd_delta_runs_floats(ctx.num_prefill_blocks, heads, dim, vdim, int(form == 2)))
-            if (3 * longest >= t + 2 * self.DELTA_RUNS_MIN_TOKENS and fits and 4 * floats <= self.DELTA_RUNS_MAX_BYTES
-                    and all(p % 16 == 0 for p in (at(keys), at(directions), at(removals), at(queries), out.data_ptr(), operands[17]))
+            if (fits and all(p % 16 == 0 for p in (at(keys), at(directions), at(removals), at(queries), out.data_ptr(), operands[17]))
                     and self.lib.psamd_delta_runs_supports(dim, vdim, base.shape[1], xv.shape[1], out.shape[1], operands[8],
-                                                           state.shape[1], int(form == 2), float(decay_least))):
+                                                           state.shape[1], int(form == 2), float(decay_least))
+                    and self.lib.psamd_delta_runs_at_once(heads, dim, vdim, int(form == 2)) > 0):
+                # Asked for by every step with a prompt, taken or not: what the largest step finds is all there ever is.
+                floats = int(self.lib.psamd_delta_runs_floats(heads, dim, vdim, int(form == 2)))
                 scratch = self.ws.get("delta.runs", (floats,), torch.float32)
-                self._ok(self.lib.psamd_delta_runs(*operands, ctx.pf_tiles.data_ptr(), ctx.pf_blocks.data_ptr(), ctx.num_prefill_blocks,
-                                                   ctx.num_items, heads, dim, vdim, form, float(decay_least), scratch.data_ptr()))
-                if ctx.num_decode == 0:
-                    return
-                most = 1                       # the single tokens are left
+                starts = ctx.host["item_start"]
+                lengths = np.diff(starts)
+                short = max(1, min(self.DELTA_RUNS_SHORT, self.DELTA_RUNS_MIN_TOKENS))
+                # The walk takes 0.19 us for every token of the longest item, the runs 55 us and 0.06 (general rule: 0.09) for every
+                # token of a run: one item of 256 tokens 54 us against 78 (gated; general 53 and 63), of 512 102 against 91 (101
+                # and 76), of 2,048 391 against 182 (393 and 193); two of 1,024 200 against 140, four of 1,024 253 against 277, four
+                # of 512 133 against 141.
+                in_whole_runs = 64 * int(((lengths[lengths > short] + 63) // 64).sum())
+                if 3 * int(lengths.max()) >= in_whole_runs + 2 * self.DELTA_RUNS_MIN_TOKENS:
+                    self._ok(self.lib.psamd_delta_runs(*operands[:19], starts.ctypes.data, operands[20], ctx.num_items, short, heads, dim,
+                                                       vdim, form, float(decay_least), scratch.data_ptr()))
+                    if int(lengths.min()) > short:
+                        return
+                    most = short               # the single tokens and the short items are left
         self._ok(self.lib.psamd_delta_scan(*operands, ctx.num_items, heads, dim, vdim, 2 if no_removal else int(reads_decayed), most))
 
     def heads_norm_gate(self, o, heads: int, vdim: int, weight, weight_per_head: bool, eps: float, gate_rows, gate_col: int,

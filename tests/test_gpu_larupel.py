@@ -607,3 +607,57 @@ def test_recurrences_in_runs_of_64_tokens(ops, monkeypatch, form, heads, groups,
         print(form, dim, runs, off[runs])
     assert off[True] != off[False]                          # the sums were made in another order
     assert all(b < max(2.0 * a, 3e-7) for a, b in zip(off[False], off[True])), off
+
+
+def recurrence(ops, form, lengths, heads, groups, dim, vdim, slots):
+    """A step of items of these lengths, and ``delta_scan``'s operands of one of the three forms for it: the values, the state
+    in front of the step, and a function of the values that gives the outputs and the state behind it."""
+    from prefixserve_amd.engine.batch import GroupMeta, StepItem, StepPacker
+
+    t = sum(lengths)
+    pages = [-(-n // 16) for n in lengths]
+    first = np.cumsum([0] + pages)
+    pk = StepPacker(torch.device(DEV), [GroupMeta(sum(pages))], 10, 8192, slots, ops.PREFILL_TILE_Q, skew_rule=ops.decode_is_skewed)
+    ctx = pk.pack([StepItem(i, [1] * n, 0, [list(range(first[i], first[i + 1]))], slot=slots - 1 - i) for i, n in enumerate(lengths)])
+    k = rnd(t, groups, dim, seed=1)
+    k = k / k.norm(dim=-1, keepdim=True)
+    r, x, state = rnd(t, groups, dim, seed=2, scale=dim ** -0.5), rnd(t, heads * vdim, seed=3), rnd(slots, heads * vdim * dim, seed=4)
+    args = dict(key_groups=groups, ctx=ctx, heads=heads, dim=dim, vdim=vdim, state_offset=0)
+    if form == "general":
+        d = torch.exp(-math.exp(-0.5) * torch.sigmoid(2.0 * rnd(t, heads, dim, seed=7)))
+        rows = torch.cat([v.reshape(t, -1) for v in (r, k, k, -torch.sigmoid(rnd(t, heads, dim, seed=5)) * k, d)], 1).contiguous()
+        s = heads * dim
+        args.update(keys=(rows, s), queries=(rows, 0), directions=(rows, 2 * s), removals=(rows, 3 * s), decay_vectors=(rows, 4 * s),
+                    decay=None, removal_scale=None, value_scale=None, reads_decayed=False, decay_least=math.exp(-math.exp(-0.5)))
+    else:
+        rows = torch.cat([r.reshape(t, -1), k.reshape(t, -1)], 1).contiguous()
+        xs = torch.sigmoid(rnd(t, heads, seed=6) + 1.0)
+        coef = torch.cat([torch.exp(-0.2 * rnd(t, heads, seed=5).abs()), -xs if form == "gated" else torch.zeros_like(xs), xs], 1).contiguous()
+        kc = (rows, groups * dim)
+        args.update(keys=kc, directions=kc, removals=kc, queries=(rows, 0), decay_vectors=None, decay=(coef, 0),
+                    removal_scale=(coef, heads), value_scale=(coef, 2 * heads), reads_decayed=True, no_removal=form == "plain")
+
+    def run(values, in_runs):
+        out, after = torch.empty(t, heads * vdim, device=DEV), state.clone()
+        ops.delta_scan(values=(values, 0), out=out, state=after, in_runs=in_runs, **args)
+        return out, after
+
+    return x, rows, run
+
+
+@pytest.mark.parametrize("form,heads,groups,dim,vdim", [("gated", 4, 2, 128, 128), ("plain", 4, 1, 128, 64), ("general", 4, 4, 64, 64)])
+def test_a_step_of_many_prompts_takes_no_more_scratch_than_a_long_one(form, heads, groups, dim, vdim):
+    """The scratch of the runs is asked for once: a long prompt beside many short ones, several long ones, and one longer than the
+    scratch holds at a time use what one long prompt has left, and give what the walk gives."""
+    from prefixserve_amd.kernels.ops import HipOps
+    from prefixserve_amd.parts.base import Workspace
+
+    ops = HipOps(torch.device(DEV), Workspace(torch.device(DEV)))
+    version = None
+    for lengths in ([2], [1500], [1000] + [17] * 61, [1, 900, 3, 450, 1, 64, 65, 1100], [7000, 130]):
+        x, _, run = recurrence(ops, form, lengths, heads, groups, dim, vdim, len(lengths))
+        got, want = run(x, True), run(x, False)
+        version = version or ops.ws.version
+        assert ops.ws.version == version and ops.ws.nbytes() <= 128 << 20
+        for a, b in zip(got, want):
+            assert float((a - b).norm() / b.norm()) < 3e-6
