@@ -18,7 +18,9 @@
 // Numerics: everything is float32. T is built by substitution, 16 x 16 on the diagonal and block by block below it (a product
 // of powers of L is shorter and loses everything where keys repeat). The gated form's ratios D_t / D_s are products of the
 // decays between the two tokens, so a decay may be 0; the general form divides by D_s and is only taken where the decays'
-// floor keeps D_s far from underflow.
+// floor keeps D_s far from underflow. A product over tokens multiplies those behind a token by zeros, which does not hide what is
+// not finite: it then stands in that token's W, and the chain walks such a run token by token for the 16 value channels it
+// concerns, as delta_scan_kernel would have.
 //
 // Operand layout of a 16 x 16 x 4 instruction: lane (r = l % 16, g = l / 16) gives k = 4 g + i, i = 0..3, of row r and of column
 // r, and receives rows 4 g .. 4 g + 3 of column r: what it receives is the column operand of a product over those rows.
@@ -72,7 +74,7 @@ struct RunList {
 
 // Where a run's arrays lie in its scratch.
 struct RunLayout {
-  int kt, kd, qd, w, p, s0, z, dc, total;
+  int kt, kd, qd, w, p, s0, z, dc, walked, total;
 };
 __host__ __device__ constexpr RunLayout run_layout(int dim, int vdim, bool general) {
   RunLayout l{};
@@ -85,6 +87,7 @@ __host__ __device__ constexpr RunLayout run_layout(int dim, int vdim, bool gener
   l.s0 = at, at += dim * vdim;                           // [vdim][dim]
   l.z = at, at += general ? dim * vdim : 0;              // [vdim][dim]
   l.dc = at, at += dim;
+  l.walked = at, at += 16;                               // [vdim / 16]: not 0 where these channels' outputs are finished
   l.total = at;
   return l;
 }
@@ -357,6 +360,8 @@ __global__ __launch_bounds__(256, 1) void runs_chain_kernel(DeltaRuns c, RunList
   constexpr bool GENERAL = FORM == kGeneralForm, SOLVES = FORM != kPlainForm;
   __shared__ __align__(16) float st_s[16 * LD];          // the state, [value channel][key channel]
   __shared__ f32x4 w_s[kRunTiles][64];
+  __shared__ int odd_s[kRunTiles];                       // per wave: W is not finite
+  __shared__ float sum_s[2][2][kRunTiles][16];
   const int item = list.item[blockIdx.x], first = list.first[blockIdx.x], runs = list.runs[blockIdx.x];
   const int h = blockIdx.y, j0 = blockIdx.z * 16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -397,6 +402,53 @@ __global__ __launch_bounds__(256, 1) void runs_chain_kernel(DeltaRuns c, RunList
       if constexpr (GENERAL) a.z[o] = *reinterpret_cast<const f32x4*>(q + lay.z + (j0 + r) * D + 16 * it + 4 * g);
     }
   };
+  // Sum over all key channels of a value channel, in every thread of its column.
+  auto column_sum = [&](float v, float (*parts)[16]) {
+    v += __shfl_xor(v, 16, kWave);
+    v += __shfl_xor(v, 32, kWave);
+    if (g == 0) parts[wave][r] = v;
+    lds_barrier();
+    return parts[0][r] + parts[1][r] + parts[2][r] + parts[3][r];
+  };
+  // A run token by token, outputs included.
+  auto walk_tokens = [&](int run) {
+    const int64_t t0 = list.t0[first + run];
+    const int n = list.tokens[first + run];
+    for (int t = 0; t < n; ++t) {
+      const int64_t scal = (t0 + t) * c.scal_row + h, head = (t0 + t) * c.out_row + static_cast<int64_t>(h) * c.vdim + j0 + r;
+      const int64_t key = (t0 + t) * c.key_row + static_cast<int64_t>(h / c.heads_per_group) * D + 4 * g;
+      const float xs = c.xscal != nullptr ? c.xscal[scal] : 1.f, ps = c.pscal != nullptr ? c.pscal[scal] : 1.f;
+      const float x = xs * c.x[(t0 + t) * c.x_row + static_cast<int64_t>(h) * c.vdim + j0 + r];
+      const float ds = !GENERAL && c.dscal != nullptr ? c.dscal[scal] : 1.f;
+      auto row = [&](const float* v, int it) { return *reinterpret_cast<const f32x4*>(v + key + 16 * it); };
+      auto dot = [](f32x4 a, f32x4 b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2] + a[3] * b[3]; };
+      float taken = 0.f, read = 0.f;
+#pragma unroll
+      for (int o = 0; o < OWN; ++o) {
+        const int it = wave + 4 * o;
+        if (it >= DT) break;
+        if constexpr (GENERAL) {
+          taken += dot(s[o], row(c.cvec, it));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[o][i] *= c.dvec[(t0 + t) * c.dvec_row + static_cast<int64_t>(h) * D + 16 * it + 4 * g + i];
+        } else {
+          s[o] = s[o] * ds;
+          if constexpr (SOLVES) taken += dot(s[o], row(c.kvec, it));
+        }
+      }
+      if constexpr (SOLVES) taken = ps * column_sum(taken, sum_s[0][t & 1]);
+#pragma unroll
+      for (int o = 0; o < OWN; ++o) {
+        const int it = wave + 4 * o;
+        if (it >= DT) break;
+        if constexpr (SOLVES) s[o] += taken * row(c.pvec, it);
+        s[o] += x * row(c.kvec, it);
+        read += dot(s[o], row(c.rvec, it));
+      }
+      read = column_sum(read, sum_s[1][t & 1]);
+      if (wave == 0 && g == 0) c.out[head] = read;
+    }
+  };
   auto walk = [&](Operands& a, int run) {
     float* q = sc + run * run_stride;
 #pragma unroll
@@ -416,15 +468,24 @@ __global__ __launch_bounds__(256, 1) void runs_chain_kernel(DeltaRuns c, RunList
       *reinterpret_cast<f32x4*>(q + lay.w + (j0 + r) * kRunTokens + 16 * wave + 4 * g) = w;
     }
     w_s[wave][lane] = w;
+    const float zeros = fmaf(w[0], 0.f, w[1] * 0.f) + fmaf(w[2], 0.f, w[3] * 0.f);
+    const bool odd = __any(zeros != 0.f);
+    if (lane == 0) odd_s[wave] = odd;
     ask_front(a, run + 2);
     lds_barrier();
+    const bool by_token = (odd_s[0] | odd_s[1] | odd_s[2] | odd_s[3]) != 0;
+    if (threadIdx.x == 0) q[lay.walked + blockIdx.z] = by_token ? 1.f : 0.f;
+    if (by_token) {
+      walk_tokens(run);
+    } else {
 #pragma unroll
-    for (int o = 0; o < OWN; ++o) {
-      f32x4 sum = zero;
+      for (int o = 0; o < OWN; ++o) {
+        f32x4 sum = zero;
 #pragma unroll
-      for (int t = 0; t < kRunTiles; ++t) sum = mma(a.kd[o][t], w_s[t][lane], sum);
-      if constexpr (GENERAL) sum += a.z[o];
-      s[o] = s[o] * a.dc[o] + sum;
+        for (int t = 0; t < kRunTiles; ++t) sum = mma(a.kd[o][t], w_s[t][lane], sum);
+        if constexpr (GENERAL) sum += a.z[o];
+        s[o] = s[o] * a.dc[o] + sum;
+      }
     }
     ask_back(a, run + 2);
   };
@@ -461,8 +522,10 @@ __global__ __launch_bounds__(256) void runs_output_kernel(DeltaRuns c, RunList l
 #pragma unroll
   for (int st = 0; st < kRunTiles; ++st)
     p[st] = st <= wave ? *reinterpret_cast<const f32x4*>(sc + lay.p + t * kRunTokens + 16 * st + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint64_t walked = __ballot(lane < c.vdim / 16 && sc[lay.walked + lane % 16] != 0.f);
   float* o = c.out + (t0 + t) * c.out_row + static_cast<int64_t>(h) * c.vdim + 4 * g;
   for (int j0 = 0; j0 < c.vdim; j0 += 16) {
+    if ((walked >> (j0 / 16) & 1) != 0) continue;
     f32x4 a[DT], w[kRunTiles];
 #pragma unroll
     for (int d = 0; d < DT; ++d) a[d] = *reinterpret_cast<const f32x4*>(sc + lay.s0 + (j0 + r) * D + 16 * d + 4 * g);

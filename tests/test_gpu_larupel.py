@@ -645,6 +645,29 @@ def recurrence(ops, form, lengths, heads, groups, dim, vdim, slots):
     return x, rows, run
 
 
+@pytest.mark.parametrize("form,heads,dim,vdim", [("gated", 2, 128, 64), ("plain", 2, 64, 32), ("general", 2, 64, 64)])
+def test_runs_of_values_that_are_not_finite(ops, monkeypatch, form, heads, dim, vdim):
+    """What is not finite in a token reaches what the walk lets it reach and no token in front of it, although a run sums over
+    all of its tokens: the same outputs and states are finite, and those agree (both are within a few times 1e-6 of 64 bits)."""
+    monkeypatch.setattr(ops, "DELTA_RUNS_MIN_TOKENS", -10000)
+    x, rows, run = recurrence(ops, form, [200, 1, 70], heads, heads, dim, vdim, 4)
+    s = heads * dim
+    for bad in (float("inf"), float("nan")):
+        for at in (0, 5, 70, 127, 199, 201 + 66):
+            for what in ("value", "key", "query"):
+                values, kept = x.clone(), rows.clone()
+                if what == "value":
+                    values[at, vdim + 3] = bad                                 # one value channel of the second head
+                else:
+                    rows[at, (s if what == "key" else 0) + 7] = bad            # a channel of the first head
+                walk, runs = run(values, False), run(values, True)
+                rows.copy_(kept)
+                for a, b, name in ((walk[0], runs[0], "outputs"), (walk[1], runs[1], "states")):
+                    ok = torch.isfinite(a)
+                    assert torch.equal(ok, torch.isfinite(b)), (what, bad, at, name)
+                    assert float((a[ok] - b[ok]).abs().max()) < 1e-5 * float(a[ok].abs().max()), (what, bad, at, name)
+
+
 @pytest.mark.parametrize("form,heads,groups,dim,vdim", [("gated", 4, 2, 128, 128), ("plain", 4, 1, 128, 64), ("general", 4, 4, 64, 64)])
 def test_a_step_of_many_prompts_takes_no_more_scratch_than_a_long_one(form, heads, groups, dim, vdim):
     """The scratch of the runs is asked for once: a long prompt beside many short ones, several long ones, and one longer than the
