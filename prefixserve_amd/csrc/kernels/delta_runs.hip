@@ -64,6 +64,7 @@ struct DeltaRuns {
 // The runs that one round of launches makes, in the order of their tokens, and the items that they are of. The host lists them (it
 // has the items' lengths) and hands the list over as a kernel argument.
 constexpr int kMaxRuns = 64;
+constexpr int64_t kRunScratch = 384LL << 20;             // bytes
 struct RunList {
   int32_t t0[kMaxRuns];        // a run's first token of the step
   int32_t tokens[kMaxRuns];    // how many it has
@@ -586,11 +587,12 @@ int psamd_delta_runs_supports(int dim, int vdim, int64_t key_row, int64_t x_row,
 }
 
 // How many runs of a recurrence of this shape the scratch holds at a time, and its floats. Both follow from the shape alone: the
-// scratch is at most 128 MiB whatever a step holds (a step with more runs makes them in several rounds of launches), so that it
-// never grows once a first prompt has been run. 39 runs of 16 heads of 128 x 128, 64 of 32 heads of 64 x 64.
+// scratch is at most 384 MiB whatever a step holds (a step with more runs makes them in several rounds of launches), so that it
+// never grows once a first prompt has been run. 64 runs of 16 heads of 128 x 128 (219 MB), 58 of 32 heads, 28 of 64. With 128 MiB
+// 2,048 tokens of 32 heads took a second round (300 us instead of 273; 32 heads of 128 x 64 without removal 201 instead of 146).
 int psamd_delta_runs_at_once(int heads, int dim, int vdim, int general) {
   const int64_t run = sizeof(float) * static_cast<int64_t>(heads) * run_layout(dim, vdim, general != 0).total;
-  return static_cast<int>(std::min<int64_t>(kMaxRuns, (128LL << 20) / run));
+  return static_cast<int>(std::min<int64_t>(kMaxRuns, kRunScratch / run));
 }
 int64_t psamd_delta_runs_floats(int heads, int dim, int vdim, int general) {
   return static_cast<int64_t>(psamd_delta_runs_at_once(heads, dim, vdim, general)) * heads * run_layout(dim, vdim, general != 0).total;

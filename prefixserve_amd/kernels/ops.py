@@ -13,6 +13,7 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import logging
+import math
 import os
 from typing import Any, Sequence
 
@@ -158,7 +159,7 @@ class HipOps:
     MOE_ROUTE_FUSED_MAX_TOKENS = 0   # up to here one kernel computes router logits and choice; above, product + choice
     MOE_CHOICE_SORTS_MAX_TOKENS = 16 # up to here the workgroup that chooses a step's experts also sorts the pairs
     MOE_PAIRWISE_MAX_TOKENS = 2     # up to here a bfloat16 step's experts run pair by pair; above, grouped by expert
-    DELTA_RUNS_MIN_TOKENS = 425     # from this length on a lone prompt's recurrence goes in runs of 64 tokens (where the caller allows it)
+    DELTA_RUNS_MIN_TOKENS = 340     # what a round of launches of the recurrences' runs costs, in tokens walked (see _runs_pay)
     DELTA_RUNS_SHORT = 64           # items of up to this many tokens beside it are walked: each would cost a whole run
     MFMA_ATTENTION_EXTRAS = True    # whether the matrix-core attention takes a sink and a bias by distance
     name = "hip"
@@ -1287,18 +1288,43 @@ class HipOps:
                 starts = ctx.host["item_start"]
                 lengths = np.diff(starts)
                 short = max(1, min(self.DELTA_RUNS_SHORT, self.DELTA_RUNS_MIN_TOKENS))
-                # The walk takes 0.19 us for every token of the longest item, the runs 55 us and 0.06 (general rule: 0.09) for every
-                # token of a run: one item of 256 tokens 54 us against 78 (gated; general 53 and 63), of 512 102 against 91 (101
-                # and 76), of 2,048 391 against 182 (393 and 193); two of 1,024 200 against 140, four of 1,024 253 against 277, four
-                # of 512 133 against 141.
-                in_whole_runs = 64 * int(((lengths[lengths > short] + 63) // 64).sum())
-                if 3 * int(lengths.max()) >= in_whole_runs + 2 * self.DELTA_RUNS_MIN_TOKENS:
+                if self._runs_pay(lengths, short, form, heads, dim, vdim, floats):
                     self._ok(self.lib.psamd_delta_runs(*operands[:19], starts.ctypes.data, operands[20], ctx.num_items, short, heads, dim,
                                                        vdim, form, float(decay_least), scratch.data_ptr()))
                     if int(lengths.min()) > short:
                         return
                     most = short               # the single tokens and the short items are left
         self._ok(self.lib.psamd_delta_scan(*operands, ctx.num_items, heads, dim, vdim, 2 if no_removal else int(reads_decayed), most))
+
+    def _runs_pay(self, lengths: np.ndarray, short: int, form: int, heads: int, dim: int, vdim: int, floats: int) -> bool:
+        """Whether a step's recurrence is faster in runs than walked, both in tokens of the walk (0.14 to 0.3 us each).
+
+        The walk: the longest item, or the throughput of 256 compute units with a workgroup per head and 16 value channels, or
+        that of the dies that the longest item's workgroups lie on (every n-th of the grid, n items). The runs: a round of
+        launches (``DELTA_RUNS_MIN_TOKENS``), 8 for every run of the longest item, which follow each other, and 5.5 for every
+        MB of scratch beyond 30; the plain form four fifths of that. us, runs / walk, one item unless it says more:
+
+        * gated, 16 heads of 128 x 128: 256 tokens 77 / 52, 512 91 / 100, 2,048 179 / 386; 4 x 512 143 / 133, 2 x 1,024 140 / 200.
+          32 heads: 1,024 136 / 198, 2 x 1,024 273 / 255. 64 heads: 512 136 / 129, 2,048 611 / 528. 16 of 64 x 64: 384 50 / 57.
+        * general, 32 heads of 64 x 64: 320 65 / 64, 512 75 / 100, 2,048 202 / 386, 4 x 512 173 / 126. 64 heads: 1,024 171 / 197,
+          2,048 392 / 390. 16 of 128 x 128: 448 136 / 132, 1,024 163 / 299.
+        * plain, 32 heads of 128 x 64: 320 59 / 58, 512 67 / 90, 2,048 146 / 352, 4 x 512 125 / 121. 80 heads: 512 103 / 112,
+          2,048 425 / 448, 2 x 1,024 414 / 320.
+
+        Over 448 steps of 16 such shapes its choice is on average 2% over the faster one and at worst 16% over the walk."""
+        long = lengths[lengths > short]
+        if len(long) == 0:
+            return False
+        longest = int(long.max())
+        at_once = int(self.lib.psamd_delta_runs_at_once(heads, dim, vdim, int(form == 2)))
+        runs = int(((long + 63) // 64).sum())
+        groups = heads * vdim / 16
+        share = 0.6 if form == 2 or dim > 64 else 0.42            # of a workgroup's time, where several share a compute unit
+        walk = max(longest, share * int(lengths.sum()) * groups / 256,
+                   share * longest * groups * math.gcd(len(lengths), 8) / 256)
+        cost = (-(-runs // at_once) * self.DELTA_RUNS_MIN_TOKENS + 8 * -(-longest // 64)
+                + 5.5 * max(0.0, 4e-6 * floats / at_once * runs - 30))
+        return walk > (0.8 if form == 1 else 1.0) * cost
 
     def heads_norm_gate(self, o, heads: int, vdim: int, weight, weight_per_head: bool, eps: float, gate_rows, gate_col: int,
                         activation: str, out) -> None:
