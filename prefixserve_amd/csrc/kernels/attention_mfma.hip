@@ -1147,13 +1147,20 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(
 
 // ------------------------------------------------------------------ decode (split keys)
 
-// A float that workgroups on different dies pass to each other inside a launch: past the caches that they do not share.
-__device__ __forceinline__ void shared_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ __forceinline__ float shared_load(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// Two floats that workgroups on different dies pass to each other inside a launch: past the caches that they do not share
+// (relaxed atomics of the whole agent go to and come from memory that all dies see).
+__device__ __forceinline__ void shared_store(float* p, float2 v) {
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 shared_load(const float* p) {
+  return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
 
 // NS = D / 16, CT = ceil(group / 16) column tiles of query heads.
-// part_o[dec][head][split][D], part_ml[dec][head][split][2] = (max, sum); arrived[dec][kv head]: how many of a request's
-// workgroups have written their runs, zero between launches.
+// part_o[dec][head][split][D], part_ml[dec][head][split][2] = (max, sum); arrived[dec][kv head][split]: which of a request's
+// workgroups have written their runs (or, in the first, how many), zero between launches.
+constexpr int kCounted = 8;              // runs that count in one integer
+constexpr int kMergeHeads = 8;           // the most query heads a kv head has where the decode kernel merges its runs
 template <int NS, int CT, bool P3 = false, bool MERGE = false>
 __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
     const bf16_t* __restrict__ qkv, int q_stride, const bf16_t* __restrict__ kv, bf16_t* __restrict__ out,
@@ -1199,12 +1206,13 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
   const int my_lo = tile_lo + split * tps;
   const int my_hi = min(my_lo + tps, tile_hi + 1);
   if (my_lo >= my_hi) {
-    // No keys left for this split (only with nsplit > 1): an empty sum and, for the merge kernel, an output of zeros, which it
-    // multiplies by a weight of zero (what lay there before might be NaN). The merge in this kernel does not read it.
+    if (MERGE) return;
+    // No keys left for this split (only with nsplit > 1): an empty sum and an output of zeros,
+    // which the merge kernel multiplies by a weight of zero (what lay there before might be NaN).
     for (int idx = threadIdx.x; idx < group * D; idx += blockDim.x) {
       const int hh = idx / D, d = idx - hh * D;
       const int64_t slot = (static_cast<int64_t>(di) * hq + kvh * group + hh) * nsplit + split;
-      if (!MERGE) part_o[slot * D + d] = 0.f;
+      part_o[slot * D + d] = 0.f;
       if (d == 0) {
         part_ml[slot * 2 + 0] = -INFINITY;
         part_ml[slot * 2 + 1] = 0.f;
@@ -1351,12 +1359,13 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
   }
   __syncthreads();
   const int runs = MERGE ? (tile_hi - tile_lo + tps) / tps : 1;        // of this request that have keys
-  for (int idx = threadIdx.x; idx < group * D; idx += blockDim.x) {
-    const int hh = idx / D, d = idx - hh * D;
-    float mm = -INFINITY;
+  // The workgroup's result for dimension d of head hh, not yet divided by its sum: the waves' results merged.
+  auto combined = [&](int hh, int d, float& mm, float& ll) {
+    mm = -INFINITY;
 #pragma unroll
     for (int w = 0; w < 4; ++w) mm = fmaxf(mm, sm_m[w * group + hh]);
-    float acc = 0.f, ll = 0.f;
+    float acc = 0.f;
+    ll = 0.f;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float mw = sm_m[w * group + hh];
@@ -1364,66 +1373,118 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
       acc += wgt * sm_o[(static_cast<int64_t>(w) * group + hh) * D + d];
       ll += wgt * sm_l[w * group + hh];
     }
-    if (MERGE ? runs == 1 : nsplit == 1) {     // nothing to merge with: this is the result
-      if (ex.sink != nullptr) ll += __expf(ex.sink[kvh * group + hh] - mm);
-      const int64_t at = static_cast<int64_t>(kvh * group + hh) * D + d;
-      if (ex.gate != nullptr) acc *= 1.f / (1.f + __expf(-bf16_to_float(ex.gate[t * ex.gate_row + at])));
-      out[t * (static_cast<int64_t>(hq) * D) + at] = float_to_bf16(acc / ll);
-      continue;
-    }
-    const int64_t slot = (static_cast<int64_t>(di) * hq + kvh * group + hh) * nsplit + split;
-    if constexpr (!MERGE) {                               // a kernel behind this one merges
-      part_o[slot * D + d] = acc;
+    return acc;
+  };
+  auto put = [&](int hh, int d, float y, float l) {
+    const int64_t at = static_cast<int64_t>(kvh * group + hh) * D + d;
+    if (ex.gate != nullptr) y *= 1.f / (1.f + __expf(-bf16_to_float(ex.gate[t * ex.gate_row + at])));
+    out[t * (static_cast<int64_t>(hq) * D) + at] = float_to_bf16(y / l);
+  };
+  if (!MERGE || runs == 1) {
+    for (int idx = threadIdx.x; idx < group * D; idx += blockDim.x) {
+      const int hh = idx / D, d = idx - hh * D;
+      float mm, ll;
+      const float acc = combined(hh, d, mm, ll);
+      if (MERGE || nsplit == 1) {               // nothing to merge with: this is the result
+        if (ex.sink != nullptr) ll += __expf(ex.sink[kvh * group + hh] - mm);
+        if (MERGE) put(hh, d, 1.f / ll * acc, 1.f);   // as a merge of one run
+        else put(hh, d, acc, ll);
+        continue;
+      }
+      const int64_t slot = (static_cast<int64_t>(di) * hq + kvh * group + hh) * nsplit + split;
+      part_o[slot * D + d] = acc;               // a kernel behind this one merges
       if (d == 0) {
         part_ml[slot * 2 + 0] = mm;
         part_ml[slot * 2 + 1] = ll;
       }
-      continue;
     }
-    shared_store(part_o + slot * D + d, acc);
-    if (d == 0) {
-      shared_store(part_ml + slot * 2 + 0, mm);
-      shared_store(part_ml + slot * 2 + 1, ll);
-    }
+    return;
   }
-  if (!MERGE || runs == 1) return;
+  // The last of a request's workgroups to get here merges its runs, as attn_decode_merge_kernel does and with the same bits. The
+  // partial results pass between dies, which no barrier or fence here makes them do: what orders them is that stores, counter and
+  // flags all go past the dies' caches, that a wave waits for its stores to have arrived (vmcnt counts them until they have)
+  // before the barrier in front of the workgroup's count or flag, and that results are loaded past the caches too, behind the
+  // answer. Up to eight runs count in one integer; more would queue for it (0.15 us each: 32 runs 4.6 us over the kernel behind,
+  // 1.1 so) and raise a flag each: whoever then sees all of them merges, two workgroups at once if it comes to that, which write
+  // the same.
+  const int64_t base = (static_cast<int64_t>(di) * hq + kvh * group) * nsplit;
+  for (int idx = 2 * threadIdx.x; idx < group * D; idx += 2 * blockDim.x) {
+    const int hh = idx / D, d = idx - hh * D;
+    const int64_t slot = base + static_cast<int64_t>(hh) * nsplit + split;
+    float mm, ll;
+    const float first = combined(hh, d, mm, ll);
+    shared_store(part_o + slot * D + d, float2{first, combined(hh, d + 1, mm, ll)});
+    if (d == 0) shared_store(part_ml + slot * 2, float2{mm, ll});
+  }
   __shared__ int last_s;
-  // The last of a request's workgroups to get here merges the runs. The partial results pass between dies: they are written and read past the dies' caches,
-  // the writes have arrived before the workgroup counts itself, and whoever counts last reads all of them.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  int32_t* counter = arrived + static_cast<int64_t>(di) * hkv + kvh;
-  if (threadIdx.x == 0) last_s = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == runs - 1;
-  __syncthreads();
-  if (!last_s) return;
-  if (threadIdx.x == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
-  const int64_t base = (static_cast<int64_t>(di) * hq + kvh * group) * nsplit;
-  float* run_m = smem;                                    // [group][runs], then the sums
-  float* run_l = smem + group * runs;
-  for (int idx = threadIdx.x; idx < group * runs; idx += blockDim.x) {
-    const int64_t slot = base + static_cast<int64_t>(idx / runs) * nsplit + idx % runs;
-    run_m[idx] = shared_load(part_ml + slot * 2);
-    run_l[idx] = shared_load(part_ml + slot * 2 + 1);
+  int32_t* flags = arrived + (static_cast<int64_t>(di) * hkv + kvh) * nsplit;   // all zero between launches
+  if (wave == 0) {
+    bool last;
+    if (runs <= kCounted) {
+      last = lane == 0 && __hip_atomic_fetch_add(flags, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == runs - 1;
+    } else {
+      if (lane == 0) __hip_atomic_store(flags + split, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      last = __all(lane < runs ? __hip_atomic_load(flags + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 1);
+    }
+    if (lane == 0) last_s = last;
   }
   __syncthreads();
-  for (int idx = threadIdx.x; idx < group * D; idx += blockDim.x) {
+  if (!last_s) return;
+  if (static_cast<int>(threadIdx.x) < runs) __hip_atomic_store(flags + threadIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
+  // A thread merges two dimensions at a time. The first ones' results of the first runs are asked for together with the
+  // statistics, the others sixteen runs at a time: a trip past the caches is what this costs.
+  constexpr int kEarly = 8, kAhead = 16, kHeads = kMergeHeads / 4;     // heads a wave makes the weights of
+  auto ask = [&](int idx, int s) {
     const int hh = idx / D, d = idx - hh * D;
-    const float* ms = run_m + hh * runs;
-    const float* ls = run_l + hh * runs;
-    const float* po = part_o + (base + static_cast<int64_t>(hh) * nsplit) * D + d;
-    float mm = -INFINITY;
-    for (int s = 0; s < runs; ++s) mm = fmaxf(mm, ms[s]);
-    float acc = 0.f, ll = 0.f;
-#pragma unroll 8
-    for (int s = 0; s < runs; ++s) {
-      const float wgt = __expf(ms[s] - mm);
-      acc += wgt * shared_load(po + static_cast<int64_t>(s) * D);
-      ll += wgt * ls[s];
-    }
+    return shared_load(part_o + (base + static_cast<int64_t>(hh) * nsplit + s) * D + d);
+  };
+  float2 early[kEarly], stats[kHeads];
+#pragma unroll
+  for (int i = 0; i < kHeads; ++i) {
+    const int hh = wave + 4 * i;
+    stats[i] = hh < group && lane < runs ? shared_load(part_ml + (base + static_cast<int64_t>(hh) * nsplit + lane) * 2) : float2{-INFINITY, 0.f};
+  }
+#pragma unroll
+  for (int s = 0; s < kEarly; ++s)
+    early[s] = s < runs && 2 * static_cast<int>(threadIdx.x) < group * D ? ask(2 * threadIdx.x, s) : float2{0.f, 0.f};
+  float* weight = smem;                                  // [group][runs]
+#pragma unroll
+  for (int i = 0; i < kHeads; ++i) {
+    const int hh = wave + 4 * i;
+    if (hh >= group) break;
+    const float mm = wave_max(stats[i].x);
+    const float w = stats[i].x == -INFINITY ? 0.f : __expf(stats[i].x - mm);
+    float ll = wave_sum(w * stats[i].y);
     if (ex.sink != nullptr) ll += __expf(ex.sink[kvh * group + hh] - mm);
-    const int64_t at = static_cast<int64_t>(kvh * group + hh) * D + d;
-    if (ex.gate != nullptr) acc *= 1.f / (1.f + __expf(-bf16_to_float(ex.gate[t * ex.gate_row + at])));
-    out[t * (static_cast<int64_t>(hq) * D) + at] = float_to_bf16(acc / ll);
+    if (lane < runs) weight[hh * runs + lane] = w / ll;
+  }
+  __syncthreads();
+  for (int idx = 2 * threadIdx.x; idx < group * D; idx += 2 * blockDim.x) {
+    const int hh = idx / D, d = idx - hh * D;
+    const float* wgt = weight + hh * runs;
+    float2 acc = {0.f, 0.f};
+    auto add = [&](float w, float2 v) {
+      acc.x = fmaf(w, v.x, acc.x);
+      acc.y = fmaf(w, v.y, acc.y);
+    };
+    int s0 = 0;
+    if (idx == 2 * static_cast<int>(threadIdx.x)) {
+#pragma unroll
+      for (int s = 0; s < kEarly; ++s) add(s < runs ? wgt[s] : 0.f, early[s]);
+      s0 = kEarly;
+    }
+    for (; s0 < runs; s0 += kAhead) {
+      float2 v[kAhead];
+#pragma unroll
+      for (int s = 0; s < kAhead; ++s) v[s] = s0 + s < runs ? ask(idx, s0 + s) : float2{0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < kAhead; ++s) add(s0 + s < runs ? wgt[s0 + s] : 0.f, v[s]);
+    }
+    put(hh, d, acc.x, 1.f);
+    put(hh, d + 1, acc.y, 1.f);
   }
 }
 
@@ -1850,8 +1911,8 @@ int psamd_attention_decode_plan(int n_dec, int kv_len, int skewed, int hkv, int 
 // results of every decode step, so that the buffers never grow.
 int psamd_attention_decode_max_parts(int max_requests) { return std::max({4096, 512, max_requests}); }
 
-// part_o needs n_dec * hq * nsplit * head_dim floats, part_ml n_dec * hq * nsplit * 2, arrived n_dec * hkv integers that are
-// zero and are left zero. Launches that share them follow each other on one stream.
+// part_o needs n_dec * hq * nsplit * head_dim floats, part_ml n_dec * hq * nsplit * 2, arrived n_dec * hkv * nsplit integers
+// that are zero and are left zero. Launches that share them follow each other on one stream.
 // min_split_keys: a request's keys are cut into runs no shorter than this (a multiple of 32), so
 // that nsplit can follow the longest request of a step without cutting the short ones to pieces.
 int psamd_attention_decode(void* stream, const void* qkv, int q_stride, void* out, const void* kv, float* part_o,
@@ -1870,10 +1931,18 @@ int psamd_attention_decode(void* stream, const void* qkv, int q_stride, void* ou
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int group = hq / hkv;
   const int ct = group <= 16 ? 1 : (group <= 32 ? 2 : 4);
-  // Where a kv head's runs are few numbers, the last of its workgroups merges them: attention + merge of one request behind 300
-  // tokens 9.5 -> 7.3 us, of eight behind 2,048 15.6 -> 13.5 (4 heads of 64 a kv head). 16 heads of 256 in 32 runs would be half
-  // a megabyte past the caches for one workgroup: 24.6 -> 47 us, and a merge kernel with a block per head stays.
-  if (nsplit == 1 || ct > 1 || static_cast<int64_t>(group) * head_dim * nsplit > 16384) arrived = nullptr;
+  // Where a kv head's runs are few numbers, the last of its workgroups merges them. us of attention and merge in a captured step
+  // of up to 4,096 keys, with the kernel behind / in one launch, behind 100, 300, 1,000, 2,048 and 4,000 keys:
+  //   32 heads of 64 on 8,  1 request   8.0 / 4.2   8.0 / 6.4   8.0 / 6.6    8.1 / 8.2    8.2 / 9.2     (32 runs at most)
+  //                         4           7.9 / 4.4   8.0 / 6.8   8.5 / 7.4    9.2 / 10.1  11.0 / 11.3    (16)
+  //                         8           7.4 / 4.6   7.3 / 6.6   8.3 / 7.8   11.2 / 10.7  17.0 / 16.3    (8)
+  //                        16           8.0 / 5.3   7.9 / 7.3  10.4 / 10.3  17.9 / 17.0  26.2 / 25.4    (4)
+  //   32 heads of 128 on 8, 1          10.3 / 5.3  10.6 / 7.5  10.6 / 8.0   10.7 / 9.7   10.8 / 11.0
+  //                         8           9.3 / 5.8   9.4 / 7.9  12.1 / 10.8  19.4 / 18.2  28.0 / 26.3
+  // It loses about 1 us where more than eight runs have few numbers to merge (64 runs: 2). With 16 heads of 64 a kv head it lost from
+  // 300 keys on (3.5 us behind 2,048), and 16 heads of 256 in 32 runs would be half a megabyte past the caches for one workgroup:
+  // there a merge kernel with a block per head stays.
+  if (nsplit == 1 || group > kMergeHeads || static_cast<int64_t>(group) * head_dim * nsplit > 16384) arrived = nullptr;
   int rc;
 #define PSAMD_DEC_NS(NS_)                                                                                          \
   rc = exact_weights ? dispatch_decode_ct<NS_, true>(ct, s, qkv, q_stride, kv, out, part_o, part_ml, arrived, dec_items, n_dec, \

@@ -588,7 +588,7 @@ int psamd_delta_runs_supports(int dim, int vdim, int64_t key_row, int64_t x_row,
 
 // How many runs of a recurrence of this shape the scratch holds at a time, and its floats. Both follow from the shape alone: the
 // scratch is at most 384 MiB whatever a step holds (a step with more runs makes them in several rounds of launches), so that it
-// never grows once a first prompt has been run. 64 runs of 16 heads of 128 x 128 (219 MB), 58 of 32 heads, 28 of 64. With 128 MiB
+// never grows once a first prompt has been run. 64 runs of 16 heads of 128 x 128 (219 MB), 58 of 32 heads, 29 of 64. With 128 MiB
 // 2,048 tokens of 32 heads took a second round (300 us instead of 273; 32 heads of 128 x 64 without removal 201 instead of 146).
 int psamd_delta_runs_at_once(int heads, int dim, int vdim, int general) {
   const int64_t run = sizeof(float) * static_cast<int64_t>(heads) * run_layout(dim, vdim, general != 0).total;

@@ -1265,3 +1265,26 @@ def test_float32_attention_takes_the_tiles_the_step_was_cut_into(ops, monkeypatc
     for tile in (16, 64):
         monkeypatch.setattr(ops, "PREFILL_TILE_Q", tile)
         assert torch.equal(paged_case(ops, torch.float32, hq, hkv, 32, [100, 1, 37], [0, 50, 70], seed=3)[0], want)
+
+
+@pytest.mark.parametrize("d", [48, 64, 128])
+@pytest.mark.parametrize("old", [(0, 100, 127, 128), (500, 1100, 1023, 40), (2900, 2047, 130, 4000), (4000,)])
+@pytest.mark.parametrize("extras", [False, True])
+def test_decode_attention_merges_its_runs_as_the_kernel_behind_it_does(ops, d, old, extras):
+    """Sixteen heads on one kv head have their runs merged by a kernel of its own, eight of them in the launch that makes them
+    (one run, counted ones, more with a flag each): the same runs, so the same bits."""
+    n = len(old)
+    first = np.cumsum([0] + [-(-(o + 1) // 16) for o in old])
+    pk = StepPacker(torch.device(DEV), [GroupMeta(int(first[-1]))], 10, 100000, 8, ops.PREFILL_TILE_Q, skew_rule=ops.decode_is_skewed)
+    ctx = pk.pack([StepItem(i, [1], o, [list(range(first[i], first[i + 1]))], slot=i) for i, o in enumerate(old)])
+    kv = rnd(int(first[-1]), 2, 1, 16 * d, dtype=torch.bfloat16, seed=d)
+    q, rest = rnd(n, 16, d, dtype=torch.bfloat16, seed=1), rnd(n, 2 * d, dtype=torch.bfloat16, seed=2)
+    sink, gate = rnd(16, seed=3), rnd(n, 16 * d, dtype=torch.bfloat16, seed=4)
+    outs = []
+    for heads in (16, 8):
+        out = torch.empty(n, heads * d, dtype=torch.bfloat16, device=DEV)
+        more = dict(sink=sink[:heads].contiguous(), out_gate=(gate[:, :heads * d].contiguous(), 0)) if extras else {}
+        ops.paged_attention(torch.cat([q[:, :heads].reshape(n, -1), rest], 1).contiguous(), out, kv, ctx, 0, heads, 1, d, d ** -0.5, None, **more)
+        outs.append(out)
+    assert torch.equal(outs[0][:, :8 * d], outs[1])
+    assert int(ops.ws._bufs["attn.arrived"].abs().max()) == 0
