@@ -1206,13 +1206,12 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
   const int my_lo = tile_lo + split * tps;
   const int my_hi = min(my_lo + tps, tile_hi + 1);
   if (my_lo >= my_hi) {
-    if (MERGE) return;
-    // No keys left for this split (only with nsplit > 1): an empty sum and an output of zeros,
-    // which the merge kernel multiplies by a weight of zero (what lay there before might be NaN).
+    // No keys left for this split (only with nsplit > 1): an empty sum and, for the merge kernel, an output of zeros, which it
+    // multiplies by a weight of zero (what lay there before might be NaN). The merge in this kernel does not read it.
     for (int idx = threadIdx.x; idx < group * D; idx += blockDim.x) {
       const int hh = idx / D, d = idx - hh * D;
       const int64_t slot = (static_cast<int64_t>(di) * hq + kvh * group + hh) * nsplit + split;
-      part_o[slot * D + d] = 0.f;
+      if (!MERGE) part_o[slot * D + d] = 0.f;
       if (d == 0) {
         part_ml[slot * 2 + 0] = -INFINITY;
         part_ml[slot * 2 + 1] = 0.f;
