@@ -30,6 +30,7 @@
 // slices up afterwards (the order of the additions differs from run to run).
 
 #include <algorithm>
+#include <cmath>
 
 #include "api.h"
 #include "common.h"
@@ -915,11 +916,29 @@ static bool tiles_take(int64_t tokens, int64_t pairs, int K, int F) {
   return K % 64 == 0 && F % 64 == 0 && 2 * tokens * K <= most && 2 * pairs * F <= most && 4LL * K * F <= most;
 }
 
-// ... and their rows: 0 where the kernel above takes the step. Both products and the sorting, 32 experts of 1,024 x 2,048,
-// us in tiles of 256 x 256 / 128 x 128 / the kernel above: 512 pairs an expert 323 / 374 / 428, 448 pairs 307 / 299 / 366,
-// 340 pairs 322 / 246 / 302, 150 pairs - / 157 / 240, 50 pairs - / 114 / 153, 25 pairs - / 145 / 130. The large tile wants
-// half the bytes per product, but one workgroup fills a compute unit and few rounds of them leave the last one half empty.
-static int wide_tile_rows(int64_t pairs, int experts) { return pairs >= 480LL * experts ? 256 : (pairs >= 48LL * experts ? 128 : 0); }
+// ... and their rows: 0 where the kernel above takes the step (from 48 pairs an expert on it is the slower one everywhere; below,
+// the router's kernel may have sorted the pairs into its tiles). Tiles of 256 x 256 ask for half the bytes per product, but one
+// workgroup of them fills a compute unit, two of 128 x 128 share one, and the last round of either is as long as a full one:
+// the time is that of the rounds, K long in the first product and F in the second, and a round of large tiles takes about one and a
+// half of small ones. An expert is taken to have what few have more of when the choices fall at random. us of both products
+// and the sorting, 256 x 256 / 128 x 128 / the kernel above (E experts of K x F):
+//   32 of 2,048 x 1,024:  60 pairs an expert 117 / 113 / 156, 200 144 / 163 / 269, 512 321 / 339 / 396, 700 334 / 411 / 481, 2,000 928 / 1,124 / 1,245
+//    8 of 2,048 x 1,024:  60 60 / 47 / 78, 300 89 / 56 / 96, 700 94 / 100 / 129, 1,000 177 / 151 / 193, 3,000 315 / 406 / 468
+//    8 of 4,096 x 3,584:  60 216 / 189 / 258, 300 341 / 453 / 443, 600 585 / 795 / 710, 2,000 1,575 / 2,192 / 1,930
+//   24 of 1,024 x 320:    300 61 / 49 / 67, 768 116 / 86 / 110, 3,000 303 / 318 / 380
+//    4 of 1,024 x 512:    60 37 / 29 / 44, 512 61 / 36 / 60, 3,000 72 / 74 / 91
+// Over 133 such steps of seven shapes the choice is on average 1% over the faster one (one bound at 480 pairs an expert: 9%, and in
+// seven of them slower than the kernel above), at worst 37%, where the rounds are just full.
+static int wide_tile_rows(int64_t pairs, int experts, int K, int F, int kind) {
+  if (pairs < 48LL * experts) return 0;
+  const double mean = static_cast<double>(pairs) / experts;
+  auto rounds = [&](int rows, int at_once) {
+    const int64_t tiles = experts * static_cast<int64_t>(std::ceil((mean + 2.0 * std::sqrt(mean)) / rows));
+    const int64_t first = tiles * ceil_div(F, kind == kExpertGated ? rows / 2 : rows), second = tiles * ceil_div(K, rows);
+    return static_cast<double>(ceil_div(first, at_once)) * K + static_cast<double>(ceil_div(second, at_once)) * F;
+  };
+  return 1.5 * rounds(256, 256) < rounds(128, 512) ? 256 : 128;
+}
 
 template <typename A>
 static int launch_experts_rows(hipStream_t s, const ExpertCall& c) {
@@ -1071,7 +1090,7 @@ int psamd_moe_experts_grouped(void* stream, const void* x, const int32_t* chosen
   const int64_t pairs = tokens * top;
   const int buckets = experts + (identity > 0 ? 1 : 0);      // all identity pairs lie in one, behind the experts'
   // Pairs that the router's kernel has sorted lie in the tiles of a small step.
-  const int wide = grouped_already == 0 && tiles_take(tokens, pairs, K, F) ? wide_tile_rows(pairs, buckets) : 0;
+  const int wide = grouped_already == 0 && tiles_take(tokens, pairs, K, F) ? wide_tile_rows(pairs, buckets, K, F, kind) : 0;
   const int rows = wide != 0 ? wide : psamd_moe_grouped_tile_rows(pairs, buckets);
   const int max_tiles = static_cast<int>(std::min<int64_t>(ceil_div(pairs, rows) + buckets, pairs));
   PSAMD_REQUIRE(max_tiles <= 65535, "too many tiles for one launch");

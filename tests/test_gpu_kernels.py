@@ -1288,3 +1288,51 @@ def test_decode_attention_merges_its_runs_as_the_kernel_behind_it_does(ops, d, o
         outs.append(out)
     assert torch.equal(outs[0][:, :8 * d], outs[1])
     assert int(ops.ws._bufs["attn.arrived"].abs().max()) == 0
+
+
+@pytest.mark.parametrize("pairs,top,k,f,experts", [
+    (90, 3, 192, 320, 8),           # tiles of 128 pairs, an expert's only one not full
+    (300, 2, 128, 192, 9),
+    (400, 4, 1024, 512, 32),        # tiles of 256 pairs: gated, and without a gate where there are identity experts
+    (600, 4, 1024, 512, 32),        # without a gate
+])
+@pytest.mark.parametrize("kind,on_output,identity,into", [("gated", False, 0, False), ("gated", True, 3, False), ("squared_relu", True, 2, False),
+                                                          ("gated", True, 2, True), ("squared_relu", False, 0, True)])
+def test_experts_with_many_pairs_and_several_choices_a_token(ops, pairs, top, k, f, experts, kind, on_output, identity, into):
+    """Several choices a token, all of them different: a pair reads the row of its token and writes the slice of its choice (or adds
+    into the token's row of the stream, times a factor per column), with and without identity experts among the choices. Against
+    float64 with the activations rounded to bfloat16, as above; what the stream held is added to in float32."""
+    t = -(-pairs * experts // top)
+    gen = torch.Generator().manual_seed(pairs + k)
+    x = rnd(t, k, dtype=torch.bfloat16, seed=1)
+    w_in = rnd(experts, (2 if kind == "gated" else 1) * f, k, dtype=torch.bfloat16, seed=2, scale=k ** -0.5)
+    down = rnd(experts, k, f, dtype=torch.bfloat16, seed=3, scale=f ** -0.5)
+    chosen = torch.rand(t, experts + identity, generator=gen).topk(top, 1).indices.to(torch.int32).contiguous().to(DEV)
+    weight = (0.4 + 0.6 * torch.rand(t, top, generator=gen)).to(DEV)
+    want = torch.empty(top, t, k, dtype=torch.float64, device=DEV)
+    for e in range(experts + identity):
+        rows, j = (chosen == e).nonzero(as_tuple=True)
+        h, w = x[rows].double(), weight[rows, j].double()[:, None]
+        if e >= experts:
+            want[j, rows] = w * h
+            continue
+        z = (h if on_output else w * h) @ w_in[e].double().T
+        if kind == "gated":
+            g, u = z[:, :f].clamp(max=5.0), z[:, f:].clamp(-5.0, 5.0)
+            a = g * torch.sigmoid(1.702 * g) * (u + 1.0)
+        else:
+            a = torch.relu(z).square()
+        want[j, rows] = (w if on_output else 1.0) * (a.to(torch.bfloat16).double() @ down[e].double().T)
+    act = torch.empty(t * top, f, dtype=torch.bfloat16, device=DEV)
+    args = (x, chosen, weight, w_in, down, act)
+    how = dict(weight_on_output=on_output, kind=kind, identity=identity)
+    if into:
+        stream, scale = rnd(t + 1, k, seed=4), rnd(k, seed=5)
+        got = stream.clone()
+        ops.moe_experts(*args, None, 1.702, 5.0, 1.0, residual=got[:t], col_scale=scale, **how)
+        assert rel(got[:t], stream[:t].double() + scale.double() * want.sum(0)) < 3e-3 and torch.equal(got[t], stream[t])
+    else:
+        out = torch.full((top, t, k), 7.0, device=DEV)
+        ops.moe_experts(*args, out, 1.702, 5.0, 1.0, **how)
+        for j in range(top):
+            assert rel(out[j], want[j]) < 3e-3, f"choice {j}"
