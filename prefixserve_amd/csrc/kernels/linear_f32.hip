@@ -210,6 +210,52 @@ __global__ __launch_bounds__(512) void rows_f32_kernel(const float* __restrict__
   if (wave < MT && m < M) put_columns(out, m, n0 + 4 * g, N, total);
 }
 
+// The same where K is one segment: 16 rows of w per workgroup, a wave for each of its chains, which one wave then adds in
+// ascending order. Of the eight waves above one had all the work (a chain is 0.2 us of matrix instructions). us at 1 token, by
+// fused multiply-adds / above / here: 16,384 columns of K = 64 4.2 / 12.4 / 4.0, of 256 8.5 / 13.1 / 6.5, 1,024 of 256 4.5 / 5.2 / 4.7; at
+// 64 tokens 34.8 / 7.9 / 4.9.
+template <int MT>
+__global__ __launch_bounds__(kSegment) void rows_short_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                  float* __restrict__ out, int M, int N, int K) {
+  constexpr int U = kChain / 16;
+  __shared__ f32x4 red[kSegment / kChain][MT][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, chains = blockDim.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16 * MT, k0 = wave * kChain + 4 * g;
+  const float* wrow = w + static_cast<int64_t>(min(n0 + r, N - 1)) * K + k0;
+  float4 a[U], b[MT][U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const bool in = k0 + 16 * u < K;                                   // K is a multiple of 4
+    a[u] = in ? *reinterpret_cast<const float4*>(wrow + 16 * u) : float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const float* xrow = x + static_cast<int64_t>(min(m0 + mt * 16 + r, M - 1)) * K + k0;
+      b[mt][u] = in ? *reinterpret_cast<const float4*>(xrow + 16 * u) : float4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc = mma16(a[u], b[mt][u], acc);
+    red[wave][mt][lane] = acc;
+  }
+  __syncthreads();
+  for (int mt = wave; mt < MT; mt += chains) {
+    f32x4 total = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < chains; ++i) total += red[i][mt][lane];
+    const int m = m0 + mt * 16 + r;
+    if (m < M) put_columns(out, m, n0 + 4 * g, N, total);
+  }
+}
+
+template <int MT>
+static void launch_rows_short(hipStream_t s, const float* x, const float* w, float* out, int M, int N, int K) {
+  const dim3 grid(static_cast<unsigned>(ceil_div(N, 16)), static_cast<unsigned>(ceil_div(M, 16 * MT)));
+  rows_short_f32_kernel<MT><<<grid, dim3(64 * static_cast<unsigned>(ceil_div(K, kChain))), 0, s>>>(x, w, out, M, N, K);
+}
+
 template <int MT>
 static void launch_rows(hipStream_t s, const float* x, const float* w, float* out, int M, int N, int K) {
   const dim3 grid(static_cast<unsigned>(ceil_div(N, 16)), static_cast<unsigned>(ceil_div(M, 16 * MT)));
@@ -229,6 +275,7 @@ bool linear_f32_takes(const void* x, const void* w, int64_t M, int N, int K) {
 }
 
 // Which kernel, us at one MI355X (K = 2,048 unless given; every one gives the same bits):
+//  * K of one segment, and up to 16 tokens or so few tiles as below: a wave per chain.
 //  * up to 8 tokens, or 16 where the columns are fewer than 16,384: 16 rows of w per workgroup. 2,048 columns at 8 tokens 13
 //    (tiles of 32 tokens 36), 128,256 at 1 token 187 (234); at 16 tokens 282 (224).
 //  * fewer tiles of 32 tokens than half the compute units: the same kernel with 32 tokens. 64 tokens x 2,048 columns 16
@@ -237,7 +284,9 @@ bool linear_f32_takes(const void* x, const void* w, int64_t M, int N, int K) {
 //    267 (319); 600 x 3,072 97 (85); from there on tiles of 64: 600 x 16,384 404 (422), 100 TFLOP/s.
 int launch_linear_f32(hipStream_t s, const float* x, const float* w, float* out, int M, int N, int K) {
   const int64_t tiles64 = ceil_div(M, 64) * ceil_div(N, 64), tiles32 = ceil_div(M, 32) * ceil_div(N, 64);
-  if (M <= 8 || (M <= 16 && N < 16384)) launch_rows<1>(s, x, w, out, M, N, K);
+  if (K <= kSegment && M <= 16) launch_rows_short<1>(s, x, w, out, M, N, K);
+  else if (K <= kSegment && tiles32 <= 128) launch_rows_short<2>(s, x, w, out, M, N, K);
+  else if (M <= 8 || (M <= 16 && N < 16384)) launch_rows<1>(s, x, w, out, M, N, K);
   else if (tiles32 <= 128) launch_rows<2>(s, x, w, out, M, N, K);
   else if (tiles64 <= 384) launch_tiles<32>(s, x, w, out, M, N, K);
   else launch_tiles<64>(s, x, w, out, M, N, K);
