@@ -154,7 +154,7 @@ class HipOps:
     PREFILL_TILE_Q = 32    # queries per workgroup of the prefill attention kernel (its 4 waves split the keys)
     SKINNY_MAX_ROWS = 64
     STREAM_MAX_ROWS = 128           # whole 64-element steps of K and aligned operands: the products with both operands through LDS
-    FUSED_SWIGLU_MAX_ROWS = 32      # above it (to SKINNY_MAX_ROWS) gate/up goes to the library, where there is one
+    FUSED_SWIGLU_MAX_ROWS = 32      # above it what _through_lds does not take goes to the library, where there is one (o, down, q/k/v: above SKINNY_MAX_ROWS)
     LIBRARY_ADD_MIN_ROWS = 1024     # from here on a product that feeds the residual stream adds into it in the library
     MOE_ROUTE_FUSED_MAX_TOKENS = 0   # up to here one kernel computes router logits and choice; above, product + choice
     MOE_CHOICE_SORTS_MAX_TOKENS = 16 # up to here the workgroup that chooses a step's experts also sorts the pairs
@@ -659,7 +659,7 @@ class HipOps:
                 return
             x = self.normed(x)
         if (x.dtype == torch.bfloat16 and k % 8 == 0 and d % 16 == 0
-                and (0 < m <= self.SKINNY_MAX_ROWS or self._through_lds(x, w_qkv, qkv, m, qkv.shape[1], k))):
+                and (0 < m <= self.SKINNY_MAX_ROWS or self._through_lds(x, w_qkv, qkv, m, qkv.shape[1], k, "qkv"))):
             self._need(w_qkv.shape == ((hq + 2 * hkv) * d, k) and qkv.shape == (m, (hq + 2 * hkv) * d), "qkv: shapes")
             self._need(x.is_contiguous() and w_qkv.is_contiguous() and qkv.is_contiguous(), "qkv: contiguous operands")
             self._need(positions.dtype == torch.int32 and positions.numel() == m, "qkv: positions")
@@ -679,13 +679,30 @@ class HipOps:
 
     # ---------------------------------------------------------------- products
 
-    def _through_lds(self, x, w, out, m: int, n: int, k: int, gated: bool = False) -> bool:
-        """Whether the products of 17 to 128 tokens with both operands through LDS take this one. At the 1B shape they
-        take, against the library's product (and the kernels behind it), at 77 tokens: o 5.0 us for 8.5, down 11.4 for 20.8,
-        gate/up with its activation 21.4 for 23.1."""
-        return (self.FUSED_SWIGLU_MAX_ROWS < m <= self.STREAM_MAX_ROWS and x.dtype == torch.bfloat16
+    def _through_lds(self, x, w, out, m: int, n: int, k: int, form: str) -> bool:
+        """Whether a product of 33 to 128 tokens goes to the kernels with both operands through LDS instead of the library: "residual"
+        (out for the stream, in slices of K), "gated" or "qkv". A workgroup there walks all of K for its rows of w (for the
+        stream an eighth of it at least), so few rows and a long K leave the chip idle where the library cuts K.
+        us, library and what follows it / here:
+
+        * residual, 77 tokens (n x k): 1,024 x 8,192 14.1 / 8.7, 4,096 x 8,192 29.3 / 23.9, 8,192 x 3,584 24.5 / 21.2, x 8,192 39.6 / 43.5.
+        * gated, 48 tokens: 128 x 2,048 8.4 / 9.8, 192 x 2,048 11.1 / 9.8, 1,024 x 2,048 11.7 / 10.0, x 4,096 15.5 / 17.6, 2,048 x 4,096 17.2 / 18.1,
+          x 7,168 27.2 / 29.4, 3,072 x 4,096 21.6 / 20.4, x 14,336 61.3 / 59.4. 77 tokens: 256 x 1,024 8.3 / 8.8, 1,024 x 1,024 11.5 / 9.0, x 2,048 11.8 / 14.0,
+          x 4,096 16.0 / 24.6, 1,536 x 2,048 15.4 / 14.6, x 4,096 24.9 / 25.0, 3,072 x 4,096 27.2 / 26.4, x 7,168 38.7 / 42.5.
+        * qkv, 77 tokens: 768 x 1,536 11.9 / 11.6, x 2,048 12.8 / 13.5, x 8,192 18.5 / 37.3, 1,536 x 4,096 16.8 / 22.0,
+          3,072 x 2,048 16.8 / 14.4, x 4,096 26.3 / 22.8, 6,144 x 4,096 29.8 / 26.4, x 8,192 41.1 / 45.8."""
+        if form == "gated":
+            if m <= self.SKINNY_MAX_ROWS:
+                pays = k <= 1024 or (k <= 2048 and n >= 160) or n >= 2560
+            else:
+                pays = k <= 512 or (k <= 1024 and n >= 320) or n >= max(1536, 0.75 * k)
+        elif form == "qkv":
+            pays = k <= 1536 or (n >= 3072 and k <= 4096)
+        else:
+            pays = n * k <= 6e7
+        return (pays and self.FUSED_SWIGLU_MAX_ROWS < m <= self.STREAM_MAX_ROWS and x.dtype == torch.bfloat16
                 and w.dtype == torch.bfloat16 and out.dtype == torch.bfloat16
-                and bool(self.lib.psamd_linear_skinny_takes(x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, int(gated))))
+                and bool(self.lib.psamd_linear_skinny_takes(x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, int(form == "gated"))))
 
     def linear(self, x, w, out) -> None:
         m, k = x.shape
@@ -758,7 +775,7 @@ class HipOps:
             if rc != 2:                          # 2: no algorithm for this shape: the ways below
                 self._ok(rc)
                 return None
-        if x.dtype == torch.bfloat16 and k % 8 == 0 and (0 < m <= self.SKINNY_MAX_ROWS or self._through_lds(x, w, x, m, n, k)):
+        if x.dtype == torch.bfloat16 and k % 8 == 0 and (0 < m <= self.SKINNY_MAX_ROWS or self._through_lds(x, w, x, m, n, k, "residual")):
             ksplit = self.lib.psamd_linear_skinny_ksplit(m, n, k)
             if ksplit > 1:
                 self._need(w.shape[1] == k and x.is_contiguous() and w.is_contiguous(), "linear_to_residual: operands")
@@ -793,7 +810,7 @@ class HipOps:
                 return
             x = self.normed(x)
         self._need(x.is_contiguous() and w_gate_up.is_contiguous() and out.is_contiguous(), "linear_swiglu: contiguous operands")
-        lds = self._through_lds(x, w_gate_up, out, m, inter, k, True)
+        lds = self._through_lds(x, w_gate_up, out, m, inter, k, "gated")
         small = x.dtype == torch.bfloat16 and k % 8 == 0 and (m <= self.SKINNY_MAX_ROWS or lds)
         if small and m > self.FUSED_SWIGLU_MAX_ROWS and not lds and self._direct_library:
             # Between these row counts the library's product and the activation kernel behind it

@@ -619,6 +619,25 @@ def test_qkv_of_17_to_128_tokens(ops, m, hq, hkv, d, k, rotate):
     assert torch.equal(kv, expected)
 
 
+@pytest.mark.parametrize("m", [17, 24, 32, 33, 64, 65, 128])
+@pytest.mark.parametrize("hq,hkv,d,k", [(4, 2, 16, 1088), (8, 2, 64, 1600), (32, 8, 128, 64), (40, 20, 64, 128)])
+def test_qkv_on_both_sides_of_its_rules(ops, m, hq, hkv, d, k):
+    """Up to 24 tokens the tiles in LDS need 320 row tiles, from 33 to 64 as many or enough to multiply (K = 1,088 has it from 62
+    tokens on), above 64 a K that the library does not cut better."""
+    test_qkv_of_17_to_128_tokens(ops, m, hq, hkv, d, k, True)
+
+
+@pytest.mark.parametrize("m", [33, 64, 65, 128])
+@pytest.mark.parametrize("n,k", [(64, 2112), (2564, 2112), (48, 1088), (1536, 2048)])
+def test_gated_products_on_both_sides_of_their_rule(ops, m, n, k):
+    """Through LDS or through the library with the activation behind it: bfloat16 rounds at 2^-9."""
+    x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd(2 * n, k, dtype=torch.bfloat16, seed=2, scale=0.05)
+    prod = x.double() @ w.double().T
+    out = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.linear_swiglu(x, w, out[:m])
+    assert rel(out[:m], torch.nn.functional.silu(prod[:, :n]) * prod[:, n:]) < 1e-2 and torch.all(out[m] == 7.0)
+
+
 # -------------------------------------------------------------------- attention
 
 def paged_case(ops, act, hq, hkv, d, lens_new, lens_old, window=None, seed=0, num_blocks=64, poison=1e30, give_back=False,
