@@ -534,3 +534,48 @@ def test_random_configurations_in_both_dtypes(seed, tmp_path):
             assert max(errors) < F32_TOL, (cfg, max(errors))
         else:
             check_rows(errors, dtype, bf16_bars(folder, truth, reqs))
+
+
+def test_long_prompts_go_through_the_runs(tmp_path, monkeypatch):
+    """A state space layer of 128, a gated delta rule of 64 and a matrix memory of 64 (whose normalizer is a value channel more)
+    in a bfloat16 model: a prompt long enough for the runs, its continuation beside another such prompt, single tokens behind
+    both. The layers ask for the form that their recurrence is, and the logits are as near the plain model as those of short
+    prompts."""
+    def slow(tensors):
+        for name, t in tensors.items():
+            if name.endswith(".A_log"):
+                t.fill_(-5.0)
+            if name.endswith(".f.b"):
+                t.fill_(5.0)
+
+    cfg = model(80, 64, 1e-5, [
+        layer(mamba2(4, 32, 128, 2, 4, 1), None),
+        layer(side_by_side("parallel", attention(4, 2, 32, 32, 0.2, 300), delta(4, 2, 64, 48, 4), 1.0, 0.5), 32),
+        layer(side_by_side("parallel_2", attention(4, 2, 32, 32, 0.2, 300), memory(4, 64, 31, 15.0), 1.0, 0.5), None),
+    ], streams=2, taps=3, mult=0.5)
+    folder = write_fubelorn(tmp_path, cfg, seed=5, std=0.3, edit=slow)
+    rng = np.random.default_rng(6)
+    reqs = [rng.integers(0, 80, 1710).tolist(), rng.integers(0, 80, 460).tolist()]
+    truth = [truth_of(folder, t) for t in reqs]
+    runner = runner_for(folder, 160, "bfloat16")
+    taken, rule = [], type(runner.ops)._runs_pay
+
+    def noting(ops, lengths, short, form, heads, dim, vdim, floats):
+        pays = rule(ops, lengths, short, form, heads, dim, vdim, floats)
+        taken.append((form, heads, dim, vdim, pays))
+        return pays
+
+    monkeypatch.setattr(type(runner.ops), "_runs_pay", noting)
+    a, b = reqs
+    steps = [{"step": 0, "entries": [{"id": "a", "tokens": a[:1000], "want": list(range(4, 1000, 5))}], "end": []},
+             {"step": 1, "entries": [{"id": "a", "tokens": a[1000:1700], "want": list(range(0, 700, 5))},
+                                     {"id": "b", "tokens": b[:450], "want": list(range(0, 450, 5))}], "end": []}]
+    expect = [[(0, p) for p in range(4, 1000, 5)], [(0, 1000 + p) for p in range(0, 700, 5)] + [(1, p) for p in range(0, 450, 5)]]
+    for i in range(10):
+        steps.append({"step": 2 + i, "entries": [{"id": "a", "tokens": [a[1700 + i]], "want": [0]},
+                                                 {"id": "b", "tokens": [b[450 + i]], "want": [0]}], "end": []})
+        expect.append([(0, 1700 + i), (1, 450 + i)])
+    errors: list = []
+    traces.compare(TraceReplayer(runner).run_step, steps, expect, truth, 1.0, errors)
+    check_rows(errors, "bfloat16", bf16_bars(folder, truth, reqs))
+    assert taken == [(1, 4, 128, 32, True), (0, 4, 64, 48, True), (1, 4, 64, 32, True)] * 2

@@ -684,3 +684,44 @@ def test_a_step_of_many_prompts_takes_no_more_scratch_than_a_long_one(form, head
         assert ops.ws.version == version and ops.ws.nbytes() <= 128 << 20
         for a, b in zip(got, want):
             assert float((a - b).norm() / b.norm()) < 3e-6
+
+
+def test_long_prompts_go_through_the_runs(tmp_path, monkeypatch):
+    """Heads of 128 (gated) and of 64 (general) in a bfloat16 model: a prompt long enough for the runs, its continuation beside
+    another such prompt, single tokens behind both. The layers ask for the form that their recurrence is, and the logits are as
+    near the plain model as those of short prompts."""
+    def slow(tensors):
+        for name, t in tensors.items():
+            if name.endswith(".A_log"):
+                t.fill_(-5.0)
+            if name.endswith(".w0"):
+                t.fill_(-4.0)
+
+    cfg = model(80, 64, 1e-5, [layer(delta(4, 2, 128, 64, 4), dense(32)), layer(general_delta(2, 64, 6), None)])
+    folder = write_larupel(tmp_path, cfg, seed=5, std=0.3, edit=slow)
+    rng = np.random.default_rng(6)
+    reqs = [rng.integers(0, 80, 1710).tolist(), rng.integers(0, 80, 460).tolist()]
+    pm = plain.PlainLarupel.from_dir(folder)
+    truth = [pm.logits(t) for t in reqs]
+    runner = runner_for(folder, 160, "bfloat16")
+    taken, rule = [], type(runner.ops)._runs_pay
+
+    def noting(ops, lengths, short, form, heads, dim, vdim, floats):
+        pays = rule(ops, lengths, short, form, heads, dim, vdim, floats)
+        taken.append((form, heads, dim, vdim, pays))
+        return pays
+
+    monkeypatch.setattr(type(runner.ops), "_runs_pay", noting)
+    a, b = reqs
+    steps = [{"step": 0, "entries": [{"id": "a", "tokens": a[:1000], "want": list(range(4, 1000, 5))}], "end": []},
+             {"step": 1, "entries": [{"id": "a", "tokens": a[1000:1700], "want": list(range(0, 700, 5))},
+                                     {"id": "b", "tokens": b[:450], "want": list(range(0, 450, 5))}], "end": []}]
+    expect = [[(0, p) for p in range(4, 1000, 5)], [(0, 1000 + p) for p in range(0, 700, 5)] + [(1, p) for p in range(0, 450, 5)]]
+    for i in range(10):
+        steps.append({"step": 2 + i, "entries": [{"id": "a", "tokens": [a[1700 + i]], "want": [0]},
+                                                 {"id": "b", "tokens": [b[450 + i]], "want": [0]}], "end": []})
+        expect.append([(0, 1700 + i), (1, 450 + i)])
+    errors: list = []
+    traces.compare(TraceReplayer(runner).run_step, steps, expect, truth, 1.0, errors)
+    check_rows(errors, "bfloat16", bf16_bars(folder, truth, reqs))
+    assert taken == [(0, 4, 128, 64, True), (2, 2, 64, 64, True)] * 2
