@@ -918,26 +918,29 @@ static bool tiles_take(int64_t tokens, int64_t pairs, int K, int F) {
 
 // ... and their rows: 0 where the kernel above takes the step (from 48 pairs an expert on it is the slower one everywhere; below,
 // the router's kernel may have sorted the pairs into its tiles). Tiles of 256 x 256 ask for half the bytes per product, but one
-// workgroup of them fills a compute unit, two of 128 x 128 share one, and the last round of either is as long as a full one:
-// the time is that of the rounds, K long in the first product and F in the second, and a round of large tiles takes about one and a
-// half of small ones. An expert is taken to have what few have more of when the choices fall at random. us of both products
+// workgroup of them fills a compute unit, two of 128 x 128 share one, and a last round that is not full costs nearly as much as one
+// that is: the time is that of the rounds, K long in the first product and F in the second, and a round of large tiles takes
+// about one and a half of small ones. An expert's last tile is half empty on average. us of both products
 // and the sorting, 256 x 256 / 128 x 128 / the kernel above (E experts of K x F):
 //   32 of 2,048 x 1,024:  60 pairs an expert 117 / 113 / 156, 200 144 / 163 / 269, 512 321 / 339 / 396, 700 334 / 411 / 481, 2,000 928 / 1,124 / 1,245
 //    8 of 2,048 x 1,024:  60 60 / 47 / 78, 300 89 / 56 / 96, 700 94 / 100 / 129, 1,000 177 / 151 / 193, 3,000 315 / 406 / 468
 //    8 of 4,096 x 3,584:  60 216 / 189 / 258, 300 341 / 453 / 443, 600 585 / 795 / 710, 2,000 1,575 / 2,192 / 1,930
 //   24 of 1,024 x 320:    300 61 / 49 / 67, 768 116 / 86 / 110, 3,000 303 / 318 / 380
 //    4 of 1,024 x 512:    60 37 / 29 / 44, 512 61 / 36 / 60, 3,000 72 / 74 / 91
-// Over 133 such steps of seven shapes the choice is on average 1% over the faster one (one bound at 480 pairs an expert: 9%, and in
-// seven of them slower than the kernel above), at worst 37%, where the rounds are just full.
+// Over 480 steps of eight shapes, 60 to 2,000 pairs an expert, choices at random, uneven and very uneven, the choice is on average
+// 1.6% over the faster tile and in none slower than the kernel above (one bound at 480 pairs an expert: 4.4%, nine); at worst 34%,
+// where a round is just full or just not.
 static int wide_tile_rows(int64_t pairs, int experts, int K, int F, int kind) {
   if (pairs < 48LL * experts) return 0;
-  const double mean = static_cast<double>(pairs) / experts;
   auto rounds = [&](int rows, int at_once) {
-    const int64_t tiles = experts * static_cast<int64_t>(std::ceil((mean + 2.0 * std::sqrt(mean)) / rows));
-    const int64_t first = tiles * ceil_div(F, kind == kExpertGated ? rows / 2 : rows), second = tiles * ceil_div(K, rows);
-    return static_cast<double>(ceil_div(first, at_once)) * K + static_cast<double>(ceil_div(second, at_once)) * F;
+    const double tiles = std::max<double>(experts, static_cast<double>(pairs) / rows + 0.5 * experts);
+    auto of = [&](int64_t columns) {
+      const double full = tiles * columns / at_once;
+      return 0.5 * (std::ceil(full) + std::max(full, 1.0));
+    };
+    return of(ceil_div(F, kind == kExpertGated ? rows / 2 : rows)) * K + of(ceil_div(K, rows)) * F;
   };
-  return 1.5 * rounds(256, 256) < rounds(128, 512) ? 256 : 128;
+  return 1.55 * rounds(256, 256) < rounds(128, 512) ? 256 : 128;
 }
 
 template <typename A>

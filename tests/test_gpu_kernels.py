@@ -1201,7 +1201,7 @@ def test_kernels_refuse_what_they_do_not_take(ops):
 
 
 @pytest.mark.parametrize("counts,k,f", [
-    ((0, 127, 128, 129, 255, 256, 257, 512, 1900, 1500), 192, 320),  # tiles of 256 pairs: empty experts, edges, halves without pairs
+    ((0, 127, 128, 129, 255, 256, 257, 512, 1900, 1500), 192, 320),  # empty experts, edges, parts without pairs
     ((1700, 0, 3, 511), 64, 64),                                    # one step of k, fewer columns than a tile
     ((0, 1, 63, 64, 65, 127, 128, 129, 10), 128, 192),              # tiles of 128 pairs
     ((200, 130, 97, 0, 90), 320, 128),
@@ -1309,11 +1309,17 @@ def test_decode_attention_merges_its_runs_as_the_kernel_behind_it_does(ops, d, o
     assert int(ops.ws._bufs["attn.arrived"].abs().max()) == 0
 
 
+@pytest.mark.parametrize("kind,on_output,identity", [("gated", False, 0), ("gated", True, 2), ("squared_relu", True, 0)])
+def test_experts_with_many_pairs_each_in_large_tiles(ops, kind, on_output, identity):
+    """Enough rows and columns that tiles of 256 pairs are taken: empty experts, edges, halves without pairs."""
+    test_experts_with_many_pairs_each(ops, (0, 127, 128, 129, 255, 256, 257, 512, 1900, 1500), 2048, 2048, kind, on_output, identity)
+
+
 @pytest.mark.parametrize("pairs,top,k,f,experts", [
     (90, 3, 192, 320, 8),           # tiles of 128 pairs, an expert's only one not full
     (300, 2, 128, 192, 9),
-    (400, 4, 1024, 512, 32),        # tiles of 256 pairs: gated, and without a gate where there are identity experts
-    (600, 4, 1024, 512, 32),        # without a gate
+    (400, 4, 1024, 512, 32),        # the most rounds of those tiles that two of 256 pairs are not worth
+    (600, 4, 1024, 512, 32),        # tiles of 256 pairs
 ])
 @pytest.mark.parametrize("kind,on_output,identity,into", [("gated", False, 0, False), ("gated", True, 3, False), ("squared_relu", True, 2, False),
                                                           ("gated", True, 2, True), ("squared_relu", False, 0, True)])
