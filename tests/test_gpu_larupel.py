@@ -545,8 +545,8 @@ def test_random_configurations_in_both_dtypes(seed, tmp_path):
 def test_recurrences_in_runs_of_64_tokens(ops, monkeypatch, form, heads, groups, dim, vdim):
     """Items shorter than, as long as and longer than one and two runs, single tokens among them (they are walked), each from
     a state of its own, run by run and token by token against float64. Keys that repeat (the systems to solve are then full),
-    decays of zero (gated, plain) and decays at their floor (general) included. The sums differ in order alone: the runs may be as
-    far off as the walk, twice for the chance of it."""
+    decays of zero (gated, plain) and decays at their floor (general) included. The sums are of another order, and
+    operands that carry a decay are rounded once more: a third further off than the walk at most, a half for the chance of it."""
     from prefixserve_amd.engine.batch import GroupMeta, StepItem, StepPacker
 
     lengths = [1, 2, 63, 64, 65, 128, 1, 200, 17]
@@ -606,7 +606,7 @@ def test_recurrences_in_runs_of_64_tokens(ops, monkeypatch, form, heads, groups,
         off[runs] = (gap(out[:t].view(t, heads, vdim), want), gap(st[:, 4:], want_state[:, 4:]))
         print(form, dim, runs, off[runs])
     assert off[True] != off[False]                          # the sums were made in another order
-    assert all(b < max(2.0 * a, 3e-7) for a, b in zip(off[False], off[True])), off
+    assert all(b < 1.5 * a for a, b in zip(off[False], off[True])), off
 
 
 def recurrence(ops, form, lengths, heads, groups, dim, vdim, slots):
