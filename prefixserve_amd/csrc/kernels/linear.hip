@@ -2,7 +2,8 @@
 //
 // * gemm_tiled: LDS-tiled FMA kernel for any element types with float accumulation: the fallback for
 //   shapes that the kernels of linear_f32.hip (32-bit) and the bfloat16 kernels below refuse.
-// * skinny_mfma: bfloat16 product for M <= 64 rows (decode steps and small portions). It is
+// * skinny_mfma: bfloat16 product for M <= 16 rows (decode steps), and up to 64 where the kernels of
+//   linear_stream.hip do not take the operands (K no multiple of 64, off a 16-byte boundary). It is
 //   bound by reading w once from HBM, so each wave streams 16 rows of w through the
 //   16x16x32 matrix-core instruction with the M tokens as the other operand. Optional
 //   epilogue: SwiGLU over a fused [gate; up] matrix, or float32 output for logits.

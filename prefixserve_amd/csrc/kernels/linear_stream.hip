@@ -262,7 +262,6 @@ __global__ __launch_bounds__(64 * W) void stream_tiles_kernel(const bf16_t* __re
   }
 }
 
-// 80 KB of buffers: two workgroups a compute unit.
 // The most rows of w per workgroup, which read the tokens least often, that still leave most of the 256 compute units one
 // (64, 32 and 16 rows at 64 tokens: 2 x 14,336 x 4,096 49.5, 50.5 and 62 us; 2 x 8,192 x 2,048 24.1, 18.6 and 20.1;
 // 2 x 4,096 x 2,048 20.3, 13.9 and 12.0; 16,384 x 2,048 16.8, 18.6 and 26.0; 4,096 x 2,048 12.6, 10.1 and 9.2). With K-slices,
@@ -272,6 +271,8 @@ static int stream_columns(int N, int ksplit) {
   return ceil_div(N, 64) * ksplit >= kEnough ? 64 : (ceil_div(N, 32) * ksplit >= kEnough ? 32 : 16);
 }
 
+// 80 KB of buffers, so that two workgroups share a compute unit; at least three, which for 128 tokens and 64 rows of gate and up are
+// 96 KB: one.
 constexpr int stream_stages(int stage) { return std::min(8, std::max(3, 80 * 1024 / stage)); }
 
 template <int TM, int TN, int W, int FORM>

@@ -159,6 +159,7 @@ class HipOps:
     MOE_ROUTE_FUSED_MAX_TOKENS = 0   # up to here one kernel computes router logits and choice; above, product + choice
     MOE_CHOICE_SORTS_MAX_TOKENS = 16 # up to here the workgroup that chooses a step's experts also sorts the pairs
     MOE_PAIRWISE_MAX_TOKENS = 2     # up to here a bfloat16 step's experts run pair by pair; above, grouped by expert
+    DELTA_RUNS = True               # delta_scan takes ``in_runs``
     DELTA_RUNS_MIN_TOKENS = 340     # what a round of launches of the recurrences' runs costs, in tokens walked (see _runs_pay)
     DELTA_RUNS_SHORT = 64           # items of up to this many tokens beside it are walked: each would cost a whole run
     MFMA_ATTENTION_EXTRAS = True    # whether the matrix-core attention takes a sink and a bias by distance

@@ -24,7 +24,7 @@ UNIT_EPS = 1e-6          # inside the root when a key or query is made a unit ve
 def in_runs(rt: Runtime, decay_least: float = 0.0) -> dict[str, Any]:
     """What a mixer adds to its ``delta_scan`` call: a serving step may sum a prompt run by run; the exact mode sums token by
     token, so that a position's bits do not depend on how its sequence was cut."""
-    if rt.dtype != torch.bfloat16 or not hasattr(rt.ops, "DELTA_RUNS_MIN_TOKENS"):
+    if rt.dtype != torch.bfloat16 or not getattr(rt.ops, "DELTA_RUNS", False):
         return {}
     return {"in_runs": True, "decay_least": decay_least}
 
