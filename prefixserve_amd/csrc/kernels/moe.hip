@@ -34,6 +34,7 @@
 
 #include "api.h"
 #include "common.h"
+#include "tile_product.h"
 
 namespace psamd {
 
@@ -390,27 +391,111 @@ __global__ __launch_bounds__(256) void moe_down_rows_kernel(
 
 // ------------------------------------------------------------------ experts, grouped by expert
 
-// One workgroup sorts the step's pairs by expert and lists the tiles of `tile_rows` pairs the
-// products run over. ints: sorted[pairs] (pair indices, expert by expert), then per tile slot
+// How an expert's pairs are cut into tiles: up to `rows` of them each, the last with what is left, or, with rows 0, evenly into
+// tiles of up to the limit that is best for this step's counts (tiles_time).
+struct TileRule {
+  int rows;
+  int columns[2], length[2];           // rows == 0: columns of tiles and length of a tile's sums in the two products
+};
+
+// The time of a tile of the 512-thread kernel below by its pairs, in 1/64 of a full one's (measured there).
+__device__ __forceinline__ int tile_cost(int pairs) { return pairs <= 64 ? 32 : pairs <= 128 ? 42 : pairs <= 192 ? 54 : 64; }
+
+// The time of the step's tiles under a limit of pairs, computed by one wave: every die runs an eighth of the tiles, 32 at once, and a
+// round of them takes as long as its tiles do on average.
+__device__ __forceinline__ int64_t tiles_time(const int32_t* count, int experts, int limit, const TileRule& rule, int lane) {
+  int tiles = 0, cost = 0;
+  for (int e = lane; e < experts; e += kWave) {
+    const int n = (count[e] + limit - 1) / limit;
+    tiles += n;
+    cost += n > 0 ? n * tile_cost((count[e] + n - 1) / n) : 0;
+  }
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    tiles += __shfl_xor(tiles, o, kWave);
+    cost += __shfl_xor(cost, o, kWave);
+  }
+  int64_t time = 0;
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+    time += static_cast<int64_t>(((tiles * rule.columns[p] + 7) / 8 + 31) / 32) * rule.length[p] * (64 * cost / max(tiles, 1));
+  return time;
+}
+
+constexpr int kGroupCounters = 4096;   // counters of the sorting, in rows of `experts`
+
+__host__ __device__ constexpr int group_counter_rows(int experts) {
+  return experts * 16 <= kGroupCounters ? 16 : (experts * 4 <= kGroupCounters ? 4 : 1);
+}
+constexpr size_t group_smem_ints(int experts) { return static_cast<size_t>(3 + group_counter_rows(experts)) * experts + 5; }
+constexpr int kGroupStaged = 16384;    // up to here the sorted pairs are laid out in LDS before they leave, in whole lines
+
+// One workgroup of 16 waves sorts the step's pairs by expert and lists the tiles that the products run over.
+// ints: sorted[pairs] (pair indices, expert by expert), then per tile slot
 // tile_expert, tile_first (index into sorted), tile_count; slots past the last tile hold -1; then the number of tiles.
 // The order of an expert's pairs among themselves is whatever the atomics gave: every pair's
 // result is computed from its own row alone, so it does not matter which rows share a tile.
-// `count`, `start`, `tstart`, `cursor` are LDS arrays of `experts` integers each.
-__device__ __forceinline__ void group_pairs(const int32_t* __restrict__ chosen, int pairs, int experts, int tile_rows,
+// `identity`: the pairs of the last of the `experts` buckets have no tiles; where they begin in `sorted` stands in tile_first
+// behind the last tile. Up to 16 waves count in counters of their own, and
+// the sorted pairs leave LDS in whole lines (16,384 pairs over 32 experts 13.1 us -> 11.2).
+__device__ __forceinline__ void group_pairs(const int32_t* __restrict__ chosen, int pairs, int experts, const TileRule& rule, bool identity,
                                             int max_tiles, int32_t* __restrict__ sorted, int32_t* __restrict__ tile_expert,
                                             int32_t* __restrict__ tile_first, int32_t* __restrict__ tile_count,
-                                            int32_t* tiles_out, int32_t* count, int32_t* start, int32_t* tstart, int32_t* cursor,
-                                            int32_t* n_tiles) {
-  for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = cursor[e] = 0;
+                                            int32_t* tiles_out, int32_t* smem, int32_t* staged) {
+  const int rows = group_counter_rows(experts);
+  int32_t *count = smem, *start = smem + experts, *tstart = smem + 2 * experts, *cursor = smem + 3 * experts;
+  int32_t *listed = smem + (3 + rows) * experts, *own = cursor + static_cast<int>(threadIdx.x >> 6) % rows * experts;
+  const int tiled = identity ? experts - 1 : experts;                            // buckets that have tiles
+  for (int e = threadIdx.x; e < rows * experts; e += blockDim.x) cursor[e] = 0;
   __syncthreads();
-  for (int p = threadIdx.x; p < pairs; p += blockDim.x) atomicAdd(&count[min(max(chosen[p], 0), experts - 1)], 1);
+  // Four choices a load, all of a step's first 16 x 1,024 asked for at once and kept for the second look.
+  constexpr int kKept = 4;
+  const int quads = reinterpret_cast<uintptr_t>(chosen) % 16 == 0 ? pairs / 4 : 0;
+  auto bucket = [&](int c) { return min(max(c, 0), experts - 1); };
+  int4 kept[kKept];
+#pragma unroll
+  for (int i = 0; i < kKept; ++i) {
+    const int q = threadIdx.x + i * blockDim.x;
+    kept[i] = q < quads ? reinterpret_cast<const int4*>(chosen)[q] : int4{0, 0, 0, 0};
+  }
+#pragma unroll
+  for (int i = 0; i < kKept; ++i) {
+    if (static_cast<int>(threadIdx.x + i * blockDim.x) >= quads) break;
+    atomicAdd(&own[bucket(kept[i].x)], 1);
+    atomicAdd(&own[bucket(kept[i].y)], 1);
+    atomicAdd(&own[bucket(kept[i].z)], 1);
+    atomicAdd(&own[bucket(kept[i].w)], 1);
+  }
+  const int done = 4 * min(quads, kKept * static_cast<int>(blockDim.x));
+#pragma unroll 4
+  for (int p = done + threadIdx.x; p < pairs; p += blockDim.x) atomicAdd(&own[bucket(chosen[p])], 1);
   __syncthreads();
+  for (int e = threadIdx.x; e < experts; e += blockDim.x) {
+    int sum = 0;
+    for (int w = 0; w < rows; ++w) sum += cursor[w * experts + e];
+    count[e] = sum;
+  }
+  __syncthreads();
+  if (rule.rows == 0) {                          // a wave each for limits of 256, 192 and 128 pairs
+    if (const int w = threadIdx.x >> 6; w < 3) {
+      const int64_t time = tiles_time(count, tiled, 256 - 64 * w, rule, threadIdx.x & 63);
+      if ((threadIdx.x & 63) == 0) listed[2 + w] = static_cast<int>(min(time >> 8, static_cast<int64_t>(INT32_MAX)));
+    }
+    __syncthreads();
+  }
   if (threadIdx.x < kWave) {                     // where every expert's pairs and tiles begin: sums over the wave's lanes
     const int lane = threadIdx.x;
+    int limit = rule.rows;
+    if (limit == 0) {
+      int best = 0;
+      for (int w = 1; w < 3; ++w)
+        if (listed[2 + w] < listed[2 + best]) best = w;
+      limit = 256 - 64 * best;
+    }
     int at = 0, nt = 0;                          // of the experts in front of this run of 64
     for (int e0 = 0; e0 < experts; e0 += kWave) {
       const int e = e0 + lane;
-      const int pairs_e = e < experts ? count[e] : 0, tiles_e = (pairs_e + tile_rows - 1) / tile_rows;
+      const int pairs_e = e < experts ? count[e] : 0, tiles_e = e < tiled ? (pairs_e + limit - 1) / limit : 0;
       int p_sum = pairs_e, t_sum = tiles_e;
 #pragma unroll
       for (int o = 1; o < kWave; o <<= 1) {
@@ -427,32 +512,58 @@ __device__ __forceinline__ void group_pairs(const int32_t* __restrict__ chosen, 
       at += __shfl(p_sum, kWave - 1, kWave);
       nt += __shfl(t_sum, kWave - 1, kWave);
     }
-    if (lane == 0) *n_tiles = min(nt, max_tiles);
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < experts; e += blockDim.x) {
-    int nt = tstart[e];
-    for (int r0 = 0; r0 < count[e] && nt < max_tiles; r0 += tile_rows, ++nt) {
-      tile_expert[nt] = e;
-      tile_first[nt] = start[e] + r0;
-      tile_count[nt] = min(tile_rows, count[e] - r0);
+    if (lane == 0) {
+      listed[0] = min(nt, max_tiles);
+      listed[1] = limit;
     }
   }
-  if (threadIdx.x == 0) *tiles_out = *n_tiles;
-  for (int nt = *n_tiles + threadIdx.x; nt < max_tiles; nt += blockDim.x) tile_expert[nt] = -1;
-  for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
-    const int e = min(max(chosen[p], 0), experts - 1);
-    sorted[start[e] + atomicAdd(&cursor[e], 1)] = p;
+  __syncthreads();
+  const int n_tiles = listed[0], limit = listed[1];
+  for (int e = threadIdx.x; e < experts; e += blockDim.x) {
+    int at = start[e];
+    for (int w = 0; w < rows; ++w) {
+      const int counted = cursor[w * experts + e];
+      cursor[w * experts + e] = at;
+      at += counted;
+    }
+    const int c = e < tiled ? count[e] : 0, n = (c + limit - 1) / limit;
+    const int each = rule.rows != 0 ? limit : (c + max(n, 1) - 1) / max(n, 1);
+    int nt = tstart[e];
+    for (int r0 = 0; r0 < c && nt < max_tiles; r0 += each, ++nt) {
+      tile_expert[nt] = e;
+      tile_first[nt] = start[e] + r0;
+      tile_count[nt] = min(each, c - r0);
+    }
   }
+  if (threadIdx.x == 0) *tiles_out = n_tiles;
+  for (int nt = n_tiles + threadIdx.x; nt < max_tiles; nt += blockDim.x) tile_expert[nt] = -1;
+  if (tiled < experts && threadIdx.x == 0 && n_tiles < max_tiles) tile_first[n_tiles] = start[tiled];
+  __syncthreads();
+  int32_t* to = staged != nullptr ? staged : sorted;
+#pragma unroll
+  for (int i = 0; i < kKept; ++i) {
+    const int q = threadIdx.x + i * blockDim.x;
+    if (q >= quads) break;
+    to[atomicAdd(&own[bucket(kept[i].x)], 1)] = 4 * q;
+    to[atomicAdd(&own[bucket(kept[i].y)], 1)] = 4 * q + 1;
+    to[atomicAdd(&own[bucket(kept[i].z)], 1)] = 4 * q + 2;
+    to[atomicAdd(&own[bucket(kept[i].w)], 1)] = 4 * q + 3;
+  }
+#pragma unroll 4
+  for (int p = done + threadIdx.x; p < pairs; p += blockDim.x) to[atomicAdd(&own[bucket(chosen[p])], 1)] = p;
+  if (staged == nullptr) return;
+  __syncthreads();
+#pragma unroll 4
+  for (int p = threadIdx.x; p < pairs; p += blockDim.x) sorted[p] = staged[p];
 }
 
 __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t* __restrict__ chosen, int pairs, int experts,
-                                                         int tile_rows, int max_tiles, int32_t* __restrict__ sorted,
+                                                         TileRule rule, int identity, int max_tiles, int32_t* __restrict__ sorted,
                                                          int32_t* __restrict__ tile_expert, int32_t* __restrict__ tile_first,
                                                          int32_t* __restrict__ tile_count) {
-  extern __shared__ int32_t group_smem[];      // count, start, tstart, cursor [experts] each, n_tiles
-  group_pairs(chosen, pairs, experts, tile_rows, max_tiles, sorted, tile_expert, tile_first, tile_count, tile_count + max_tiles, group_smem,
-              group_smem + experts, group_smem + 2 * experts, group_smem + 3 * experts, group_smem + 4 * experts);
+  extern __shared__ int32_t group_smem[];
+  group_pairs(chosen, pairs, experts, rule, identity != 0, max_tiles, sorted, tile_expert, tile_first, tile_count, tile_count + max_tiles,
+              group_smem, pairs <= kGroupStaged ? group_smem + group_smem_ints(experts) : nullptr);
 }
 
 // The choice from logits and the sorting in one workgroup of 16 waves, for steps of so few tokens
@@ -463,8 +574,8 @@ __global__ __launch_bounds__(1024) void moe_topk_group_kernel(const float* __res
                                                               int32_t* __restrict__ tile_expert, int32_t* __restrict__ tile_first,
                                                               int32_t* __restrict__ tile_count, const float* __restrict__ bias,
                                                               RouterRule rule) {
-  extern __shared__ int32_t group_smem[];      // as above, then score[16][experts]
-  float* score = reinterpret_cast<float*>(group_smem + 4 * experts + 1) + (threadIdx.x >> 6) * experts;
+  extern __shared__ int32_t group_smem[];      // the sorting's integers, then score[16][experts]
+  float* score = reinterpret_cast<float*>(group_smem + group_smem_ints(buckets)) + (threadIdx.x >> 6) * experts;
   const int lane = threadIdx.x & (kWave - 1);
   for (int t = threadIdx.x >> 6; t < tokens; t += 16) {
     for (int e = lane; e < experts; e += kWave) score[e] = router_score(z[static_cast<int64_t>(t) * experts + e], bias, e, rule.mode);
@@ -474,8 +585,8 @@ __global__ __launch_bounds__(1024) void moe_topk_group_kernel(const float* __res
   }
   __threadfence_block();
   __syncthreads();                             // the workgroup's own writes of `chosen` are read below
-  group_pairs(chosen, tokens * top, buckets, tile_rows, max_tiles, sorted, tile_expert, tile_first, tile_count, tile_count + max_tiles, group_smem,
-              group_smem + experts, group_smem + 2 * experts, group_smem + 3 * experts, group_smem + 4 * experts);
+  group_pairs(chosen, tokens * top, buckets, TileRule{tile_rows, {0, 0}, {0, 0}}, false, max_tiles, sorted, tile_expert, tile_first, tile_count,
+              tile_count + max_tiles, group_smem, nullptr);
 }
 
 // k per staging round: with one tile of pairs a round of 64 leaves a wave two pieces of its matrix in flight, too few to
@@ -677,22 +788,24 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
 
 // ------------------------------------------------------------------ experts, many pairs each
 
-// A tile of TM pairs by TN rows of the expert's matrix per workgroup of WM x WN waves, both operands through LDS 64 k at a
-// time. The matrices of all experts are read at the rate the matrix cores use them only if a workgroup multiplies each byte
-// often: 256 x 256 asks for half the bytes per product of the kernel above, whose rows of the matrix go from memory to
-// registers for one tile of 128 pairs (14 TB/s out of the L2s at 16,384 pairs over 32 experts of 1,024 x 2,048: 250 us for
-// the first product, 143 for the second; here 187 and 123). What it does about each bound:
-//  * memory to LDS without registers (global_load_lds, 16 bytes a lane), the step after next always under way;
-//  * LDS rows of 128 bytes with the 16-byte pieces exchanged by row / 2, so that the 16 rows a read touches lie on all
-//    banks (the exchange is done by which piece a lane fetches: the copy itself writes lanes side by side);
-//  * the operands of half a step are read from LDS between the matrix instructions of the half before, and the one
-//    barrier of a step stands between its halves, where the matrix cores still have work;
-//  * an expert's tiles run on one die (its L2 then holds the expert's rows): die d takes the d-th eighth of the tiles;
-//  * the waves for pairs that a tile does not have skip the arithmetic, so an expert's last tile costs what it holds to
-//    half a tile.
+// A tile of up to TM pairs by TN rows of the expert's matrix per workgroup of WM x WN waves, both operands through LDS 64 k at a
+// time (tile_product.h has the loop). The matrices of all experts are read at the rate the matrix cores use them only if a workgroup
+// multiplies each byte often: 256 x 256 asks for half the bytes per product of the kernel above, whose rows of the matrix go
+// from memory to registers for one tile of 128 pairs (14 TB/s out of the L2s). What it does about each bound:
+//  * an expert's tiles run on one die (its L2 then holds the expert's rows): die d takes the d-th eighth of the work;
+//  * a chip of 256 units runs large tiles in a few rounds, whose last one is seldom full, and an expert with a few pairs more than
+//    whole tiles costs one more: with TM 256 the sorting cuts every expert's pairs evenly under the limit (256, 192 or 128) that
+//    gives the step's counts the least time, and a tile runs the loop that is made for its size (us of the first and second
+//    product at 16,384 pairs over 32 experts of 2,048 x 1,024, choices at random: 190 + 124 in tiles of 256, 170 + 111 so; at 14,336
+//    pairs in tiles of 128 163 + 117);
+//  * as many workgroups as there are units stay and walk the tiles: the grid of the most tiles there could be had half of its
+//    workgroups leave at once, each from a unit of its own;
+//  * the waves for pairs that a tile does not have skip the arithmetic.
 // GATED: a wave's 64 rows are 32 gate rows and the 32 up rows of the same columns.
-typedef __attribute__((address_space(1))) const void* global_ptr;
-typedef __attribute__((address_space(3))) void* lds_ptr;
+
+// LDS of the steps of a workgroup's tile: two of the largest, as many of a smaller one as fit there.
+constexpr int tile_smem_steps(int tm, int tn) { return 2 * (tm + tn) * 128 + (tm == 256 ? 16 * 1024 : 0); }
+constexpr int tile_stages(int tm, int tn, int rows) { return std::min(3, tile_smem_steps(tm, tn) / ((rows + tn) * 128)); }
 
 template <int TM, int TN, int WM, int WN, int FORM>
 __global__ __launch_bounds__(64 * WM * WN, 2) void moe_tile_kernel(
@@ -700,144 +813,116 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void moe_tile_kernel(
     const int32_t* __restrict__ sorted, const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_first,
     const int32_t* __restrict__ tile_count, const int32_t* __restrict__ n_tiles, bf16_t* __restrict__ out_act,
     float* __restrict__ out_f32, int64_t tokens, int K, int N, int top, float gate_alpha, float limit, float up_shift,
-    int into_stream, const float* __restrict__ col_scale, int experts, const bf16_t* __restrict__ x,
+    int into_stream, const float* __restrict__ col_scale, int identity_to, const bf16_t* __restrict__ x,
     const float* __restrict__ weight, int column_tiles) {
   constexpr bool GATED = FORM == kFormGated;
-  constexpr int WV = WM * WN, BK = 64, RM = TM / WM / 16, RN = TN / WN / 16, WROWS = TN / WN;
+  constexpr int WV = WM * WN, BK = 64, RN = TN / WN / 16, WROWS = TN / WN;
   constexpr int COLS = GATED ? TN / 2 : TN, WCOLS = GATED ? WROWS / 2 : WROWS;   // columns of the workgroup, of a wave
-  constexpr int LA = TM / 8 / WV, LB = TN / 8 / WV;                              // copies of 8 rows per wave and step
-  __shared__ __align__(16) bf16_t a0[TM * BK], a1[TM * BK], b0[TN * BK], b1[TN * BK];
-  __shared__ int32_t pair_s[TM];
-  const int tiles = *n_tiles, per_die = (tiles + 7) / 8;
-  const int at = static_cast<int>(blockIdx.x >> 3), slot = static_cast<int>(blockIdx.x & 7) * per_die + at / column_tiles;
-  if (at / column_tiles >= per_die || slot >= tiles) return;                     // uniform for the workgroup
-  const int n0 = at % column_tiles * COLS;
-  const int e = tile_expert[slot], first = tile_first[slot], count = tile_count[slot];
-  if (e >= experts) {                           // a tile of identity pairs: the tokens themselves times their weights
-    if (FORM != kFormDown) return;
-    for (int idx = threadIdx.x; idx < count * COLS; idx += 64 * WV) {
-      const int pair = sorted[first + idx / COLS], n = n0 + idx % COLS;
-      if (n >= N) continue;
-      const int64_t t = pair / top;
-      const float y = weight[pair] * bf16_to_float(x[t * N + n]);
-      if (into_stream) add_float(out_f32 + t * N + n, col_scale != nullptr ? col_scale[n] * y : y);
-      else out_f32[(static_cast<int64_t>(pair % top) * tokens + t) * N + n] = y;
-    }
-    return;
-  }
+  constexpr int LB = TN / 8 / WV;                                                // copies of 8 rows of the matrix per wave and step
+  extern __shared__ __align__(16) unsigned char tile_smem[];                     // the steps of tile_product, then int32_t[TM]
+  int32_t* pair_s = reinterpret_cast<int32_t*>(tile_smem + tile_smem_steps(TM, TN));
+  // The work of this workgroup's die: an eighth of all (tile, columns).
+  const int tiles = *n_tiles, die = static_cast<int>(blockIdx.x & 7);
+  const int from = static_cast<int>(static_cast<int64_t>(tiles) * column_tiles * die / 8);
+  const int to = static_cast<int>(static_cast<int64_t>(tiles) * column_tiles * (die + 1) / 8);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int r = lane & 15, g = lane >> 4;
-  const int wm = wave / WN * (TM / WM), wn = wave % WN;                          // waves of a SIMD share no rows of pairs
-  for (int i = threadIdx.x; i < TM; i += 64 * WV) pair_s[i] = i < count ? sorted[first + i] : -1;
-  // What this lane copies: piece p of row 8 j + lane / 8 of an operand lies at place lane % 8 of that row.
-  const char* a_base = reinterpret_cast<const char*>(a);
-  const char* w_base = reinterpret_cast<const char*>(w + static_cast<int64_t>(e) * (GATED ? 2 : 1) * N * K);
-  uint32_t a_off[LA], b_off[LB];
+  const int wn = wave % WN;
+  for (int at = from + static_cast<int>(blockIdx.x >> 3); at < to; at += static_cast<int>(gridDim.x >> 3)) {   // uniform for the workgroup
+    const int slot = at / column_tiles, n0 = at % column_tiles * COLS;
+    const int e = tile_expert[slot], first = tile_first[slot], count = min(tile_count[slot], TM);
+    const char* w_base = reinterpret_cast<const char*>(w + static_cast<int64_t>(e) * (GATED ? 2 : 1) * N * K);
+    __syncthreads();                            // everybody is done with the tile before: its pairs, its last step in LDS
+    for (int i = threadIdx.x; i < TM; i += 64 * WV) pair_s[i] = i < count ? sorted[first + i] : -1;
+    __syncthreads();
+    // RM tiles of 16 pairs for each of the WM waves that share columns.
+    auto product = [&](auto rm) {
+      constexpr int RM = decltype(rm)::value, ROWS = RM * 16 * WM, LA = ROWS / 8 / WV;
+      static_assert(LA * 8 * WV == ROWS && LB * 8 * WV == TN, "whole copies per wave");
+      uint32_t a_off[LA], b_off[LB];
 #pragma unroll
-  for (int i = 0; i < LA; ++i) {
-    const int row = (wave * LA + i) * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
-    const int pair = sorted[first + min(row, count - 1)];
-    a_off[i] = static_cast<uint32_t>(FORM != kFormDown ? pair / top : pair) * (2u * K) + 16u * piece;
-  }
-#pragma unroll
-  for (int i = 0; i < LB; ++i) {
-    const int row = (wave * LB + i) * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
-    const int col = min(n0 + (row / WROWS) * WCOLS + row % WCOLS, N - 1);
-    b_off[i] = static_cast<uint32_t>(GATED && row % WROWS >= WCOLS ? N + col : col) * (2u * K) + 16u * piece;
-  }
-  auto copy = [&](int k0, bf16_t* as, bf16_t* bs) {
-#pragma unroll
-    for (int i = 0; i < LA; ++i)
-      __builtin_amdgcn_global_load_lds((global_ptr)(a_base + a_off[i] + 2 * k0), (lds_ptr)(as + (wave * LA + i) * 8 * BK), 16, 0, 0);
-#pragma unroll
-    for (int i = 0; i < LB; ++i)
-      __builtin_amdgcn_global_load_lds((global_ptr)(w_base + b_off[i] + 2 * k0), (lds_ptr)(bs + (wave * LB + i) * 8 * BK), 16, 0, 0);
-  };
-  f32x4 acc[RN][RM];
-#pragma unroll
-  for (int i = 0; i < RN; ++i)
-#pragma unroll
-    for (int j = 0; j < RM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const bool works = wm < count;
-  const int swap = (r >> 1) & 7;
-  bf16x8 fa[2][RM], fb[2][RN];
-  auto operands = [&](const bf16_t* as, const bf16_t* bs, int half) {
-    const int c = ((half * 4 + g) ^ swap) * 8;
-#pragma unroll
-    for (int i = 0; i < RN; ++i) fb[half][i] = *reinterpret_cast<const bf16x8*>(bs + (wn * WROWS + i * 16 + r) * BK + c);
-#pragma unroll
-    for (int j = 0; j < RM; ++j) fa[half][j] = *reinterpret_cast<const bf16x8*>(as + (wm + j * 16 + r) * BK + c);
-  };
-  auto multiply = [&](int half) {
-#pragma unroll
-    for (int i = 0; i < RN; ++i)
-#pragma unroll
-      for (int j = 0; j < RM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[half][i], fa[half][j], acc[i][j], 0, 0, 0);
-#pragma unroll
-    for (int q = 0; q < RM + RN; ++q) {                                          // one read of the other half's operands, then
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                         // the matrix instructions it hides behind
-      __builtin_amdgcn_sched_group_barrier(0x008, RM * RN / (RM + RN), 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, RM * RN, 0);
-  };
-  const int steps = K / BK;
-  auto step = [&](bf16_t* ca, bf16_t* cb, bf16_t* na, bf16_t* nb, int t) {
-    if (works) {
-      operands(ca, cb, 1);
-      multiply(0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();                            // step t + 1 has arrived, and everybody has read step t
-    if (t + 2 < steps) copy((t + 2) * BK, ca, cb);
-    __builtin_amdgcn_sched_barrier(0);
-    if (works) {
-      operands(na, nb, 0);                      // behind the last step: what lies there, not used
-      multiply(1);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  copy(0, a0, b0);
-  __syncthreads();
-  if (steps > 1) copy(BK, a1, b1);
-  __builtin_amdgcn_sched_barrier(0);
-  if (works) operands(a0, b0, 0);
-  for (int t = 0; t < steps; t += 2) {
-    step(a0, b0, a1, b1, t);
-    if (t + 1 < steps) step(a1, b1, a0, b0, t + 1);
-  }
-  if (!works) return;
-  // Lane (r, g) holds, for the pair in row wm + 16 j + r, columns 4 g .. + 3 of every 16 of the wave's.
-#pragma unroll
-  for (int j = 0; j < RM; ++j) {
-    const int pair = pair_s[wm + j * 16 + r];
-    if (pair < 0) continue;
-    const float pw = pair_weight != nullptr ? pair_weight[pair] : 1.f;           // on the input's sums (GATED) or on the output's
-#pragma unroll
-    for (int i = 0; i < WCOLS / 16; ++i) {
-      const int nc = n0 + wn * WCOLS + i * 16 + 4 * g;
-      if (nc >= N) continue;                                                     // N is a multiple of 8
-      if (FORM != kFormDown) {
-        bf16_t res[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          if (!GATED) {
-            const float p = fmaxf(pw * acc[i][j][v], 0.f);
-            res[v] = float_to_bf16(p * p);
-            continue;
-          }
-          const float gg = fminf(pw * acc[i][j][v], limit);
-          const float uu = fminf(fmaxf(pw * acc[(i + RN / 2) % RN][j][v], -limit), limit);
-          res[v] = float_to_bf16(gg / (1.f + __expf(-gate_alpha * gg)) * (uu + up_shift));
-        }
-        *reinterpret_cast<ushort4*>(out_act + static_cast<int64_t>(pair) * N + nc) = ushort4{res[0], res[1], res[2], res[3]};
-      } else if (into_stream) {
-        float* o = out_f32 + static_cast<int64_t>(pair / top) * N + nc;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) add_float(o + v, (col_scale != nullptr ? col_scale[nc + v] : 1.f) * (pw * acc[i][j][v]));
-      } else {
-        float* o = out_f32 + (static_cast<int64_t>(pair % top) * tokens + pair / top) * N + nc;
-        *reinterpret_cast<float4*>(o) = float4{pw * acc[i][j][0], pw * acc[i][j][1], pw * acc[i][j][2], pw * acc[i][j][3]};
+      for (int i = 0; i < LA; ++i) {
+        const int row = (wave * LA + i) * 8 + (lane >> 3);
+        const int pair = pair_s[min(row, count - 1)];
+        a_off[i] = static_cast<uint32_t>(FORM != kFormDown ? pair / top : pair) * (2u * K) + 16u * tile_copy_piece(row, lane);
       }
+#pragma unroll
+      for (int i = 0; i < LB; ++i) {
+        const int row = (wave * LB + i) * 8 + (lane >> 3);
+        const int col = min(n0 + (row / WROWS) * WCOLS + row % WCOLS, N - 1);
+        b_off[i] = static_cast<uint32_t>(GATED && row % WROWS >= WCOLS ? N + col : col) * (2u * K) + 16u * tile_copy_piece(row, lane);
+      }
+      const int wm = wave / WN * (RM * 16);                                      // waves of a SIMD share no rows of pairs
+      const bool works = wm < count;
+      tile_f32x4 acc[RN][RM];
+#pragma unroll
+      for (int i = 0; i < RN; ++i)
+#pragma unroll
+        for (int j = 0; j < RM; ++j) acc[i][j] = tile_f32x4{0.f, 0.f, 0.f, 0.f};
+      tile_product<tile_stages(TM, TN, ROWS), ROWS, TN>(acc, tile_smem, reinterpret_cast<const char*>(a), w_base, a_off, b_off, wm,
+                                                         wn * WROWS, wave, lane, K / BK, works);
+      if (!works) return;
+      // Lane (r, g) holds, for the pair in row wm + 16 j + r, columns 4 g .. + 3 of every 16 of the wave's.
+#pragma unroll
+      for (int j = 0; j < RM; ++j) {
+        const int pair = pair_s[wm + j * 16 + r];
+        if (pair < 0) continue;
+        const float pw = pair_weight != nullptr ? pair_weight[pair] : 1.f;       // on the input's sums (GATED) or on the output's
+#pragma unroll
+        for (int i = 0; i < WCOLS / 16; ++i) {
+          const int nc = n0 + wn * WCOLS + i * 16 + 4 * g;
+          if (nc >= N) continue;                                                 // N is a multiple of 8
+          if (FORM != kFormDown) {
+            bf16_t res[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              if (!GATED) {
+                const float p = fmaxf(pw * acc[i][j][v], 0.f);
+                res[v] = float_to_bf16(p * p);
+                continue;
+              }
+              const float gg = fminf(pw * acc[i][j][v], limit);
+              const float uu = fminf(fmaxf(pw * acc[(i + RN / 2) % RN][j][v], -limit), limit);
+              res[v] = float_to_bf16(gg / (1.f + __expf(-gate_alpha * gg)) * (uu + up_shift));
+            }
+            *reinterpret_cast<ushort4*>(out_act + static_cast<int64_t>(pair) * N + nc) = ushort4{res[0], res[1], res[2], res[3]};
+          } else if (into_stream) {
+            float* o = out_f32 + static_cast<int64_t>(pair / top) * N + nc;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) add_float(o + v, (col_scale != nullptr ? col_scale[nc + v] : 1.f) * (pw * acc[i][j][v]));
+          } else {
+            float* o = out_f32 + (static_cast<int64_t>(pair % top) * tokens + pair / top) * N + nc;
+            *reinterpret_cast<float4*>(o) = float4{pw * acc[i][j][0], pw * acc[i][j][1], pw * acc[i][j][2], pw * acc[i][j][3]};
+          }
+        }
+      }
+    };
+    constexpr int MOST = TM / WM / 16;
+    if constexpr (MOST == 8) {
+      if (count <= TM / 4) product(std::integral_constant<int, MOST / 4>{});
+      else if (count <= TM / 2) product(std::integral_constant<int, MOST / 2>{});
+      else if (count <= TM / 4 * 3) product(std::integral_constant<int, MOST / 4 * 3>{});
+      else product(std::integral_constant<int, MOST>{});
+    } else {
+      product(std::integral_constant<int, MOST>{});
+    }
+  }
+  // The identity pairs lie behind the experts' and have no tiles: the tokens themselves times their weights, dealt out over all threads.
+  if (FORM != kFormDown || identity_to == 0) return;
+  const int begin = tile_first[tiles], quads = N / 4;                            // N is a multiple of 8
+  const int64_t all = static_cast<int64_t>(identity_to - begin) * quads;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * (64 * WV) + threadIdx.x; i < all; i += static_cast<int64_t>(gridDim.x) * (64 * WV)) {
+    const int pair = sorted[begin + i / quads], n = static_cast<int>(i % quads) * 4;
+    const int64_t t = pair / top;
+    const float wt = weight[pair];
+    const ushort4 in = *reinterpret_cast<const ushort4*>(x + t * N + n);
+    const float4 y{wt * bf16_to_float(in.x), wt * bf16_to_float(in.y), wt * bf16_to_float(in.z), wt * bf16_to_float(in.w)};
+    if (into_stream) {
+      const float* ys = &y.x;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) add_float(out_f32 + t * N + n + v, col_scale != nullptr ? col_scale[n + v] * ys[v] : ys[v]);
+    } else {
+      *reinterpret_cast<float4*>(out_f32 + (static_cast<int64_t>(pair % top) * tokens + t) * N + n) = y;
     }
   }
 }
@@ -852,7 +937,7 @@ struct ExpertCall {
   void* act;
   float* out;
   int64_t tokens;
-  int K, F, experts, top, kind;        // experts: those with matrices
+  int K, F, experts, identity, top, kind;        // experts: those with matrices
   float gate_alpha, limit, up_shift;
   int weight_on_output, into_stream;
   const float* col_scale;
@@ -884,7 +969,11 @@ static int launch_grouped(hipStream_t s, const ExpertCall& c, const int32_t* int
 }
 
 template <int TM, int TN, int WM, int WN, int FORM>
-static void run_tiles(hipStream_t s, const ExpertCall& c, const int32_t* ints, int max_tiles) {
+static int run_tiles(hipStream_t s, const ExpertCall& c, const int32_t* ints, int max_tiles) {
+  constexpr size_t kSmem = tile_smem_steps(TM, TN) + TM * sizeof(int32_t);
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(moe_tile_kernel<TM, TN, WM, WN, FORM>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                          static_cast<int>(kSmem)) != hipSuccess)
+    return fail("psamd_moe_experts_grouped: " + std::to_string(kSmem) + " bytes of LDS were refused");
   const int32_t* sorted = ints;
   const int32_t* t_e = ints + c.tokens * c.top;
   const int32_t* t_f = t_e + max_tiles;
@@ -892,21 +981,24 @@ static void run_tiles(hipStream_t s, const ExpertCall& c, const int32_t* ints, i
   constexpr bool down = FORM == kFormDown;
   const int N = down ? c.K : c.F, K = down ? c.F : c.K;
   const int column_tiles = static_cast<int>(ceil_div(N, FORM == kFormGated ? TN / 2 : TN));
-  const dim3 grid(static_cast<unsigned>(8 * ceil_div(max_tiles, 8) * column_tiles));
-  moe_tile_kernel<TM, TN, WM, WN, FORM><<<grid, dim3(64 * WM * WN), 0, s>>>(
+  // Of the large tiles one workgroup fills a compute unit: as many as there are units walk the tiles. The small ones come one each.
+  const int64_t most = 8 * ceil_div(static_cast<int64_t>(max_tiles) * column_tiles, 8);
+  const dim3 grid(static_cast<unsigned>(TM == 256 ? std::min<int64_t>(most, 256) : most));
+  moe_tile_kernel<TM, TN, WM, WN, FORM><<<grid, dim3(64 * WM * WN), kSmem, s>>>(
       static_cast<const bf16_t*>(down ? c.act : c.x), (c.weight_on_output != 0) == down ? c.weight : nullptr,
       static_cast<const bf16_t*>(down ? c.w_down : c.w_in), sorted, t_e, t_f, t_c, t_c + max_tiles,
       down ? nullptr : static_cast<bf16_t*>(c.act), down ? c.out : nullptr, c.tokens, K, N, c.top, c.gate_alpha, c.limit,
-      c.up_shift, c.into_stream, c.col_scale, c.experts, static_cast<const bf16_t*>(c.x), c.weight, column_tiles);
+      c.up_shift, c.into_stream, c.col_scale, c.identity > 0 ? static_cast<int>(c.tokens * c.top) : 0,
+      static_cast<const bf16_t*>(c.x), c.weight, column_tiles);
+  return check_launch("psamd_moe_experts_grouped (tiles)");
 }
 
 template <int TM, int TN, int WM, int WN>
 static int launch_tiles(hipStream_t s, const ExpertCall& c, const int32_t* ints, int max_tiles) {
-  if (c.kind == kExpertGated) run_tiles<TM, TN, WM, WN, kFormGated>(s, c, ints, max_tiles);
-  else run_tiles<TM, TN, WM, WN, kFormSquaredRelu>(s, c, ints, max_tiles);
-  if (check_launch("psamd_moe_experts_grouped (in)")) return 1;
-  run_tiles<TM, TN, WM, WN, kFormDown>(s, c, ints, max_tiles);
-  return check_launch("psamd_moe_experts_grouped (down)");
+  if (c.kind == kExpertGated ? run_tiles<TM, TN, WM, WN, kFormGated>(s, c, ints, max_tiles)
+                             : run_tiles<TM, TN, WM, WN, kFormSquaredRelu>(s, c, ints, max_tiles))
+    return 1;
+  return run_tiles<TM, TN, WM, WN, kFormDown>(s, c, ints, max_tiles);
 }
 
 // Whether the tiles of the kernel for many pairs take these experts: whole steps of 64 k in both products, and offsets inside
@@ -917,30 +1009,31 @@ static bool tiles_take(int64_t tokens, int64_t pairs, int K, int F) {
 }
 
 // ... and their rows: 0 where the kernel above takes the step (from 48 pairs an expert on it is the slower one everywhere; below,
-// the router's kernel may have sorted the pairs into its tiles). Tiles of 256 x 256 ask for half the bytes per product, but one
-// workgroup of them fills a compute unit, two of 128 x 128 share one, and a last round that is not full costs nearly as much as one
-// that is: the time is that of the rounds, K long in the first product and F in the second, and a round of large tiles takes
-// about one and a half of small ones. An expert's last tile is half empty on average. us of both products
-// and the sorting, 256 x 256 / 128 x 128 / the kernel above (E experts of K x F):
-//   32 of 2,048 x 1,024:  60 pairs an expert 117 / 113 / 156, 200 144 / 163 / 269, 512 321 / 339 / 396, 700 334 / 411 / 481, 2,000 928 / 1,124 / 1,245
-//    8 of 2,048 x 1,024:  60 60 / 47 / 78, 300 89 / 56 / 96, 700 94 / 100 / 129, 1,000 177 / 151 / 193, 3,000 315 / 406 / 468
-//    8 of 4,096 x 3,584:  60 216 / 189 / 258, 300 341 / 453 / 443, 600 585 / 795 / 710, 2,000 1,575 / 2,192 / 1,930
-//   24 of 1,024 x 320:    300 61 / 49 / 67, 768 116 / 86 / 110, 3,000 303 / 318 / 380
-//    4 of 1,024 x 512:    60 37 / 29 / 44, 512 61 / 36 / 60, 3,000 72 / 74 / 91
-// Over 480 steps of eight shapes, 60 to 2,000 pairs an expert, choices at random, uneven and very uneven, the choice is on average
-// 1.6% over the faster tile and in none slower than the kernel above (one bound at 480 pairs an expert: 4.4%, nine); at worst 34%,
-// where a round is just full or just not.
+// the router's kernel may have sorted the pairs into its tiles), 256 where the device chooses tiles of up to 256 x 256 by the step's
+// counts. Those ask for half the bytes per product, but one workgroup of them fills a compute unit, two of 128 x 128 share one, and a
+// last round that is not full costs nearly as much as one that is: the time is that of the rounds, K long in the first product and F
+// in the second, and 300 more for what a large tile does in front of and behind its loop, which the two small ones on a unit do beside
+// each other's. An expert's last tile is half empty on average. us of both products and the sorting, 256 / 128 / the kernel above
+// (E experts of K x F, choices at random):
+//   32 of 2,048 x 1,024:  50 pairs an expert 116 / 111 / 119, 140 141 / 156 / 228, 260 195 / 218 / 265, 448 257 / 284 / 345, 1,000 559 / 591 / 683
+//    8 of 2,048 x 1,024:  64 48 / 46 / 79, 300 68 / 61 / 100, 512 91 / 104 / 135, 1,000 163 / 163 / 229, 2,000 243 / 265 / 344
+//    8 of 4,096 x 3,584:  64 167 / 158 / 263, 260 325 / 422 / 418, 448 383 / 531 / 547, 1,000 757 / 1,007 / 942
+//   24 of 1,024 x 320:    64 33 / 33 / 47, 512 80 / 75 / 97, 2,000 245 / 203 / 270
+//    4 of 1,024 x 512:    64 31 / 28 / 43, 512 48 / 37 / 61, 2,000 65 / 61 / 81
+//   64 of 2,048 x 1,408:  64 263 / 261 / 373, 448 635 / 734 / 897, 2,000 2,529 / 3,044 / 3,354
+// Over these shapes at 15 sizes, choices at random and uneven, the choice is on average 0.5% over the faster (always 256: 6.6%, always
+// 128: 6.7%), at worst 12%.
 static int wide_tile_rows(int64_t pairs, int experts, int K, int F, int kind) {
   if (pairs < 48LL * experts) return 0;
-  auto rounds = [&](int rows, int at_once) {
+  auto rounds = [&](int rows, int at_once, int beside) {
     const double tiles = std::max<double>(experts, static_cast<double>(pairs) / rows + 0.5 * experts);
     auto of = [&](int64_t columns) {
       const double full = tiles * columns / at_once;
       return 0.5 * (std::ceil(full) + std::max(full, 1.0));
     };
-    return of(ceil_div(F, kind == kExpertGated ? rows / 2 : rows)) * K + of(ceil_div(K, rows)) * F;
+    return of(ceil_div(F, kind == kExpertGated ? rows / 2 : rows)) * (K + beside) + of(ceil_div(K, rows)) * (F + beside);
   };
-  return 1.55 * rounds(256, 256) < rounds(128, 512) ? 256 : 128;
+  return 1.2 * rounds(256, 256, 300) < rounds(128, 512, 0) ? 256 : 128;
 }
 
 template <typename A>
@@ -1040,7 +1133,7 @@ int psamd_moe_topk_group(void* stream, const float* logits, int32_t* chosen, flo
   const int64_t pairs = tokens * top;
   const int rows = psamd_moe_grouped_tile_rows(pairs, buckets);
   const int max_tiles = psamd_moe_grouped_max_tiles(pairs, buckets);
-  moe_topk_group_kernel<<<dim3(1), dim3(1024), sizeof(int32_t) * (4 * experts + 1) + sizeof(float) * 16 * experts,
+  moe_topk_group_kernel<<<dim3(1), dim3(1024), sizeof(int32_t) * group_smem_ints(buckets) + sizeof(float) * 16 * experts,
                           static_cast<hipStream_t>(stream)>>>(logits, chosen, weight, static_cast<int>(tokens), experts, buckets, top, rows,
                                                               max_tiles, ints, ints + pairs, ints + pairs + max_tiles,
                                                               ints + pairs + 2 * max_tiles, bias, rule);
@@ -1057,7 +1150,7 @@ int psamd_moe_experts_rows(void* stream, const void* x, const int32_t* chosen, c
   PSAMD_REQUIRE(tokens * top <= 2147483647LL && ceil_div(std::max(K, F), kRowsPerBlock) <= 65535, "too large for one launch");
   if (tokens == 0) return 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const ExpertCall c{x, chosen, weight, w_in, w_down, act, out, tokens, K, F, experts, top, kind,
+  const ExpertCall c{x, chosen, weight, w_in, w_down, act, out, tokens, K, F, experts, identity, top, kind,
                      gate_alpha, limit, up_shift, weight_on_output, into_stream, col_scale};
   if (dtype == kBF16) return launch_experts_rows<bf16_t>(s, c);
   if (dtype == kF32) return launch_experts_rows<float>(s, c);
@@ -1095,15 +1188,22 @@ int psamd_moe_experts_grouped(void* stream, const void* x, const int32_t* chosen
   // Pairs that the router's kernel has sorted lie in the tiles of a small step.
   const int wide = grouped_already == 0 && tiles_take(tokens, pairs, K, F) ? wide_tile_rows(pairs, buckets, K, F, kind) : 0;
   const int rows = wide != 0 ? wide : psamd_moe_grouped_tile_rows(pairs, buckets);
-  const int max_tiles = static_cast<int>(std::min<int64_t>(ceil_div(pairs, rows) + buckets, pairs));
+  const int least = rows == 256 ? 128 : rows;                // the device may cut into tiles of 128
+  const int max_tiles = static_cast<int>(std::min<int64_t>(ceil_div(pairs, least) + buckets, pairs));
   PSAMD_REQUIRE(max_tiles <= 65535, "too many tiles for one launch");
   if (grouped_already == 0) {
-    moe_group_kernel<<<dim3(1), dim3(1024), sizeof(int32_t) * (4 * buckets + 1), s>>>(
-        chosen, static_cast<int>(pairs), buckets, rows, max_tiles, ints, ints + pairs, ints + pairs + max_tiles,
+    const TileRule rule{rows == 256 ? 0 : rows,
+                        {static_cast<int>(ceil_div(F, kind == kExpertGated ? 128 : 256)), static_cast<int>(ceil_div(K, 256))}, {K, F}};
+    const size_t smem = sizeof(int32_t) * (group_smem_ints(buckets) + (pairs <= kGroupStaged ? pairs : 0));
+    if (smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(moe_group_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                static_cast<int>(smem)) != hipSuccess)
+      return fail("psamd_moe_experts_grouped: " + std::to_string(smem) + " bytes of LDS were refused");
+    moe_group_kernel<<<dim3(1), dim3(1024), smem, s>>>(
+        chosen, static_cast<int>(pairs), buckets, rule, identity > 0 && wide != 0, max_tiles, ints, ints + pairs, ints + pairs + max_tiles,
         ints + pairs + 2 * max_tiles);
     if (check_launch("psamd_moe_experts_grouped (grouping)")) return 1;
   }
-  const ExpertCall c{x, chosen, weight, w_in, w_down, act, out, tokens, K, F, experts, top, kind,
+  const ExpertCall c{x, chosen, weight, w_in, w_down, act, out, tokens, K, F, experts, identity, top, kind,
                      gate_alpha, limit, up_shift, weight_on_output, into_stream, col_scale};
   if (wide == 256) return launch_tiles<256, 256, 2, 4>(s, c, ints, max_tiles);
   if (wide == 128) return launch_tiles<128, 128, 2, 2>(s, c, ints, max_tiles);

@@ -1240,6 +1240,17 @@ def test_experts_with_many_pairs_each(ops, counts, k, f, kind, on_output, identi
     assert rel(out[0, :t], want) < 3e-3 and torch.all(out[0, t] == 7.0)
 
 
+@pytest.mark.parametrize("counts,kind,identity", [
+    ((0, 1, 63, 64, 65, 127, 128, 129, 192, 193, 255, 256, 257, 0, 300, 512, 513, 514), "gated", 0),   # every size of tile, and none
+    ((200, 193, 192, 257, 0, 190, 191, 250, 64, 300, 201, 202, 203, 204, 205, 206, 207, 208, 209), "gated", 3),
+    ((520, 513, 512, 1, 530, 519, 521, 522, 523, 524, 525, 1040), "gated", 0),
+    ((520, 513, 512, 1, 530, 519, 521, 522, 523, 524, 525, 1040, 600, 0, 511, 640, 512, 512, 514, 700), "squared_relu", 2),
+])
+def test_experts_in_tiles_cut_by_the_counts(ops, counts, kind, identity):
+    """Sizes at which the device chooses how every expert's pairs are cut into tiles, against the same float64."""
+    test_experts_with_many_pairs_each(ops, counts, 2048, 1024, kind, True, identity)
+
+
 @pytest.mark.parametrize("hq,hkv,d,window", [(8, 2, 64, None), (16, 1, 16, None), (8, 4, 32, 130), (4, 4, 128, 33), (8, 1, 64, 16)])
 @pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
 def test_float32_attention_of_values_that_are_not_finite(ops, hq, hkv, d, window, bad):
