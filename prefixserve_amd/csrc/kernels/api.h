@@ -315,6 +315,19 @@ int psamd_qkv_rope_append(void* stream, const void* x, const void* w, void* qkv_
                           int head_dim, const int32_t* positions, const float* table, void* kv,
                           const int32_t* write_slot);
 
+// bfloat16 products of more than 128 tokens in tiles, fused with what follows them, where they are faster than the library's product
+// and the kernels behind it (all pointers on 16 bytes, K a multiple of 64, n_out of 16). psamd_linear_tile_slices: for a product
+// that is added to the float32 residual stream, -1 (take the library), 0 (psamd_linear_tile_stream adds it into `out`, the stream) or
+// the number of float32 K-slices [slices][M, n_out] that it leaves in `out` (slices x M stays within 4,608). The others return 2
+// where the library is to be taken: _plain leaves bfloat16 to the norm behind it; w of _gated is [gate; up] and activation
+// 0 (silu), 1 (relu) or 2 (gelu, tanh form); _qkv takes what psamd_qkv_rope_append does.
+int psamd_linear_tile_slices(const void* x, const void* w, int M, int n_out, int K);
+int psamd_linear_tile_stream(void* stream, const void* x, const void* w, float* out, int M, int n_out, int K);
+int psamd_linear_tile_plain(void* stream, const void* x, const void* w, void* out, int M, int n_out, int K);
+int psamd_linear_tile_gated(void* stream, const void* x, const void* w, void* out, int M, int n_out, int K, int activation);
+int psamd_linear_tile_qkv(void* stream, const void* x, const void* w, void* qkv_out, int M, int K, int hq, int hkv, int head_dim,
+                          const int32_t* positions, const float* table, void* kv, const int32_t* write_slot);
+
 // Small steps without a norm kernel and without partial slices to add up (bfloat16, M <= 16):
 // the products that feed the residual stream add into it (psamd_linear_skinny_add: float atomics, each
 // column times col_scale [n_out] where that is given,

@@ -51,6 +51,11 @@ _SIGNATURES = {
     "psamd_swiglu": [_vp, _vp, _vp, _i32, _i64, _i32, _i32],
     "psamd_rope_kv_append": [_vp, _vp, _i32, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp],
     "psamd_linear": [_vp, _vp, _i32, _vp, _i32, _vp, _i32, _i64, _i32, _i32],
+    "psamd_linear_tile_slices": [_vp, _vp, _i32, _i32, _i32],
+    "psamd_linear_tile_stream": [_vp, _vp, _vp, _vp, _i32, _i32, _i32],
+    "psamd_linear_tile_plain": [_vp, _vp, _vp, _vp, _i32, _i32, _i32],
+    "psamd_linear_tile_gated": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32],
+    "psamd_linear_tile_qkv": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp],
     "psamd_gemm_lt": [_vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _i32],
     "psamd_linear_skinny": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32],
     "psamd_linear_skinny_ksplit": [_i32, _i32, _i32],
@@ -155,6 +160,7 @@ class HipOps:
     SKINNY_MAX_ROWS = 64
     STREAM_MAX_ROWS = 128           # whole 64-element steps of K and aligned operands: the products with both operands through LDS
     FUSED_SWIGLU_MAX_ROWS = 32      # above it what _through_lds does not take goes to the library, where there is one (o, down, q/k/v: above SKINNY_MAX_ROWS)
+    TILE_SLICE_ROWS = 4608          # K-slices x tokens of a product of more tokens than that whose sums the norm behind it adds up
     LIBRARY_ADD_MIN_ROWS = 1024     # from here on a product that feeds the residual stream adds into it in the library
     MOE_ROUTE_FUSED_MAX_TOKENS = 0   # up to here one kernel computes router logits and choice; above, product + choice
     MOE_CHOICE_SORTS_MAX_TOKENS = 16 # up to here the workgroup that chooses a step's experts also sorts the pairs
@@ -639,7 +645,8 @@ class HipOps:
 
     def qkv_rope_append(self, x, w_qkv, qkv, hq: int, hkv: int, d: int, positions, table, kv, write_slot) -> None:
         """qkv = x @ w_qkv^T, q and k rotated, k and v written to their pages. One kernel for a
-        bfloat16 step of at most 64 tokens (128: ``_through_lds``); otherwise the product followed by ``rope_kv_append``."""
+        bfloat16 step of at most 64 tokens (128: ``_through_lds``; more: where the tiles of linear_tile.hip are the faster);
+        otherwise the product followed by ``rope_kv_append``."""
         m, k = x.shape
         if isinstance(x, NormedRows):
             if (x.rows is None and d % 16 == 0 and qkv.dtype == torch.bfloat16 and self.fuses_norm(m, k, x.dtype)):
@@ -659,8 +666,9 @@ class HipOps:
                     positions.data_ptr(), _ptr(table), _ptr(kv), None if kv is None else write_slot.data_ptr()))
                 return
             x = self.normed(x)
+        tiles = m > self.STREAM_MAX_ROWS and self._in_tiles(x, w_qkv, qkv) and d % 16 == 0
         if (x.dtype == torch.bfloat16 and k % 8 == 0 and d % 16 == 0
-                and (0 < m <= self.SKINNY_MAX_ROWS or self._through_lds(x, w_qkv, qkv, m, qkv.shape[1], k, "qkv"))):
+                and (0 < m <= self.SKINNY_MAX_ROWS or tiles or self._through_lds(x, w_qkv, qkv, m, qkv.shape[1], k, "qkv"))):
             self._need(w_qkv.shape == ((hq + 2 * hkv) * d, k) and qkv.shape == (m, (hq + 2 * hkv) * d), "qkv: shapes")
             self._need(x.is_contiguous() and w_qkv.is_contiguous() and qkv.is_contiguous(), "qkv: contiguous operands")
             self._need(positions.dtype == torch.int32 and positions.numel() == m, "qkv: positions")
@@ -671,10 +679,12 @@ class HipOps:
                 self._need(kv.dtype == qkv.dtype and kv.shape[1:] == (2, hkv, 16 * d) and kv.is_contiguous(),
                            "qkv: cache must be [blocks, 2, kv_heads, 16*D] in the activation dtype")
                 self._need(write_slot.dtype == torch.int32 and write_slot.numel() == m, "qkv: write slots")
-            self._ok(self.lib.psamd_qkv_rope_append(self._stream(), x.data_ptr(), w_qkv.data_ptr(), qkv.data_ptr(), m, k,
-                                                    hq, hkv, d, positions.data_ptr(), _ptr(table), _ptr(kv),
-                                                    None if kv is None else write_slot.data_ptr()))
-            return
+            fused = self.lib.psamd_linear_tile_qkv if tiles else self.lib.psamd_qkv_rope_append
+            rc = fused(self._stream(), x.data_ptr(), w_qkv.data_ptr(), qkv.data_ptr(), m, k, hq, hkv, d, positions.data_ptr(),
+                       _ptr(table), _ptr(kv), None if kv is None else write_slot.data_ptr())
+            if not (tiles and rc == 2):          # 2: the library and the rotation behind it are the faster
+                self._ok(rc)
+                return
         self.linear(x, w_qkv, qkv)
         self.rope_kv_append(qkv, hq, hkv, d, positions, table, kv, write_slot)
 
@@ -704,6 +714,11 @@ class HipOps:
         return (pays and self.FUSED_SWIGLU_MAX_ROWS < m <= self.STREAM_MAX_ROWS and x.dtype == torch.bfloat16
                 and w.dtype == torch.bfloat16 and out.dtype == torch.bfloat16
                 and bool(self.lib.psamd_linear_skinny_takes(x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, int(form == "gated"))))
+
+    def _in_tiles(self, x, w, out) -> bool:
+        """Whether the tiles of linear_tile.hip may be asked: they need the library beside them for what they leave to it."""
+        return (self._direct_library and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and out.dtype in (torch.bfloat16, torch.float32)
+                and x.is_contiguous() and w.is_contiguous() and out.is_contiguous())
 
     def linear(self, x, w, out) -> None:
         m, k = x.shape
@@ -763,6 +778,25 @@ class HipOps:
             self._ok(self.lib.psamd_linear_skinny_add(self._stream(), x.data_ptr(), w.data_ptr(), residual.data_ptr(), m, n, k,
                                                       _ptr(col_scale)))
             return None
+        if m > self.STREAM_MAX_ROWS and self._in_tiles(x, w, x):
+            self._need(w.shape[1] == k, "linear_to_residual: operands")
+            if (residual is not None and col_scale is None and residual.dtype == torch.float32 and residual.shape == (m, n)
+                    and residual.is_contiguous() and residual.data_ptr() % 16 == 0):
+                slices = self.lib.psamd_linear_tile_slices(x.data_ptr(), w.data_ptr(), m, n, k)
+                if slices >= 0:
+                    out = residual
+                    if slices > 0:               # in a buffer for the most slices of any step, so that it does not grow with them
+                        self._need(slices * m <= self.TILE_SLICE_ROWS, "linear_to_residual: more slices than there is room for")
+                        self.ws.get(name + ".tiles", (self.TILE_SLICE_ROWS * n,), torch.float32)
+                        out = self.ws.get(name + ".tiles", (slices, m, n), torch.float32)
+                    self._ok(self.lib.psamd_linear_tile_stream(self._stream(), x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k))
+                    return None if slices == 0 else out
+            else:
+                out = self.ws.get(name, (m, n), x.dtype)
+                rc = self.lib.psamd_linear_tile_plain(self._stream(), x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k)
+                if rc != 2:                      # 2: the library is the faster
+                    self._ok(rc)
+                    return out
         if (residual is not None and col_scale is None and m >= self.LIBRARY_ADD_MIN_ROWS and x.dtype == torch.bfloat16 and k % 8 == 0
                 and residual.shape == (m, n) and residual.dtype == torch.float32 and self._direct_library):
             # A large step: the library's product adds into the float32 stream itself (out = x w^T + out),
@@ -827,6 +861,11 @@ class HipOps:
             self._ok(self.lib.psamd_linear_skinny(self._stream(), x.data_ptr(), w_gate_up.data_ptr(), out.data_ptr(),
                                                   _BF16, m, inter, k, epi, 1))
             return
+        if m > self.STREAM_MAX_ROWS and self._in_tiles(x, w_gate_up, out) and out.dtype == torch.bfloat16:
+            rc = self.lib.psamd_linear_tile_gated(self._stream(), x.data_ptr(), w_gate_up.data_ptr(), out.data_ptr(), m, inter, k, epi - 1)
+            if rc != 2:                          # 2: the library and the activation behind it are the faster
+                self._ok(rc)
+                return
         gu = self.ws.get("mlp.gate_up", (m, 2 * inter), x.dtype)
         self.linear(x, w_gate_up, gu)
         self.swiglu(gu, out, activation)

@@ -1200,6 +1200,66 @@ def test_kernels_refuse_what_they_do_not_take(ops):
         ops.swiglu(x, torch.empty(2, 4, dtype=torch.float16, device=DEV))
 
 
+# Every tile shape of the products of more than 128 tokens, with one step of k, few and many, tiles that end in the last token
+# or column or one behind it, one and several K-slices. rel() is over the largest value: a rounding to bfloat16 (8 bits) is up to 2^-8 of it.
+@pytest.mark.parametrize("act", ["silu", "relu", "gelu_tanh"])
+@pytest.mark.parametrize("m,n,k", [(129, 48, 64), (193, 256, 192), (257, 4112, 128), (250, 8208, 64), (384, 8192, 2048), (1000, 8192, 2048)])
+def test_gated_products_in_tiles(ops, m, n, k, act):
+    x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd(2 * n, k, dtype=torch.bfloat16, seed=2, scale=k ** -0.5)
+    out = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    assert ops.lib.psamd_linear_tile_gated(ops._stream(), x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, {"silu": 0, "relu": 1, "gelu_tanh": 2}[act]) == 0
+    z = x.double() @ w.double().T
+    f = {"silu": torch.nn.functional.silu, "relu": torch.relu, "gelu_tanh": lambda v: torch.nn.functional.gelu(v, approximate="tanh")}[act]
+    want = f(z[:, :n]) * z[:, n:]
+    assert rel(out[:m], want) < 3 * 2 ** -8 and torch.all(out[m] == 7.0)      # gate, up and the result are rounded
+    plain = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    ops.linear_swiglu(x, w, plain, act)
+    assert torch.equal(plain, out[:m])
+
+
+@pytest.mark.parametrize("m,n,k", [(129, 16, 64), (131, 2048, 1088), (257, 272, 4160), (600, 2048, 8192), (383, 4096, 2048), (1000, 4096, 14336),
+                                   (1537, 2048, 192), (5000, 64, 128), (511, 2048, 320), (1000, 4112, 448)])
+def test_products_in_tiles_for_the_residual_stream(ops, m, n, k):
+    """Added into the stream, or left in slices for the norm: sums of k products in 32 bits. Without the stream, and where columns are
+    scaled, in bfloat16."""
+    x, w = rnd(m, k, dtype=torch.bfloat16, seed=3), rnd(n, k, dtype=torch.bfloat16, seed=4, scale=k ** -0.5)
+    stream = rnd(m + 1, n, seed=5)
+    want = x.double() @ w.double().T
+    got = stream.clone()
+    delta = ops.linear_to_residual(x, w, "tiles", got[:m])
+    total = got[:m].double() + (delta.double() if delta is not None and delta.dim() == 2 else 0.0 if delta is None else delta.double().sum(0))
+    assert ops.lib.psamd_linear_tile_slices(x.data_ptr(), w.data_ptr(), m, n, k) >= 0 and (delta is None or delta.dtype == torch.float32)
+    assert rel(total, stream[:m].double() + want) < 2e-6 and torch.equal(got[m], stream[m])
+    plain = ops.linear_to_residual(x, w, "tiles.plain")
+    assert plain.dtype == torch.bfloat16 and rel(plain, want) < 2 ** -8
+    scaled = ops.linear_to_residual(x, w, "tiles.scaled", got[:m], torch.ones(n, device=DEV))
+    assert torch.equal(scaled, plain)
+
+
+@pytest.mark.parametrize("m,hq,hkv,d,k", [(129, 2, 2, 16, 64), (255, 32, 8, 64, 192), (300, 3, 1, 96, 320), (1030, 8, 2, 128, 1024), (780, 32, 8, 128, 1024),
+                                          (500, 32, 8, 128, 1024), (513, 16, 16, 32, 128)])
+@pytest.mark.parametrize("cached,rotated", [(True, True), (True, False), (False, True)])
+def test_qkv_products_in_tiles(ops, m, hq, hkv, d, k, cached, rotated):
+    """Projection, rotation and pages in one kernel against the product and the kernel behind it: the same order of roundings."""
+    n, blocks = (hq + 2 * hkv) * d, m // 16 + 3
+    x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2, scale=0.1)
+    pos = torch.tensor([(7 * i + 3) % 150 for i in range(m)], dtype=torch.int32, device=DEV)
+    slots = torch.tensor(np.random.default_rng(m).permutation(blocks * 16)[:m].tolist(), dtype=torch.int32, device=DEV)
+    table = rnd(150, d // 2, 2, seed=9) if rotated else None
+    kv = torch.full((blocks, 2, hkv, 16 * d), 3.0, dtype=torch.bfloat16, device=DEV) if cached else None
+    kv_want = None if kv is None else kv.clone()
+    out = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    assert ops.lib.psamd_linear_tile_qkv(ops._stream(), x.data_ptr(), w.data_ptr(), out.data_ptr(), m, k, hq, hkv, d, pos.data_ptr(),
+                                         table.data_ptr() if rotated else None, kv.data_ptr() if cached else None,
+                                         slots.data_ptr() if cached else None) == 0
+    plain = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    plain.copy_(x.double() @ w.double().T)
+    ops.rope_kv_append(plain, hq, hkv, d, pos, table, kv_want, slots if cached else None)
+    assert rel(out[:m], plain) < 2 ** -7 and torch.all(out[m] == 7.0)          # a last bit in front of the rotation and one behind it
+    if cached:
+        assert rel(kv, kv_want) < 2 ** -7 and torch.equal(kv == 3.0, kv_want == 3.0)
+
+
 @pytest.mark.parametrize("counts,k,f", [
     ((0, 127, 128, 129, 255, 256, 257, 512, 1900, 1500), 192, 320),  # empty experts, edges, parts without pairs
     ((1700, 0, 3, 511), 64, 64),                                    # one step of k, fewer columns than a tile
