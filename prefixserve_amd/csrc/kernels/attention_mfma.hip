@@ -116,6 +116,30 @@ __device__ __forceinline__ WeightTerms split_weight(float p) {
   return w;
 }
 
+// The same for eight weights, in pairs: one conversion for two numbers.
+struct Weights {
+  bf16x8 hi, mid, lo;
+};
+template <bool P3>
+__device__ __forceinline__ Weights split_weights(const float (&p)[8]) {
+  typedef __attribute__((ext_vector_type(2))) float f32x2;
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  uint4 hi{}, mid{}, lo{};
+  uint32_t *h = &hi.x, *m = &mid.x, *l = &lo.x;
+  auto pack = [](f32x2 v) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2)); };
+  auto rest = [](f32x2 v, uint32_t of) { return f32x2{v[0] - __uint_as_float(of << 16), v[1] - __uint_as_float(of & 0xffff0000u)}; };
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x2 v{p[2 * i], p[2 * i + 1]};
+    h[i] = pack(v);
+    if (!P3) continue;
+    const f32x2 r1 = rest(v, h[i]);
+    m[i] = pack(r1);
+    l[i] = pack(rest(r1, m[i]));
+  }
+  return Weights{__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, mid), __builtin_bit_cast(bf16x8, lo)};
+}
+
 // Per wave the loop is unrolled by two with two register sets: the keys and values of the
 // wave's next tile are loaded before the current one is computed. The block table is staged
 // in LDS once (a page id fetched from global memory inside the loop would put a second,
@@ -277,27 +301,25 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(
     }
     const float m_use = m == -INFINITY ? 0.f : m;
     float rowsum = 0.f;
-    bf16x8 pb[2], pm[2], pl[2];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const float p = __builtin_amdgcn_exp2f(fmaf(s[v], c, -m_use));
-      rowsum += p;
-      const WeightTerms w = split_weight<P3>(p);
-      pb[v >> 3][v & 7] = w.hi;
-      pm[v >> 3][v & 7] = w.mid;
-      pl[v >> 3][v & 7] = w.lo;
+    for (int cpage = 0; cpage < 2; ++cpage) {
+      float p[8];
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        p[v] = __builtin_amdgcn_exp2f(fmaf(s[8 * cpage + v], c, -m_use));
+        rowsum += p[v];
+      }
+      const Weights w = split_weights<P3>(p);
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.v[cpage][dt], w.hi, o[dt], 0, 0, 0);
+      if (P3) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.v[cpage][dt], w.mid, o[dt], 0, 0, 0);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.v[cpage][dt], w.lo, o[dt], 0, 0, 0);
+      }
     }
     l += rowsum + __shfl_xor(rowsum, 32, kWave);
-#pragma unroll
-    for (int cpage = 0; cpage < 2; ++cpage)
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.v[cpage][dt], pb[cpage], o[dt], 0, 0, 0);
-        if (P3) {
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.v[cpage][dt], pm[cpage], o[dt], 0, 0, 0);
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.v[cpage][dt], pl[cpage], o[dt], 0, 0, 0);
-        }
-      }
   };
 
   {
@@ -572,27 +594,25 @@ __global__ __launch_bounds__(256) void attn_masked_mfma_kernel(
     }
     const float m_use = m == -INFINITY ? 0.f : m;
     float rowsum = 0.f;
-    bf16x8 pb[2], pm[2], pl[2];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const float p = __builtin_amdgcn_exp2f(fmaf(s[v], c, -m_use));
-      rowsum += p;
-      const WeightTerms w = split_weight<P3>(p);
-      pb[v >> 3][v & 7] = w.hi;
-      pm[v >> 3][v & 7] = w.mid;
-      pl[v >> 3][v & 7] = w.lo;
+    for (int cpage = 0; cpage < 2; ++cpage) {
+      float p[8];
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        p[v] = __builtin_amdgcn_exp2f(fmaf(s[8 * cpage + v], c, -m_use));
+        rowsum += p[v];
+      }
+      const Weights w = split_weights<P3>(p);
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.v[cpage][dt], w.hi, o[dt], 0, 0, 0);
+      if (P3) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.v[cpage][dt], w.mid, o[dt], 0, 0, 0);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.v[cpage][dt], w.lo, o[dt], 0, 0, 0);
+      }
     }
     l += rowsum + __shfl_xor(rowsum, 32, kWave);
-#pragma unroll
-    for (int cpage = 0; cpage < 2; ++cpage)
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.v[cpage][dt], pb[cpage], o[dt], 0, 0, 0);
-        if (P3) {
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.v[cpage][dt], pm[cpage], o[dt], 0, 0, 0);
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t.v[cpage][dt], pl[cpage], o[dt], 0, 0, 0);
-        }
-      }
   };
 
   {
@@ -941,28 +961,32 @@ __global__ __launch_bounds__(256 * KP, NS <= 4 ? 4 : 2) void attn_prefill_groupe
     float rowsum = 0.f;
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
-      bf16x8 pb[2], pm[2], pl[2];
+      // A page's eight weights at a time, split and multiplied before the next: the terms of both at once cost registers that
+      // there are not.
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const float p = __builtin_amdgcn_exp2f(fmaf(s[t][v], c, -m_use));
-        rowsum += p;
-        const WeightTerms w = split_weight<P3>(p);
-        pb[v >> 3][v & 7] = w.hi;
-        pm[v >> 3][v & 7] = w.mid;
-        pl[v >> 3][v & 7] = w.lo;
-      }
+      for (int cpage = 0; cpage < 2; ++cpage) {
+        float p[8];
 #pragma unroll
-      for (int cpage = 0; cpage < 2; ++cpage)
+        for (int v = 0; v < 8; ++v) {
+          p[v] = __builtin_amdgcn_exp2f(fmaf(s[t][8 * cpage + v], c, -m_use));
+          rowsum += p[v];
+        }
+        const Weights w = split_weights<P3>(p);
+        bf16x8 vv[DT];
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
           const bf16_t* vr = vd + ((2 * t + cpage) * D + min(32 * dt + col, D - 1)) * VS;
-          const bf16x8 vv = join(ld4(vr), ld4(vr + 8));
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv, pb[cpage], o[dt], 0, 0, 0);
-          if (P3) {
-            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv, pm[cpage], o[dt], 0, 0, 0);
-            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv, pl[cpage], o[dt], 0, 0, 0);
-          }
+          vv[dt] = join(ld4(vr), ld4(vr + 8));
         }
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv[dt], w.hi, o[dt], 0, 0, 0);
+        if (P3) {
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv[dt], w.mid, o[dt], 0, 0, 0);
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv[dt], w.lo, o[dt], 0, 0, 0);
+        }
+      }
     }
     l += rowsum + __shfl_xor(rowsum, 32, kWave);
   };

@@ -18,13 +18,9 @@ typedef uint16_t bf16_t;    // raw bits; arithmetic is always done in float
 
 __device__ __forceinline__ float bf16_to_float(bf16_t v) { return __uint_as_float(static_cast<uint32_t>(v) << 16); }
 
-// Round to nearest even; NaN stays NaN.
-__device__ __forceinline__ bf16_t float_to_bf16(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<bf16_t>((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return static_cast<bf16_t>(u >> 16);
-}
+// Round to nearest even; NaN stays NaN. One instruction (v_cvt_pk_bf16_f32, for two numbers where they are neighbours), which gives
+// the bits of the six in integers that stood here for all 2^32 numbers.
+__device__ __forceinline__ bf16_t float_to_bf16(float f) { return __builtin_bit_cast(bf16_t, static_cast<__bf16>(f)); }
 
 template <typename T> __device__ __forceinline__ float to_float(T v);
 template <> __device__ __forceinline__ float to_float<float>(float v) { return v; }
