@@ -523,6 +523,14 @@ __global__ void to_activation_kernel(const float* __restrict__ in, A* __restrict
 
 // ------------------------------------------------------------------ rope + unit norm + kv append
 
+// (u, v) turned by the angle whose cosine and sine are c, and a^2 + b^2, with their roundings written out: both kernels below give the
+// same bits.
+__device__ __forceinline__ void rotate_pair(float u, float v, float2 c, float& a, float& b) {
+  a = __fmaf_rn(u, c.x, -__fmul_rn(v, c.y));
+  b = __fmaf_rn(u, c.y, __fmul_rn(v, c.x));
+}
+__device__ __forceinline__ float sum_of_squares(float a, float b) { return __fmaf_rn(a, a, __fmul_rn(b, b)); }
+
 // A group of L lanes per (token, head) of a row [hq q heads | hkv k heads | hkv v heads] x d, L the
 // power of two that holds d/2 pairs (at most a wave: several heads share a wave when d < 128). A q
 // or k head is rotated (pair (i, i + d/2), table [pos][i] = (cos, sin); NULL: not rotated), then, with
@@ -577,9 +585,8 @@ __global__ __launch_bounds__(256) void rope_norm_kv_append_kernel(
         }
         float2 cs = float2{1.f, 0.f};
         if (table != nullptr) cs = table[static_cast<int64_t>(pos) * half + i];
-        a[j] = u * cs.x - v * cs.y;
-        b[j] = v * cs.x + u * cs.y;
-        ss += a[j] * a[j] + b[j] * b[j];
+        rotate_pair(u, v, cs, a[j], b[j]);
+        ss += sum_of_squares(a[j], b[j]);
       }
     }
     float inv = 1.f;
@@ -608,6 +615,93 @@ __global__ __launch_bounds__(256) void rope_norm_kv_append_kernel(
     const int vh = head - hq - hkv;
     A* vpage = kv + page * page_elems + static_cast<int64_t>(hkv) * kPage * d + off;
     for (int c = l; c < d; c += group_lanes) vpage[(static_cast<int64_t>(vh) * d + c) * kPage] = row[c];
+  }
+}
+
+// The same for many tokens in bfloat16 with heads of 16, 32, 64 or 128: a block per 16 tokens, eight pairs per thread in 16-byte
+// accesses, a head's pairs in neighbouring lanes, the values through LDS as in rope_kv_append_vec_kernel. The kernel above spends
+// a wave on two heads of 64 in accesses of two bytes and writes the transposed values one by one. The sum of squares is
+// added in its order (pairs half the head apart first), so the bits are its bits.
+__global__ __launch_bounds__(256) void rope_norm_kv_append_vec_kernel(
+    bf16_t* __restrict__ qkv, int tokens, int hq, int hkv, int d, const int32_t* __restrict__ positions,
+    const float2* __restrict__ table, int norm_dim, float eps, bf16_t* __restrict__ kv, const int32_t* __restrict__ write_slot,
+    const float* __restrict__ bias, const float* __restrict__ q_weight, const float* __restrict__ k_weight, int q_weight_stride) {
+  extern __shared__ __align__(16) bf16_t norm_v_lds[];   // [16][a share of hkv * d, and 8]
+  const int t0 = blockIdx.x * 16;
+  const int nt = min(16, tokens - t0);
+  const int half = d >> 1, per_head = half >> 3;         // lanes per head: a power of two up to 8
+  const int width = (hq + 2 * hkv) * d;
+  const int64_t page_elems = 2LL * hkv * kPage * d;
+  const int vw = hkv * d;
+  const int c_lo = static_cast<int>(static_cast<int64_t>(vw >> 3) * blockIdx.y / gridDim.y);      // 8-element columns
+  const int c_hi = static_cast<int>(static_cast<int64_t>(vw >> 3) * (blockIdx.y + 1) / gridDim.y);
+  const int nc = c_hi - c_lo, vs = 8 * nc + 8;
+  for (int idx = threadIdx.x; kv != nullptr && idx < nt * nc; idx += blockDim.x) {
+    const int j = idx / nc, c = idx - j * nc;
+    *reinterpret_cast<uint4*>(norm_v_lds + j * vs + 8 * c) =
+        *reinterpret_cast<const uint4*>(qkv + static_cast<int64_t>(t0 + j) * width + (hq + hkv) * d + 8 * (c_lo + c));
+  }
+  // Whole heads to every blockIdx.y, and every lane of a head takes part in its sum.
+  const int heads = nt * (hq + hkv);
+  const int h_lo = static_cast<int>(static_cast<int64_t>(heads) * blockIdx.y / gridDim.y);
+  const int h_hi = static_cast<int>(static_cast<int64_t>(heads) * (blockIdx.y + 1) / gridDim.y);
+  for (int idx = h_lo * per_head + threadIdx.x; idx < h_hi * per_head; idx += blockDim.x) {
+    const int which = idx / per_head, i = (idx - which * per_head) << 3;
+    const int j = which / (hq + hkv), h = which - j * (hq + hkv);
+    const int64_t t = t0 + j;
+    bf16_t* x = qkv + t * width + h * d + i;
+    const uint4 lo4 = *reinterpret_cast<const uint4*>(x), hi4 = *reinterpret_cast<const uint4*>(x + half);
+    const bf16_t *lo_in = reinterpret_cast<const bf16_t*>(&lo4), *hi_in = reinterpret_cast<const bf16_t*>(&hi4);
+    const float2* cs = table != nullptr ? table + static_cast<int64_t>(positions[t]) * half + i : nullptr;
+    const float* nw = h < hq ? (q_weight != nullptr ? q_weight + static_cast<int64_t>(h) * q_weight_stride : nullptr) : k_weight;
+    float a[8], b[8], ss[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float u = bf16_to_float(lo_in[e]), v = bf16_to_float(hi_in[e]);
+      if (bias != nullptr) {
+        u += bias[static_cast<int64_t>(h) * d + i + e];
+        v += bias[static_cast<int64_t>(h) * d + i + e + half];
+      }
+      float2 c = float2{1.f, 0.f};
+      if (cs != nullptr) c = cs[e];
+      rotate_pair(u, v, c, a[e], b[e]);
+      ss[e] = sum_of_squares(a[e], b[e]);
+    }
+    float inv = 1.f;
+    if (norm_dim > 0) {
+      for (int o = per_head >> 1; o > 0; o >>= 1)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss[e] += __shfl_xor(ss[e], o, kWave);
+#pragma unroll
+      for (int o = 4; o > 0; o >>= 1)
+#pragma unroll
+        for (int e = 0; e < o; ++e) ss[e] += ss[e + o];
+      inv = rsqrtf(ss[0] / static_cast<float>(norm_dim) + eps);
+    }
+    uint4 lo_out, hi_out;
+    bf16_t *lo = reinterpret_cast<bf16_t*>(&lo_out), *hi = reinterpret_cast<bf16_t*>(&hi_out);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      lo[e] = float_to_bf16(a[e] * inv * (nw != nullptr ? nw[i + e] : 1.f));
+      hi[e] = float_to_bf16(b[e] * inv * (nw != nullptr ? nw[i + e + half] : 1.f));
+    }
+    *reinterpret_cast<uint4*>(x) = lo_out;
+    *reinterpret_cast<uint4*>(x + half) = hi_out;
+    if (kv != nullptr && h >= hq) {
+      const int slot = write_slot[t];
+      bf16_t* dst = kv + static_cast<int64_t>(slot / kPage) * page_elems + (static_cast<int64_t>(h - hq) * kPage + slot % kPage) * d + i;
+      *reinterpret_cast<uint4*>(dst) = lo_out;
+      *reinterpret_cast<uint4*>(dst + half) = hi_out;
+    }
+  }
+  if (kv == nullptr) return;
+  __syncthreads();
+  const int j = threadIdx.x & 15;
+  if (j < nt) {
+    const int slot = write_slot[t0 + j];
+    bf16_t* vpage = kv + static_cast<int64_t>(slot / kPage) * page_elems + static_cast<int64_t>(hkv) * kPage * d + slot % kPage;
+    for (int e = threadIdx.x >> 4; e < 8 * nc; e += blockDim.x >> 4)
+      vpage[static_cast<int64_t>(8 * c_lo + e) * kPage] = norm_v_lds[j * vs + e];
   }
 }
 
@@ -875,6 +969,10 @@ int psamd_to_activation(void* stream, const float* in, void* out, int act_dtype,
   return check_launch("psamd_to_activation");
 }
 
+// From here on the kernel for many tokens. us, one by one / 16 tokens a block: 32 heads of 64 on 8 at 300 tokens 5.2 / 6.5, 600 7.9 /
+// 8.2, 1,531 16.1 / 9.9, 2,048 20.2 / 12.1 (queries alone 12.8 / 6.6); 16 of 128 on 8 at 513 9.2 / 9.6, on 4 at 2,048 20.6 / 12.3.
+constexpr int64_t kNormVecMinTokens = 1024;
+
 int psamd_qk_prepare_kv_append(void* stream, void* qkv, int act_dtype, int64_t tokens, int hq, int hkv, int head_dim,
                                const int32_t* positions, const float* table, int norm_dim, float eps, const float* bias,
                                const float* q_weight, const float* k_weight, int v_from_k, void* kv,
@@ -894,6 +992,20 @@ int psamd_qk_prepare_kv_append(void* stream, void* qkv, int act_dtype, int64_t t
   const int heads_per_block = 4 * (64 / group_lanes);
   PSAMD_REQUIRE(ceil_div(row_heads, heads_per_block) <= 65535, "too many heads for one launch");
   const dim3 grid(static_cast<unsigned>(tokens), static_cast<unsigned>(ceil_div(row_heads, heads_per_block)));
+  const auto aligned = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
+  const bool whole_lanes = head_dim == 16 || head_dim == 32 || head_dim == 64 || head_dim == 128;
+  if (act_dtype == kBF16 && tokens >= kNormVecMinTokens && whole_lanes && !v_from_k && aligned(qkv) && aligned(kv)) {
+    const int64_t groups = ceil_div(tokens, 16);
+    // Enough blocks for every compute unit, each with at least a round of work for its threads.
+    const int64_t ny = std::min<int64_t>({ceil_div(1024, groups), 16, ceil_div(static_cast<int64_t>(hq + hkv) * head_dim, 256)});
+    const size_t smem = sizeof(bf16_t) * 16 * (8 * static_cast<size_t>(ceil_div(static_cast<int64_t>(hkv) * head_dim / 8, ny)) + 8);
+    if (smem <= 64 * 1024 && groups * 16 * (hq + hkv) * (head_dim / 16) < (1LL << 31)) {
+      rope_norm_kv_append_vec_kernel<<<dim3(static_cast<unsigned>(groups), static_cast<unsigned>(ny)), dim3(256), smem, s>>>(
+          static_cast<bf16_t*>(qkv), static_cast<int>(tokens), hq, hkv, head_dim, positions, tab, norm_dim, eps, static_cast<bf16_t*>(kv),
+          write_slot, bias, q_weight, k_weight, q_weight_stride);
+      return check_launch("psamd_qk_prepare_kv_append");
+    }
+  }
   if (act_dtype == kBF16) {
     rope_norm_kv_append_kernel<bf16_t><<<grid, dim3(256), 0, s>>>(static_cast<bf16_t*>(qkv), hq, hkv, head_dim, positions,
                                                                  tab, norm_dim, eps, static_cast<bf16_t*>(kv), write_slot,

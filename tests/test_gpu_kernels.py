@@ -1260,6 +1260,26 @@ def test_qkv_products_in_tiles(ops, m, hq, hkv, d, k, cached, rotated):
         assert rel(kv, kv_want) < 2 ** -7 and torch.equal(kv == 3.0, kv_want == 3.0)
 
 
+@pytest.mark.parametrize("hq,hkv,d,norm_dim", [(32, 8, 64, 64), (4, 2, 16, 16), (3, 1, 32, 20), (16, 4, 128, 0), (5, 0, 64, 64)])
+@pytest.mark.parametrize("weights", [False, True])
+def test_rotation_and_norm_of_many_tokens_equal_those_of_few(ops, hq, hkv, d, norm_dim, weights):
+    """From 1,024 tokens on 16 tokens a block: the bits of the kernel for fewer, on a last block that is not full."""
+    m, width, blocks = 1029, (hq + 2 * hkv) * d, 70
+    rows = rnd(m, width, dtype=torch.bfloat16, seed=d)
+    pos = torch.tensor([(7 * i + 3) % 150 for i in range(m)], dtype=torch.int32, device=DEV)
+    slots = torch.tensor(np.random.default_rng(m).permutation(blocks * 16)[:m].tolist(), dtype=torch.int32, device=DEV)
+    table = rnd(150, d // 2, 2, seed=9)
+    how = {"bias": rnd((hq + hkv) * d, seed=1), "q_weight": rnd(hq * d, seed=2), "k_weight": rnd(d, seed=3), "q_weight_per_head": True} if weights else {}
+    kv = [torch.full((blocks, 2, hkv, 16 * d), 3.0, dtype=torch.bfloat16, device=DEV) if hkv else None for _ in range(2)]
+    many, few = torch.cat((rows, rows[:1])), rows.clone()
+    ops.rope_norm_kv_append(many[:m], hq, hkv, d, pos, table, kv[0], slots if hkv else None, norm_dim, 1e-5, **how)
+    for a in range(0, m, 500):
+        b = min(m, a + 500)
+        ops.rope_norm_kv_append(few[a:b], hq, hkv, d, pos[a:b], table, kv[1], slots[a:b] if hkv else None, norm_dim, 1e-5, **how)
+    assert torch.equal(many[:m], few) and torch.equal(many[m], rows[0])
+    assert not hkv or torch.equal(kv[0], kv[1])
+
+
 @pytest.mark.parametrize("counts,k,f", [
     ((0, 127, 128, 129, 255, 256, 257, 512, 1900, 1500), 192, 320),  # empty experts, edges, parts without pairs
     ((1700, 0, 3, 511), 64, 64),                                    # one step of k, fewer columns than a tile
