@@ -161,7 +161,7 @@ class HipOps:
     STREAM_MAX_ROWS = 128           # whole 64-element steps of K and aligned operands: the products with both operands through LDS
     FUSED_SWIGLU_MAX_ROWS = 32      # above it what _through_lds does not take goes to the library, where there is one (o, down, q/k/v: above SKINNY_MAX_ROWS)
     TILE_SLICE_ROWS = 4608          # K-slices x tokens of a product of more tokens than that whose sums the norm behind it adds up
-    LIBRARY_ADD_MIN_ROWS = 1024     # from here on a product that feeds the residual stream adds into it in the library
+    LIBRARY_ADD_MIN_ROWS = 1024     # from here on a product that feeds the residual stream adds into it, in tiles or in the library
     MOE_ROUTE_FUSED_MAX_TOKENS = 0   # up to here one kernel computes router logits and choice; above, product + choice
     MOE_CHOICE_SORTS_MAX_TOKENS = 16 # up to here the workgroup that chooses a step's experts also sorts the pairs
     MOE_PAIRWISE_MAX_TOKENS = 2     # up to here a bfloat16 step's experts run pair by pair; above, grouped by expert
@@ -760,8 +760,8 @@ class HipOps:
                            col_scale: torch.Tensor | None = None) -> torch.Tensor | None:
         """x @ w^T for a consumer that adds it to the residual stream (the fused add+norm).
         Returns [T, N] in the activation dtype or, for a small bfloat16 step whose product has
-        few output columns, [S, T, N] float32 partial sums of a K-split, which the consumer adds
-        up: splitting K over workgroups is what lets such a product use the whole chip. With the
+        few output columns (and, given the stream, one of up to 1,023 tokens), [S, T, N] float32 partial sums of a K-split, which the
+        consumer adds up: splitting K over workgroups is what lets such a product use the whole chip. With the
         stream itself given as ``residual`` (float32 [T, N]), a step small enough to run without
         norm kernels adds the product into it here, K-slice by K-slice, and returns None.
         ``col_scale`` (float32 [N]): what is added into ``residual`` here is multiplied by it column by
