@@ -427,7 +427,7 @@ constexpr int kGroupCounters = 4096;   // counters of the sorting, in rows of `e
 __host__ __device__ constexpr int group_counter_rows(int experts) {
   return experts * 16 <= kGroupCounters ? 16 : (experts * 4 <= kGroupCounters ? 4 : 1);
 }
-constexpr size_t group_smem_ints(int experts) { return static_cast<size_t>(3 + group_counter_rows(experts)) * experts + 5; }
+constexpr size_t group_smem_ints(int experts, int rows) { return static_cast<size_t>(3 + rows) * experts + 5; }
 constexpr int kGroupStaged = 16384;    // up to here the sorted pairs are laid out in LDS before they leave, in whole lines
 
 // One workgroup of 16 waves sorts the step's pairs by expert and lists the tiles that the products run over.
@@ -436,13 +436,12 @@ constexpr int kGroupStaged = 16384;    // up to here the sorted pairs are laid o
 // The order of an expert's pairs among themselves is whatever the atomics gave: every pair's
 // result is computed from its own row alone, so it does not matter which rows share a tile.
 // `identity`: the pairs of the last of the `experts` buckets have no tiles; where they begin in `sorted` stands in tile_first
-// behind the last tile. Up to 16 waves count in counters of their own, and
+// behind the last tile. Up to 16 waves (`rows`) count in counters of their own, and
 // the sorted pairs leave LDS in whole lines (16,384 pairs over 32 experts 13.1 us -> 11.2).
 __device__ __forceinline__ void group_pairs(const int32_t* __restrict__ chosen, int pairs, int experts, const TileRule& rule, bool identity,
                                             int max_tiles, int32_t* __restrict__ sorted, int32_t* __restrict__ tile_expert,
                                             int32_t* __restrict__ tile_first, int32_t* __restrict__ tile_count,
-                                            int32_t* tiles_out, int32_t* smem, int32_t* staged) {
-  const int rows = group_counter_rows(experts);
+                                            int32_t* tiles_out, int32_t* smem, int rows, int32_t* staged) {
   int32_t *count = smem, *start = smem + experts, *tstart = smem + 2 * experts, *cursor = smem + 3 * experts;
   int32_t *listed = smem + (3 + rows) * experts, *own = cursor + static_cast<int>(threadIdx.x >> 6) % rows * experts;
   const int tiled = identity ? experts - 1 : experts;                            // buckets that have tiles
@@ -563,7 +562,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t* __restri
                                                          int32_t* __restrict__ tile_count) {
   extern __shared__ int32_t group_smem[];
   group_pairs(chosen, pairs, experts, rule, identity != 0, max_tiles, sorted, tile_expert, tile_first, tile_count, tile_count + max_tiles,
-              group_smem, pairs <= kGroupStaged ? group_smem + group_smem_ints(experts) : nullptr);
+              group_smem, group_counter_rows(experts), pairs <= kGroupStaged ? group_smem + group_smem_ints(experts, group_counter_rows(experts)) : nullptr);
 }
 
 // The choice from logits and the sorting in one workgroup of 16 waves, for steps of so few tokens
@@ -575,7 +574,7 @@ __global__ __launch_bounds__(1024) void moe_topk_group_kernel(const float* __res
                                                               int32_t* __restrict__ tile_count, const float* __restrict__ bias,
                                                               RouterRule rule) {
   extern __shared__ int32_t group_smem[];      // the sorting's integers, then score[16][experts]
-  float* score = reinterpret_cast<float*>(group_smem + group_smem_ints(buckets)) + (threadIdx.x >> 6) * experts;
+  float* score = reinterpret_cast<float*>(group_smem + group_smem_ints(buckets, 1)) + (threadIdx.x >> 6) * experts;
   const int lane = threadIdx.x & (kWave - 1);
   for (int t = threadIdx.x >> 6; t < tokens; t += 16) {
     for (int e = lane; e < experts; e += kWave) score[e] = router_score(z[static_cast<int64_t>(t) * experts + e], bias, e, rule.mode);
@@ -586,7 +585,7 @@ __global__ __launch_bounds__(1024) void moe_topk_group_kernel(const float* __res
   __threadfence_block();
   __syncthreads();                             // the workgroup's own writes of `chosen` are read below
   group_pairs(chosen, tokens * top, buckets, TileRule{tile_rows, {0, 0}, {0, 0}}, false, max_tiles, sorted, tile_expert, tile_first, tile_count,
-              tile_count + max_tiles, group_smem, nullptr);
+              tile_count + max_tiles, group_smem, 1, nullptr);
 }
 
 // k per staging round: with one tile of pairs a round of 64 leaves a wave two pieces of its matrix in flight, too few to
@@ -1133,7 +1132,7 @@ int psamd_moe_topk_group(void* stream, const float* logits, int32_t* chosen, flo
   const int64_t pairs = tokens * top;
   const int rows = psamd_moe_grouped_tile_rows(pairs, buckets);
   const int max_tiles = psamd_moe_grouped_max_tiles(pairs, buckets);
-  moe_topk_group_kernel<<<dim3(1), dim3(1024), sizeof(int32_t) * group_smem_ints(buckets) + sizeof(float) * 16 * experts,
+  moe_topk_group_kernel<<<dim3(1), dim3(1024), sizeof(int32_t) * group_smem_ints(buckets, 1) + sizeof(float) * 16 * experts,
                           static_cast<hipStream_t>(stream)>>>(logits, chosen, weight, static_cast<int>(tokens), experts, buckets, top, rows,
                                                               max_tiles, ints, ints + pairs, ints + pairs + max_tiles,
                                                               ints + pairs + 2 * max_tiles, bias, rule);
@@ -1194,7 +1193,7 @@ int psamd_moe_experts_grouped(void* stream, const void* x, const int32_t* chosen
   if (grouped_already == 0) {
     const TileRule rule{rows == 256 ? 0 : rows,
                         {static_cast<int>(ceil_div(F, kind == kExpertGated ? 128 : 256)), static_cast<int>(ceil_div(K, 256))}, {K, F}};
-    const size_t smem = sizeof(int32_t) * (group_smem_ints(buckets) + (pairs <= kGroupStaged ? pairs : 0));
+    const size_t smem = sizeof(int32_t) * (group_smem_ints(buckets, group_counter_rows(buckets)) + (pairs <= kGroupStaged ? pairs : 0));
     if (smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(moe_group_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                 static_cast<int>(smem)) != hipSuccess)
       return fail("psamd_moe_experts_grouped: " + std::to_string(smem) + " bytes of LDS were refused");

@@ -13,7 +13,8 @@ typedef __attribute__((ext_vector_type(4))) float tile_f32x4;
 // 64 lanes x 16 bytes from base + offset (a lane's own) to LDS at `to`, side by side: no register receives them. Written out because
 // the compiler waits for every copy under way in front of any read of LDS that it sees; whoever reads them waits for them itself.
 __device__ __forceinline__ void copy_to_lds(uint32_t to, uint32_t offset, const char* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(offset), "s"(base) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(offset), "s"(base)
+               : "memory", "m0");
 }
 
 constexpr int wait_for_copies(int left) { return (left & 15) | ((left >> 4) << 14) | (7 << 4); }   // s_waitcnt vmcnt(left) lgkmcnt(0)

@@ -1260,6 +1260,29 @@ def test_qkv_products_in_tiles(ops, m, hq, hkv, d, k, cached, rotated):
         assert rel(kv, kv_want) < 2 ** -7 and torch.equal(kv == 3.0, kv_want == 3.0)
 
 
+@pytest.mark.parametrize("e", [33, 256, 760])
+def test_the_choice_among_many_experts_that_sorts_its_pairs(ops, e):
+    """A decode step's choice and sorting in one workgroup, whose scores and counters have to fit LDS together, and the experts behind it."""
+    t, k, f, top = 8, 64, 64, 4
+    x, router = rnd(t, k, dtype=torch.bfloat16, seed=1), rnd(e, k, dtype=torch.bfloat16, seed=2, scale=0.1)
+    chosen, weight = torch.empty(t, top, dtype=torch.int32, device=DEV), torch.empty(t, top, device=DEV)
+    ops.moe_route(x, router.float(), chosen, weight, router)
+    z = torch.sigmoid(x.double() @ router.double().T)
+    # of scores that are one number in 32 bits either may be taken: a sum of 64 products and a sigmoid, 2^-24 each at random
+    assert rel(weight, torch.topk(z, top).values) < 1e-6 and rel(weight, z.gather(1, chosen.long())) < 1e-6
+    assert all(len(set(row)) == top for row in chosen.tolist())
+    w_in, down = rnd(e, 2 * f, k, dtype=torch.bfloat16, seed=3, scale=0.1), rnd(e, k, f, dtype=torch.bfloat16, seed=4, scale=0.1)
+    out = torch.empty(top, t, k, device=DEV)
+    ops.moe_experts(x, chosen, weight, w_in, down, torch.empty(t * top, f, dtype=torch.bfloat16, device=DEV), out, 1.0, float("inf"), 0.0, weight_on_output=True)
+    got = torch.zeros(t, k, dtype=torch.float64, device=DEV)
+    for j in range(top):
+        for i in range(t):
+            h = w_in[int(chosen[i, j])].double() @ x[i].double()
+            a = (torch.nn.functional.silu(h[:f]) * h[f:]).to(torch.bfloat16).double()
+            got[i] += weight[i, j].double() * (down[int(chosen[i, j])].double() @ a)
+    assert rel(out.sum(0), got) < 3e-3
+
+
 @pytest.mark.parametrize("hq,hkv,d,norm_dim", [(32, 8, 64, 64), (4, 2, 16, 16), (3, 1, 32, 20), (16, 4, 128, 0), (5, 0, 64, 64)])
 @pytest.mark.parametrize("weights", [False, True])
 def test_rotation_and_norm_of_many_tokens_equal_those_of_few(ops, hq, hkv, d, norm_dim, weights):
