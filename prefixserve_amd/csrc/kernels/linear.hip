@@ -955,13 +955,9 @@ int psamd_linear_skinny(void* stream, const void* x, const void* w, void* out, i
 int psamd_qkv_rope_append(void* stream, const void* x, const void* w, void* qkv_out, int M, int K, int hq, int hkv,
                           int head_dim, const int32_t* positions, const float* table, void* kv,
                           const int32_t* write_slot) {
-  // From 25 tokens on both operands go through LDS, from 17 on where there are 320 tiles (3,072 x 2,048: 7.7 us here and 8.2
-  // there at 17 tokens, 8.4 and 8.2 at 24, 13.4 and 10.5 at 64; 6,144 x 4,096: 19.5 and 15.8 at 17, 30.6 and 20.4 at 64). The
-  // tile of 64 tokens, which 33 need too, only pays with fewer row tiles where there is enough to multiply: 1,536 rows at 33, 48
-  // and 64 tokens with K = 512 4.8, 5.2 and 5.7 here, 5.5, 5.6 and 5.7 there; 1,024 6.2, 6.9 and 7.9, 6.9, 7.0 and 7.2; 2,048
-  // 9.0, 10.4 and 12.3, 9.6, 9.7 and 9.9; 4,096 16.5, 20.0 and 23.5, 15.5, 15.7 and 16.0.
-  const bool many_tiles = (hq + 2 * hkv) * (head_dim / 16) >= 320;
-  const bool stream_takes = hq > 0 && hkv > 0 && (many_tiles || (M > 24 && (M <= 32 || M > 64 || static_cast<int64_t>(K) * (M - 16) >= 48 * 1024))) &&
+  // From 17 tokens on both operands go through LDS where that kernel takes them (rows x K, us at 17, 32 and 64 tokens, here and there:
+  // 3,072 x 2,048 7.6, 8.3, 10.3 and 6.2, 6.4, 7.8; 1,536 x 512 4.2, 4.4, 5.8 and 4.0, 4.2, 4.9; 1,536 x 2,048 7.4, 8.2, 10.1 and 5.9, 6.2, 7.6).
+  const bool stream_takes = hq > 0 && hkv > 0 &&
                             linear_stream_takes(x, w, qkv_out, M, (hq + 2 * hkv) * head_dim, K, false);
   PSAMD_REQUIRE(M >= 1 && (M <= 64 || stream_takes), "M must be in [1, 64]");
   PSAMD_REQUIRE(K > 0 && K % 8 == 0, "K must be a positive multiple of 8");

@@ -698,21 +698,22 @@ class HipOps:
         stream an eighth of it at least), so few rows and a long K leave the chip idle where the library cuts K.
         us, library and what follows it / here:
 
-        * residual, 77 tokens (n x k): 1,024 x 8,192 14.1 / 8.7, 4,096 x 8,192 29.3 / 23.9, 8,192 x 3,584 24.5 / 21.2, x 8,192 39.6 / 43.5.
-        * gated, 48 tokens: 128 x 2,048 8.4 / 9.8, 192 x 2,048 11.1 / 9.8, 1,024 x 2,048 11.7 / 10.0, x 4,096 15.5 / 17.6, 2,048 x 4,096 17.2 / 18.1,
-          x 7,168 27.2 / 29.4, 3,072 x 4,096 21.6 / 20.4, x 14,336 61.3 / 59.4. 77 tokens: 256 x 1,024 8.3 / 8.8, 1,024 x 1,024 11.5 / 9.0, x 2,048 11.8 / 14.0,
-          x 4,096 16.0 / 24.6, 1,536 x 2,048 15.4 / 14.6, x 4,096 24.9 / 25.0, 3,072 x 4,096 27.2 / 26.4, x 7,168 38.7 / 42.5.
-        * qkv, 77 tokens: 768 x 1,536 11.9 / 11.6, x 2,048 12.8 / 13.5, x 8,192 18.5 / 37.3, 1,536 x 4,096 16.8 / 22.0,
-          3,072 x 2,048 16.8 / 14.4, x 4,096 26.3 / 22.8, 6,144 x 4,096 29.8 / 26.4, x 8,192 41.1 / 45.8."""
+        * residual (n x k), 40 tokens: 5,120 x 14,336 55.2 / 37.8, 8,192 x 4,096 24.1 / 25.4, x 8,192 38.4 / 43.2, x 14,336 64.6 / 52.9. 77 tokens:
+          1,024 x 8,192 14.1 / 8.7, 8,192 x 3,584 24.5 / 21.2, x 8,192 43.7 / 45.9, x 14,336 74.7 / 62.3.
+        * gated, 64 tokens: 256 x 4,096 14.7 / 11.5, x 8,192 12.9 / 18.9, 1,024 x 4,096 14.2 / 11.7, x 8,192 25.8 / 27.0, 2,048 x 8,192 26.6 / 27.6,
+          3,072 x 8,192 32.1 / 31.2, 5,632 x 8,192 46.6 / 48.4. 77 tokens: 256 x 1,024 8.4 / 6.1, x 2,048 8.5 / 10.3, 768 x 2,048 11.9 / 10.7, x 4,096 12.5 / 17.3,
+          1,536 x 4,096 23.8 / 23.2, 2,048 x 4,096 19.8 / 24.3, 3,072 x 8,192 37.2 / 44.1.
+        * qkv, 64 tokens: 768 x 4,096 16.1 / 10.7, x 8,192 15.6 / 16.7, 1,536 x 8,192 26.7 / 22.8 (40: 18.1 / 19.8), 2,560 x 8,192 27.3 / 24.6, 9,216 x 8,192 45.8 / 42.5
+          (40). 77 tokens: 768 x 2,048 12.5 / 10.0, 1,536 x 4,096 13.8 / 16.3, 2,560 x 4,096 16.5 / 19.1, 3,072 x 4,096 21.1 / 17.6, x 8,192 44.5 / 34.2, 4,608 x 8,192 32.7 / 35.2."""
         if form == "gated":
             if m <= self.SKINNY_MAX_ROWS:
-                pays = k <= 1024 or (k <= 2048 and n >= 160) or n >= 2560
+                pays = k <= 4096 or n >= 2560
             else:
-                pays = k <= 512 or (k <= 1024 and n >= 320) or n >= max(1536, 0.75 * k)
+                pays = k <= 1024 or (k <= 2048 and n >= 640) or n >= max(1536, 0.75 * k)
         elif form == "qkv":
-            pays = k <= 1536 or (n >= 3072 and k <= 4096)
+            pays = (k <= 4096 or n >= 2560) if m <= self.SKINNY_MAX_ROWS else (k <= 2048 or (n >= 3072 and k <= 4096))
         else:
-            pays = n * k <= 6e7
+            pays = n * k <= 6e7 or k >= 14336
         return (pays and self.FUSED_SWIGLU_MAX_ROWS < m <= self.STREAM_MAX_ROWS and x.dtype == torch.bfloat16
                 and w.dtype == torch.bfloat16 and out.dtype == torch.bfloat16
                 and bool(self.lib.psamd_linear_skinny_takes(x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, int(form == "gated"))))
