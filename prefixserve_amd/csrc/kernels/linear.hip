@@ -15,6 +15,7 @@
 #include "common.h"
 #include "linear_f32.h"
 #include "linear_stream.h"
+#include "stream_operands.h"
 
 namespace psamd {
 
@@ -262,19 +263,6 @@ __global__ __launch_bounds__(64 * WV) void skinny_mfma_kernel(const bf16_t* __re
     }
   }
 }
-
-// Where the tokens of a small step come from: bfloat16 rows x[M][K], or (x == nullptr) rows of the
-// float32 residual stream that the kernel normalizes itself on the way in (RMS norm: statistics
-// in 32-bit, eps inside the root, times the norm's weight), row rows[m] for token m (rows ==
-// nullptr: row m). A kernel that reads its tokens this way needs no norm kernel in front of it.
-struct Tokens {
-  const bf16_t* x;
-  const float* resid;
-  const void* norm_w;
-  const int32_t* rows;
-  float eps;
-  int norm_w_bf16;      // the norm's weight is bfloat16 (else float32)
-};
 
 // Stages the M <= ROWS tokens of a small step in LDS for a workgroup of WV waves, from rows of
 // the float32 residual stream: xs[row][k] = bfloat16(resid[row][k] * norm_w[k]), and the rows'
@@ -1022,6 +1010,8 @@ int psamd_linear_normed(void* stream, const float* resid, const int32_t* rows, c
   PSAMD_REQUIRE(norm_w_dtype == kBF16 || norm_w_dtype == kF32, "the norm's weight is bfloat16 or float32");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const Tokens tk{nullptr, resid, norm_w, rows, eps, norm_w_dtype == kBF16 ? 1 : 0};
+  const int form = epilogue == 1 ? kGated : (out_dtype == kF32 ? kSlices : kPlain);
+  if (linear_normed_takes(w, out, form, M, n_out, K)) return launch_linear_normed(s, tk, w, out, form, M, n_out, K, g_gate_act);
   const int64_t groups = ceil_div(n_out, 16);
   const bool eight = M <= 8;
   if (epilogue == 1) {
@@ -1061,6 +1051,8 @@ int psamd_qkv_rope_append_normed(void* stream, const float* resid, const void* n
   const float2* tab = reinterpret_cast<const float2*>(table);
   bf16_t* kvp = static_cast<bf16_t*>(kv);
   const int n_tiles = (hq + 2 * hkv) * (head_dim / 16);
+  if (linear_normed_takes(w, qkv_out, kQkv, M, 16 * n_tiles, K))
+    return launch_linear_normed(s, tk, w, qkv_out, kQkv, M, 16 * n_tiles, K, 0, QkvOut{hq, hkv, head_dim, positions, tab, kvp, write_slot});
   if (M <= 8) return launch_qkv_normed<1, 8>(s, tk, wp, op, M, K, hq, hkv, head_dim, positions, tab, kvp, write_slot);
   if (n_tiles >= 320) return launch_qkv_normed<2, 16>(s, tk, wp, op, M, K, hq, hkv, head_dim, positions, tab, kvp, write_slot);
   return launch_qkv_normed<1, 16>(s, tk, wp, op, M, K, hq, hkv, head_dim, positions, tab, kvp, write_slot);
