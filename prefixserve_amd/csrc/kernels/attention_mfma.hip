@@ -1185,8 +1185,8 @@ __device__ __forceinline__ float2 shared_load(const float* p) {
 // workgroups have written their runs (or, in the first, how many), zero between launches.
 constexpr int kCounted = 8;              // runs that count in one integer
 constexpr int kMergeHeads = 8;           // the most query heads a kv head has where the decode kernel merges its runs
-template <int NS, int CT, bool P3 = false, bool MERGE = false>
-__global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
+template <int NS, int CT, bool P3 = false, bool MERGE = false, int WV = 4>
+__global__ __launch_bounds__(64 * WV) void attn_decode_mfma_kernel(
     const bf16_t* __restrict__ qkv, int q_stride, const bf16_t* __restrict__ kv, bf16_t* __restrict__ out,
     float* part_o, float* part_ml, int32_t* arrived, const int32_t* __restrict__ dec_items,
     const int32_t* __restrict__ item_start,
@@ -1195,6 +1195,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
     int n_dec, Extras ex) {
   constexpr int D = 16 * NS;
   constexpr int KS = (D + 31) / 32;
+  static_assert(!MERGE || WV == 4, "four waves merge the runs");
   extern __shared__ float smem[];
   // Workgroups are handed out in the order of blockIdx.x, round robin over the eight dies. The
   // (request, split) pairs are laid out eight at a time, one per die, with the kv heads of a pair
@@ -1270,7 +1271,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
     for (int ds = 0; ds < NS; ++ds) o[ct][ds] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  for (int tile = my_lo + wave; tile < my_hi; tile += 4) {
+  for (int tile = my_lo + wave; tile < my_hi; tile += WV) {
     // The tile is the same for all lanes of a wave: said so, its page ids come through the scalar
     // cache instead of as vector loads that every lane repeats (32 requests x 8 kv heads, 2,048
     // keys: 25.9 -> 22.0 us). Asking for the next tile's keys and values before multiplying the
@@ -1361,10 +1362,10 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
     }
   }
 
-  // ---- merge the 4 waves: smem = m[4][group], l[4][group], o[4][group][D]
+  // ---- merge the waves: smem = m[WV][group], l[WV][group], o[WV][group][D]
   float* sm_m = smem;
-  float* sm_l = smem + 4 * group;
-  float* sm_o = smem + 8 * group;
+  float* sm_l = smem + WV * group;
+  float* sm_o = smem + 2 * WV * group;
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
     const int hh = ct * 16 + r;
@@ -1386,11 +1387,11 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
   auto combined = [&](int hh, int d, float& mm, float& ll) {
     mm = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) mm = fmaxf(mm, sm_m[w * group + hh]);
+    for (int w = 0; w < WV; ++w) mm = fmaxf(mm, sm_m[w * group + hh]);
     float acc = 0.f;
     ll = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < WV; ++w) {
       const float mw = sm_m[w * group + hh];
       const float wgt = mw == -INFINITY ? 0.f : __expf(mw - mm);
       acc += wgt * sm_o[(static_cast<int64_t>(w) * group + hh) * D + d];
@@ -1718,6 +1719,18 @@ static int launch_prefill(hipStream_t s, const void* qkv, int q_stride, void* ou
   return launch_prefill_merge(s, part_o, part_ml, out, pf_tiles, item_start, n_tiles, hq, 16 * NS, nsplit);
 }
 
+// From kOneRun to 256 (request, kv head) pairs a workgroup of eight waves takes all keys of one: it has its compute unit (nearly) to itself, and
+// nothing is merged behind it. us a layer behind 300, 1,000, 2,049 and uneven up to 2,900 keys, as before (two runs of four waves below 256 pairs,
+// one from there on) / so, 32 heads on 8:
+//   head size 64,  22 requests   9.6, 16.3, 25.7, 27.6 / 6.9, 13.8, 21.9, 24.4      head size 128, 22    14.3, 27.2, 47.5, 46.0 / 11.1, 23.5, 41.0, 46.8
+//                  24            9.8, 16.7, 26.6, 27.2 / 6.9, 14.1, 22.9, 24.3                     28    14.6, 29.9, 50.3, 48.8 / 12.1, 26.9, 46.4, 50.0
+//                  30           10.6, 18.2, 29.8, 28.1 / 7.9, 16.0, 26.9, 25.5                     32    14.1, 30.0, 53.0, 52.0 / 12.9, 29.0, 51.4, 51.2
+//                  32            9.1, 17.8, 30.5, 35.2 / 8.1, 16.7, 28.1, 26.5      head size 32,  24     8.2, 12.5, 19.1, 21.1 /  6.0, 10.3, 17.2, 18.9
+// At 20 and 21 requests three runs stay the faster for uneven contexts (21.7 / 24.0); above 256 pairs some units have two such workgroups
+// (33 requests behind 2,049 keys: 35.0 / 39.0). The same keys cut evenly over the chip whatever the requests' lengths gained nothing (64 uneven
+// requests: 46.2 / 46.6): a launch pays 7 us for its trips to memory one after the other, and then streams at 5.2 TB/s either way.
+constexpr int kOneRun = 176;
+
 template <int NS, int CT, bool P3>
 static int launch_decode(hipStream_t s, const void* qkv, int q_stride, const void* kv, void* out, float* part_o,
                          float* part_ml, int32_t* arrived, const int32_t* dec_items, int n_dec, const int32_t* item_start, const int32_t* item_end,
@@ -1727,18 +1740,21 @@ static int launch_decode(hipStream_t s, const void* qkv, int q_stride, const voi
   // The waves' results, and for the merge two numbers per head and run.
   const size_t smem = sizeof(float) * std::max<size_t>(8 * group + 4 * static_cast<size_t>(group) * 16 * NS, 2 * static_cast<size_t>(group) * nsplit);
   const int64_t groups_of_8 = ceil_div(static_cast<int64_t>(n_dec) * nsplit, 8);
-  auto run = [&](auto kernel) {
+  auto run = [&](auto kernel, int waves, size_t smem) {
     if (!lds_allowed(kernel, smem)) return fail("psamd_attention_decode: " + std::to_string(smem) + " bytes of LDS were refused");
-    kernel<<<dim3(8 * hkv, static_cast<unsigned>(groups_of_8)), dim3(256), smem, s>>>(
+    kernel<<<dim3(8 * hkv, static_cast<unsigned>(groups_of_8)), dim3(64 * waves), smem, s>>>(
         static_cast<const bf16_t*>(qkv), q_stride, static_cast<const bf16_t*>(kv), static_cast<bf16_t*>(out), part_o,
         part_ml, arrived, dec_items, item_start, item_end, table_off, block_ids, hq, hkv, nsplit, scale, window, min_tiles, n_dec,
         g_extras);
     return check_launch("psamd_attention_decode");
   };
   if constexpr (CT == 1) {
-    if (arrived != nullptr) return run(attn_decode_mfma_kernel<NS, CT, P3, true>);
+    if (arrived != nullptr) return run(attn_decode_mfma_kernel<NS, CT, P3, true>, 4, smem);
+    const int64_t pairs = static_cast<int64_t>(n_dec) * hkv;
+    if (nsplit == 1 && pairs >= kOneRun && pairs <= 256)
+      return run(attn_decode_mfma_kernel<NS, CT, P3, false, 8>, 8, sizeof(float) * 8 * (2 + 16 * NS) * static_cast<size_t>(group));
   }
-  return run(attn_decode_mfma_kernel<NS, CT, P3>);
+  return run(attn_decode_mfma_kernel<NS, CT, P3>, 4, smem);
 }
 
 template <int NS, bool P3>
@@ -1913,13 +1929,13 @@ int psamd_attention_decode_skewed(int n_dec, int longest, int64_t total) {
 
 // How psamd_attention_decode should cut the keys of a step of n_dec single-token items whose
 // longest context is kv_len (for a captured step: the longest there can be): *nsplit runs per
-// request, none shorter than *min_run keys. Two workgroups per compute unit; from one per compute
-// unit on, no split and no merge kernel (32 requests x 8 kv heads at head size 128: 48 -> 41 us).
+// request, none shorter than *min_run keys. Two workgroups per compute unit; from two thirds of one per
+// compute unit on (kOneRun), no split and no merge.
 int psamd_attention_decode_plan(int n_dec, int kv_len, int skewed, int hkv, int window, int* nsplit, int* min_run) {
   PSAMD_REQUIRE(n_dec >= 1 && kv_len >= 1 && hkv >= 1 && nsplit != nullptr && min_run != nullptr, "decode plan: bad sizes");
   if (window > 0) kv_len = std::min(kv_len, window);
   const int64_t pairs = static_cast<int64_t>(n_dec) * hkv;
-  int n = pairs >= 256 ? 1 : static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({64, 512 / pairs, ceil_div(kv_len, 128)})));
+  int n = pairs >= kOneRun ? 1 : static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({64, 512 / pairs, ceil_div(kv_len, 128)})));
   int run = 128;
   if (skewed && window <= 0) {
     n = std::max(n, static_cast<int>(std::min<int64_t>({64, 4096 / n_dec, ceil_div(kv_len, 1024)})));
