@@ -10,9 +10,12 @@
 // The chains are short because the matrix instruction rounds more than a fused multiply-add does: at K = 252 one chain is
 // 4.5e-7 off the product in 64 bits where a chain of fused multiply-adds is 2.8e-7 off.
 
+#include <algorithm>
+
 #include "api.h"
 #include "common.h"
 #include "linear_f32.h"
+#include "tile_product.h"
 
 namespace psamd {
 
@@ -43,102 +46,115 @@ __device__ __forceinline__ void put_columns(float* __restrict__ out, int64_t m, 
 
 // ------------------------------------------------------------------ many tokens
 
-// A workgroup of four waves makes 64 columns x BM tokens (a wave 32 x 32, or 16 x 32), both operands through LDS 64 k at a
-// time, the next ones on their way in registers. Bound by the matrix instructions: 2,048 cycles of them per step and wave
-// at 64 x 64 against 16 LDS reads of 16 bytes; 64 k a step because 32 k's instructions are over before the next step's
-// rows arrive (one workgroup on a compute unit, K = 2,048: 57 -> 46 us). Rows of LDS are 68 floats apart: the 16 rows a read
-// touches lie on 16 different groups of four banks. Tiles that share rows of w run on one die (its L2 serves them): die d
-// takes the d-th eighth of the tiles, tokens fastest.
-// 600 tokens x 16,384 columns x 2,048: 404 us, 100 TFLOP/s, where tiles of 64 x 64 by fused multiply-adds took 1,034.
-constexpr int kColumns = 64;
-
-template <int BM>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                       float* __restrict__ out, int M, int N, int K, int m_tiles, int tiles,
-                                                       int per_die) {
-  constexpr int BN = kColumns, BK = 64, LD = BK + 4, RT = BN * BM / 2048, MT = 2;
-  constexpr int CH = BK / 4, ROWS = 256 / CH;                          // 16-byte pieces per row, rows the workgroup brings at once
-  constexpr int PW = BN / ROWS, PX = BM / ROWS;                        // pieces per thread
-  static_assert(BM == 64 || BM == 32, "a wave takes 32 tokens");
-  __shared__ __align__(16) float ws[2][BN * LD];
-  __shared__ __align__(16) float xs[2][BM * LD];
+// A workgroup of WM x WN waves makes BN columns x BM tokens, both operands through LDS 64 k, a chain, at a time: the next chain's rows are copied
+// there while this one is multiplied (copy_to_lds: no register holds them), a wave's operands are read 32 k ahead of the matrix
+// instructions, and a chain's first instruction takes zero for its sums. A row of LDS is 256 bytes, its sixteen 16-byte pieces exchanged by
+// the row's number, so that the 16 rows a read touches lie on all banks. Tiles that share rows of w run on one die (its L2 serves
+// them): die d takes the d-th eighth of the tiles, tokens fastest. Bound by the matrix instructions, whose rate on this card is 150 TFLOP/s (a loop of
+// them and nothing else); what is left of it goes to the wait for a chain's first operands behind the barrier, which the other
+// workgroups of the compute unit fill. us, with rows on their way in registers and operands read as they are needed / so:
+// 600 tokens x 16,384 columns x 2,048 424 / 343 (117 TFLOP/s), 600 x 3,072 91 / 72, 600 x 2,048 75 / 55, 600 x 2,048 x 8,192 267 / 199, 300 x 2,048 52 / 32,
+// 150 x 2,048 x 8,192 130 / 90, 2,048 x 16,384 1,299 / 1,059 (130). A third buffer costs workgroups and is slower everywhere (600 x 2,048 65).
+template <int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                float* __restrict__ out, int M, int N, int K, int m_tiles, int tiles,
+                                                                int per_die) {
+  constexpr int W = WM * WN, RT = BN / 16 / WN, MT = BM / 16 / WM, LW = BN / 4 / W, LX = BM / 4 / W, STAGE = (BM + BN) * 256;
+  static_assert(LW * 4 * W == BN && LX * 4 * W == BM && RT * 16 * WN == BN && MT * 16 * WM == BM, "whole copies and tiles per wave");
+  __shared__ __align__(16) unsigned char buffers[2 * STAGE];           // 2 x [BN rows of w, BM of x][64 k]
   const int local = static_cast<int>(blockIdx.x >> 3), tile = static_cast<int>(blockIdx.x & 7) * per_die + local;
   if (local >= per_die || tile >= tiles) return;
   const int n0 = tile / m_tiles * BN, m0 = tile % m_tiles * BM;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int r = lane & 15, g = lane >> 4;
-  const int wn = (BM == 64 ? wave >> 1 : wave) * (RT * 16), wm = BM == 64 ? (wave & 1) * 32 : 0;   // this wave's part of the tile
-
-  const float* wsrc[PW];
-  const float* xsrc[PX];
-  const int c4 = 4 * (tid % CH), row0 = tid / CH;                                        // first k of this thread's pieces
+  const int wn = wave % WN * (RT * 16), wm = wave / WN * (MT * 16);    // this wave's part of the tile
+  const char* wb = reinterpret_cast<const char*>(w + static_cast<int64_t>(n0) * K);
+  const char* xb = reinterpret_cast<const char*>(x + static_cast<int64_t>(m0) * K);
+  uint32_t w_off[LW], x_off[LX];                                       // copy i of this wave brings four rows; a lane its 16 bytes of them
+  const int row0 = lane >> 4, last_w = N - 1 - n0, last_x = M - 1 - m0;
+  auto piece = [&](int row) { return (lane & 15) ^ (row & 15); };
 #pragma unroll
-  for (int p = 0; p < PW; ++p) wsrc[p] = w + static_cast<int64_t>(min(n0 + row0 + ROWS * p, N - 1)) * K + c4;
+  for (int i = 0; i < LW; ++i) {
+    const int row = (wave * LW + i) * 4 + row0;
+    w_off[i] = static_cast<uint32_t>(min(row, last_w)) * (4u * K) + 16u * piece(row);
+  }
 #pragma unroll
-  for (int p = 0; p < PX; ++p) xsrc[p] = x + static_cast<int64_t>(min(m0 + row0 + ROWS * p, M - 1)) * K + c4;
-  float4 wr[PW], xr[PX];
-  auto ask = [&](int k0) {
-    const bool in = k0 + c4 < K;                                       // K is a multiple of 4
+  for (int i = 0; i < LX; ++i) {
+    const int row = (wave * LX + i) * 4 + row0;
+    x_off[i] = static_cast<uint32_t>(min(row, last_x)) * (4u * K) + 16u * piece(row);
+  }
+  const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)buffers));
+  auto copy = [&](int t, int to) {
 #pragma unroll
-    for (int p = 0; p < PW; ++p) wr[p] = in ? *reinterpret_cast<const float4*>(wsrc[p] + k0) : float4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < LW; ++i) copy_to_lds(base + to + (wave * LW + i) * 1024, w_off[i], wb + static_cast<int64_t>(t) * 256);
 #pragma unroll
-    for (int p = 0; p < PX; ++p) xr[p] = in ? *reinterpret_cast<const float4*>(xsrc[p] + k0) : float4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < LX; ++i) copy_to_lds(base + to + BN * 256 + (wave * LX + i) * 1024, x_off[i], xb + static_cast<int64_t>(t) * 256);
   };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int p = 0; p < PW; ++p) *reinterpret_cast<float4*>(ws[buf] + (row0 + ROWS * p) * LD + c4) = wr[p];
-#pragma unroll
-    for (int p = 0; p < PX; ++p) *reinterpret_cast<float4*>(xs[buf] + (row0 + ROWS * p) * LD + c4) = xr[p];
-  };
-  f32x4 acc[RT][MT], part[RT][MT], total[RT][MT];                      // of the chain, the segment, all of K
+  f32x4 part[RT][MT], total[RT][MT];                                   // of the segment, of all of K
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = part[rt][mt] = total[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  ask(0);
-  stage(0);
-  __syncthreads();
-  int buf = 0;
-  for (int k0 = 0; k0 < K; k0 += BK, buf ^= 1) {
-    const bool more = k0 + BK < K;
-    if (more) ask(k0 + BK);
-    const float* wl = ws[buf] + (wn + r) * LD + 4 * g;
-    const float* xl = xs[buf] + (wm + r) * LD + 4 * g;
+    for (int mt = 0; mt < MT; ++mt) part[rt][mt] = total[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int whole = K / kChain, chains = (K + kChain - 1) / kChain;
+  auto multiply = [&](int t, int at) {
+    f32x4 a[4][RT], b[4][MT], acc[RT][MT];
+    auto operands = [&](int q) {                                       // of k = 16 q .. 16 q + 15
+      const unsigned char* from = buffers + at + r * 256 + 16 * ((4 * q + g) ^ r);
 #pragma unroll
-    for (int kk = 0; kk < BK; kk += 16) {
-      f32x4 a[RT], b[MT];
+      for (int rt = 0; rt < RT; ++rt) a[q][rt] = *reinterpret_cast<const f32x4*>(from + (wn + 16 * rt) * 256);
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) a[rt] = *reinterpret_cast<const f32x4*>(wl + rt * 16 * LD + kk);
+      for (int mt = 0; mt < MT; ++mt) b[q][mt] = *reinterpret_cast<const f32x4*>(from + (BN + wm + 16 * mt) * 256);
+    };
+    operands(0);
+    operands(1);
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) b[mt] = *reinterpret_cast<const f32x4*>(xl + mt * 16 * LD + kk);
+    for (int q = 0; q < 4; ++q) {
+      if (q < 2) operands(q + 2);
+      __builtin_amdgcn_sched_barrier(0);
       // One k of every tile after the other: neighbouring instructions do not wait for each other's sums.
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rt][i], b[mt][i], acc[rt][mt], 0, 0, 0);
+          for (int mt = 0; mt < MT; ++mt)
+            acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q][rt][i], b[q][mt][i], q == 0 && i == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[rt][mt], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    if (((k0 + BK) & (kChain - 1)) == 0 || !more) {                    // a chain is complete
+    constexpr int kChains = kSegment / kChain;
+    const bool ends = t % kChains == kChains - 1 || t + 1 == chains;
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          part[rt][mt] += acc[rt][mt];
-          acc[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-    }
-    if (((k0 + BK) & (kSegment - 1)) == 0 || !more) {
+      for (int mt = 0; mt < MT; ++mt) {
+        part[rt][mt] = (t % kChains == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : part[rt][mt]) + acc[rt][mt];
+        if (ends) total[rt][mt] += part[rt][mt];
+      }
+  };
+  if (whole > 0) copy(0, 0);
+  int at = 0;
+  for (int t = 0; t < whole; ++t, at ^= STAGE) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(wait_for_copies(0));
+    __builtin_amdgcn_s_barrier();                                      // chain t has arrived, and everybody has read the one before
+    __builtin_amdgcn_sched_barrier(0);
+    if (t + 1 < whole) copy(t + 1, at ^ STAGE);
+    asm volatile("" ::: "memory");                                     // what the copies brought is read behind the barrier
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(t, at);
+  }
+  if (whole < chains) {                                                // the last chain in part: zeros behind K, a multiple of 4
+    auto put = [&](int to, const char* from, uint32_t off, int row) {
+      const int k = kChain * whole + 4 * piece(row);
+      *reinterpret_cast<f32x4*>(buffers + at + to + lane * 16) =
+          k < K ? *reinterpret_cast<const f32x4*>(from + static_cast<int64_t>(whole) * 256 + off) : f32x4{0.f, 0.f, 0.f, 0.f};
+    };
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
+    for (int i = 0; i < LW; ++i) put((wave * LW + i) * 1024, wb, w_off[i], (wave * LW + i) * 4 + row0);
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          total[rt][mt] += part[rt][mt];
-          part[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-    }
-    if (more) stage(buf ^ 1);                                          // last read before the barrier in front of this step
-    __syncthreads();
+    for (int i = 0; i < LX; ++i) put(BN * 256 + (wave * LX + i) * 1024, xb, x_off[i], (wave * LX + i) * 4 + row0);
+    __syncthreads();                                                   // (this buffer was last read in front of the barrier before)
+    multiply(whole, at);
   }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
@@ -262,34 +278,41 @@ static void launch_rows(hipStream_t s, const float* x, const float* w, float* ou
   rows_f32_kernel<MT><<<grid, dim3(512), 0, s>>>(x, w, out, M, N, K);
 }
 
-template <int BM>
+template <int BM, int BN, int WM, int WN>
 static void launch_tiles(hipStream_t s, const float* x, const float* w, float* out, int M, int N, int K) {
-  const int m_tiles = static_cast<int>(ceil_div(M, BM)), tiles = static_cast<int>(ceil_div(N, kColumns)) * m_tiles;
+  const int m_tiles = static_cast<int>(ceil_div(M, BM)), tiles = static_cast<int>(ceil_div(N, BN)) * m_tiles;
   const int per_die = static_cast<int>(ceil_div(tiles, 8));
-  gemm_f32_kernel<BM><<<dim3(static_cast<unsigned>(8 * per_die)), dim3(256), 0, s>>>(x, w, out, M, N, K, m_tiles, tiles, per_die);
+  gemm_f32_kernel<BM, BN, WM, WN><<<dim3(static_cast<unsigned>(8 * per_die)), dim3(64 * WM * WN), 0, s>>>(x, w, out, M, N, K, m_tiles, tiles, per_die);
 }
 
 bool linear_f32_takes(const void* x, const void* w, int64_t M, int N, int K) {
   const uintptr_t bits = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w);
-  return K % 4 == 0 && bits % 16 == 0 && M <= (1 << 24) && ceil_div(M, 64) * ceil_div(N, 64) < (1LL << 31) - 8;
+  return K % 4 == 0 && bits % 16 == 0 && M <= (1 << 24) && K <= (1 << 23) &&
+         ceil_div(M, 32) * ceil_div(N, 32) < (1LL << 31) - 8;              // a tile's offsets of 32 bits
 }
 
 // Which kernel, us at one MI355X (K = 2,048 unless given; every one gives the same bits):
 //  * K of one segment, and up to 16 tokens or so few tiles as below: a wave per chain.
 //  * up to 8 tokens, or 16 where the columns are fewer than 16,384: 16 rows of w per workgroup. 2,048 columns at 8 tokens 13
 //    (tiles of 32 tokens 36), 128,256 at 1 token 187 (234); at 16 tokens 282 (224).
-//  * fewer tiles of 32 tokens than half the compute units: the same kernel with 32 tokens. 64 tokens x 2,048 columns 16
-//    (35), K = 8,192 54 (128); 200 tokens 50 (35).
-//  * tiles of 32 tokens while those of 64 are so few that their last round is mostly empty: 600 x 2,048 71 (84), K = 8,192
-//    267 (319); 600 x 3,072 97 (85); from there on tiles of 64: 600 x 16,384 404 (422), 100 TFLOP/s.
+//  * tiles of 32 tokens x 64 columns for a quarter of the compute units at most: the same kernel with 32 tokens. 64 tokens x 2,048 columns 17 (tiles 18),
+//    33 x 2,048 x 8,192 53 (62), 24 x 3,072 15 (18).
+//  * tiles: what the compute unit with the most of them takes, in columns x tokens over the share of its rate that a shape gets from as many
+//    workgroups as it has. 600 x 16,384 in tiles of 64 x 64 / 32 x 64 / 32 x 32 343 / 331 to 372 / -, 2,048 x 16,384 1,059 / 1,100 / -, 600 x 2,048 68 / 55 / 59,
+//    x 8,192 258 / 199 / 238, 300 x 2,048 - / 39 / 32, 150 x 2,048 x 8,192 - / 101 / 90, 17 x 16,384 - / 37 / 33, 128 x 3,072 - / 30 / 26.
 int launch_linear_f32(hipStream_t s, const float* x, const float* w, float* out, int M, int N, int K) {
-  const int64_t tiles64 = ceil_div(M, 64) * ceil_div(N, 64), tiles32 = ceil_div(M, 32) * ceil_div(N, 64);
+  const int64_t tiles32 = ceil_div(M, 32) * ceil_div(N, 64);
+  auto cost = [&](int bm, int bn, double share) {
+    const int64_t each = ceil_div(ceil_div(M, bm) * ceil_div(N, bn), 256);
+    return static_cast<double>(each) * bm * bn / (share * (bm * bn > 2048 || each > 2 ? 1.0 : (each == 2 ? 0.85 : 0.62)));
+  };
   if (K <= kSegment && M <= 16) launch_rows_short<1>(s, x, w, out, M, N, K);
   else if (K <= kSegment && tiles32 <= 128) launch_rows_short<2>(s, x, w, out, M, N, K);
   else if (M <= 8 || (M <= 16 && N < 16384)) launch_rows<1>(s, x, w, out, M, N, K);
-  else if (tiles32 <= 128) launch_rows<2>(s, x, w, out, M, N, K);
-  else if (tiles64 <= 384) launch_tiles<32>(s, x, w, out, M, N, K);
-  else launch_tiles<64>(s, x, w, out, M, N, K);
+  else if (tiles32 <= 64) launch_rows<2>(s, x, w, out, M, N, K);
+  else if (cost(64, 64, 1.0) <= std::min(cost(32, 64, 0.94), cost(32, 32, 0.78))) launch_tiles<64, 64, 2, 4>(s, x, w, out, M, N, K);
+  else if (cost(32, 64, 0.94) <= cost(32, 32, 0.78)) launch_tiles<32, 64, 1, 4>(s, x, w, out, M, N, K);
+  else launch_tiles<32, 32, 2, 2>(s, x, w, out, M, N, K);
   return check_launch("psamd_linear");
 }
 
