@@ -34,6 +34,8 @@
 
 #include "api.h"
 #include "common.h"
+#include "linear_stream.h"
+#include "stream_operands.h"
 #include "tile_product.h"
 
 namespace psamd {
@@ -782,6 +784,151 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(
   }
 }
 
+// The same tiles of up to 16 pairs with both operands through LDS in whole lines, for K and F multiples of 64 (the kernel above loads its matrix as a
+// matrix instruction's operand, 16 rows x 64 bytes, one round ahead). TN columns a workgroup; steps, units, buffers and waves as in
+// stream_tiles_kernel (linear_stream.hip). Bound by reading the used experts' matrices once; each workgroup begins at another place of K, as rows
+// of w lie a power of two apart (that alone gave the kernel above 10%). us of routing and experts, above / here (TB/s of the used experts' matrices):
+//   32 experts of 2,048 x 1,024, 8 choices, 1, 2, 4, 8, 16 and 64 tokens   45.8, 52.5, 78.0, 96.6, 104.7, 126.6 / 34.7, 42.9, 69.0, 81.1, 88.3 (4.6), 101.7
+//    the same without gates                                              32.4, 43.6, 65.7, 75.5,  74.0,  85.2 / 26.7, 38.9, 57.2, 65.2, 65.8, 76.1
+//    8 of 4,096 x 3,584, 2 choices, 1, 8, 16, 64                         78.1, 145.9, 158.8, 210.5 / 51.0, 122.3, 134.8 (5.2), 160.5
+//   64 of 2,048 x 1,408, 6 choices, 1, 2, 8, 16                          39.5, 57.9, 140.9, 206.0 / 33.0, 62.4, 110.7, 169.9
+// (1 and 2 tokens: pair by pair before.)
+template <int TN, int KG, int STAGES, int FORM>
+__global__ __launch_bounds__(64 * (TN / 16) * KG) void moe_stream_kernel(
+    const bf16_t* __restrict__ a, const float* __restrict__ pair_weight, const bf16_t* __restrict__ w,
+    const int32_t* __restrict__ sorted, const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_first,
+    const int32_t* __restrict__ tile_count, bf16_t* __restrict__ out_act, float* __restrict__ out_f32, int64_t tokens,
+    int K, int N, int top, float gate_alpha, float limit, float up_shift, int into_stream,
+    const float* __restrict__ col_scale, int experts, const bf16_t* __restrict__ x, const float* __restrict__ weight) {
+  constexpr bool GATED = FORM == kFormGated;
+  constexpr int CT = TN / 16, RT = GATED ? 2 : 1, ROWS = TN * RT, W = CT * KG, LW = KG * ROWS / 8 / W;
+  constexpr int XC = 2 * KG, LX = (XC + W - 1) / W;                              // copies of 8 pairs a step, of a wave
+  constexpr int W_STEP = KG * ROWS * 128, STEP = W_STEP + KG * 2048;
+  static_assert(LW * 8 * W == KG * ROWS && (XC % W == 0 || W % XC == 0), "whole copies per wave");
+  static_assert(W * RT * 1024 <= STAGES * STEP, "the sums of the units' waves fit where the steps were");
+  extern __shared__ __align__(16) unsigned char moe_smem[];                      // STAGES x [KG][ROWS rows of w][128], [KG][16 pairs][128]
+  const int slot = blockIdx.y;
+  const int e = tile_expert[slot];
+  if (e < 0) return;                            // uniform for the workgroup
+  const int first = tile_first[slot], count = tile_count[slot];
+  const int n0 = static_cast<int>(blockIdx.x) * TN;
+  if (e >= experts) {                           // a tile of identity pairs: the tokens themselves times their weights
+    if (FORM != kFormDown) return;
+    for (int idx = threadIdx.x; idx < count * TN; idx += blockDim.x) {
+      const int pair = sorted[first + idx / TN], n = n0 + idx % TN;
+      if (n >= N) continue;
+      const int64_t t = pair / top;
+      const float y = weight[pair] * bf16_to_float(x[t * N + n]);
+      if (into_stream) add_float(out_f32 + t * N + n, col_scale != nullptr ? col_scale[n] * y : y);
+      else out_f32[(static_cast<int64_t>(pair % top) * tokens + t) * N + n] = y;
+    }
+    return;
+  }
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int r = lane & 15, g = lane >> 4;
+  const char* wb = reinterpret_cast<const char*>(w + static_cast<int64_t>(e) * (GATED ? 2 : 1) * N * K);
+  const char* ab = reinterpret_cast<const char*>(a);
+  uint32_t w_off[LW], x_off[LX];
+#pragma unroll
+  for (int i = 0; i < LW; ++i) {
+    const int row = (wave * LW + i) % (ROWS / 8) * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+    const int col = min(n0 + row % TN, N - 1);
+    w_off[i] = static_cast<uint32_t>(row >= TN ? N + col : col) * (2u * K) + 16u * piece;
+  }
+#pragma unroll
+  for (int i = 0; i < LX; ++i) {                // where waves outnumber the copies, some bring the same rows to the same place
+    const int row = (wave * LX + i) % 2 * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+    const int pair = sorted[first + min(row, count - 1)];
+    x_off[i] = static_cast<uint32_t>(FORM != kFormDown ? pair / top : pair) * (2u * K) + 16u * piece;
+  }
+  const int units = K / 64, steps = (units + KG - 1) / KG, end = units * 128;
+  int from = static_cast<int>((blockIdx.x + 5u * blockIdx.y) % static_cast<unsigned>(units)) * 128, to = 0;
+  auto unit_at = [&](int unit) {
+    const int k = from + unit * 128;
+    return min(k >= end ? k - end : k, end - 128);
+  };
+  auto copy = [&]() {
+#pragma unroll
+    for (int i = 0; i < LW; ++i) {
+      const int at = wave * LW + i;
+      __builtin_amdgcn_global_load_lds((global_ptr)(wb + unit_at(at / (ROWS / 8)) + w_off[i]), (lds_ptr)(moe_smem + to + at * 1024), 16, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < LX; ++i) {
+      const int at = (wave * LX + i) % XC;
+      __builtin_amdgcn_global_load_lds((global_ptr)(ab + unit_at(at / 2) + x_off[i]), (lds_ptr)(moe_smem + to + W_STEP + at * 1024), 16, 0, 0);
+    }
+    from = min(from + KG * 128 >= end ? from + KG * 128 - end : from + KG * 128, end - 128);
+    to = to + STEP == STAGES * STEP ? 0 : to + STEP;
+  };
+#pragma unroll
+  for (int t = 0; t < STAGES - 1; ++t)
+    if (t < steps) copy();
+  f32x4 acc[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) acc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int tile = wave % CT, unit = wave / CT;
+  const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_bytes)moe_smem)), piece0 = 16u * (g ^ ((r >> 1) & 7));
+  const uint32_t w_at = base + (unit * ROWS + 16 * tile + r) * 128 + piece0, x_at = base + W_STEP + (unit * 16 + r) * 128 + piece0;
+  uint32_t at = 0;
+  for (int t = 0; t < steps; ++t) {
+    __builtin_amdgcn_sched_barrier(0);
+    wait_for_step<LW + LX, STAGES - 2>(steps - 1 - t);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (t + STAGES - 1 < steps) copy();
+    __builtin_amdgcn_sched_barrier(0);
+    if (t * KG + unit < units) {
+      Operands<TN, RT, 1> ops;
+      ops.read(w_at + at, x_at + at);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ops.w[h][rt], ops.x[h][0], acc[rt], 0, 0, 0);
+    }
+    at = at + STEP == STAGES * STEP ? 0 : at + STEP;
+  }
+  f32x4* const parts = reinterpret_cast<f32x4*>(moe_smem);                       // [KG][CT][RT][64 lanes]
+  __syncthreads();
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) parts[(wave * RT + rt) * 64 + lane] = acc[rt];
+  __syncthreads();
+  if (wave >= CT) return;
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    acc[rt] = parts[(wave * RT + rt) * 64 + lane];
+#pragma unroll
+    for (int q = 1; q < KG; ++q) acc[rt] += parts[((q * CT + wave) * RT + rt) * 64 + lane];
+  }
+  // Lane (r, g) holds, for the pair in row r, columns 4 g .. + 3 of its wave's sixteen.
+  const int nc = n0 + 16 * tile + 4 * g;
+  if (r >= count || nc >= N) return;                                             // N is a multiple of 8
+  const int pair = sorted[first + r];
+  const float pw = pair_weight != nullptr ? pair_weight[pair] : 1.f;             // on the input's sums (GATED) or on the output's
+  if (FORM != kFormDown) {
+    bf16_t res[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      if (!GATED) {
+        const float p = fmaxf(pw * acc[0][v], 0.f);
+        res[v] = float_to_bf16(p * p);
+        continue;
+      }
+      const float gg = fminf(pw * acc[0][v], limit);
+      const float uu = fminf(fmaxf(pw * acc[RT - 1][v], -limit), limit);
+      res[v] = float_to_bf16(gg / (1.f + __expf(-gate_alpha * gg)) * (uu + up_shift));
+    }
+    *reinterpret_cast<ushort4*>(out_act + static_cast<int64_t>(pair) * N + nc) = ushort4{res[0], res[1], res[2], res[3]};
+  } else if (into_stream) {
+    float* o = out_f32 + static_cast<int64_t>(pair / top) * N + nc;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) add_float(o + v, (col_scale != nullptr ? col_scale[nc + v] : 1.f) * (pw * acc[0][v]));
+  } else {
+    *reinterpret_cast<float4*>(out_f32 + (static_cast<int64_t>(pair % top) * tokens + pair / top) * N + nc) =
+        float4{pw * acc[0][0], pw * acc[0][1], pw * acc[0][2], pw * acc[0][3]};
+  }
+}
+
 // ------------------------------------------------------------------ experts, many pairs each
 
 // A tile of up to TM pairs by TN rows of the expert's matrix per workgroup of WM x WN waves, both operands through LDS 64 k at a
@@ -973,6 +1120,42 @@ static int launch_grouped(hipStream_t s, const ExpertCall& c, const int32_t* int
   return check_launch("psamd_moe_experts_grouped (down)");
 }
 
+template <int TN, int FORM>
+static int run_stream(hipStream_t s, const ExpertCall& c, const int32_t* ints, int max_tiles) {
+  constexpr int KG = 128 / TN, STAGES = FORM == kFormGated ? 2 : 3;              // two workgroups share a compute unit
+  constexpr size_t smem = static_cast<size_t>(STAGES) * KG * ((FORM == kFormGated ? 2 : 1) * TN + 16) * 128;
+  auto kernel = moe_stream_kernel<TN, KG, STAGES, FORM>;
+  if (smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              static_cast<int>(smem)) != hipSuccess)
+    return fail("psamd_moe_experts_grouped: " + std::to_string(smem) + " bytes of LDS were refused");
+  const int32_t* t_e = ints + c.tokens * c.top;
+  constexpr bool down = FORM == kFormDown;
+  const int N = down ? c.K : c.F, K = down ? c.F : c.K;
+  kernel<<<dim3(static_cast<unsigned>(ceil_div(N, TN)), static_cast<unsigned>(max_tiles)), dim3(512), smem, s>>>(
+      static_cast<const bf16_t*>(down ? c.act : c.x), (c.weight_on_output != 0) == down ? c.weight : nullptr,
+      static_cast<const bf16_t*>(down ? c.w_down : c.w_in), ints, t_e, t_e + max_tiles, t_e + 2 * max_tiles,
+      down ? nullptr : static_cast<bf16_t*>(c.act), down ? c.out : nullptr, c.tokens, K, N, c.top, c.gate_alpha, c.limit, c.up_shift,
+      c.into_stream, c.col_scale, c.experts, static_cast<const bf16_t*>(c.x), c.weight);
+  return check_launch("psamd_moe_experts_grouped (small tiles)");
+}
+
+// Columns a workgroup: the most that leave it a few hundred workgroups, were there a tile a slot. us of a whole step's experts (sorting included), columns
+// of the first product / the second: 32 experts of 2,048 x 1,024, 8 tokens x 8 choices 32/64 74.8, 32/32 75.0, 64/64 77.1, 16/64 85.8, 16/16 101; 24 of
+// 1,024 x 320, 8 x 4 17.4, 18.1, 19.1, 18.6, 23.7; 4 of 1,024 x 512, 5 x 2 14.8, 14.0, 17.1, 13.8, 13.1.
+template <int FORM>
+static int launch_stream_form(hipStream_t s, const ExpertCall& c, const int32_t* ints, int max_tiles) {
+  const int64_t N = FORM == kFormDown ? c.K : c.F;
+  if (FORM == kFormDown && ceil_div(N, 64) * max_tiles >= 384) return run_stream<64, FORM>(s, c, ints, max_tiles);
+  if (ceil_div(N, 32) * max_tiles >= 192) return run_stream<32, FORM>(s, c, ints, max_tiles);
+  return run_stream<16, FORM>(s, c, ints, max_tiles);
+}
+
+static int launch_stream(hipStream_t s, const ExpertCall& c, const int32_t* ints, int max_tiles) {
+  if (c.kind == kExpertGated ? launch_stream_form<kFormGated>(s, c, ints, max_tiles) : launch_stream_form<kFormSquaredRelu>(s, c, ints, max_tiles))
+    return 1;
+  return launch_stream_form<kFormDown>(s, c, ints, max_tiles);
+}
+
 template <int TM, int TN, int WM, int WN, int FORM>
 static int run_tiles(hipStream_t s, const ExpertCall& c, const int32_t* ints, int max_tiles) {
   constexpr size_t kSmem = tile_smem_steps(TM, TN) + TM * sizeof(int32_t);
@@ -1013,13 +1196,17 @@ static bool tiles_take(int64_t tokens, int64_t pairs, int K, int F) {
   return K % 64 == 0 && F % 64 == 0 && 2 * tokens * K <= most && 2 * pairs * F <= most && 4LL * K * F <= most;
 }
 
-// ... and their rows: 0 where the kernel above takes the step (from 48 pairs an expert on it is the slower one everywhere; below,
-// the router's kernel may have sorted the pairs into its tiles), 256 where the device chooses tiles of up to 256 x 256 by the step's
+// From how many pairs an expert on a step that sorts its pairs itself takes the large tiles; below, moe_stream_kernel reads an expert once per 16 pairs. us of
+// routing and experts, small tiles / large: 32 experts of 2,048 x 1,024 at 16, 20, 24, 28, 46 pairs each 102, 113, 117, 122, 149 / 112, 116, 116, 117, 123; 8 of
+// 4,096 x 3,584 at 16, 24, 46 161, 182, 238 / 181, 181, 186; 24 of 1,024 x 320 at 16, 28, 46 31, 38, 43 / 35, 37, 39; 64 of 2,048 x 1,408 at 12, 16, 24 224, 248, 315 / 233, 239, 244.
+constexpr int64_t kTilesFromPairs = 24;
+
+// ... and their rows: 0 where the kernel for small tiles takes the step, 256 where the device chooses tiles of up to 256 x 256 by the step's
 // counts. Those ask for half the bytes per product, but one workgroup of them fills a compute unit, two of 128 x 128 share one, and a
 // last round that is not full costs nearly as much as one that is: the time is that of the rounds, K long in the first product and F
 // in the second, and 300 more for what a large tile does in front of and behind its loop, which the two small ones on a unit do beside
 // each other's. An expert's last tile is half empty on average. us of both products and the sorting, 256 / 128 / the kernel above
-// (E experts of K x F, choices at random):
+// (E experts of K x F, choices at random; the kernel above is moe_grouped_kernel, in front of moe_stream_kernel):
 //   32 of 2,048 x 1,024:  50 pairs an expert 109 / 109 / 152, 140 126 / 146 / 227, 260 163 / 194 / 269, 448 232 / 261 / 337, 1,000 580 / 594 / 693
 //    8 of 2,048 x 1,024:  64 59 / 58 / 90, 260 70 / 66 / 110, 512 92 / 107 / 141, 1,000 166 / 156 / 235, 2,000 262 / 279 / 373
 //    8 of 4,096 x 3,584:  64 156 / 159 / 255, 260 301 / 397 / 441, 448 377 / 547 / 567, 1,000 848 / 1,128 / 1,048
@@ -1029,7 +1216,7 @@ static bool tiles_take(int64_t tokens, int64_t pairs, int K, int F) {
 // Over eight shapes at 17 sizes, choices even and uneven, the choice is on average 1.0% over the faster (always 256: 2.9%, always
 // 128: 7.8%), at worst 17%.
 static int wide_tile_rows(int64_t pairs, int experts, int K, int F, int kind) {
-  if (pairs < 48LL * experts) return 0;
+  if (pairs < kTilesFromPairs * experts) return 0;
   auto rounds = [&](int rows, int at_once, int beside) {
     const double tiles = std::max<double>(experts, static_cast<double>(pairs) / rows + 0.5 * experts);
     auto of = [&](int64_t columns) {
@@ -1215,6 +1402,7 @@ int psamd_moe_experts_grouped(void* stream, const void* x, const int32_t* chosen
   if (wide == 128) return launch_tiles<128, 128, 2, 2>(s, c, ints, max_tiles);
   if (rows == 128) return launch_grouped<8, 2>(s, c, ints, max_tiles);
   if (rows == 64) return launch_grouped<4, 2>(s, c, ints, max_tiles);
+  if (tiles_take(tokens, pairs, K, F)) return launch_stream(s, c, ints, max_tiles);
   return launch_grouped<1, 1>(s, c, ints, max_tiles);
 }
 

@@ -164,7 +164,7 @@ class HipOps:
     LIBRARY_ADD_MIN_ROWS = 1024     # from here on a product that feeds the residual stream adds into it in the library
     MOE_ROUTE_FUSED_MAX_TOKENS = 0   # up to here one kernel computes router logits and choice; above, product + choice
     MOE_CHOICE_SORTS_MAX_TOKENS = 16 # up to here the workgroup that chooses a step's experts also sorts the pairs
-    MOE_PAIRWISE_MAX_TOKENS = 2     # up to here a bfloat16 step's experts run pair by pair; above, grouped by expert
+    MOE_PAIRWISE_MAX_TOKENS = 2     # up to here the experts of a bfloat16 step whose width is no multiple of 64 run pair by pair; else grouped by expert
     DELTA_RUNS = True               # delta_scan takes ``in_runs``
     DELTA_RUNS_MIN_TOKENS = 340     # what a round of launches of the recurrences' runs costs, in tokens walked (see _runs_pay)
     DELTA_RUNS_SHORT = 64           # items of up to this many tokens beside it are walked: each would cost a whole run
@@ -933,7 +933,7 @@ class HipOps:
 
     def _groups_pairs(self, dtype: torch.dtype, t: int, k: int) -> bool:
         """Whether a step of ``t`` tokens of width ``k`` runs its experts grouped by expert."""
-        return dtype == torch.bfloat16 and t > self.MOE_PAIRWISE_MAX_TOKENS and k % 8 == 0
+        return dtype == torch.bfloat16 and t > 0 and k % 8 == 0 and (t > self.MOE_PAIRWISE_MAX_TOKENS or k % 64 == 0)
 
     def _group_ints(self, t: int, top: int, e: int) -> torch.Tensor:
         tiles = int(self.lib.psamd_moe_grouped_max_tiles(t * top, e))
