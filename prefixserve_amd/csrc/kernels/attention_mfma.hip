@@ -1192,7 +1192,7 @@ __global__ __launch_bounds__(64 * WV) void attn_decode_mfma_kernel(
     const int32_t* __restrict__ item_start,
     const int32_t* __restrict__ item_end, const int32_t* __restrict__ table_off,
     const int32_t* __restrict__ block_ids, int hq, int hkv, int nsplit, float scale, int window, int min_tiles,
-    int n_dec, Extras ex) {
+    int n_dec, int ld, Extras ex) {
   constexpr int D = 16 * NS;
   constexpr int KS = (D + 31) / 32;
   static_assert(!MERGE || WV == 4, "four waves merge the runs");
@@ -1362,7 +1362,8 @@ __global__ __launch_bounds__(64 * WV) void attn_decode_mfma_kernel(
     }
   }
 
-  // ---- merge the waves: smem = m[WV][group], l[WV][group], o[WV][group][D]
+  // ---- merge the waves: smem = m[WV][group], l[WV][group], o[WV][group][ld]. Rows of o are ld = D + 4 floats apart where that fits: D apart, the 16 heads
+  // that a store touches lay on the same four banks.
   float* sm_m = smem;
   float* sm_l = smem + WV * group;
   float* sm_o = smem + 2 * WV * group;
@@ -1375,16 +1376,41 @@ __global__ __launch_bounds__(64 * WV) void attn_decode_mfma_kernel(
         sm_l[wave * group + hh] = l[ct];
       }
 #pragma unroll
-      for (int ds = 0; ds < NS; ++ds)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          sm_o[(static_cast<int64_t>(wave) * group + hh) * D + 16 * ds + 4 * g4 + v] = o[ct][ds][v];
+      for (int ds = 0; ds < NS; ++ds) *reinterpret_cast<f32x4*>(sm_o + (wave * group + hh) * ld + 16 * ds + 4 * g4) = o[ct][ds];
     }
   }
   __syncthreads();
+  // Many numbers of many heads (16 heads of 256: 4,096, sixteen a thread): the waves' weights once per head, in place of their maxima.
+  const bool many = !MERGE && group * D > 1024;
+  float head_m = 0.f, head_l = 0.f;
+  if (many) {
+    const int hh = threadIdx.x;
+    if (hh < group) {
+      head_m = -INFINITY;
+#pragma unroll
+      for (int w = 0; w < WV; ++w) head_m = fmaxf(head_m, sm_m[w * group + hh]);
+#pragma unroll
+      for (int w = 0; w < WV; ++w) {
+        const float mw = sm_m[w * group + hh], wgt = mw == -INFINITY ? 0.f : __expf(mw - head_m);
+        head_l += wgt * sm_l[w * group + hh];
+        sm_m[w * group + hh] = wgt;
+      }
+      sm_l[hh] = head_m;                         // (its own head's numbers alone: read above)
+      if (WV > 1) sm_l[group + hh] = head_l;
+    }
+    __syncthreads();
+  }
   const int runs = MERGE ? (tile_hi - tile_lo + tps) / tps : 1;        // of this request that have keys
   // The workgroup's result for dimension d of head hh, not yet divided by its sum: the waves' results merged.
   auto combined = [&](int hh, int d, float& mm, float& ll) {
+    if (many) {
+      mm = sm_l[hh];
+      ll = sm_l[group + hh];
+      float acc = 0.f;
+#pragma unroll
+      for (int w = 0; w < WV; ++w) acc += sm_m[w * group + hh] * sm_o[(w * group + hh) * ld + d];
+      return acc;
+    }
     mm = -INFINITY;
 #pragma unroll
     for (int w = 0; w < WV; ++w) mm = fmaxf(mm, sm_m[w * group + hh]);
@@ -1394,7 +1420,7 @@ __global__ __launch_bounds__(64 * WV) void attn_decode_mfma_kernel(
     for (int w = 0; w < WV; ++w) {
       const float mw = sm_m[w * group + hh];
       const float wgt = mw == -INFINITY ? 0.f : __expf(mw - mm);
-      acc += wgt * sm_o[(static_cast<int64_t>(w) * group + hh) * D + d];
+      acc += wgt * sm_o[(w * group + hh) * ld + d];
       ll += wgt * sm_l[w * group + hh];
     }
     return acc;
@@ -1512,44 +1538,45 @@ __global__ __launch_bounds__(64 * WV) void attn_decode_mfma_kernel(
   }
 }
 
-// One block (64 threads) per (decode item, head): merges the splits and writes bfloat16.
-// Lane s first loads the statistics of split s, so the weights of all splits come from one
-// round of loads; then every lane sums its dimensions over the splits with loads that do
-// not depend on each other.
-__global__ __launch_bounds__(64) void attn_decode_merge_kernel(
+// One block (a thread per dimension, 64 to 256) per (decode item, head): merges the splits and writes bfloat16. Lane s of every wave loads
+// the statistics of split s, so the weights of all splits come from one round of loads; the first splits' partial outputs are asked for
+// together with them, the others sixteen at a time: a trip to memory is what this costs (16 heads of 256 in 12 runs: with 64 threads, eight
+// loads at a time and four dimensions a thread one after the other 8.1 us).
+__global__ __launch_bounds__(256) void attn_decode_merge_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, bf16_t* __restrict__ out,
     const int32_t* __restrict__ dec_items, const int32_t* __restrict__ item_start, int hq, int d, int nsplit, Extras ex) {
-  __shared__ float wgt_s[64];
-  const int di = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
+  __shared__ float wgt_s[4][64];
+  const int di = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & (kWave - 1), i = threadIdx.x;
   const int64_t t = item_start[dec_items[di]];
   const int64_t base = (static_cast<int64_t>(di) * hq + h) * nsplit;
   const bool has = lane < nsplit;                       // nsplit <= 64
   const float ms = has ? part_ml[(base + lane) * 2] : -INFINITY;
   const float ls = has ? part_ml[(base + lane) * 2 + 1] : 0.f;
-  // The first splits' partial outputs are asked for together with the statistics, not after them.
-  constexpr int kEarly = 8;
-  float early[kEarly];
+  constexpr int kAhead = 16;
+  float early[kAhead];
 #pragma unroll
-  for (int s = 0; s < kEarly; ++s) early[s] = (s < nsplit && lane < d) ? part_o[(base + s) * d + lane] : 0.f;
+  for (int s = 0; s < kAhead; ++s) early[s] = (s < nsplit && i < d) ? part_o[(base + s) * d + i] : 0.f;
   const float mm = wave_max(ms);
   const float w = ms == -INFINITY ? 0.f : __expf(ms - mm);
   float ll = wave_sum(w * ls);
   if (ex.sink != nullptr) ll += __expf(ex.sink[h] - mm);
-  wgt_s[lane] = w / ll;
-  __syncthreads();
-  for (int i = lane; i < d; i += kWave) {
-    float acc = 0.f;
-    int s0 = 0;
-    if (i == lane) {
+  float* wgt = wgt_s[threadIdx.x >> 6];                 // each wave its own: no barrier
+  wgt[lane] = w / ll;
+  __builtin_amdgcn_wave_barrier();
+  __threadfence_block();
+  if (i >= d) return;
+  float acc = 0.f;
 #pragma unroll
-      for (int s = 0; s < kEarly; ++s) acc += (s < nsplit ? wgt_s[s] : 0.f) * early[s];
-      s0 = kEarly;
-    }
-#pragma unroll 8
-    for (int s = s0; s < nsplit; ++s) acc += wgt_s[s] * part_o[(base + s) * d + i];
-    if (ex.gate != nullptr) acc *= 1.f / (1.f + __expf(-bf16_to_float(ex.gate[t * ex.gate_row + h * d + i])));
-    out[t * (static_cast<int64_t>(hq) * d) + h * d + i] = float_to_bf16(acc);
+  for (int s = 0; s < kAhead; ++s) acc += (s < nsplit ? wgt[s] : 0.f) * early[s];
+  for (int s0 = kAhead; s0 < nsplit; s0 += kAhead) {
+    float v[kAhead];
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) v[s] = s0 + s < nsplit ? part_o[(base + s0 + s) * d + i] : 0.f;
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) acc += (s0 + s < nsplit ? wgt[s0 + s] : 0.f) * v[s];
   }
+  if (ex.gate != nullptr) acc *= 1.f / (1.f + __expf(-bf16_to_float(ex.gate[t * ex.gate_row + h * d + i])));
+  out[t * (static_cast<int64_t>(hq) * d) + h * d + i] = float_to_bf16(acc);
 }
 
 // Bytes of LDS the grouped kernel needs for head size D, kt 32-key tiles per wave and
@@ -1738,23 +1765,27 @@ static int launch_decode(hipStream_t s, const void* qkv, int q_stride, const voi
                          int window, int min_tiles) {
   const int group = hq / hkv;
   // The waves' results, and for the merge two numbers per head and run.
-  const size_t smem = sizeof(float) * std::max<size_t>(8 * group + 4 * static_cast<size_t>(group) * 16 * NS, 2 * static_cast<size_t>(group) * nsplit);
+  auto bytes = [&](int waves, int ld) {
+    return sizeof(float) * std::max<size_t>(waves * static_cast<size_t>(group) * (2 + ld), 2 * static_cast<size_t>(group) * nsplit);
+  };
   const int64_t groups_of_8 = ceil_div(static_cast<int64_t>(n_dec) * nsplit, 8);
-  auto run = [&](auto kernel, int waves, size_t smem) {
+  auto run = [&](auto kernel, int waves) {
+    const int ld = 16 * NS + (bytes(waves, 16 * NS + 4) <= 160 * 1024 ? 4 : 0);
+    const size_t smem = bytes(waves, ld);
     if (!lds_allowed(kernel, smem)) return fail("psamd_attention_decode: " + std::to_string(smem) + " bytes of LDS were refused");
     kernel<<<dim3(8 * hkv, static_cast<unsigned>(groups_of_8)), dim3(64 * waves), smem, s>>>(
         static_cast<const bf16_t*>(qkv), q_stride, static_cast<const bf16_t*>(kv), static_cast<bf16_t*>(out), part_o,
         part_ml, arrived, dec_items, item_start, item_end, table_off, block_ids, hq, hkv, nsplit, scale, window, min_tiles, n_dec,
-        g_extras);
+        ld, g_extras);
     return check_launch("psamd_attention_decode");
   };
   if constexpr (CT == 1) {
-    if (arrived != nullptr) return run(attn_decode_mfma_kernel<NS, CT, P3, true>, 4, smem);
+    if (arrived != nullptr) return run(attn_decode_mfma_kernel<NS, CT, P3, true>, 4);
     const int64_t pairs = static_cast<int64_t>(n_dec) * hkv;
     if (nsplit == 1 && pairs >= kOneRun && pairs <= 256)
-      return run(attn_decode_mfma_kernel<NS, CT, P3, false, 8>, 8, sizeof(float) * 8 * (2 + 16 * NS) * static_cast<size_t>(group));
+      return run(attn_decode_mfma_kernel<NS, CT, P3, false, 8>, 8);
   }
-  return run(attn_decode_mfma_kernel<NS, CT, P3>, 4, smem);
+  return run(attn_decode_mfma_kernel<NS, CT, P3>, 4);
 }
 
 template <int NS, bool P3>
@@ -2006,7 +2037,7 @@ int psamd_attention_decode(void* stream, const void* qkv, int q_stride, void* ou
   }
 #undef PSAMD_DEC_NS
   if (rc != 0 || nsplit == 1 || arrived != nullptr) return rc;
-  attn_decode_merge_kernel<<<dim3(n_dec, hq), dim3(64), 0, s>>>(part_o, part_ml, static_cast<bf16_t*>(out), dec_items,
+  attn_decode_merge_kernel<<<dim3(n_dec, hq), dim3(static_cast<unsigned>(64 * ceil_div(head_dim, 64))), 0, s>>>(part_o, part_ml, static_cast<bf16_t*>(out), dec_items,
                                                                item_start, hq, head_dim, nsplit, g_extras);
   return check_launch("psamd_attention_decode(merge)");
 }
