@@ -253,6 +253,105 @@ __global__ __launch_bounds__(256) void general_delta_prepare_kernel(
   }
 }
 
+// The same for more tokens, 16 of one head a workgroup, head sizes up to 64 C: a lane owns C columns, of which it holds sixteen
+// rows of the map at a time for its wave's four tokens, and its rows are under way before the first sum. Above, every thread
+// walks the whole map for its one number: a load, an LDS read and one dependent multiply-add after the other. The sums keep
+// their order, so the bits are the same. 32 heads of 64, rank 64, bfloat16: 600 tokens 26.7 -> 15.9 us, 2,048 70.8 -> 37.0 (2.7
+// TB/s of what is written). Eight tokens a wave: 18.9 and 37.5, two: 18.6 and 43.6.
+constexpr int kBlockTokens = 16;
+
+template <typename A, int C>
+__global__ __launch_bounds__(256) void general_delta_prepare_block_kernel(
+    const A* __restrict__ rows, int64_t in_row, int r_col, int k_col, int v_col, int a_col, int l_col,
+    const float* __restrict__ a_bias, const float* __restrict__ w2, const float* __restrict__ w0, float* __restrict__ ops,
+    int64_t tokens, int heads, int dim, int rank, float decay_floor, float unit_eps) {
+  constexpr int MINE = kBlockTokens / 4, RUN = 16;
+  extern __shared__ __align__(16) float prep_block_smem[];                       // tanh(l)[16][padded], zeros behind the rank
+  const int padded = (rank + RUN - 1) / RUN * RUN;
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kBlockTokens, hd = static_cast<int64_t>(heads) * dim;
+  const int nt = static_cast<int>(min(static_cast<int64_t>(kBlockTokens), tokens - t0));
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+  const int first = wave * MINE;                                                 // of this wave's tokens; those behind nt repeat the last
+  int64_t hc[C];
+  bool in[C];
+  float low[MINE][C], w[RUN][C], bias[C];
+  A r[MINE][C], k[MINE][C], v[MINE][C], rate[MINE][C];
+  auto load_map = [&](int j0) {
+#pragma unroll
+    for (int j = 0; j < RUN; ++j)
+#pragma unroll
+      for (int c = 0; c < C; ++c) w[j][c] = j0 + j < rank ? w2[(j0 + j) * hd + hc[c]] : 0.f;
+  };
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    in[c] = lane + kWave * c < dim;
+    hc[c] = static_cast<int64_t>(blockIdx.y) * dim + min(lane + kWave * c, dim - 1);
+    bias[c] = a_bias[hc[c]];
+#pragma unroll
+    for (int m = 0; m < MINE; ++m) low[m][c] = w0[hc[c]];
+  }
+  for (int idx = threadIdx.x; idx < nt * padded; idx += blockDim.x) {
+    const int tk = idx / padded, j = idx - tk * padded;
+    prep_block_smem[idx] = j < rank ? tanhf(to_float<A>(rows[(t0 + tk) * in_row + l_col + j])) : 0.f;
+  }
+  load_map(0);
+#pragma unroll
+  for (int m = 0; m < MINE; ++m) {
+    const A* row = rows + (t0 + min(first + m, nt - 1)) * in_row;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      r[m][c] = row[r_col + hc[c]];
+      k[m][c] = row[k_col + hc[c]];
+      v[m][c] = row[v_col + hc[c]];
+      rate[m][c] = row[a_col + hc[c]];
+    }
+  }
+  __syncthreads();
+  for (int j0 = 0; j0 < rank; j0 += RUN) {
+    if (j0 > 0) load_map(j0);
+#pragma unroll
+    for (int m = 0; m < MINE; ++m) {
+      const float4* th = reinterpret_cast<const float4*>(prep_block_smem + min(first + m, nt - 1) * padded + j0);
+#pragma unroll
+      for (int q = 0; q < RUN / 4; ++q) {
+        const float4 x = th[q];
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+          low[m][c] = fmaf(w[4 * q][c], x.x, low[m][c]);
+          low[m][c] = fmaf(w[4 * q + 1][c], x.y, low[m][c]);
+          low[m][c] = fmaf(w[4 * q + 2][c], x.z, low[m][c]);
+          low[m][c] = fmaf(w[4 * q + 3][c], x.w, low[m][c]);
+        }
+      }
+    }
+  }
+  float inv[MINE];
+#pragma unroll
+  for (int m = 0; m < MINE; ++m) {
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+      if (in[c]) ss = fmaf(to_float<A>(k[m][c]), to_float<A>(k[m][c]), ss);
+    inv[m] = 1.f / sqrtf(wave_sum(ss) + unit_eps);
+  }
+#pragma unroll
+  for (int m = 0; m < MINE; ++m) {
+    if (first + m >= nt) break;                                                  // uniform for the wave
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      if (!in[c]) continue;
+      const float key = to_float<A>(k[m][c]), unit = key * inv[m];
+      float* o = ops + (t0 + first + m) * 6 * hd + hc[c];
+      o[0] = to_float<A>(r[m][c]);
+      o[hd] = key;
+      o[2 * hd] = to_float<A>(v[m][c]);
+      o[3 * hd] = expf(-decay_floor * sigmoidf_(low[m][c]));
+      o[4 * hd] = -sigmoidf_(to_float<A>(rate[m][c]) + bias[c]) * unit;
+      o[5 * hd] = unit;
+    }
+  }
+}
+
 // ------------------------------------------------------------------ the recurrence
 
 // Sum over the 16 lanes of a row, in every lane, by four data-parallel moves inside the vector unit (lane
@@ -591,16 +690,27 @@ int psamd_general_delta_prepare(void* stream, const void* rows, int act_dtype, i
                 "columns outside the rows");
   if (tokens == 0) return 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid(static_cast<unsigned>(ceil_div(tokens, kPrepTokens)), static_cast<unsigned>(heads));
-  const size_t smem = sizeof(float) * kPrepTokens * (static_cast<size_t>(rank) + 1);
+  // Sixteen tokens a workgroup where that leaves the chip full. Below, the four of the other kernel are ahead: 300 workgroups
+  // (600 tokens, 8 heads) 10.8 us against 9.0; from 450 (600 tokens, 12 heads: 12.4 against 13.6) they are behind. 32 KB of LDS
+  // hold the tokens' values of a rank of 512.
+  const size_t block_smem = sizeof(float) * kBlockTokens * ((static_cast<size_t>(rank) + 15) / 16 * 16);
+  const bool blocks = ceil_div(tokens, kBlockTokens) * heads >= 448 && dim <= 2 * kWave && block_smem <= 32 * 1024;
+  auto run = [&](auto kernel, auto type, int per_block, size_t smem) {
+    using A = decltype(type);
+    kernel<<<dim3(static_cast<unsigned>(ceil_div(tokens, per_block)), static_cast<unsigned>(heads)), dim3(256), smem, s>>>(
+        static_cast<const A*>(rows), in_row, r_col, k_col, v_col, a_col, l_col, a_bias, w2, w0, ops, tokens, heads, dim, rank,
+        decay_floor, unit_eps);
+  };
+  auto pick = [&](auto type) {
+    using A = decltype(type);
+    if (!blocks) return run(general_delta_prepare_kernel<A>, type, kPrepTokens, sizeof(float) * kPrepTokens * (rank + 1u));
+    if (dim <= kWave) return run(general_delta_prepare_block_kernel<A, 1>, type, kBlockTokens, block_smem);
+    run(general_delta_prepare_block_kernel<A, 2>, type, kBlockTokens, block_smem);
+  };
   if (act_dtype == kBF16) {
-    general_delta_prepare_kernel<bf16_t><<<grid, dim3(256), smem, s>>>(static_cast<const bf16_t*>(rows), in_row, r_col, k_col,
-                                                                      v_col, a_col, l_col, a_bias, w2, w0, ops, tokens, heads,
-                                                                      dim, rank, decay_floor, unit_eps);
+    pick(bf16_t{});
   } else if (act_dtype == kF32) {
-    general_delta_prepare_kernel<float><<<grid, dim3(256), smem, s>>>(static_cast<const float*>(rows), in_row, r_col, k_col,
-                                                                     v_col, a_col, l_col, a_bias, w2, w0, ops, tokens, heads, dim,
-                                                                     rank, decay_floor, unit_eps);
+    pick(float{});
   } else {
     return fail("psamd_general_delta_prepare: activation dtype must be float32 or bfloat16");
   }

@@ -725,3 +725,39 @@ def test_long_prompts_go_through_the_runs(tmp_path, monkeypatch):
     traces.compare(TraceReplayer(runner).run_step, steps, expect, truth, 1.0, errors)
     check_rows(errors, "bfloat16", bf16_bars(folder, truth, reqs))
     assert taken == [(0, 4, 128, 64, True), (2, 2, 64, 64, True)] * 2
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,dim,rank,tokens", [(28, 64, 64, 241), (7, 128, 16, 1024), (23, 100, 13, 331), (32, 40, 17, 257),
+                                                   (448, 64, 1, 3), (7, 65, 512, 1009)])
+def test_general_delta_operands_of_many_tokens(ops, dtype, heads, dim, rank, tokens):
+    """From 448 workgroups of sixteen tokens and a head on another kernel makes them: the sums in the same order, so the bits of
+    calls of a few tokens. Heads that do not fill their lanes, ranks that do not fill a step, tokens behind the last sixteen."""
+    torch.manual_seed(0)
+    hd, floor, eps = heads * dim, 0.6, 1e-6
+    rows = torch.randn(tokens, 5 * hd + rank + 3, device=DEV).to(dtype)
+    w2, w0, bias = torch.randn(rank, hd, device=DEV) * 0.2, torch.randn(hd, device=DEV), torch.randn(hd, device=DEV)
+
+    def make(x):
+        out = torch.full((x.shape[0], 6 * hd), float("nan"), device=DEV)
+        ops.general_delta_prepare(x, 0, hd, 2 * hd, 3 * hd, 5 * hd + 3, bias, w2, w0, out, heads, dim, floor, eps)
+        return out
+
+    got = make(rows)
+    few = 448 // heads * 16 - 16
+    if heads < 448:
+        assert torch.equal(got, torch.cat([make(rows[i: i + few]) for i in range(0, tokens, few)]))
+    x = rows.double()
+    r, k, v, a = (x[:, i * hd: (i + 1) * hd] for i in range(4))
+    th = torch.tanh(x[:, 5 * hd + 3:])
+    low, size = th @ w2.double() + w0.double(), th.abs() @ w2.double().abs() + w0.double().abs()
+    kh = k.view(tokens, heads, dim)
+    c = (kh / torch.sqrt((kh * kh).sum(-1, keepdim=True) + eps)).view(tokens, hd)
+    u = 2.0 ** -24
+    # Each term's tanh 2 u off, the sum's rank roundings: low (rank + 4) u of its terms' sizes; w moves by at most floor / 4 of
+    # that, and by sigmoid, product and exp, 8 u of at most 1. Directions: a sum of dim squares, its root, quotient, product.
+    assert torch.equal(got[:, : 3 * hd], torch.cat([r, k, v], -1).float())
+    assert ((got[:, 3 * hd: 4 * hd] - torch.exp(-floor * torch.sigmoid(low))).abs() <= u * (floor / 4 * (rank + 4) * size + 8)).all()
+    assert ((got[:, 5 * hd:] - c).abs() <= u * (dim / 2 + 4) * c.abs()).all()
+    p = -torch.sigmoid(a + bias.double()) * c
+    assert ((got[:, 4 * hd: 5 * hd] - p).abs() <= u * (dim / 2 + 4 + 8 + (a + bias.double()).abs()) * c.abs()).all()
