@@ -12,7 +12,7 @@
 //     L_ts = (c_t D_{t-1}) . (p_s / D_s), W = U (what is taken out), Wx = T (M X), M_ts = (c_t D_{t-1}) . (k_s / D_s),
 //     Kt = T (c D_{-1}), and what the values alone leave in the output (Y) and the state (Z).
 // Three launches: runs_prepare (all runs side by side: everything that does not need S0), runs_chain (an item's runs in turn:
-// two small products each), runs_output (all runs side by side). 2,048 tokens as above: 66 + 94 + 30 us (gated), 126 + 59 + 25
+// two small products each), runs_output (all runs side by side). 2,048 tokens as above: 41 + 93 + 28 us (gated), 107 + 60 + 24
 // (general). The chain is what bounds a long prompt: 64 matrix instructions and two barriers a run, 2.9 us of 32 runs in turn.
 //
 // Numerics: everything is float32. T is built by substitution, 16 x 16 on the diagonal and block by block below it (a product
@@ -113,7 +113,11 @@ __device__ __forceinline__ void lds_barrier() {
 
 constexpr int kGatedForm = 0, kPlainForm = 1, kGeneralForm = 2;   // plain: the gated form with nothing taken out
 
-// grid (runs, heads), four waves: wave w makes the rows of tokens 16 w .. 16 w + 15.
+// grid (runs, heads), four waves: wave w makes the rows of tokens 16 w .. 16 w + 15 of what is between tokens, then the columns
+// 16 w, 64 + 16 w, .. of Wx, Kt, Kd and Z. With one to three waves a SIMD, what bounds it is each wave's chain of loads and
+// products: 16 heads of 128, 2,048 tokens, 65 -> 41 us with the columns divided (wave 3 was at it 74 us while wave 0 took 42) and
+// the operands asked for ahead; the general form's 32 heads of 64 126 -> 107. There the divisions by D_s, the rows that
+// wave 3 has four times as many of as wave 0 and two workgroups of 70 KB of LDS a compute unit are left. Same sums, same bits.
 template <int DT, int FORM>
 __global__ __launch_bounds__(256) void runs_prepare_kernel(DeltaRuns c, RunList list) {
   constexpr int D = DT * 16, LD = D + 4;
@@ -127,13 +131,27 @@ __global__ __launch_bounds__(256) void runs_prepare_kernel(DeltaRuns c, RunList 
   const int64_t t0 = list.t0[blockIdx.x];
   const int n = list.tokens[blockIdx.x];
   const int h = blockIdx.y, grp = h / c.heads_per_group;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
   const RunLayout lay = run_layout(D, c.vdim, GENERAL);
   float* sc = c.scratch + (static_cast<int64_t>(blockIdx.x) * c.heads + h) * lay.total;
   const int64_t key0 = t0 * c.key_row + static_cast<int64_t>(grp) * D;
   const int64_t x0 = t0 * c.x_row + static_cast<int64_t>(h) * c.vdim;
 
+  // The run's products over the key channels, a lane's rows and columns read 16 bytes at a time. What is read is asked for ahead
+  // of where it is used and without a branch, behind the run the last token again; zeros are used for it.
+  const int t = 16 * wave + r;
+  const bool has = t < n;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  auto row4 = [&](const float* v, int tok, int d) {      // dimensions 16 d + 4 g .. of a token's vector
+    return *reinterpret_cast<const f32x4*>(v + key0 + min(tok, n - 1) * c.key_row + 16 * d + 4 * g);
+  };
+  f32x4 ct[DT], qt[DT];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) {
+    ct[d] = row4(GENERAL ? c.cvec : c.kvec, t, d);
+    qt[d] = row4(c.rvec, t, d);
+  }
   if (threadIdx.x < kRunTokens) {
     const int t = threadIdx.x;
     const int64_t at = (t0 + t) * c.scal_row + h;
@@ -144,7 +162,8 @@ __global__ __launch_bounds__(256) void runs_prepare_kernel(DeltaRuns c, RunList 
   if constexpr (GENERAL) {
     for (int idx = threadIdx.x; idx < kRunTokens * D; idx += 256) {
       const int t = idx / D, i = idx % D;
-      ds[t * LD + i] = t < n ? c.dvec[(t0 + t) * c.dvec_row + static_cast<int64_t>(h) * D + i] : 1.f;
+      const float w = c.dvec[(t0 + min(t, n - 1)) * c.dvec_row + static_cast<int64_t>(h) * D + i];
+      ds[t * LD + i] = t < n ? w : 1.f;
     }
     __syncthreads();
     if (threadIdx.x < D) {
@@ -161,9 +180,10 @@ __global__ __launch_bounds__(256) void runs_prepare_kernel(DeltaRuns c, RunList 
     if (threadIdx.x < kRunTokens) {
       const int s = threadIdx.x;
       float ratio = 1.f;
-      for (int t = s; t < kRunTokens; ++t) {
-        if (t > s) ratio *= num[0][t];
-        tm[t * kLd + s] = ratio;
+#pragma unroll 16
+      for (int t = 0; t < kRunTokens; ++t) {             // all lanes at one t: the decays are read ahead
+        ratio *= t > s ? num[0][t] : 1.f;
+        if (t >= s) tm[t * kLd + s] = ratio;
       }
       num[2][s] = ratio;
     }
@@ -172,17 +192,19 @@ __global__ __launch_bounds__(256) void runs_prepare_kernel(DeltaRuns c, RunList 
     __syncthreads();
   }
 
-  // The run's products over the key channels, a lane's rows and columns read 16 bytes at a time.
-  const int t = 16 * wave + r;
-  const bool has = t < n;
-  auto row4 = [&](const float* v, int tok, int d) {      // dimensions 16 d + 4 g .. of a token's vector, zeros behind the run
-    return tok < n ? *reinterpret_cast<const f32x4*>(v + key0 + tok * c.key_row + 16 * d + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 first[DT], second[DT];                           // a block of tokens s, asked for a block ahead
+  auto ask_rows = [&](int st) {
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      first[d] = row4(GENERAL ? c.pvec : c.kvec, 16 * st + r, d);
+      if constexpr (GENERAL) second[d] = row4(c.kvec, 16 * st + r, d);
+    }
   };
-  f32x4 ct[DT], qt[DT];
+  ask_rows(0);
 #pragma unroll
   for (int d = 0; d < DT; ++d) {
-    ct[d] = row4(GENERAL ? c.cvec : c.kvec, t, d);
-    qt[d] = row4(c.rvec, t, d);
+    ct[d] = has ? ct[d] : zero;
+    qt[d] = has ? qt[d] : zero;
     if constexpr (GENERAL) {
       if (t > 0) ct[d] *= *reinterpret_cast<const f32x4*>(ds + (t - 1) * LD + 16 * d + 4 * g);
       qt[d] *= *reinterpret_cast<const f32x4*>(ds + t * LD + 16 * d + 4 * g);
@@ -196,22 +218,27 @@ __global__ __launch_bounds__(256) void runs_prepare_kernel(DeltaRuns c, RunList 
     if (st > wave) continue;
     const int sr = 16 * st + r;                          // the row this lane supplies
     f32x4 cc = {0.f, 0.f, 0.f, 0.f}, qc = cc, ck = cc, qk = cc;
+    f32x4 one[DT], two[DT];
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
-      f32x4 first = row4(GENERAL ? c.pvec : c.kvec, sr, d);
+      one[d] = sr < n ? first[d] : zero;
+      if constexpr (GENERAL) two[d] = sr < n ? second[d] : zero;
+    }
+    if (st < wave) ask_rows(st + 1);
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
       if constexpr (GENERAL) {
         const f32x4 dd = *reinterpret_cast<const f32x4*>(ds + sr * LD + 16 * d + 4 * g);
-        f32x4 second = row4(c.kvec, sr, d);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          first[i] /= dd[i];
-          second[i] /= dd[i];
+          one[d][i] /= dd[i];
+          two[d][i] /= dd[i];
         }
-        ck = mma(second, ct[d], ck);
-        qk = mma(second, qt[d], qk);
+        ck = mma(two[d], ct[d], ck);
+        qk = mma(two[d], qt[d], qk);
       }
-      if constexpr (SOLVES) cc = mma(first, ct[d], cc);
-      qc = mma(first, qt[d], qc);
+      if constexpr (SOLVES) cc = mma(one[d], ct[d], cc);
+      qc = mma(one[d], qt[d], qc);
     }
     f32x4 l, p;
 #pragma unroll
@@ -228,31 +255,41 @@ __global__ __launch_bounds__(256) void runs_prepare_kernel(DeltaRuns c, RunList 
     if constexpr (SOLVES) *reinterpret_cast<f32x4*>(lm + t * kLd + 16 * st + 4 * g) = l;
     *reinterpret_cast<f32x4*>(sc + lay.p + t * kRunTokens + 16 * st + 4 * g) = p;
   }
-  // A lane's four tokens s of column j of the values (k = 4 g + i of the operand of either kind).
-  auto x4 = [&](int st, int j) {
+  // A lane's four tokens s of column j of the values (k = 4 g + i of the operand of either kind), a column at a time.
+  f32x4 xs[kRunTiles];
+  auto ask_x = [&](int j, int blocks) {
+#pragma unroll
+    for (int st = 0; st < kRunTiles; ++st) {
+      if (st >= blocks) continue;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) xs[st][i] = c.x[x0 + min(16 * st + 4 * g + i, n - 1) * c.x_row + j];
+    }
+  };
+  auto x4 = [&](int st) {
     f32x4 v;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int s = 16 * st + 4 * g + i;
-      v[i] = s < n ? c.x[x0 + s * c.x_row + j] : 0.f;
-    }
+    for (int i = 0; i < 4; ++i) v[i] = 16 * st + 4 * g + i < n ? xs[st][i] : 0.f;
     return v;
   };
   if constexpr (GENERAL) {
+    ask_x(r, wave + 1);
     for (int j0 = 0; j0 < c.vdim; j0 += 16) {
-      f32x4 y = {0.f, 0.f, 0.f, 0.f}, m = y;
+      f32x4 y = zero, m = zero, x[kRunTiles];
+#pragma unroll
+      for (int st = 0; st < kRunTiles; ++st) x[st] = x4(st);
+      ask_x(min(j0 + 16, c.vdim - 16) + r, wave + 1);
 #pragma unroll
       for (int st = 0; st < kRunTiles; ++st) {
         if (st > wave) continue;
-        const f32x4 xv = x4(st, j0 + r);
-        y = mma(xv, pk_reg[st], y);
-        m = mma(xv, m_reg[st], m);
+        y = mma(x[st], pk_reg[st], y);
+        m = mma(x[st], m_reg[st], m);
       }
       if (has) *reinterpret_cast<f32x4*>(c.out + (t0 + t) * c.out_row + static_cast<int64_t>(h) * c.vdim + j0 + 4 * g) = y;
 #pragma unroll
       for (int v = 0; v < 4; ++v) mx[(j0 + 4 * g + v) * kLd + t] = m[v];
     }
   }
+  if constexpr (!GENERAL) ask_x(min(16 * wave, c.vdim - 16) + r, kRunTiles);
   __syncthreads();                                       // L is whole, the ratios have been read
   if constexpr (SOLVES) {
     // T = (1 - L)^-1: the blocks on the diagonal by substitution, a column per lane, ...
@@ -289,64 +326,90 @@ __global__ __launch_bounds__(256) void runs_prepare_kernel(DeltaRuns c, RunList 
       __syncthreads();
     }
   }
-  f32x4 tr[kRunTiles];                                   // row t of T
+  // Behind here a wave has columns of its own for all four blocks of tokens: with blocks of tokens of its own wave 3 made four
+  // times the products of wave 0, and each wave fetched the operands again.
+  f32x4 tr[kRunTiles][kRunTiles];                        // rows 16 tt + r of T
+  if constexpr (SOLVES) {
 #pragma unroll
-  for (int st = 0; st < kRunTiles; ++st)
-    tr[st] = SOLVES && st <= wave ? *reinterpret_cast<const f32x4*>(tm + t * kLd + 16 * st + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int j0 = 0; j0 < c.vdim; j0 += 16) {              // Wx, rows t, column j
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int tt = 0; tt < kRunTiles; ++tt)
 #pragma unroll
-    for (int st = 0; st < kRunTiles; ++st) {
-      if (SOLVES ? st > wave : st != wave) continue;
-      f32x4 b;
-      if constexpr (GENERAL) {
-        b = *reinterpret_cast<const f32x4*>(mx + (j0 + r) * kLd + 16 * st + 4 * g);
-      } else {
-        b = x4(st, j0 + r);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) b[i] *= num[4][16 * st + 4 * g + i];
-      }
-      acc = SOLVES ? mma(tr[st], b, acc) : b;
-    }
-    *reinterpret_cast<f32x4*>(sc + lay.w + (j0 + r) * kRunTokens + 16 * wave + 4 * g) = acc;
+      for (int st = 0; st <= tt; ++st) tr[tt][st] = *reinterpret_cast<const f32x4*>(tm + (16 * tt + r) * kLd + 16 * st + 4 * g);
   }
-  for (int i0 = 0; i0 < D; i0 += 16) {                   // Kt, rows i, column t; Kd of this wave's tokens
-    const int i = i0 + r;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int j0 = 16 * wave; j0 < c.vdim; j0 += 64) {      // Wx, rows t, column j
+    f32x4 b[kRunTiles];
 #pragma unroll
     for (int st = 0; st < kRunTiles; ++st) {
-      if (st > wave) continue;
-      f32x4 a, kd;
+      if constexpr (GENERAL) {
+        b[st] = *reinterpret_cast<const f32x4*>(mx + (j0 + r) * kLd + 16 * st + 4 * g);
+      } else {
+        b[st] = x4(st);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) b[st][i] *= num[4][16 * st + 4 * g + i];
+      }
+    }
+    if constexpr (!GENERAL) ask_x(min(j0 + 64, c.vdim - 16) + r, kRunTiles);
+#pragma unroll
+    for (int tt = 0; tt < kRunTiles; ++tt) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (SOLVES) {
+#pragma unroll
+        for (int st = 0; st <= tt; ++st) acc = mma(tr[tt][st], b[st], acc);
+      } else {
+        acc = b[tt];
+      }
+      *reinterpret_cast<f32x4*>(sc + lay.w + (j0 + r) * kRunTokens + 16 * tt + 4 * g) = acc;
+    }
+  }
+  for (int i0 = 16 * wave; i0 < D; i0 += 64) {           // Kt, rows i, column t; Kd
+    const int i = i0 + r;
+    f32x4 a[kRunTiles];
+#pragma unroll
+    for (int st = 0; st < kRunTiles; ++st) {
+      f32x4 kd;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int s = 16 * st + 4 * g + v;
-        const float k = s < n ? (GENERAL ? c.cvec : c.kvec)[key0 + s * c.key_row + i] : 0.f;
-        a[v] = GENERAL ? (s > 0 ? k * ds[(s - 1) * LD + i] : k) : num[3][s] * num[1][s] * k;
-        if (st == wave) {
-          if constexpr (GENERAL) kd[v] = s < n ? c.pvec[key0 + s * c.key_row + i] * (ds[(kRunTokens - 1) * LD + i] / ds[s * LD + i]) : 0.f;
-          else kd[v] = num[2][s] * k;
+        const float key = (GENERAL ? c.cvec : c.kvec)[key0 + min(s, n - 1) * c.key_row + i], k = s < n ? key : 0.f;
+        a[st][v] = GENERAL ? (s > 0 ? k * ds[(s - 1) * LD + i] : k) : num[3][s] * num[1][s] * k;
+        if constexpr (GENERAL) {
+          const float taken = c.pvec[key0 + min(s, n - 1) * c.key_row + i];
+          kd[v] = s < n ? taken * (ds[(kRunTokens - 1) * LD + i] / ds[s * LD + i]) : 0.f;
+        } else {
+          kd[v] = num[2][s] * k;
         }
       }
-      if constexpr (SOLVES) acc = mma(a, tr[st], acc);
-      if (st == wave) *reinterpret_cast<f32x4*>(sc + lay.kd + i * kRunTokens + 16 * st + 4 * g) = kd;
+      *reinterpret_cast<f32x4*>(sc + lay.kd + i * kRunTokens + 16 * st + 4 * g) = kd;
     }
-    if constexpr (SOLVES) *reinterpret_cast<f32x4*>(sc + lay.kt + t * D + i0 + 4 * g) = acc;
+    if constexpr (SOLVES) {
+#pragma unroll
+      for (int tt = 0; tt < kRunTiles; ++tt) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int st = 0; st <= tt; ++st) acc = mma(a[st], tr[tt][st], acc);
+        *reinterpret_cast<f32x4*>(sc + lay.kt + (16 * tt + r) * D + i0 + 4 * g) = acc;
+      }
+    }
   }
   if constexpr (GENERAL) {
     for (int it = wave; it < DT; it += 4) {              // Z, rows i, column j
       f32x4 kk[kRunTiles];
+      ask_x(r, kRunTiles);
       const int i = 16 * it + r;
 #pragma unroll
       for (int st = 0; st < kRunTiles; ++st)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int s = 16 * st + 4 * g + v;
-          kk[st][v] = s < n ? c.kvec[key0 + s * c.key_row + i] * (ds[(kRunTokens - 1) * LD + i] / ds[s * LD + i]) : 0.f;
+          const float key = c.kvec[key0 + min(s, n - 1) * c.key_row + i];
+          kk[st][v] = s < n ? key * (ds[(kRunTokens - 1) * LD + i] / ds[s * LD + i]) : 0.f;
         }
       for (int j0 = 0; j0 < c.vdim; j0 += 16) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f}, x[kRunTiles];
 #pragma unroll
-        for (int st = 0; st < kRunTiles; ++st) acc = mma(kk[st], x4(st, j0 + r), acc);
+        for (int st = 0; st < kRunTiles; ++st) x[st] = x4(st);
+        ask_x(min(j0 + 16, c.vdim - 16) + r, kRunTiles);
+#pragma unroll
+        for (int st = 0; st < kRunTiles; ++st) acc = mma(kk[st], x[st], acc);
         *reinterpret_cast<f32x4*>(sc + lay.z + (j0 + r) * D + 16 * it + 4 * g) = acc;
       }
     }

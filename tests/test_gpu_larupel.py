@@ -609,6 +609,13 @@ def test_recurrences_in_runs_of_64_tokens(ops, monkeypatch, form, heads, groups,
     assert all(b < 1.5 * a for a, b in zip(off[False], off[True])), off
 
 
+@pytest.mark.parametrize("form,heads,groups,dim,vdim", [("gated", 2, 2, 64, 80), ("gated", 3, 1, 128, 256), ("plain", 2, 1, 128, 176),
+                                                        ("general", 2, 2, 64, 112), ("general", 1, 1, 128, 256)])
+def test_runs_of_more_value_channels_than_the_waves_take_at_once(ops, monkeypatch, form, heads, groups, dim, vdim):
+    """Four waves take sixteen value channels each: the last ones are fewer than four waves', or a whole second or fourth time."""
+    test_recurrences_in_runs_of_64_tokens(ops, monkeypatch, form, heads, groups, dim, vdim)
+
+
 def recurrence(ops, form, lengths, heads, groups, dim, vdim, slots):
     """A step of items of these lengths, and ``delta_scan``'s operands of one of the three forms for it: the values, the state
     in front of the step, and a function of the values that gives the outputs and the state behind it."""
