@@ -339,7 +339,7 @@ __device__ __forceinline__ float stage_scale(const Tokens& tk, const float* ss, 
 // k-steps of all RT tiles in flight together; the partial sums meet in LDS and wave rt finishes
 // tile rt. gridDim.y slices of K give partial sums out[blockIdx.y][M][n_out], as above. SWIGLU:
 // w is [gate; up] and a group is RT pairs of tiles. K must be a multiple of 32.
-// NORMED: the tokens are rows of the float32 residual stream, normalized while they are staged
+// NORMED: the tokens are rows of the float32 residual stream, normalized while they are staged, where linear_normed.hip does not take them
 // (gridDim.y must be 1: a row's statistics need the whole row). ATOMIC: the K-slices add into one
 // out[M][n_out] (see skinny_mfma_kernel).
 template <int RT, int ROWS, bool SWIGLU, typename TO, bool NORMED = false, bool ATOMIC = false>
@@ -1012,6 +1012,7 @@ int psamd_linear_normed(void* stream, const float* resid, const int32_t* rows, c
   const Tokens tk{nullptr, resid, norm_w, rows, eps, norm_w_dtype == kBF16 ? 1 : 0};
   const int form = epilogue == 1 ? kGated : (out_dtype == kF32 ? kSlices : kPlain);
   if (linear_normed_takes(w, out, form, M, n_out, K)) return launch_linear_normed(s, tk, w, out, form, M, n_out, K, g_gate_act);
+  // What is left has a K that is no multiple of 64, a w off 16 bytes, rows that do not fit in LDS beside w's, float32 outputs or few columns.
   const int64_t groups = ceil_div(n_out, 16);
   const bool eight = M <= 8;
   if (epilogue == 1) {

@@ -1352,7 +1352,7 @@ int psamd_moe_experts_rows(void* stream, const void* x, const int32_t* chosen, c
 // Pairs per tile of the grouped form for a step of this many pairs over this many experts: 128 when
 // the experts have at least twice that many pairs each on average (an expert's last tile is half
 // empty on average: 512 tokens of 8 choices over 32 experts took 204 us in tiles of 128, one full
-// and one nearly empty per expert), 64 from 48 pairs per expert on, 16 below.
+// and one nearly empty per expert), 64 from 48 pairs per expert on, 16 below. Where K and F are multiples of 64, wide_tile_rows is asked first.
 int psamd_moe_grouped_tile_rows(int64_t pairs, int experts) {
   return pairs >= 256LL * experts ? 128 : (pairs >= 48LL * experts ? 64 : 16);
 }
