@@ -842,7 +842,8 @@ __global__ __launch_bounds__(64 * (TN / 16) * KG) void moe_stream_kernel(
     x_off[i] = static_cast<uint32_t>(FORM != kFormDown ? pair / top : pair) * (2u * K) + 16u * piece;
   }
   const int units = K / 64, steps = (units + KG - 1) / KG, end = units * 128;
-  int from = static_cast<int>((blockIdx.x + 5u * blockIdx.y) % static_cast<unsigned>(units)) * 128, to = 0;
+  // By columns and expert, never by the tile: the sorting puts an expert's pairs into its tiles in any order, and a pair's sums keep theirs.
+  int from = static_cast<int>((blockIdx.x + 5u * static_cast<unsigned>(e)) % static_cast<unsigned>(units)) * 128, to = 0;
   auto unit_at = [&](int unit) {
     const int k = from + unit * 128;
     return min(k >= end ? k - end : k, end - 128);
