@@ -164,7 +164,7 @@ class HipOps:
     LIBRARY_ADD_MIN_ROWS = 1024     # from here on a product that feeds the residual stream adds into it in the library
     MOE_ROUTE_FUSED_MAX_TOKENS = 0   # up to here one kernel computes router logits and choice; above, product + choice
     MOE_CHOICE_SORTS_MAX_TOKENS = 16 # up to here the workgroup that chooses a step's experts also sorts the pairs
-    MOE_PAIRWISE_MAX_TOKENS = 2     # up to here the experts of a bfloat16 step whose width is no multiple of 64 run pair by pair; else grouped by expert
+    MOE_PAIRWISE_MAX_TOKENS = 2     # up to here a bfloat16 step's experts may run pair by pair (_groups_pairs)
     DELTA_RUNS = True               # delta_scan takes ``in_runs``
     DELTA_RUNS_MIN_TOKENS = 340     # what a round of launches of the recurrences' runs costs, in tokens walked (see _runs_pay)
     DELTA_RUNS_SHORT = 64           # items of up to this many tokens beside it are walked: each would cost a whole run
@@ -880,7 +880,8 @@ class HipOps:
     # ------------------------------------------------------------------ experts
 
     def moe_route(self, x, w_router, chosen, weight, w_router_act=None, bias=None, mode: int = 0, groups: int = 0,
-                  keep: int = 0, factor: float = 1.0, group_max: bool = False, correction=None, identity: int = 0) -> None:
+                  keep: int = 0, factor: float = 1.0, group_max: bool = False, correction=None, identity: int = 0,
+                  expert_width: int = 0) -> None:
         """chosen[t, :], weight[t, :] = the experts with the largest sigmoid(x[t] . w_router[e]) and
         those scores, largest first, the lower index among equals; scores in 32-bit. With the router
         also given in the activation dtype (``w_router_act``), a step of more than
@@ -893,7 +894,8 @@ class HipOps:
         runs of neighbours, a run's score is the sum of its two largest scores, and only experts of the ``keep`` best
         runs can be chosen. The weights are multiplied by ``factor``. ``mode`` 2: the scores are the softmax over all logits,
         the choice goes by score + ``correction`` (float32 [E]), the weights are the scores. ``group_max``: a run's score is
-        its largest alone. The last ``identity`` rows of the router are identity experts (``moe_experts``)."""
+        its largest alone. The last ``identity`` rows of the router are identity experts (``moe_experts``). ``expert_width``: F of the
+        experts that follow, where it is no multiple of 64 (a step's pairs are sorted here only if the experts take them sorted)."""
         e, top = w_router.shape[0], chosen.shape[1]
         if correction is not None:
             self._need(correction.dtype == torch.float32 and correction.numel() == e and correction.is_contiguous(),
@@ -913,7 +915,7 @@ class HipOps:
             logits = self.ws.get("moe.logits", (t, e), torch.float32)
             self.linear(x, w_router_act, logits)
             self._grouped_for = None
-            if self._groups_pairs(x.dtype, t, k) and t <= self.MOE_CHOICE_SORTS_MAX_TOKENS and e <= 1024:
+            if self._groups_pairs(x.dtype, t, k, expert_width) and t <= self.MOE_CHOICE_SORTS_MAX_TOKENS and e <= 1024:
                 # A small step: the workgroup that chooses also sorts the pairs for the experts' kernels.
                 ints = self._group_ints(t, top, buckets)
                 self._ok(self.lib.psamd_moe_topk_group(self._stream(), logits.data_ptr(), chosen.data_ptr(), weight.data_ptr(),
@@ -931,9 +933,13 @@ class HipOps:
         self._ok(self.lib.psamd_moe_route(self._stream(), x.data_ptr(), _code(x.dtype), w_router.data_ptr(),
                                           chosen.data_ptr(), weight.data_ptr(), t, k, e, top, *rule))
 
-    def _groups_pairs(self, dtype: torch.dtype, t: int, k: int) -> bool:
-        """Whether a step of ``t`` tokens of width ``k`` runs its experts grouped by expert."""
-        return dtype == torch.bfloat16 and t > 0 and k % 8 == 0 and (t > self.MOE_PAIRWISE_MAX_TOKENS or k % 64 == 0)
+    def _groups_pairs(self, dtype: torch.dtype, t: int, k: int, f: int) -> bool:
+        """Whether a step of ``t`` tokens of width ``k`` runs its experts of width ``f`` grouped by expert. One and two tokens do where
+        the kernel that copies whole lines takes both widths, multiples of 64; the other grouped kernel is the slower one for them. us of
+        routing and experts at 1 / 2 tokens, grouped and pair by pair: 32 of 2,048 x 1,000, 8 choices 56.6 / 65.9 and 47.4 / 55.0, x 1,024
+        39.0 / 48.6 and 46.5 / 56.3; 8 of 4,096 x 3,592, 2 choices - / 109 and - / 93.6."""
+        return (dtype == torch.bfloat16 and t > 0 and k % 8 == 0 and f % 8 == 0
+                and (t > self.MOE_PAIRWISE_MAX_TOKENS or (k % 64 == 0 and f % 64 == 0)))
 
     def _group_ints(self, t: int, top: int, e: int) -> torch.Tensor:
         tiles = int(self.lib.psamd_moe_grouped_max_tiles(t * top, e))
@@ -972,12 +978,12 @@ class HipOps:
             self._need(col_scale is None and out.shape == (top, t, k) and out.dtype == torch.float32 and out.is_contiguous(),
                        "moe_experts: output slices")
         tail = (int(weight_on_output), EXPERT_KINDS[kind], int(into), _ptr(col_scale))
-        if self._groups_pairs(x.dtype, t, k) and f % 8 == 0:
+        buckets = e + (1 if identity else 0)
+        done = int(getattr(self, "_grouped_for", None) == (chosen.data_ptr(), t, top, buckets))   # the router's kernel sorted them
+        self._grouped_for = None
+        if self._groups_pairs(x.dtype, t, k, f):
             # Sorted by expert and run in tiles on the matrix cores: an expert is read once per tile of pairs.
-            buckets = e + (1 if identity else 0)
             ints = self._group_ints(t, top, buckets)
-            done = int(getattr(self, "_grouped_for", None) == (chosen.data_ptr(), t, top, buckets))   # the router's kernel sorted them
-            self._grouped_for = None
             self._ok(self.lib.psamd_moe_experts_grouped(self._stream(), x.data_ptr(), chosen.data_ptr(), weight.data_ptr(),
                                                         w_in.data_ptr(), w_down.data_ptr(), act.data_ptr(),
                                                         out.data_ptr(), ints.data_ptr(), t, k, f, e, int(identity), top, float(gate_alpha),

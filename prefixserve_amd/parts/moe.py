@@ -100,6 +100,8 @@ class RoutedExperts(FeedForward):
                 self.route_options["group_max"] = True
         if weight_scale != 1.0:
             self.route_options["factor"] = float(weight_scale)
+        if self.intermediate_size % 64:
+            self.route_options["expert_width"] = self.intermediate_size
         self.expert_options: dict[str, object] = {}
         if self.identity:
             self.route_options["identity"] = self.expert_options["identity"] = self.identity

@@ -245,7 +245,7 @@ class EmulatedOps:
             kv[:, 1].view(kv.shape[0], hkv, d, PAGE)[page, :, :, off] = vals
 
     def moe_route(self, x, w_router, chosen, weight, w_router_act=None, bias=None, mode=0, groups=0, keep=0, factor=1.0,
-                  group_max=False, correction=None, identity=0) -> None:
+                  group_max=False, correction=None, identity=0, expert_width=0) -> None:
         z = x.float() @ w_router.float().T
         if bias is not None:
             z = z + bias

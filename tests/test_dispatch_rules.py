@@ -1,0 +1,63 @@
+"""Which entry points of the kernel library a call goes to: host rules, run without a GPU on a library that only notes what is called."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from prefixserve_amd.kernels.ops import HipOps
+
+
+class NotingLibrary:
+    """Every entry point returns 0 and is noted with its arguments."""
+
+    def __init__(self) -> None:
+        self.calls: list[tuple[str, tuple]] = []
+
+    def __getattr__(self, name: str):
+        def entry(*args):
+            self.calls.append((name, args))
+            return 0
+
+        return entry
+
+
+class Buffers:
+    def get(self, name, shape, dtype):
+        return torch.empty(shape, dtype=dtype)
+
+
+@pytest.fixture
+def ops():
+    made = object.__new__(HipOps)
+    made.device, made.lib, made.ws, made._step_stream = torch.device("cpu"), NotingLibrary(), Buffers(), 0
+    made.linear = lambda x, w, out: None                 # the router's logits
+    return made
+
+
+def experts_called(ops, t: int, k: int, f: int, experts: int = 8, top: int = 2) -> list[str]:
+    """The entry points of one routed layer, a grouped call marked with whether the router sorted its pairs."""
+    x = torch.empty(t, k, dtype=torch.bfloat16)
+    router = torch.empty(experts, k)
+    chosen, weight = torch.empty(t, top, dtype=torch.int32), torch.empty(t, top)
+    ops.moe_route(x, router, chosen, weight, router.to(torch.bfloat16), **({"expert_width": f} if f % 64 else {}))
+    w_in, w_down = torch.empty(experts, 2 * f, k, dtype=torch.bfloat16), torch.empty(experts, k, f, dtype=torch.bfloat16)
+    ops.moe_experts(x, chosen, weight, w_in, w_down, torch.empty(t * top, f, dtype=torch.bfloat16), torch.empty(top, t, k), 1.0, 7.0, 0.0)
+    done = {"psamd_moe_experts_grouped": lambda a: f" sorted {a[18]}"}
+    return [name + done.get(name, lambda a: "")(args) for name, args in ops.lib.calls if name != "psamd_moe_grouped_max_tiles"]
+
+
+PAIR_BY_PAIR = ["psamd_moe_topk", "psamd_moe_experts_rows"]
+SORTED_BY_THE_ROUTER = ["psamd_moe_topk_group", "psamd_moe_experts_grouped sorted 1"]
+
+
+@pytest.mark.parametrize("t,k,f,want", [
+    (1, 128, 64, SORTED_BY_THE_ROUTER), (2, 64, 192, SORTED_BY_THE_ROUTER),
+    (1, 128, 72, PAIR_BY_PAIR), (2, 64, 1000, PAIR_BY_PAIR), (2, 64, 33, PAIR_BY_PAIR), (2, 72, 64, PAIR_BY_PAIR),
+    (3, 64, 72, SORTED_BY_THE_ROUTER), (16, 72, 64, SORTED_BY_THE_ROUTER), (3, 64, 33, PAIR_BY_PAIR), (3, 36, 64, PAIR_BY_PAIR),
+    (17, 64, 72, ["psamd_moe_topk", "psamd_moe_experts_grouped sorted 0"]),
+])
+def test_one_and_two_tokens_are_grouped_where_both_widths_are_whole(ops, t, k, f, want):
+    """One and two tokens of experts whose width is no multiple of 64 ran in the slower grouped kernel; and the router sorts a step's
+    pairs exactly if the experts take them sorted."""
+    assert experts_called(ops, t, k, f) == want
