@@ -164,6 +164,7 @@ class HipOps:
     LIBRARY_ADD_MIN_ROWS = 1024     # from here on a product that feeds the residual stream adds into it in the library
     MOE_ROUTE_FUSED_MAX_TOKENS = 0   # up to here one kernel computes router logits and choice; above, product + choice
     MOE_CHOICE_SORTS_MAX_TOKENS = 16 # up to here the workgroup that chooses a step's experts also sorts the pairs
+    MOE_CHOICE_SORTS_MAX_EXPERTS = 1024   # ... among as many as its counters in LDS hold
     MOE_PAIRWISE_MAX_TOKENS = 2     # up to here a bfloat16 step's experts may run pair by pair (_groups_pairs)
     DELTA_RUNS = True               # delta_scan takes ``in_runs``
     DELTA_RUNS_MIN_TOKENS = 340     # what a round of launches of the recurrences' runs costs, in tokens walked (see _runs_pay)
@@ -915,7 +916,7 @@ class HipOps:
             logits = self.ws.get("moe.logits", (t, e), torch.float32)
             self.linear(x, w_router_act, logits)
             self._grouped_for = None
-            if self._groups_pairs(x.dtype, t, k, expert_width) and t <= self.MOE_CHOICE_SORTS_MAX_TOKENS and e <= 1024:
+            if self._groups_pairs(x.dtype, t, k, expert_width, e - identity) and t <= self.MOE_CHOICE_SORTS_MAX_TOKENS and e <= self.MOE_CHOICE_SORTS_MAX_EXPERTS:
                 # A small step: the workgroup that chooses also sorts the pairs for the experts' kernels.
                 ints = self._group_ints(t, top, buckets)
                 self._ok(self.lib.psamd_moe_topk_group(self._stream(), logits.data_ptr(), chosen.data_ptr(), weight.data_ptr(),
@@ -933,13 +934,14 @@ class HipOps:
         self._ok(self.lib.psamd_moe_route(self._stream(), x.data_ptr(), _code(x.dtype), w_router.data_ptr(),
                                           chosen.data_ptr(), weight.data_ptr(), t, k, e, top, *rule))
 
-    def _groups_pairs(self, dtype: torch.dtype, t: int, k: int, f: int) -> bool:
-        """Whether a step of ``t`` tokens of width ``k`` runs its experts of width ``f`` grouped by expert. One and two tokens do where
-        the kernel that copies whole lines takes both widths, multiples of 64; the other grouped kernel is the slower one for them. us of
+    def _groups_pairs(self, dtype: torch.dtype, t: int, k: int, f: int, experts: int) -> bool:
+        """Whether a step of ``t`` tokens of width ``k`` runs its ``experts`` of width ``f`` grouped by expert. One and two tokens do where
+        the kernel that copies whole lines takes both widths, multiples of 64 (the other grouped kernel is the slower one for them), and
+        the router's kernel may have sorted the pairs (the sorting on its own takes 4,096 experts and no more; pair by pair any number). us of
         routing and experts at 1 / 2 tokens, grouped and pair by pair: 32 of 2,048 x 1,000, 8 choices 56.6 / 65.9 and 47.4 / 55.0, x 1,024
         39.0 / 48.6 and 46.5 / 56.3; 8 of 4,096 x 3,592, 2 choices - / 109 and - / 93.6."""
         return (dtype == torch.bfloat16 and t > 0 and k % 8 == 0 and f % 8 == 0
-                and (t > self.MOE_PAIRWISE_MAX_TOKENS or (k % 64 == 0 and f % 64 == 0)))
+                and (t > self.MOE_PAIRWISE_MAX_TOKENS or (k % 64 == 0 and f % 64 == 0 and experts <= self.MOE_CHOICE_SORTS_MAX_EXPERTS)))
 
     def _group_ints(self, t: int, top: int, e: int) -> torch.Tensor:
         tiles = int(self.lib.psamd_moe_grouped_max_tiles(t * top, e))
@@ -981,7 +983,7 @@ class HipOps:
         buckets = e + (1 if identity else 0)
         done = int(getattr(self, "_grouped_for", None) == (chosen.data_ptr(), t, top, buckets))   # the router's kernel sorted them
         self._grouped_for = None
-        if self._groups_pairs(x.dtype, t, k, f):
+        if self._groups_pairs(x.dtype, t, k, f, e):
             # Sorted by expert and run in tiles on the matrix cores: an expert is read once per tile of pairs.
             ints = self._group_ints(t, top, buckets)
             self._ok(self.lib.psamd_moe_experts_grouped(self._stream(), x.data_ptr(), chosen.data_ptr(), weight.data_ptr(),

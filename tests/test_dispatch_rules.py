@@ -61,3 +61,12 @@ def test_one_and_two_tokens_are_grouped_where_both_widths_are_whole(ops, t, k, f
     """One and two tokens of experts whose width is no multiple of 64 ran in the slower grouped kernel; and the router sorts a step's
     pairs exactly if the experts take them sorted."""
     assert experts_called(ops, t, k, f) == want
+
+
+@pytest.mark.parametrize("t,experts,want", [
+    (2, 1024, SORTED_BY_THE_ROUTER), (1, 1025, PAIR_BY_PAIR), (2, 4097, PAIR_BY_PAIR),
+    (3, 1025, ["psamd_moe_topk", "psamd_moe_experts_grouped sorted 0"]),
+])
+def test_one_and_two_tokens_among_any_number_of_experts(ops, t, experts, want):
+    """The sorting refuses more than 4,096 experts, which one and two tokens did not need it for."""
+    assert experts_called(ops, t, 64, 64, experts) == want
