@@ -1756,7 +1756,11 @@ static int launch_prefill(hipStream_t s, const void* qkv, int q_stride, void* ou
 // At 20 and 21 requests three runs stay the faster for uneven contexts (21.7 / 24.0); above 256 pairs some units have two such workgroups
 // (33 requests behind 2,049 keys: 35.0 / 39.0). The same keys cut evenly over the chip whatever the requests' lengths gained nothing (64 uneven
 // requests: 46.2 / 46.6): a launch pays 7 us for its trips to memory one after the other, and then streams at 5.2 TB/s either way.
+// The kernel of eight waves is that of up to 16 query heads a kv head: with more, one run of four waves instead of two of them leaves half of
+// the waves out (256 heads of 64 on 8, 22 requests behind 2,049 keys / uneven up to 2,900: 32.5, 33.8 in two runs, 39.4, 44.3 in one; 64 on 1, 255
+// uneven: 53.5, 68.5).
 constexpr int kOneRun = 176;
+constexpr int kOneTileHeads = 16;       // query heads a kv head that are one tile of the matrix instructions
 
 template <int NS, int CT, bool P3>
 static int launch_decode(hipStream_t s, const void* qkv, int q_stride, const void* kv, void* out, float* part_o,
@@ -1960,13 +1964,14 @@ int psamd_attention_decode_skewed(int n_dec, int longest, int64_t total) {
 
 // How psamd_attention_decode should cut the keys of a step of n_dec single-token items whose
 // longest context is kv_len (for a captured step: the longest there can be): *nsplit runs per
-// request, none shorter than *min_run keys. Two workgroups per compute unit; from two thirds of one per
-// compute unit on (kOneRun), no split and no merge.
-int psamd_attention_decode_plan(int n_dec, int kv_len, int skewed, int hkv, int window, int* nsplit, int* min_run) {
-  PSAMD_REQUIRE(n_dec >= 1 && kv_len >= 1 && hkv >= 1 && nsplit != nullptr && min_run != nullptr, "decode plan: bad sizes");
+// request, none shorter than *min_run keys. Two workgroups per compute unit; from one per compute unit on, or two thirds
+// of that where the kernel of eight waves takes the layer (kOneRun), no split and no merge.
+int psamd_attention_decode_plan(int n_dec, int kv_len, int skewed, int hq, int hkv, int window, int* nsplit, int* min_run) {
+  PSAMD_REQUIRE(n_dec >= 1 && kv_len >= 1 && hkv >= 1 && hq >= hkv && nsplit != nullptr && min_run != nullptr, "decode plan: bad sizes");
   if (window > 0) kv_len = std::min(kv_len, window);
   const int64_t pairs = static_cast<int64_t>(n_dec) * hkv;
-  int n = pairs >= kOneRun ? 1 : static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({64, 512 / pairs, ceil_div(kv_len, 128)})));
+  const bool one_run = pairs >= (hq / hkv <= kOneTileHeads ? kOneRun : 256);
+  int n = one_run ? 1 : static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({64, 512 / pairs, ceil_div(kv_len, 128)})));
   int run = 128;
   if (skewed && window <= 0) {
     n = std::max(n, static_cast<int>(std::min<int64_t>({64, 4096 / n_dec, ceil_div(kv_len, 1024)})));
@@ -2000,7 +2005,7 @@ int psamd_attention_decode(void* stream, const void* qkv, int q_stride, void* ou
   if (n_dec == 0) return 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int group = hq / hkv;
-  const int ct = group <= 16 ? 1 : (group <= 32 ? 2 : 4);
+  const int ct = group <= kOneTileHeads ? 1 : (group <= 32 ? 2 : 4);
   // Where a kv head's runs are few numbers, the last of its workgroups merges them. us of attention and merge in a captured step
   // of up to 4,096 keys, with the kernel behind / in one launch, behind 100, 300, 1,000, 2,048 and 4,000 keys:
   //   32 heads of 64 on 8,  1 request   8.0 / 4.2   8.0 / 6.4   8.0 / 6.6    8.1 / 8.2    8.2 / 9.2     (32 runs at most)

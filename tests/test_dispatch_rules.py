@@ -1,11 +1,15 @@
-"""Which entry points of the kernel library a call goes to: host rules, run without a GPU on a library that only notes what is called."""
+"""Rules of the host side, run without a GPU: which entry points a call goes to, on a library that only notes what is called, and the kernel
+library's own plans."""
 
 from __future__ import annotations
+
+import ctypes
 
 import pytest
 import torch
 
-from prefixserve_amd.kernels.ops import HipOps
+from prefixserve_amd.build import ensure_kernels
+from prefixserve_amd.kernels.ops import _SIGNATURES, HipOps
 
 
 class NotingLibrary:
@@ -70,3 +74,22 @@ def test_one_and_two_tokens_are_grouped_where_both_widths_are_whole(ops, t, k, f
 def test_one_and_two_tokens_among_any_number_of_experts(ops, t, experts, want):
     """The sorting refuses more than 4,096 experts, which one and two tokens did not need it for."""
     assert experts_called(ops, t, 64, 64, experts) == want
+
+
+@pytest.fixture(scope="module")
+def planner():
+    made = object.__new__(HipOps)
+    made.lib, made._plans = ensure_kernels(), {}
+    made.lib.psamd_attention_decode_plan.argtypes = _SIGNATURES["psamd_attention_decode_plan"]
+    made.lib.psamd_last_error.restype = ctypes.c_char_p
+    return made
+
+
+@pytest.mark.parametrize("requests,hq,hkv,runs", [
+    (21, 32, 8, 3), (22, 32, 8, 1), (31, 128, 8, 1), (32, 32, 8, 1), (40, 32, 8, 1), (176, 16, 1, 1),
+    (22, 136, 8, 2), (31, 256, 8, 2), (32, 256, 8, 1), (176, 17, 1, 2), (255, 64, 1, 2), (256, 64, 1, 1), (90, 48, 2, 2),
+])
+def test_keys_stay_whole_where_the_kernel_of_eight_waves_takes_them(planner, requests, hq, hkv, runs):
+    """From 176 (request, kv head) pairs on there is one run of all keys, but more than 16 query heads a kv head, which that kernel
+    does not take, keep two until there is a workgroup for every compute unit."""
+    assert planner.decode_plan(requests, 2000, False, hkv, 0, hq) == (runs, 128)
