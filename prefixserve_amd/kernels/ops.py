@@ -695,15 +695,16 @@ class HipOps:
 
     def _through_lds(self, x, w, out, m: int, n: int, k: int, form: str) -> bool:
         """Whether a product of 33 to 128 tokens goes to the kernels with both operands through LDS instead of the library: "residual"
-        (out for the stream, in slices of K), "gated" or "qkv". A workgroup there walks all of K for its rows of w (for the
-        stream an eighth of it at least), so few rows and a long K leave the chip idle where the library cuts K.
+        (out for the stream, in slices of K; asked from 65 tokens on), "gated" or "qkv". A workgroup there walks all of K for its rows
+        of w (for the stream an eighth of it at least), so few rows and a long K leave the chip idle where the library cuts K.
         us, library and what follows it / here:
 
-        * residual (n x k), 40 tokens: 5,120 x 14,336 55.2 / 37.8, 8,192 x 4,096 24.1 / 25.4, x 8,192 38.4 / 43.2, x 14,336 64.6 / 52.9. 77 tokens:
-          1,024 x 8,192 14.1 / 8.7, 8,192 x 3,584 24.5 / 21.2, x 8,192 43.7 / 45.9, x 14,336 74.7 / 62.3.
-        * gated, 64 tokens: 256 x 4,096 14.7 / 11.5, x 8,192 12.9 / 18.9, 1,024 x 4,096 14.2 / 11.7, x 8,192 25.8 / 27.0, 2,048 x 8,192 26.6 / 27.6,
-          3,072 x 8,192 32.1 / 31.2, 5,632 x 8,192 46.6 / 48.4. 77 tokens: 256 x 1,024 8.4 / 6.1, x 2,048 8.5 / 10.3, 768 x 2,048 11.9 / 10.7, x 4,096 12.5 / 17.3,
-          1,536 x 4,096 23.8 / 23.2, 2,048 x 4,096 19.8 / 24.3, 3,072 x 8,192 37.2 / 44.1.
+        * residual (n x k): what decides is whether the slices of 64 rows are one round of workgroups (``_slices_pay``). 5,120 rows and fewer gain also
+          where they are a little more than one: 4,608 x 8,192 (288) 33.4 / 36.3 at 72, 49.2 / 42.0 at 128, 2,816 x 8,192 (264) 40.2 / 25.0 at 72,
+          45.7 / 28.0 at 128, 5,120 x 12,288 47.4 / 37.5 at 72, 71.5 / 45.0 at 128, 2,048 x 2,048 11.9 / 10.7 at 72, 11.9 / 12.9 at 128.
+        * gated, 64 tokens: 256 x 4,096 14.7 / 11.5, x 8,192 12.9 / 18.9, 1,024 x 4,096 14.2 / 11.7, x 8,192 25.9 / 27.4, 2,048 x 8,192 27.8 / 30.7,
+          2,560 x 8,192 32.3 / 29.8, x 14,336 53.4 / 53.5, 5,632 x 8,192 46.0 / 43.7, 8,192 x 12,288 91.5 / 78.7. 77 tokens: 256 x 1,024 8.4 / 6.1,
+          x 2,048 8.5 / 10.3, 768 x 2,048 11.9 / 10.7, x 4,096 12.5 / 17.3, 1,536 x 4,096 23.8 / 23.2, 2,048 x 4,096 19.8 / 24.3, 3,072 x 8,192 37.2 / 44.1.
         * qkv, 64 tokens: 768 x 4,096 16.1 / 10.7, x 8,192 15.6 / 16.7, 1,536 x 8,192 26.7 / 22.8 (40: 18.1 / 19.8), 2,560 x 8,192 27.3 / 24.6, 9,216 x 8,192 45.8 / 42.5
           (40). 77 tokens: 768 x 2,048 12.5 / 10.0, 1,536 x 4,096 13.8 / 16.3, 2,560 x 4,096 16.5 / 19.1, 3,072 x 4,096 21.1 / 17.6, x 8,192 44.5 / 34.2, 4,608 x 8,192 32.7 / 35.2."""
         if form == "gated":
@@ -714,10 +715,28 @@ class HipOps:
         elif form == "qkv":
             pays = (k <= 4096 or n >= 2560) if m <= self.SKINNY_MAX_ROWS else (k <= 2048 or (n >= 3072 and k <= 4096))
         else:
-            pays = n * k <= 6e7 or k >= 14336
+            pays = n <= 5120 or self._slices_pay(m, n, k)
         return (pays and self.FUSED_SWIGLU_MAX_ROWS < m <= self.STREAM_MAX_ROWS and x.dtype == torch.bfloat16
                 and w.dtype == torch.bfloat16 and out.dtype == torch.bfloat16
                 and bool(self.lib.psamd_linear_skinny_takes(x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, int(form == "gated"))))
+
+    def _slices_pay(self, m: int, n: int, k: int) -> bool:
+        """Whether a product of 65 to 128 tokens and more than 5,120 rows of w is the faster in slices of K. us at 72, 96, 104 and 128 tokens, the norm behind
+        it included, library / here (workgroups):
+
+        * one round of the 256 compute units: 7,168 x 4,096 (224) 29.4, 29.9, 30.0, 32.0 / 24.3, 25.8, 27.6, 28.5, 8,192 x 13,824 (256) 62.1, 69.8, 67.6, 83.2 / 55.0,
+          58.7, 64.2, 66.8; but not where w is large and its rows a power of two apart, so that all workgroups ask the same memory channels:
+          8,192 x 8,192 41.4, 45.8, 43.8, 53.6 / 43.3, 45.0, 47.3, 49.5, x 16,384 71.6, 80.2, 76.0, 96.2 / 77.9, 81.4, 85.6, 89.7;
+        * the start of a second round: 6,144 x 4,096 (288) 27.1, 27.5, 27.8, 30.0 / 27.7, 29.1, 28.5, 30.2, x 8,192 39.5, 43.3, 41.1, 50.3 / 42.3, 45.1, 47.3, 51.1,
+          x 16,384 64.3, 74.6, 68.2, 88.3 / 72.4, 76.9, 80.7, 87.0, 10,240 x 5,120 (320) 76.1, 65.0, 64.1, 69.7 / 73.8, 78.5, 79.1, 83.6;
+        * the library's time doubles behind a K of 16,384, which outweighs the second round of three slices, not of two: 6,144 x 18,432 149 to 155 / 84 to 94,
+          8,192 x 32,768 209, 191, 214, 219 / 125, 129, 149, 155, 10,240 x 24,576 189, 179, 191, 194 / 192, 206, 216, 228."""
+        slices = int(self.lib.psamd_linear_skinny_ksplit(m, n, k))
+        if slices <= 1:
+            return False
+        if -(-n // 64) * slices <= 256:
+            return n * k <= 6e7 or k > 16384 or k & (k - 1) != 0
+        return k > 16384 and slices > 2
 
     def _in_tiles(self, x, w, out) -> bool:
         """Whether the tiles of linear_tile.hip may be asked: bfloat16 in and out, and the library beside them for what they leave to it."""
