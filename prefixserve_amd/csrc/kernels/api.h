@@ -388,7 +388,7 @@ int psamd_attention_prefill(void* stream, const void* qkv, int q_stride, void* o
 // than the rest), into how many runs of at least how many keys each request's keys are cut, and
 // the most (requests x runs) any plan gives (part_o: that many x hq x head_dim floats).
 int psamd_attention_decode_skewed(int n_dec, int longest, int64_t total);
-int psamd_attention_decode_plan(int n_dec, int kv_len, int skewed, int hq, int hkv, int window, int* nsplit, int* min_run);
+int psamd_attention_decode_plan(int n_dec, int kv_len, int skewed, int hq, int hkv, int head_dim, int window, int* nsplit, int* min_run);
 int psamd_attention_decode_max_parts(int max_requests);
 
 int psamd_attention_decode(void* stream, const void* qkv, int q_stride, void* out, const void* kv, float* part_o,

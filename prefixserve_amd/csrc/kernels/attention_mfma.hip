@@ -1746,20 +1746,27 @@ static int launch_prefill(hipStream_t s, const void* qkv, int q_stride, void* ou
   return launch_prefill_merge(s, part_o, part_ml, out, pf_tiles, item_start, n_tiles, hq, 16 * NS, nsplit);
 }
 
-// From kOneRun to 256 (request, kv head) pairs a workgroup of eight waves takes all keys of one: it has its compute unit (nearly) to itself, and
-// nothing is merged behind it. us a layer behind 300, 1,000, 2,049 and uneven up to 2,900 keys, as before (two runs of four waves below 256 pairs,
-// one from there on) / so, 32 heads on 8:
-//   head size 64,  22 requests   9.6, 16.3, 25.7, 27.6 / 6.9, 13.8, 21.9, 24.4      head size 128, 22    14.3, 27.2, 47.5, 46.0 / 11.1, 23.5, 41.0, 46.8
-//                  24            9.8, 16.7, 26.6, 27.2 / 6.9, 14.1, 22.9, 24.3                     28    14.6, 29.9, 50.3, 48.8 / 12.1, 26.9, 46.4, 50.0
-//                  30           10.6, 18.2, 29.8, 28.1 / 7.9, 16.0, 26.9, 25.5                     32    14.1, 30.0, 53.0, 52.0 / 12.9, 29.0, 51.4, 51.2
-//                  32            9.1, 17.8, 30.5, 35.2 / 8.1, 16.7, 28.1, 26.5      head size 32,  24     8.2, 12.5, 19.1, 21.1 /  6.0, 10.3, 17.2, 18.9
+// From kOneRun to 256 (request, kv head) pairs of heads of up to 64 a workgroup of eight waves takes all keys of one: it has its compute unit (nearly) to
+// itself, and nothing is merged behind it. us a layer behind 300, 1,000, 2,049 and uneven up to 2,900 keys, as before (two runs of four waves below
+// 256 pairs, one from there on) / so, 32 heads on 8:
+//   head size 64,  22 requests   9.6, 16.3, 25.7, 27.6 / 6.9, 13.8, 21.9, 24.4
+//                  24            9.8, 16.7, 26.6, 27.2 / 6.9, 14.1, 22.9, 24.3      head size 32,  24     8.2, 12.5, 19.1, 21.1 /  6.0, 10.3, 17.2, 18.9
+//                  30           10.6, 18.2, 29.8, 28.1 / 7.9, 16.0, 26.9, 25.5
+//                  32            9.1, 17.8, 30.5, 35.2 / 8.1, 16.7, 28.1, 26.5
 // At 20 and 21 requests three runs stay the faster for uneven contexts (21.7 / 24.0); above 256 pairs some units have two such workgroups
 // (33 requests behind 2,049 keys: 35.0 / 39.0). The same keys cut evenly over the chip whatever the requests' lengths gained nothing (64 uneven
 // requests: 46.2 / 46.6): a launch pays 7 us for its trips to memory one after the other, and then streams at 5.2 TB/s either way.
+// Wider heads keep their two runs below 256 pairs: a compute unit reads 32 KB a us, so that the longest of uneven contexts on one unit outlasts the others,
+// and the plan does not know how uneven they are. Two runs / one, mean of the contexts half of the longest: 12 requests on 16 kv heads, head size 64 22.9 / 20.8,
+// 80 27.4 / 29.0, 96 28.8 / 30.8, 112 31.4 / 39.3, 128 30.9 / 40.8, 192 48.0 / 60.4, 256 53.8 / 89.4; 90 on 2, 128 41.5 / 45.2, 192 63.0 / 67.5; 22 on 8, 96 31.5 / 31.5,
+// 128 40.6 / 40.8, 256 55.6 / 87.3. (Contexts of one length would gain, 128, 22 on 8 behind 300 and 2,049: 12.4, 48.0 / 9.6, 41.4.)
 // The kernel of eight waves is that of up to 16 query heads a kv head: with more, one run of four waves instead of two of them leaves half of
 // the waves out (256 heads of 64 on 8, 22 requests behind 2,049 keys / uneven up to 2,900: 32.5, 33.8 in two runs, 39.4, 44.3 in one; 64 on 1, 255
-// uneven: 53.5, 68.5).
+// uneven: 53.5, 68.5). And of head sizes up to 192: at 256 its registers do not hold the sums (44 bytes of scratch a lane; 32 requests on 8 behind 300 and 2,049
+// keys and uneven: four waves 21.8, 96.5, 91.3, eight 25.4, 102.3, 108.1; at 192 18.3, 78.7, 84.1 and 16.7, 73.1, 70.6; at 128 13.6, 51.2, 47.9 and 12.3, 49.4, 48.9).
 constexpr int kOneRun = 176;
+constexpr int kOneRunDim = 64;          // the largest head size that takes one run below 256 pairs
+constexpr int kEightWavesDim = 192;     // ... and that eight waves take at all
 constexpr int kOneTileHeads = 16;       // query heads a kv head that are one tile of the matrix instructions
 
 template <int NS, int CT, bool P3>
@@ -1786,8 +1793,9 @@ static int launch_decode(hipStream_t s, const void* qkv, int q_stride, const voi
   if constexpr (CT == 1) {
     if (arrived != nullptr) return run(attn_decode_mfma_kernel<NS, CT, P3, true>, 4);
     const int64_t pairs = static_cast<int64_t>(n_dec) * hkv;
-    if (nsplit == 1 && pairs >= kOneRun && pairs <= 256)
-      return run(attn_decode_mfma_kernel<NS, CT, P3, false, 8>, 8);
+    if constexpr (16 * NS <= kEightWavesDim) {
+      if (nsplit == 1 && pairs >= kOneRun && pairs <= 256) return run(attn_decode_mfma_kernel<NS, CT, P3, false, 8>, 8);
+    }
   }
   return run(attn_decode_mfma_kernel<NS, CT, P3>, 4);
 }
@@ -1965,12 +1973,12 @@ int psamd_attention_decode_skewed(int n_dec, int longest, int64_t total) {
 // How psamd_attention_decode should cut the keys of a step of n_dec single-token items whose
 // longest context is kv_len (for a captured step: the longest there can be): *nsplit runs per
 // request, none shorter than *min_run keys. Two workgroups per compute unit; from one per compute unit on, or two thirds
-// of that where the kernel of eight waves takes the layer (kOneRun), no split and no merge.
-int psamd_attention_decode_plan(int n_dec, int kv_len, int skewed, int hq, int hkv, int window, int* nsplit, int* min_run) {
-  PSAMD_REQUIRE(n_dec >= 1 && kv_len >= 1 && hkv >= 1 && hq >= hkv && nsplit != nullptr && min_run != nullptr, "decode plan: bad sizes");
+// of that where the kernel of eight waves is the faster for any contexts (kOneRun), no split and no merge.
+int psamd_attention_decode_plan(int n_dec, int kv_len, int skewed, int hq, int hkv, int head_dim, int window, int* nsplit, int* min_run) {
+  PSAMD_REQUIRE(n_dec >= 1 && kv_len >= 1 && hkv >= 1 && hq >= hkv && head_dim >= 1 && nsplit != nullptr && min_run != nullptr, "decode plan: bad sizes");
   if (window > 0) kv_len = std::min(kv_len, window);
   const int64_t pairs = static_cast<int64_t>(n_dec) * hkv;
-  const bool one_run = pairs >= (hq / hkv <= kOneTileHeads ? kOneRun : 256);
+  const bool one_run = pairs >= (hq / hkv <= kOneTileHeads && head_dim <= kOneRunDim ? kOneRun : 256);
   int n = one_run ? 1 : static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({64, 512 / pairs, ceil_div(kv_len, 128)})));
   int run = 128;
   if (skewed && window <= 0) {

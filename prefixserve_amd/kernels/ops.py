@@ -75,7 +75,7 @@ _SIGNATURES = {
     "psamd_attention_prefill_nsplit": [_i32, _i32, _i32, _i32, _i32],
     "psamd_attention_prefill_part_rows": [_i32, _i32, _i32],
     "psamd_attention_decode_skewed": [_i32, _i32, _i64],
-    "psamd_attention_decode_plan": [_i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp],
+    "psamd_attention_decode_plan": [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp],
     "psamd_attention_decode_max_parts": [_i32],
     "psamd_attention_prefill": [_vp, _vp, _i32, _vp, _vp, _vp, _i32, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32,
                                 _f32, _i32, _vp, _vp, _i32, _i32],
@@ -1442,15 +1442,15 @@ class HipOps:
         longest needs). A captured decode step is keyed by it."""
         return bool(self.lib.psamd_attention_decode_skewed(int(count), int(longest), int(total)))
 
-    def decode_plan(self, count: int, kv_len: int, skewed: bool, hkv: int, window: int, hq: int | None = None) -> tuple[int, int]:
+    def decode_plan(self, count: int, kv_len: int, skewed: bool, hkv: int, window: int, hq: int | None = None, d: int = 64) -> tuple[int, int]:
         """(runs per request, shortest run in keys) for a step of ``count`` single-token items; ``hq`` None: as many query heads
-        as kv heads."""
+        as kv heads; ``d``: their size."""
         hq = hkv if hq is None else hq
-        key = (count, kv_len, skewed, hq, hkv, window)
+        key = (count, kv_len, skewed, hq, hkv, d, window)
         plan = self._plans.get(key)
         if plan is None:
             nsplit, min_run = ctypes.c_int(0), ctypes.c_int(0)
-            self._ok(self.lib.psamd_attention_decode_plan(count, kv_len, int(skewed), hq, hkv, window, ctypes.byref(nsplit),
+            self._ok(self.lib.psamd_attention_decode_plan(count, kv_len, int(skewed), hq, hkv, d, window, ctypes.byref(nsplit),
                                                           ctypes.byref(min_run)))
             if len(self._plans) > 4096:
                 self._plans.clear()
@@ -1555,7 +1555,7 @@ class HipOps:
             if ctx.num_decode:
                 kv_len = self.fixed_kv_len or ctx.max_kv_len
                 skewed = self.fixed_skew if self.fixed_kv_len else ctx.decode_skewed
-                nsplit, min_run = self.decode_plan(ctx.num_decode, kv_len, skewed, hkv, win, hq)
+                nsplit, min_run = self.decode_plan(ctx.num_decode, kv_len, skewed, hkv, win, hq, d)
                 # Room for the (request, run) pairs of any plan: asked for once, never grown.
                 parts = self._bounds.get(ctx.num_decode)
                 if parts is None:

@@ -86,14 +86,16 @@ def planner():
     return made
 
 
-@pytest.mark.parametrize("requests,hq,hkv,runs", [
-    (21, 32, 8, 3), (22, 32, 8, 1), (31, 128, 8, 1), (32, 32, 8, 1), (40, 32, 8, 1), (176, 16, 1, 1),
-    (22, 136, 8, 2), (31, 256, 8, 2), (32, 256, 8, 1), (176, 17, 1, 2), (255, 64, 1, 2), (256, 64, 1, 1), (90, 48, 2, 2),
+@pytest.mark.parametrize("requests,hq,hkv,d,runs", [
+    (21, 32, 8, 64, 3), (22, 32, 8, 64, 1), (31, 128, 8, 32, 1), (32, 32, 8, 64, 1), (40, 32, 8, 64, 1), (176, 16, 1, 64, 1),
+    (22, 136, 8, 64, 2), (31, 256, 8, 64, 2), (32, 256, 8, 64, 1), (176, 17, 1, 64, 2), (255, 64, 1, 64, 2), (256, 64, 1, 64, 1), (90, 48, 2, 64, 2),
+    (22, 32, 8, 80, 2), (31, 32, 8, 128, 2), (12, 16, 16, 256, 2), (32, 32, 8, 128, 1), (32, 8, 8, 256, 1), (17, 32, 8, 256, 3),
 ])
-def test_keys_stay_whole_where_the_kernel_of_eight_waves_takes_them(planner, requests, hq, hkv, runs):
+def test_keys_stay_whole_where_the_kernel_of_eight_waves_takes_them(planner, requests, hq, hkv, d, runs):
     """From 176 (request, kv head) pairs on there is one run of all keys, but more than 16 query heads a kv head, which that kernel
-    does not take, keep two until there is a workgroup for every compute unit."""
-    assert planner.decode_plan(requests, 2000, False, hkv, 0, hq) == (runs, 128)
+    does not take, and heads of more than 64, where the longest of uneven contexts would outlast the others, keep two until there is
+    a workgroup for every compute unit."""
+    assert planner.decode_plan(requests, 2000, False, hkv, 0, hq, d) == (runs, 128)
 
 
 @pytest.mark.parametrize("m,n,k,here", [
