@@ -210,14 +210,19 @@ __global__ __launch_bounds__(64 * (TN / 16) * TG * KG) void stream_tiles_kernel(
   }
 }
 
+constexpr int kUnits = 256;                                                    // compute units
+
 // The most rows of w per workgroup, which read the tokens least often, that still give about half of the 256 compute units one and
 // leave no second round of workgroups that take a whole unit's LDS: 5,632 gated columns are 352 workgroups of 16 (23.1 us at 77 tokens) or 176
 // of 32 (18.0), 11,008 344 of 32 (54.4) or 172 of 64 (43.2), 4,608 rows of q/k/v 288 of 16 (33.5) or 144 of 32 (19.5); the six fastest
 // forms tried for 8,192 gated columns x 2,048 were all 256 of 32, not 128 of 64. With K-slices, which linear_stream_ksplit chooses for 64 rows,
-// fewer only where even eight slices leave units idle (1,024 x 1,024: 3.5, 3.2, 3.2).
+// fewer only where even eight slices leave units idle (1,024 x 1,024: 3.5, 3.2, 3.2) and those of fewer rows, one to a unit, are still one round.
+// us with the norm behind it, two rounds of 32 / one of 64: 1,408 x 1,536 at 33 tokens 9.9 / 8.4, at 128 13.6 / 11.3, 1,280 x 2,048 at 97 12.4 / 10.4, 5,632 x 256 at
+// 33 12.3 / 10.9; of 16 / of 32: 2,816 x 256 at 128 11.6 / 9.7.
 static int stream_columns(int N, int ksplit) {
-  const int kEnough = ksplit > 1 ? 192 : 136;
-  return ceil_div(N, 64) * ksplit >= kEnough ? 64 : (ceil_div(N, 32) * ksplit >= kEnough ? 32 : 16);
+  const int64_t of64 = ceil_div(N, 64) * ksplit, of32 = ceil_div(N, 32) * ksplit, of16 = ceil_div(N, 16) * ksplit;
+  if (ksplit > 1) return of64 >= 192 || of32 > kUnits ? 64 : (of32 >= 192 || of16 > kUnits ? 32 : 16);
+  return of64 >= 136 ? 64 : (of32 >= 136 ? 32 : 16);
 }
 
 // How a tile of TM tokens and TN rows is shared out: TG, KG and the number of buffers. Few rows a workgroup (16, 32) leave a unit of
@@ -264,8 +269,10 @@ static int launch_stream_tokens(hipStream_t s, const void* x, const void* w, voi
                                 const QkvOut& q) {
   if (M <= 32) return launch_stream_tiles<32, TN, FORM>(s, x, w, out, M, N, K, ksplit, act, q);
   if (M <= 64) return launch_stream_tiles<64, TN, FORM>(s, x, w, out, M, N, K, ksplit, act, q);
+  // Tiles of 96 tokens, whose slices have a unit each to themselves, not where that makes a second round: those of 128 share one (2,816 x 4,096, 264
+  // workgroups, the norm behind it included, 77 tokens 18.7 / 16.0 us, x 512 at 65 11.9 / 10.5).
   if constexpr (!(FORM == kGated && TN == 64)) {       // (2 x 14,336 x 4,096 gated at 96 tokens: 45.4 us as 96, 46.3 as 128; 2 x 11,008 43.7, 41.9)
-    if (M <= 96 && (TN < 64 || ceil_div(K / 64, ksplit) >= 8)) return launch_stream_tiles<96, TN, FORM>(s, x, w, out, M, N, K, ksplit, act, q);
+    if (M <= 96 && (TN < 64 || (ceil_div(K / 64, ksplit) >= 8 && ceil_div(N, 64) * ksplit <= kUnits))) return launch_stream_tiles<96, TN, FORM>(s, x, w, out, M, N, K, ksplit, act, q);
   }
   return launch_stream_tiles<128, TN, FORM>(s, x, w, out, M, N, K, ksplit, act, q);
 }
