@@ -729,14 +729,16 @@ class HipOps:
           8,192 x 8,192 41.4, 45.8, 43.8, 53.6 / 43.3, 45.0, 47.3, 49.5, x 16,384 71.6, 80.2, 76.0, 96.2 / 77.9, 81.4, 85.6, 89.7;
         * the start of a second round: 6,144 x 4,096 (288) 27.1, 27.5, 27.8, 30.0 / 27.7, 29.1, 28.5, 30.2, x 8,192 39.5, 43.3, 41.1, 50.3 / 42.3, 45.1, 47.3, 51.1,
           x 16,384 64.3, 74.6, 68.2, 88.3 / 72.4, 76.9, 80.7, 87.0, 10,240 x 5,120 (320) 76.1, 65.0, 64.1, 69.7 / 73.8, 78.5, 79.1, 83.6;
-        * the library's time doubles behind a K of 16,384, which outweighs the second round of three slices, not of two: 6,144 x 18,432 149 to 155 / 84 to 94,
-          8,192 x 32,768 209, 191, 214, 219 / 125, 129, 149, 155, 10,240 x 24,576 189, 179, 191, 194 / 192, 206, 216, 228."""
+        * the library's time doubles behind a K of 16,384, and it takes half as long again for one that is no multiple of 128, which outweighs the second round of
+          three slices, not of two: 6,144 x 18,432 150, 150, 155, 159 / 86, 92, 95, 101, 8,192 x 32,768 209, 191, 214, 219 / 125, 129, 149, 155, 10,240 x 24,576 189,
+          179, 191, 194 / 192, 206, 216, 228; 6,144 x 3,072 23.8, 24.4, 24.6, 26.8 / 24.4, 26.2, 26.5, 28.7, x 2,880 33.3, 32.6, 33.3, 33.4 / 23.7, 25.3, 25.9, 27.4,
+          x 13,888 78.9, 78.7, 79.2, 86.8 / 65.2, 71.1, 73.1, 78.9, 9,216 x 2,880 53.0, 53.5, 54.8, 54.3 / 55.0, 55.3, 55.6, 58.2."""
         slices = int(self.lib.psamd_linear_skinny_ksplit(m, n, k))
         if slices <= 1:
             return False
         if -(-n // 64) * slices <= 256:
             return n * k <= 6e7 or k > 16384 or k & (k - 1) != 0
-        return k > 16384 and slices > 2
+        return slices > 2 and (k > 16384 or k % 128 != 0)
 
     def _in_tiles(self, x, w, out) -> bool:
         """Whether the tiles of linear_tile.hip may be asked: bfloat16 in and out, and the library beside them for what they leave to it."""

@@ -103,7 +103,7 @@ def test_keys_stay_whole_where_the_kernel_of_eight_waves_takes_them(planner, req
     (66, 5184, 4096, True), (96, 8192, 7296, True), (96, 8192, 14336, True), (128, 7168, 4096, True),   # one round of workgroups
     (72, 8192, 4096, True), (72, 8192, 8192, False), (104, 8192, 16384, False), (72, 8192, 32768, True),  # rows a power of two apart
     (104, 6144, 8192, False), (104, 6144, 14336, False), (104, 6144, 16384, False), (96, 10240, 2048, False),   # a second round
-    (72, 6144, 18432, True), (104, 10240, 24576, False), (77, 12288, 4096, False), (77, 16384, 20480, False),
+    (72, 6144, 18432, True), (72, 5632, 2880, True), (128, 6144, 13888, True), (104, 10240, 24576, False), (72, 9216, 2880, False), (77, 12288, 4096, False), (77, 16384, 20480, False),
 ])
 def test_slices_of_k_are_taken_where_they_are_one_round(planner, m, n, k, here):
     """Products for the stream of 65 to 128 tokens: any K from 14,336 on was taken, also where the slices begin a second round of workgroups, up to 18%
