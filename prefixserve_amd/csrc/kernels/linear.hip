@@ -1012,7 +1012,8 @@ int psamd_linear_normed(void* stream, const float* resid, const int32_t* rows, c
   const Tokens tk{nullptr, resid, norm_w, rows, eps, norm_w_dtype == kBF16 ? 1 : 0};
   const int form = epilogue == 1 ? kGated : (out_dtype == kF32 ? kSlices : kPlain);
   if (linear_normed_takes(w, out, form, M, n_out, K)) return launch_linear_normed(s, tk, w, out, form, M, n_out, K, g_gate_act);
-  // What is left has a K that is no multiple of 64, a w off 16 bytes, rows that do not fit in LDS beside w's, float32 outputs or few columns.
+  // What is left has a K that is no multiple of 64, a w off 16 bytes, rows that do not fit in LDS beside w's, float32 outputs, or sizes at which
+  // these kernels are the faster (normed_pays).
   const int64_t groups = ceil_div(n_out, 16);
   const bool eight = M <= 8;
   if (epilogue == 1) {

@@ -241,17 +241,44 @@ int launch_normed(hipStream_t s, const Tokens& tk, const void* w, void* out, int
 
 }  // namespace
 
-// Where every compute unit's one workgroup has rows enough to hide the staging of the tokens. us at 1, 4, 8 and 16 tokens, kernels of linear.hip and here:
-//   gated 2 x 8,192 x 2,048   16.5, 17.5, 18.2, 20.8 -> 14.8, 15.9, 16.7, 18.9    plain 512 x 2,048     6.4, 6.5, 6.6, 8.0 -> 5.0, 5.3, 6.3, 7.6
-//   gated 2 x 14,336 x 4,096  51.4, 52.2, 53.2 -> 44.9, 46.4, 47.5               plain 2,048 x 2,048   6.6, 7.0, 6.9, 8.4 -> 5.8, 6.3, 7.2, 8.5
-//   gated 2 x 1,024 x 2,048    8.6, 9.0, 8.9, 10.2 -> 6.1, 6.6, 7.5, 9.5           plain 3,072 x 3,072   7.7, 8.2, 8.4, 10.3 -> 7.5, 8.2, 9.7, 10.3
-//   q/k/v 4,608 x 2,048        9.2, 9.6, 10.5, 12.5 -> 7.9, 8.3, 9.2, 10.2         plain 5,376 x 2,048   9.5, 10.0, 10.4, 12.6 -> 7.7, 8.2, 9.0, 10.5
-//   q/k/v 6,144 x 4,096       16.1, 17.3, 19.0 -> 14.3, 15.9, 17.2                plain 10,752 x 2,048  14.5, 14.7, 15.6, 19.7 -> 12.1, 12.6, 13.4, 14.7
-//   q/k/v 3,072 x 2,048        6.7, 7.0, 7.4, 8.8 -> 6.9, 7.3, 8.4, 9.3
-// Not for tiles of 16 rows of q/k/v, nor plain ones from 5 tokens on. Float32 outputs (the output matrix) stay in linear.hip, whose workgroups stage the
+// Where every compute unit's one workgroup has rows enough to hide the staging of the tokens, which grows with them, and buffers enough for its rows of w:
+// beside the tokens there is room for three buffers of the gated form up to K = 4,032 (9 and more tokens: 1,984), for two behind that. us with
+// weights that are in no cache at 1, 4, 5, 8, 9 and 16 tokens, kernels of linear.hip and here (q/k/v: heads of 128):
+//   tiles of 16 rows (below 4,321)
+//     gated 2 x 1,536 x 2,048   8.8, 8.9, 9.0, 9.0, 10.1, 10.3 -> 7.6, 8.2, 9.0, 9.0, 11.3, 11.4       2 x 2,048 x 4,096  14.4, 15.0, 16.0, 15.9 -> 14.1, 16.1, 17.3, 17.2
+//           2 x 4,096 x 1,536   9.1, 9.3, 9.5, 9.3, 10.4, 10.5 -> 8.8, 9.4, 10.1, 10.1, 11.1, 11.2     2 x 2,816 x 5,120  19.1, 19.5, 21.0, 20.9 -> 18.8, 21.1, 22.6, 22.6
+//     plain 2,048 x 2,048       6.3, 6.6, 6.8, 6.7 -> 5.9, 6.4, -, -      4,096 x 4,096  10.7, 11.5 -> 9.9, 12.0      q/k/v 3,072 x 2,048  6.7, 7.0, -, 7.4, -, 8.8 -> 6.9, 7.3, -, 8.4, -, 9.3
+//   tiles of 32 (below 8,641)
+//     gated 2 x 8,192 x 2,048   17.1, 17.4, 17.9, 17.9, 20.5, 21.2 -> 15.1, 16.0, 16.7, 16.8, 19.2, 19.2     x 1,024  10.0, 10.0, 10.3, 10.4, 12.8, 13.2 -> 10.0, 10.2, 10.7, 10.8, 11.5, 11.6
+//           2 x 8,192 x 2,880   21.0, 21.8, 23.1, 22.8, 26.3, 26.8 -> 20.4, 21.7, 23.0, 22.9, 27.7, 27.9     x 4,096  34.3, 35.4, 37.2, 37.2 -> 29.1, 30.9, 32.1, 32.2
+//     q/k/v 4,608 x 2,048       9.1, 10.0, 9.8, 10.5, 11.3, 12.1 -> 8.2, 8.9, 9.6, 9.6, 10.9, 11.0           4,608 x 1,536  7.9, 8.4, 8.3, 8.8, 9.6, 10.3 -> 7.7, 8.2, 8.8, 8.8, 9.8, 10.0
+//           6,144 x 4,096       14.8, 15.4, 15.6, 16.5 -> 13.9, 15.9, 17.0, 17.1                             8,192 x 4,096  16.7, 17.8, 18.4, 19.1 -> 17.2, 19.4, 20.4, 20.4
+//           6,144 x 5,120       21.2, 22.9, 25.4, 26.1 -> 16.4, 18.6, 20.1, 20.3                             8,192 x 2,560  12.3, 13.0, 12.9, 13.6, 15.3, 16.2 -> 12.2, 13.1, 14.0, 14.2, 15.7, 15.8
+//     plain 6,144 x 2,048       9.3, 9.7, 10.1, 10.0, 11.7, 12.0 -> 8.4, 9.1, 9.8, 9.8, 11.3, 11.5           6,144 x 1,536  7.8, 8.0, 8.1, 8.2, 9.2, 9.4 -> 7.6, 8.0, 8.7, 8.7, 9.7, 9.9
+//   tiles of 64
+//     gated 2 x 14,336 x 4,096  49.2, 50.3, 51.5, 51.6 -> 43.2, 45.0, 45.9, 46.2       2 x 11,008 x 2,560  30.9, 32.4, 32.6, 32.8, 31.4, 32.2 -> 24.7, 25.5, 26.3, 26.5, 34.9, 35.2
+//     q/k/v 9,216 x 2,048       13.3, 14.6, 15.1, 15.6, 20.7, 22.0 -> 11.3, 12.1, 12.8, 12.9, 14.0, 14.2     plain  13.2, 13.6, 13.0, 13.9, 17.4, 18.4 -> 10.9, 11.6, 12.3, 12.3, 13.6, 13.8
+// Float32 outputs (the output matrix) stay in linear.hip, whose workgroups stage the
 // tokens once for several groups of rows: 32,000 x 2,048 28.7, 29.0, 31.4, 37.2 there, 29.3, 30.4, 32.4, 35.5 here, 128,256 x 2,048 93.9 to 112 there, 101 to 131 here.
+static bool normed_pays(int form, int M, int n_out, int K) {
+  const int64_t of16 = ceil_div(n_out, 16), of32 = ceil_div(n_out, 32);
+  const bool narrow = of32 < kEnoughBlocks, wide = ceil_div(n_out, 64) >= kEnoughBlocks;   // tiles of 16 and of 64 rows
+  if (form == kGated) {
+    const bool three = 96 * 1024 + normed_tokens_bytes(M <= 8 ? 8 : 16, K) <= 160 * 1024;  // buffers
+    if (narrow) return M <= 2 || (three && (M <= 4 || K > 1536 || of16 < 160));            // few steps do not pay for many tokens
+    if (wide) return M <= 8 || three || K <= 2048;
+    return M <= 8 ? (M <= 4 || K > 1024 || of32 <= 200) : (three || K <= 2560);
+  }
+  if (narrow) return form == kPlain && (M <= 2 || (M <= 4 && (K <= 2816 || of16 <= 160)));
+  if (wide || K >= 4608) return true;
+  if (K < 2048) return M <= 4 && (K <= 512 || (K >= 1536 && of32 <= 192));
+  if (K <= 2816) return M <= 4 || M > 8 || of32 <= 192;
+  if (M > 8) return form == kPlain || of32 <= 192;
+  return of32 <= 192 && M <= (of32 <= 176 ? 4 : 2);
+}
+
 bool linear_normed_takes(const void* w, const void* out, int form, int M, int n_out, int K) {
-  if (form == kSlices || (form != kGated && ceil_div(n_out, 32) < kEnoughBlocks && (form == kQkv || M > 4))) return false;
+  if (form == kSlices || !normed_pays(form, M, n_out, K)) return false;
   return M >= 1 && M <= 16 && n_out > 0 && n_out % 4 == 0 && K >= 64 && K % 64 == 0 && (form == kGated ? 4LL : 2LL) * n_out * K < (1LL << 32) &&
          64 * 1024 + normed_tokens_bytes(M <= 8 ? 8 : 16, K) <= 160 * 1024 &&
          (reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
