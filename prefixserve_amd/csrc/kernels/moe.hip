@@ -1197,27 +1197,36 @@ static bool tiles_take(int64_t tokens, int64_t pairs, int K, int F) {
   return K % 64 == 0 && F % 64 == 0 && 2 * tokens * K <= most && 2 * pairs * F <= most && 4LL * K * F <= most;
 }
 
-// From how many pairs an expert on a step that sorts its pairs itself takes the large tiles; below, moe_stream_kernel reads an expert once per 16 pairs. us of
-// routing and experts, small tiles / large: 32 experts of 2,048 x 1,024 at 16, 20, 24, 28, 46 pairs each 102, 113, 117, 122, 149 / 112, 116, 116, 117, 123; 8 of
-// 4,096 x 3,584 at 16, 24, 46 161, 182, 238 / 181, 181, 186; 24 of 1,024 x 320 at 16, 28, 46 31, 38, 43 / 35, 37, 39; 64 of 2,048 x 1,408 at 12, 16, 24 224, 248, 315 / 233, 239, 244.
-constexpr int64_t kTilesFromPairs = 24;
+// From how many pairs an expert on a step that sorts its pairs itself takes the large tiles; below, moe_stream_kernel reads an expert once per 16 pairs. The
+// large tiles take nearly the same time at any of these counts, which is that of their steps of K one after the other, if there are too few of them: `filled`
+// counts those of 128 columns that the smaller of the two products has with one tile an expert. us of routing and experts, small tiles / large, at 24, 32, 40 and 47
+// pairs an expert (filled):
+//   64 of 2,048 x 1,408 gated (1,024) 230, 273, 313, 339 / 197, 202, 218, 228       32 of 2,048 x 1,024 gated (512) 122, 134, 150, 160 / 118, 120, 122, 123
+//    8 of 4,096 x 3,584 gated (256)   182, 209, 235, 244 / 185, 188, 189, 191       16 of 2,048 x 2,816 gated (256) 152, 170, 188, 201 / 168, 171, 174, 176
+//   24 of 1,024 x 320 gated (120)      34, 39, 41, 42 / 38, 39, 40, 40                8 of 2,048 x 1,024 gated (128)  38, 44, 44, 47 / 53, 55, 55, 56
+//   16 of 4,096 x 1,024 ungated (128)  78, 87, 99, 103 / 98, 102, 109, 114            8 of 1,024 x 8,192 gated (64)  124, 154, 165, 177 / 178, 181, 183, 184
+//    4 of 1,024 x 512 gated (32)       18, 19, 21, 22 / 31, 32, 33, 35               32 of 512 x 256 ungated (64)     23, 27, 29, 31 / 30, 32, 35, 36
+static int64_t tiles_from_pairs(int experts, int K, int F, int kind) {
+  const int64_t filled = experts * std::min(ceil_div(K, 128), ceil_div(F, kind == kExpertGated ? 64 : 128));
+  return filled >= 320 ? 24 : (filled >= 200 ? 28 : 48);
+}
 
 // ... and their rows: 0 where the kernel for small tiles takes the step, 256 where the device chooses tiles of up to 256 x 256 by the step's
 // counts. Those ask for half the bytes per product, but one workgroup of them fills a compute unit, two of 128 x 128 share one, and a
 // last round that is not full costs nearly as much as one that is: the time is that of the rounds, K long in the first product and F
 // in the second, and 300 more for what a large tile does in front of and behind its loop, which the two small ones on a unit do beside
-// each other's. An expert's last tile is half empty on average. us of both products and the sorting, 256 / 128 / the kernel above
-// (E experts of K x F, choices at random; the kernel above is moe_grouped_kernel, in front of moe_stream_kernel):
-//   32 of 2,048 x 1,024:  50 pairs an expert 109 / 109 / 152, 140 126 / 146 / 227, 260 163 / 194 / 269, 448 232 / 261 / 337, 1,000 580 / 594 / 693
-//    8 of 2,048 x 1,024:  64 59 / 58 / 90, 260 70 / 66 / 110, 512 92 / 107 / 141, 1,000 166 / 156 / 235, 2,000 262 / 279 / 373
-//    8 of 4,096 x 3,584:  64 156 / 159 / 255, 260 301 / 397 / 441, 448 377 / 547 / 567, 1,000 848 / 1,128 / 1,048
-//   24 of 1,024 x 320:    64 38 / 33 / 47, 512 75 / 72 / 96, 2,000 247 / 204 / 273
-//    4 of 1,024 x 512:    64 36 / 29 / 44, 512 43 / 34 / 57, 2,000 54 / 50 / 70
-//   64 of 2,048 x 1,408:  64 266 / 277 / 345, 448 639 / 750 / 921, 1,000 1,303 / 1,527 / 1,818
+// each other's. An expert's last tile is half empty on average. us of both products and the sorting, 256 / 128 (E experts of K x F,
+// choices at random):
+//   32 of 2,048 x 1,024:  50 pairs an expert 109 / 109, 140 126 / 146, 260 163 / 194, 448 232 / 261, 1,000 580 / 594
+//    8 of 2,048 x 1,024:  64 59 / 58, 260 70 / 66, 512 92 / 107, 1,000 166 / 156, 2,000 262 / 279
+//    8 of 4,096 x 3,584:  64 156 / 159, 260 301 / 397, 448 377 / 547, 1,000 848 / 1,128
+//   24 of 1,024 x 320:    64 38 / 33, 512 75 / 72, 2,000 247 / 204
+//    4 of 1,024 x 512:    64 36 / 29, 512 43 / 34, 2,000 54 / 50
+//   64 of 2,048 x 1,408:  64 266 / 277, 448 639 / 750, 1,000 1,303 / 1,527
 // Over eight shapes at 17 sizes, choices even and uneven, the choice is on average 1.0% over the faster (always 256: 2.9%, always
 // 128: 7.8%), at worst 17%.
 static int wide_tile_rows(int64_t pairs, int experts, int K, int F, int kind) {
-  if (pairs < kTilesFromPairs * experts) return 0;
+  if (pairs < tiles_from_pairs(experts, K, F, kind) * experts) return 0;
   auto rounds = [&](int rows, int at_once, int beside) {
     const double tiles = std::max<double>(experts, static_cast<double>(pairs) / rows + 0.5 * experts);
     auto of = [&](int64_t columns) {
