@@ -692,9 +692,10 @@ int psamd_general_delta_prepare(void* stream, const void* rows, int act_dtype, i
   hipStream_t s = static_cast<hipStream_t>(stream);
   // Sixteen tokens a workgroup where that leaves the chip full. Below, the four of the other kernel are ahead: 300 workgroups
   // (600 tokens, 8 heads) 10.8 us against 9.0; from 450 (600 tokens, 12 heads: 12.4 against 13.6) they are behind. 32 KB of LDS
-  // hold the tokens' values of a rank of 512.
+  // hold the tokens' values of a rank of 512. Lanes without a column count as missing workgroups: 16 heads of 32, rank 64
+  // 600 tokens 11.1 us by the other kernel, 11.7 here, 1,200 18.3 and 16.1; rank 512 38 and 43, 72 and 83, 2,048 tokens 117 and 93.
   const size_t block_smem = sizeof(float) * kBlockTokens * ((static_cast<size_t>(rank) + 15) / 16 * 16);
-  const bool blocks = ceil_div(tokens, kBlockTokens) * heads >= 448 && dim <= 2 * kWave && block_smem <= 32 * 1024;
+  const bool blocks = ceil_div(tokens, kBlockTokens) * heads * std::min(dim, kWave) >= 448 * kWave && dim <= 2 * kWave && block_smem <= 32 * 1024;
   auto run = [&](auto kernel, auto type, int per_block, size_t smem) {
     using A = decltype(type);
     kernel<<<dim3(static_cast<unsigned>(ceil_div(tokens, per_block)), static_cast<unsigned>(heads)), dim3(256), smem, s>>>(

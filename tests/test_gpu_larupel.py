@@ -736,9 +736,9 @@ def test_long_prompts_go_through_the_runs(tmp_path, monkeypatch):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads,dim,rank,tokens", [(28, 64, 64, 241), (7, 128, 16, 1024), (23, 100, 13, 331), (32, 40, 17, 257),
-                                                   (448, 64, 1, 3), (7, 65, 512, 1009)])
+                                                   (32, 40, 17, 400), (20, 32, 64, 720), (448, 64, 1, 3), (7, 65, 512, 1009)])
 def test_general_delta_operands_of_many_tokens(ops, dtype, heads, dim, rank, tokens):
-    """From 448 workgroups of sixteen tokens and a head on another kernel makes them: the sums in the same order, so the bits of
+    """From 448 workgroups of sixteen tokens and a head on (more where a head leaves lanes out) another kernel makes them: the sums in the same order, so the bits of
     calls of a few tokens. Heads that do not fill their lanes, ranks that do not fill a step, tokens behind the last sixteen."""
     torch.manual_seed(0)
     hd, floor, eps = heads * dim, 0.6, 1e-6
