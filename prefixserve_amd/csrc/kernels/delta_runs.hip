@@ -12,7 +12,7 @@
 //     L_ts = (c_t D_{t-1}) . (p_s / D_s), W = U (what is taken out), Wx = T (M X), M_ts = (c_t D_{t-1}) . (k_s / D_s),
 //     Kt = T (c D_{-1}), and what the values alone leave in the output (Y) and the state (Z).
 // Three launches: runs_prepare (all runs side by side: everything that does not need S0), runs_chain (an item's runs in turn:
-// two small products each), runs_output (all runs side by side). 2,048 tokens as above: 41 + 93 + 28 us (gated), 107 + 60 + 24
+// two small products each), runs_output (all runs side by side). 2,048 tokens as above: 39 + 90 + 27 us (gated), 106 + 60 + 24
 // (general). The chain is what bounds a long prompt: 64 matrix instructions and two barriers a run, 2.9 us of 32 runs in turn.
 //
 // Numerics: everything is float32. T is built by substitution, 16 x 16 on the diagonal and block by block below it (a product
@@ -115,8 +115,8 @@ constexpr int kGatedForm = 0, kPlainForm = 1, kGeneralForm = 2;   // plain: the 
 
 // grid (runs, heads), four waves: wave w makes the rows of tokens 16 w .. 16 w + 15 of what is between tokens, then the columns
 // 16 w, 64 + 16 w, .. of Wx, Kt, Kd and Z. With one to three waves a SIMD, what bounds it is each wave's chain of loads and
-// products: 16 heads of 128, 2,048 tokens, 65 -> 41 us with the columns divided (wave 3 was at it 74 us while wave 0 took 42) and
-// the operands asked for ahead; the general form's 32 heads of 64 126 -> 107. There the divisions by D_s, the rows that
+// products: 16 heads of 128, 2,048 tokens, 61 -> 39 us with the columns divided (wave 3 was at it 74 us while wave 0 took 42) and
+// the operands asked for ahead; the general form's 32 heads of 64 118 -> 106. There the divisions by D_s, the rows that
 // wave 3 has four times as many of as wave 0 and two workgroups of 70 KB of LDS a compute unit are left. Same sums, same bits.
 template <int DT, int FORM>
 __global__ __launch_bounds__(256) void runs_prepare_kernel(DeltaRuns c, RunList list) {

@@ -52,9 +52,10 @@ __device__ __forceinline__ void put_columns(float* __restrict__ out, int64_t m, 
 // the row's number, so that the 16 rows a read touches lie on all banks. Tiles that share rows of w run on one die (its L2 serves
 // them): die d takes the d-th eighth of the tiles, tokens fastest. Bound by the matrix instructions, whose rate on this card is 150 TFLOP/s (a loop of
 // them and nothing else); what is left of it goes to the wait for a chain's first operands behind the barrier, which the other
-// workgroups of the compute unit fill. us, with rows on their way in registers and operands read as they are needed / so:
-// 600 tokens x 16,384 columns x 2,048 424 / 343 (117 TFLOP/s), 600 x 3,072 91 / 72, 600 x 2,048 75 / 55, 600 x 2,048 x 8,192 267 / 199, 300 x 2,048 52 / 32,
-// 150 x 2,048 x 8,192 130 / 90, 2,048 x 16,384 1,299 / 1,059 (130). A third buffer costs workgroups and is slower everywhere (600 x 2,048 65).
+// workgroups of the compute unit fill. us with weights that are in no cache, with rows on their way in registers and operands read as they are needed / so, both
+// on a card that copies 1 GiB at 5.16 TB/s: 600 tokens x 16,384 columns x 2,048 411 / 346 (116 TFLOP/s), 600 x 3,072 86 / 73, 600 x 2,048 71 / 56, 600 x 2,048 x
+// 8,192 266 / 209, 300 x 2,048 50 / 34, 150 x 2,048 x 8,192 127 / 90, 2,048 x 16,384 1,301 / 1,093 (126). A third buffer costs workgroups and is slower everywhere
+// (600 x 2,048 65).
 template <int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                 float* __restrict__ out, int M, int N, int K, int m_tiles, int tiles,
@@ -295,11 +296,11 @@ bool linear_f32_takes(const void* x, const void* w, int64_t M, int N, int K) {
 //  * K of one segment, and up to 16 tokens or so few tiles as below: a wave per chain.
 //  * up to 8 tokens, or 16 where the columns are fewer than 16,384: 16 rows of w per workgroup. 2,048 columns at 8 tokens 13
 //    (tiles of 32 tokens 36), 128,256 at 1 token 187 (234); at 16 tokens 282 (224).
-//  * tiles of 32 tokens x 64 columns for a quarter of the compute units at most: the same kernel with 32 tokens. 64 tokens x 2,048 columns 17 (tiles 18),
-//    33 x 2,048 x 8,192 53 (62), 24 x 3,072 15 (18).
+//  * tiles of 32 tokens x 64 columns for a quarter of the compute units at most: the same kernel with 32 tokens. 64 tokens x 2,048 columns 16 (tiles 17),
+//    33 x 2,048 x 8,192 50 (79), 24 x 3,072 16 (24).
 //  * tiles: what the compute unit with the most of them takes, in columns x tokens over the share of its rate that a shape gets from as many
-//    workgroups as it has. 600 x 16,384 in tiles of 64 x 64 / 32 x 64 / 32 x 32 343 / 331 to 372 / -, 2,048 x 16,384 1,059 / 1,100 / -, 600 x 2,048 68 / 55 / 59,
-//    x 8,192 258 / 199 / 238, 300 x 2,048 - / 39 / 32, 150 x 2,048 x 8,192 - / 101 / 90, 17 x 16,384 - / 37 / 33, 128 x 3,072 - / 30 / 26.
+//    workgroups as it has. 600 x 16,384 in tiles of 64 x 64 / 32 x 64 / 32 x 32 346 / 335 / 366, 2,048 x 16,384 1,093 / 1,117 / 1,281, 600 x 3,072 73 / 78 / 80, 600 x 2,048
+//    71 / 56 / 60, x 8,192 271 / 210 / 231, 300 x 2,048 40 / 42 / 34, 150 x 2,048 x 8,192 153 / 100 / 90, 17 x 16,384 45 / 34 / 32, 128 x 3,072 41 / 28 / 25.
 int launch_linear_f32(hipStream_t s, const float* x, const float* w, float* out, int M, int N, int K) {
   const int64_t tiles32 = ceil_div(M, 32) * ceil_div(N, 64);
   auto cost = [&](int bm, int bn, double share) {
