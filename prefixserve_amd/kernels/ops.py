@@ -851,6 +851,8 @@ class HipOps:
                 self._ok(self.lib.psamd_linear_skinny(self._stream(), x.data_ptr(), w.data_ptr(), out.data_ptr(),
                                                       _F32, m, n, k, 0, ksplit))
                 return out
+        if self.SKINNY_MAX_ROWS < m <= self.STREAM_MAX_ROWS and x.dtype == torch.bfloat16 and k % 8 == 0:
+            self.ws.get(name + ".slices", (8 * self.STREAM_MAX_ROWS * n,), torch.float32)   # a shorter step has slices: as above
         out = self.ws.get(name, (m, n), x.dtype)
         self.linear(x, w, out)
         return out

@@ -27,8 +27,13 @@ class NotingLibrary:
 
 
 class Buffers:
+    def __init__(self) -> None:
+        self.asked: dict[str, int] = {}
+
     def get(self, name, shape, dtype):
-        return torch.empty(shape, dtype=dtype)
+        out = torch.empty(shape, dtype=dtype)
+        self.asked[name] = max(self.asked.get(name, 0), out.numel())
+        return out
 
 
 @pytest.fixture
@@ -111,3 +116,18 @@ def test_slices_of_k_are_taken_where_they_are_one_round(planner, m, n, k, here):
     x, w = torch.empty(m, 64, dtype=torch.bfloat16), torch.empty(64, 64, dtype=torch.bfloat16)   # addresses alone are looked at
     takes = planner._through_lds(x, w, x, m, n, k, "residual") and planner.lib.psamd_linear_skinny_ksplit(m, n, k) > 1
     assert takes == here
+
+
+@pytest.mark.parametrize("n,k", [(6144, 64), (2048, 64)])
+def test_a_step_left_to_the_library_asks_for_the_slices_of_a_shorter_one(ops, n, k):
+    """Up to 64 tokens a product for the stream has slices whatever its sizes: where 65 to 128 tokens go to the library, their step asks for the
+    slices' room too, so that no buffer grows behind the largest step."""
+    ops._direct_library, ops.fixed_kv_len, ops._slice_views, ops._fuses = True, None, {}, {}
+    ops.lib.psamd_linear_skinny_takes = lambda *args: 0              # the library's
+    ops.lib.psamd_linear_skinny_ksplit = lambda m, n, k: 4
+    x, w = torch.empty(100, k, dtype=torch.bfloat16), torch.empty(n, k, dtype=torch.bfloat16)
+    large = ops.linear_to_residual(x, w, "o")
+    assert large.shape == (100, n) and large.dtype == torch.bfloat16
+    asked = dict(ops.ws.asked)
+    assert ops.linear_to_residual(x[:40], w, "o").shape == (4, 40, n)
+    assert ops.ws.asked == asked
