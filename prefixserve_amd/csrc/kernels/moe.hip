@@ -37,6 +37,7 @@
 #include "linear_stream.h"
 #include "stream_operands.h"
 #include "tile_product.h"
+#include "wide_tile.h"
 
 namespace psamd {
 
@@ -413,7 +414,7 @@ struct TileCut {
   __device__ __forceinline__ int first(int tile) const { return 64 * (tile * units + min(tile, larger)); }
 };
 
-// The time of a tile of the 512-thread kernel below by its 64s of pairs, in 1/64 of a full one's (measured there).
+// The time of a large tile by its 64s of pairs, in 1/64 of a full one's (measured there).
 __device__ __forceinline__ int tile_cost(int units) { return units <= 2 ? 42 : units == 3 ? 54 : 64; }
 
 // The time of the step's tiles under a limit of pairs, computed by one wave: every die runs an eighth of the tiles, 32 at once, and a
@@ -932,139 +933,32 @@ __global__ __launch_bounds__(64 * (TN / 16) * KG) void moe_stream_kernel(
 
 // ------------------------------------------------------------------ experts, many pairs each
 
-// A tile of up to TM pairs by TN rows of the expert's matrix per workgroup of WM x WN waves, both operands through LDS 64 k at a
-// time (tile_product.h has the loop). The matrices of all experts are read at the rate the matrix cores use them only if a workgroup
-// multiplies each byte often: 256 x 256 asks for half the bytes per product of the kernel above, whose rows of the matrix go
+// A tile of up to 256 pairs by 256 rows of the expert's matrix, or 128 by 128, per workgroup, both operands through LDS 64 k at a
+// time (wide_tile.h and tile_product.h have the loops). The matrices of all experts are read at the rate the matrix cores use them only if a
+// workgroup multiplies each byte often: 256 x 256 asks for half the bytes per product of the kernel above, whose rows of the matrix go
 // from memory to registers for one tile of 128 pairs (14 TB/s out of the L2s). What it does about each bound:
 //  * an expert's tiles run on one die (its L2 then holds the expert's rows): die d takes the d-th eighth of the work;
 //  * a chip of 256 units runs large tiles in a few rounds, whose last one is seldom full, and an expert with a few pairs more than
-//    whole tiles costs one more: with TM 256 the sorting cuts every expert's pairs into near-even tiles under the limit (256, 192 or 128)
-//    that gives the step's counts the least time, and a tile runs the loop that is made for its size. (A loop more is not free: its code
-//    comes from memory in every launch, and where few tiles need it nobody has fetched it for them: one of 32 experts with 140
-//    pairs, the others 64, 140 us, 128 with one loop for all. But that one loop takes 313 us at 512 pairs an expert.);
+//    whole tiles costs one more: the sorting cuts every expert's pairs into near-even tiles under the limit (256, 192 or 128)
+//    that gives the step's counts the least time, and a tile runs the loop that is made for its size;
 //  * us of sorting and products, tiles of 256 and a rest in one loop / cut evenly by the pair / so, 32 experts of 2,048 x 1,024: 66 pairs
 //    an expert 119 / 119 / 112, 160 136 / 142 / 134, 256 208 / 189 / 164, 512 328 / 294 / 287, 1,000 552 / 561 / 584, 1,400 681 / 693 / 704; 8 of
 //    4,096 x 3,584: 256 356 / 340 / 317, 512 590 / 573 / 562, 1,400 1,165 / 1,197 / 1,182. Over 274 steps (eight shapes, 52 to 2,000 pairs, even and
-//    uneven) 0.91 of the time of tiles of 256 and a rest, 0.97 of that of the even cut;
-//  * as many workgroups as there are units stay and walk the tiles: the grid of the most tiles there could be had half of its
-//    workgroups leave at once, each from a unit of its own;
-//  * the waves for pairs that a tile does not have skip the arithmetic.
-// GATED: a wave's 64 rows are 32 gate rows and the 32 up rows of the same columns.
+//    uneven) 0.91 of the time of tiles of 256 and a rest, 0.97 of that of the even cut (all of them with the loop before wide_tile.h's);
+//  * as many workgroups as there are units stay and walk the large tiles, the copies of one under the end of the one before: that and waves of 128
+//    x 128 against eight of 128 x 64 that began each tile anew, us of sorting and both products, 32 experts of 2,048 x 1,024: 448 pairs an expert
+//    225 -> 204, 512 273 -> 249 (all even 242 -> 227), 1,024 525 -> 455; 8 of 4,096 x 3,584 at 512 526 -> 469; 64 of 2,048 x 1,408 at 192 345 -> 314.
+//    What is left of 249: gate and up 136 (one tile after the other 1.6 us a step of 64 k where the dense product takes 1.4: 268 MB of matrices come from
+//    memory meanwhile; 4 us of activations behind each tile, under which no matrix core works), down 90 (134 MB of float32 leave, 134 MB of matrices come).
+// GATED: a wave's rows of the matrix are gate rows and then the up rows of the same columns.
 
-// LDS of the steps of a workgroup's tile: two of the largest, as many of a smaller one as fit there.
-constexpr int tile_smem_steps(int tm, int tn) { return 2 * (tm + tn) * 128 + (tm == 256 ? 16 * 1024 : 0); }
-constexpr int tile_stages(int tm, int tn, int rows) { return std::min(3, tile_smem_steps(tm, tn) / ((rows + tn) * 128)); }
-
-template <int TM, int TN, int WM, int WN, int FORM>
-__global__ __launch_bounds__(64 * WM * WN, 2) void moe_tile_kernel(
-    const bf16_t* __restrict__ a, const float* __restrict__ pair_weight, const bf16_t* __restrict__ w,
-    const int32_t* __restrict__ sorted, const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_first,
-    const int32_t* __restrict__ tile_count, const int32_t* __restrict__ n_tiles, bf16_t* __restrict__ out_act,
-    float* __restrict__ out_f32, int64_t tokens, int K, int N, int top, float gate_alpha, float limit, float up_shift,
-    int into_stream, const float* __restrict__ col_scale, int identity_to, const bf16_t* __restrict__ x,
-    const float* __restrict__ weight, int column_tiles) {
-  constexpr bool GATED = FORM == kFormGated;
-  constexpr int WV = WM * WN, BK = 64, RN = TN / WN / 16, WROWS = TN / WN;
-  constexpr int COLS = GATED ? TN / 2 : TN, WCOLS = GATED ? WROWS / 2 : WROWS;   // columns of the workgroup, of a wave
-  constexpr int LB = TN / 8 / WV;                                                // copies of 8 rows of the matrix per wave and step
-  extern __shared__ __align__(16) unsigned char tile_smem[];                     // the steps of tile_product, then int32_t[TM]
-  int32_t* pair_s = reinterpret_cast<int32_t*>(tile_smem + tile_smem_steps(TM, TN));
-  // The work of this workgroup's die: an eighth of all (tile, columns).
-  const int tiles = *n_tiles, die = static_cast<int>(blockIdx.x & 7);
-  const int from = static_cast<int>(static_cast<int64_t>(tiles) * column_tiles * die / 8);
-  const int to = static_cast<int>(static_cast<int64_t>(tiles) * column_tiles * (die + 1) / 8);
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int r = lane & 15, g = lane >> 4;
-  const int wn = wave % WN;
-  // Uniform for the workgroup. Each time its place moves on by a tile's columns: an expert's last tile is often a smaller one, and a
-  // workgroup that always took the same place would have it every time, or never.
-  const int at_once = static_cast<int>(gridDim.x >> 3);
-  for (int round = 0; from + round * at_once < to; ++round) {
-    const int at = from + round * at_once + static_cast<int>((blockIdx.x >> 3) + static_cast<unsigned>(round) * column_tiles) % at_once;
-    if (at >= to) continue;
-    const int slot = at / column_tiles, n0 = at % column_tiles * COLS;
-    const int e = tile_expert[slot], first = tile_first[slot], count = min(tile_count[slot], TM);
-    const char* w_base = reinterpret_cast<const char*>(w + static_cast<int64_t>(e) * (GATED ? 2 : 1) * N * K);
-    __syncthreads();                            // everybody is done with the tile before: its pairs, its last step in LDS
-    for (int i = threadIdx.x; i < TM; i += 64 * WV) pair_s[i] = i < count ? sorted[first + i] : -1;
-    __syncthreads();
-    // RM tiles of 16 pairs for each of the WM waves that share columns.
-    auto product = [&](auto rm) {
-      constexpr int RM = decltype(rm)::value, ROWS = RM * 16 * WM, LA = ROWS / 8 / WV;
-      static_assert(LA * 8 * WV == ROWS && LB * 8 * WV == TN, "whole copies per wave");
-      uint32_t a_off[LA], b_off[LB];
-#pragma unroll
-      for (int i = 0; i < LA; ++i) {
-        const int row = (wave * LA + i) * 8 + (lane >> 3);
-        const int pair = pair_s[min(row, count - 1)];
-        a_off[i] = static_cast<uint32_t>(FORM != kFormDown ? pair / top : pair) * (2u * K) + 16u * tile_copy_piece(row, lane);
-      }
-#pragma unroll
-      for (int i = 0; i < LB; ++i) {
-        const int row = (wave * LB + i) * 8 + (lane >> 3);
-        const int col = min(n0 + (row / WROWS) * WCOLS + row % WCOLS, N - 1);
-        b_off[i] = static_cast<uint32_t>(GATED && row % WROWS >= WCOLS ? N + col : col) * (2u * K) + 16u * tile_copy_piece(row, lane);
-      }
-      const int wm = wave / WN * (RM * 16);                                      // waves of a SIMD share no rows of pairs
-      const bool works = wm < count;
-      tile_f32x4 acc[RN][RM];
-#pragma unroll
-      for (int i = 0; i < RN; ++i)
-#pragma unroll
-        for (int j = 0; j < RM; ++j) acc[i][j] = tile_f32x4{0.f, 0.f, 0.f, 0.f};
-      tile_product<tile_stages(TM, TN, ROWS), ROWS, TN>(acc, tile_smem, reinterpret_cast<const char*>(a), w_base, a_off, b_off, wm,
-                                                         wn * WROWS, wave, lane, K / BK, works);
-      if (!works) return;
-      // Lane (r, g) holds, for the pair in row wm + 16 j + r, columns 4 g .. + 3 of every 16 of the wave's.
-#pragma unroll
-      for (int j = 0; j < RM; ++j) {
-        const int pair = pair_s[wm + j * 16 + r];
-        if (pair < 0) continue;
-        const float pw = pair_weight != nullptr ? pair_weight[pair] : 1.f;       // on the input's sums (GATED) or on the output's
-#pragma unroll
-        for (int i = 0; i < WCOLS / 16; ++i) {
-          const int nc = n0 + wn * WCOLS + i * 16 + 4 * g;
-          if (nc >= N) continue;                                                 // N is a multiple of 8
-          if (FORM != kFormDown) {
-            bf16_t res[4];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-              if (!GATED) {
-                const float p = fmaxf(pw * acc[i][j][v], 0.f);
-                res[v] = float_to_bf16(p * p);
-                continue;
-              }
-              const float gg = fminf(pw * acc[i][j][v], limit);
-              const float uu = fminf(fmaxf(pw * acc[(i + RN / 2) % RN][j][v], -limit), limit);
-              res[v] = float_to_bf16(gg / (1.f + __expf(-gate_alpha * gg)) * (uu + up_shift));
-            }
-            *reinterpret_cast<ushort4*>(out_act + static_cast<int64_t>(pair) * N + nc) = ushort4{res[0], res[1], res[2], res[3]};
-          } else if (into_stream) {
-            float* o = out_f32 + static_cast<int64_t>(pair / top) * N + nc;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) add_float(o + v, (col_scale != nullptr ? col_scale[nc + v] : 1.f) * (pw * acc[i][j][v]));
-          } else {
-            float* o = out_f32 + (static_cast<int64_t>(pair % top) * tokens + pair / top) * N + nc;
-            *reinterpret_cast<float4*>(o) = float4{pw * acc[i][j][0], pw * acc[i][j][1], pw * acc[i][j][2], pw * acc[i][j][3]};
-          }
-        }
-      }
-    };
-    constexpr int MOST = TM / WM / 16;
-    if constexpr (MOST == 8) {
-      if (count <= TM / 4) product(std::integral_constant<int, MOST / 4>{});
-      else if (count <= TM / 2) product(std::integral_constant<int, MOST / 2>{});
-      else if (count <= TM / 4 * 3) product(std::integral_constant<int, MOST / 4 * 3>{});
-      else product(std::integral_constant<int, MOST>{});
-    } else {
-      product(std::integral_constant<int, MOST>{});
-    }
-  }
-  // The identity pairs lie behind the experts' and have no tiles: the tokens themselves times their weights, dealt out over all threads.
-  if (FORM != kFormDown || identity_to == 0) return;
-  const int begin = tile_first[tiles], quads = N / 4;                            // N is a multiple of 8
-  const int64_t all = static_cast<int64_t>(identity_to - begin) * quads;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * (64 * WV) + threadIdx.x; i < all; i += static_cast<int64_t>(gridDim.x) * (64 * WV)) {
+// The identity pairs lie behind the experts' and have no tiles: the tokens themselves times their weights, dealt out over all threads.
+__device__ __forceinline__ void copy_identity(const int32_t* __restrict__ sorted, int begin, int end, const bf16_t* __restrict__ x,
+                                              const float* __restrict__ weight, float* __restrict__ out_f32, int64_t tokens, int N, int top,
+                                              int into_stream, const float* __restrict__ col_scale) {
+  const int quads = N / 4;                                                       // N is a multiple of 8
+  const int64_t all = static_cast<int64_t>(end - begin) * quads, step = static_cast<int64_t>(gridDim.x) * blockDim.x;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < all; i += step) {
     const int pair = sorted[begin + i / quads], n = static_cast<int>(i % quads) * 4;
     const int64_t t = pair / top;
     const float wt = weight[pair];
@@ -1078,6 +972,265 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void moe_tile_kernel(
       *reinterpret_cast<float4*>(out_f32 + (static_cast<int64_t>(pair % top) * tokens + t) * N + n) = y;
     }
   }
+}
+
+// The small tiles: one a workgroup, two workgroups a unit.
+constexpr int kSmallTile = 128, kSmallSmem = 2 * 2 * kSmallTile * 128;
+
+template <int FORM>
+__global__ __launch_bounds__(256, 2) void moe_tile_kernel(
+    const bf16_t* __restrict__ a, const float* __restrict__ pair_weight, const bf16_t* __restrict__ w,
+    const int32_t* __restrict__ sorted, const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_first,
+    const int32_t* __restrict__ tile_count, const int32_t* __restrict__ n_tiles, bf16_t* __restrict__ out_act,
+    float* __restrict__ out_f32, int64_t tokens, int K, int N, int top, float gate_alpha, float limit, float up_shift,
+    int into_stream, const float* __restrict__ col_scale, int identity_to, const bf16_t* __restrict__ x,
+    const float* __restrict__ weight, int column_tiles) {
+  constexpr bool GATED = FORM == kFormGated;
+  constexpr int TM = kSmallTile, TN = kSmallTile, BK = 64, RM = 4, RN = 4, WROWS = TN / 2, LA = 4, LB = 4;   // four waves of 64 x 64
+  constexpr int COLS = GATED ? TN / 2 : TN, WCOLS = GATED ? WROWS / 2 : WROWS;   // columns of the workgroup, of a wave
+  extern __shared__ __align__(16) unsigned char tile_smem[];                     // two steps, then int32_t[TM]
+  int32_t* pair_s = reinterpret_cast<int32_t*>(tile_smem + kSmallSmem);
+  // The work of this workgroup's die: an eighth of all (tile, columns).
+  const int tiles = *n_tiles, die = static_cast<int>(blockIdx.x & 7);
+  const int from = static_cast<int>(static_cast<int64_t>(tiles) * column_tiles * die / 8);
+  const int to = static_cast<int>(static_cast<int64_t>(tiles) * column_tiles * (die + 1) / 8);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int r = lane & 15, g = lane >> 4, wn = wave & 1;
+  if (const int at = from + static_cast<int>(blockIdx.x >> 3); at < to) {        // uniform for the workgroup
+    const int slot = at / column_tiles, n0 = at % column_tiles * COLS;
+    const int e = tile_expert[slot], first = tile_first[slot], count = min(tile_count[slot], TM);
+    const char* w_base = reinterpret_cast<const char*>(w + static_cast<int64_t>(e) * (GATED ? 2 : 1) * N * K);
+    if (threadIdx.x < TM) pair_s[threadIdx.x] = static_cast<int>(threadIdx.x) < count ? sorted[first + threadIdx.x] : -1;
+    __syncthreads();
+    uint32_t a_off[LA], b_off[LB];
+#pragma unroll
+    for (int i = 0; i < LA; ++i) {
+      const int row = (wave * LA + i) * 8 + (lane >> 3);
+      const int pair = pair_s[min(row, count - 1)];
+      a_off[i] = static_cast<uint32_t>(FORM != kFormDown ? pair / top : pair) * (2u * K) + 16u * tile_copy_piece(row, lane);
+    }
+#pragma unroll
+    for (int i = 0; i < LB; ++i) {
+      const int row = (wave * LB + i) * 8 + (lane >> 3);
+      const int col = min(n0 + (row / WROWS) * WCOLS + row % WCOLS, N - 1);
+      b_off[i] = static_cast<uint32_t>(GATED && row % WROWS >= WCOLS ? N + col : col) * (2u * K) + 16u * tile_copy_piece(row, lane);
+    }
+    const int wm = wave / 2 * (RM * 16);
+    const bool works = wm < count;               // the waves for pairs that a tile does not have skip the arithmetic
+    tile_f32x4 acc[RN][RM];
+#pragma unroll
+    for (int i = 0; i < RN; ++i)
+#pragma unroll
+      for (int j = 0; j < RM; ++j) acc[i][j] = tile_f32x4{0.f, 0.f, 0.f, 0.f};
+    tile_product<2, TM, TN>(acc, tile_smem, reinterpret_cast<const char*>(a), w_base, a_off, b_off, wm, wn * WROWS, wave, lane, K / BK, works);
+    // Lane (r, g) holds, for the pair in row wm + 16 j + r, columns 4 g .. + 3 of every 16 of the wave's.
+#pragma unroll
+    for (int j = 0; j < RM; ++j) {
+      const int pair = pair_s[wm + j * 16 + r];
+      if (pair < 0) continue;
+      const float pw = pair_weight != nullptr ? pair_weight[pair] : 1.f;       // on the input's sums (GATED) or on the output's
+#pragma unroll
+      for (int i = 0; i < WCOLS / 16; ++i) {
+        const int nc = n0 + wn * WCOLS + i * 16 + 4 * g;
+        if (nc >= N) continue;                                                 // N is a multiple of 8
+        if (FORM != kFormDown) {
+          bf16_t res[4];
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            if (!GATED) {
+              const float p = fmaxf(pw * acc[i][j][v], 0.f);
+              res[v] = float_to_bf16(p * p);
+              continue;
+            }
+            const float gg = fminf(pw * acc[i][j][v], limit);
+            const float uu = fminf(fmaxf(pw * acc[(i + RN / 2) % RN][j][v], -limit), limit);
+            res[v] = float_to_bf16(gg / (1.f + __expf(-gate_alpha * gg)) * (uu + up_shift));
+          }
+          *reinterpret_cast<ushort4*>(out_act + static_cast<int64_t>(pair) * N + nc) = ushort4{res[0], res[1], res[2], res[3]};
+        } else if (into_stream) {
+          float* o = out_f32 + static_cast<int64_t>(pair / top) * N + nc;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) add_float(o + v, (col_scale != nullptr ? col_scale[nc + v] : 1.f) * (pw * acc[i][j][v]));
+        } else {
+          float* o = out_f32 + (static_cast<int64_t>(pair % top) * tokens + pair / top) * N + nc;
+          *reinterpret_cast<float4*>(o) = float4{pw * acc[i][j][0], pw * acc[i][j][1], pw * acc[i][j][2], pw * acc[i][j][3]};
+        }
+      }
+    }
+  }
+  if (FORM == kFormDown && identity_to != 0)
+    copy_identity(sorted, tile_first[tiles], identity_to, x, weight, out_f32, tokens, N, top, into_stream, col_scale);
+}
+
+// The large ones of these tiles (256 x 256; wide_tile.h has the loop): workgroups of four waves that stay and walk their die's eighth of the work.
+template <int FORM>
+struct ExpertTiles {
+  const float* __restrict__ pair_weight;
+  const bf16_t* __restrict__ matrices;
+  const int32_t* __restrict__ sorted;
+  const int32_t* __restrict__ tile_expert;
+  const int32_t* __restrict__ tile_first;
+  const int32_t* __restrict__ tile_count;
+  bf16_t* __restrict__ out_act;
+  float* __restrict__ out_f32;
+  const float* __restrict__ col_scale;
+  int64_t tokens;
+  int K, N, top, into_stream, column_tiles, from, to, at_once;
+  float gate_alpha, limit, up_shift;
+
+  static constexpr bool GATED = FORM == kFormGated;
+  static constexpr int WROWS = kWideTile / 2, WCOLS = GATED ? WROWS / 2 : WROWS, COLS = 2 * WCOLS;
+  struct Item {
+    int expert, first, count, n0;
+  };
+  const char* w;
+  int round, lane, wave;
+  bool has_next;
+  Item cur, nxt;                                // the tile that is multiplied, the one behind it
+  int row_pair, out_pair[2];                    // of the copies' row 64 wave + lane of the next tile; of this tile's rows of this wave
+
+  // What follows from the lane alone would be computed in front of all tiles and held through them, where no register is free.
+  __device__ __forceinline__ int own_lane() const {
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    return l;
+  }
+  // Each round its place moves on by a tile's columns: an expert's last tile is often a smaller one, and a workgroup that always took the
+  // same place would have it every time, or never.
+  __device__ __forceinline__ void look() {
+    const int at = from + round * at_once + static_cast<int>((blockIdx.x >> 3) + static_cast<unsigned>(round) * column_tiles) % at_once;
+    has_next = at < to;
+    if (!has_next) return;
+    const int slot = at / column_tiles;
+    auto one = [](int v) { return __builtin_amdgcn_readfirstlane(v); };          // uniform, where the compiler can't see it
+    nxt = Item{one(tile_expert[slot]), one(tile_first[slot]), one(min(tile_count[slot], kWideTile)), one(at % column_tiles * COLS)};
+    ++round;
+  }
+  __device__ __forceinline__ void start() {
+    lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    round = 0;
+    look();
+    if (has_next) ask_rows();
+  }
+  __device__ __forceinline__ void ask_rows() { row_pair = sorted[nxt.first + min(64 * wave + lane, nxt.count - 1)]; }
+  __device__ __forceinline__ void ahead() {
+    if (has_next) ask_rows();
+  }
+  __device__ __forceinline__ int rows() {
+    cur = nxt;
+    look();
+    const int at = (wave >> 1) * (16 * rows16(cur.count)) + lane;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) out_pair[h] = sorted[cur.first + min(at + 64 * h, cur.count - 1)];
+    return cur.count;
+  }
+  static __device__ __forceinline__ int rows16(int count) { return count <= 64 ? 2 : (count <= 128 ? 4 : (count <= 192 ? 6 : 8)); }
+  __device__ __forceinline__ bool a_rows(uint32_t (&off)[8]) {
+    if (!has_next) return false;
+    const int lane = own_lane();
+    const int at = static_cast<int>(static_cast<uint32_t>(FORM != kFormDown ? row_pair / top : row_pair) * (2u * K));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) off[i] = static_cast<uint32_t>(__shfl(at, 8 * i + (lane >> 3), kWave)) + wide_piece(8 * i + (lane >> 3), lane);
+    return true;
+  }
+  // Columns of the two bfloat16 forms: a lane's four of two neighbouring tiles of 16 stand side by side, 16 bytes of the output.
+  __device__ __forceinline__ bool w_rows(uint32_t (&off)[8]) {
+    if (!has_next) return false;
+    const int lane = own_lane();
+    w = reinterpret_cast<const char*>(matrices + static_cast<int64_t>(nxt.expert) * (GATED ? 2 : 1) * N * K);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int row = (wave * 8 + i) * 8 + (lane >> 3), in = row % WCOLS;
+      const int c = FORM == kFormDown ? in : (in & ~31) + (in >> 2 & 3) * 8 + (in >> 4 & 1) * 4 + (in & 3);
+      const int col = min(nxt.n0 + row / WROWS * WCOLS + c, N - 1);
+      off[i] = wide_row(GATED && row % WROWS >= WCOLS ? N + col : col, K) + wide_piece(8 * i + (lane >> 3), lane);
+    }
+    return true;
+  }
+  template <int RM>
+  __device__ __forceinline__ bool finish(tile_f32x4 (&acc)[8][RM]) {
+    const int lane = own_lane(), r = lane & 15, g = lane >> 4, wm = (wave >> 1) * (16 * RM);
+    int pair[RM];
+    float weight[RM];
+#pragma unroll
+    for (int j = 0; j < RM; ++j) {
+      pair[j] = __shfl(out_pair[j / 4], (16 * j + r) % kWave, kWave);
+      weight[j] = pair_weight != nullptr ? pair_weight[pair[j]] : 1.f;            // on the input's sums (GATED) or on the output's
+    }
+#pragma unroll
+    for (int j = 0; j < RM; ++j) {
+      if (wm + 16 * j + r >= cur.count) continue;
+      const float pw = weight[j];
+      const int c0 = cur.n0 + (wave & 1) * WCOLS;
+      if constexpr (FORM != kFormDown) {
+        bf16_t* o = out_act + static_cast<int64_t>(pair[j]) * N;
+#pragma unroll
+        for (int i = 0; i < WCOLS / 16; i += 2) {
+          const int nc = c0 + i * 16 + 8 * g;
+          if (nc >= N) continue;                                                 // N is a multiple of 64
+          union {
+            bf16_t h[8];
+            uint4 v;
+          } res;
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              if (!GATED) {
+                const float p = fmaxf(pw * acc[i + q][j][v], 0.f);
+                res.h[4 * q + v] = float_to_bf16(p * p);
+                continue;
+              }
+              const float gg = fminf(pw * acc[i + q][j][v], limit);
+              const float uu = fminf(fmaxf(pw * acc[(i + q + 4) % 8][j][v], -limit), limit);
+              res.h[4 * q + v] = float_to_bf16(gg / (1.f + __expf(-gate_alpha * gg)) * (uu + up_shift));
+            }
+          *reinterpret_cast<uint4*>(o + nc) = res.v;
+          __builtin_amdgcn_sched_barrier(0);                                     // a few sums at a time leave the accumulator registers
+        }
+      } else {
+        const int64_t row = into_stream ? pair[j] / top : static_cast<int64_t>(pair[j] % top) * tokens + pair[j] / top;
+        float* o = out_f32 + row * N;
+#pragma unroll
+        for (int i = 0; i < WCOLS / 16; ++i) {
+          const int nc = c0 + i * 16 + 4 * g;
+          if (nc >= N) continue;
+          const tile_f32x4 y = {pw * acc[i][j][0], pw * acc[i][j][1], pw * acc[i][j][2], pw * acc[i][j][3]};
+          if (!into_stream) {
+            *reinterpret_cast<tile_f32x4*>(o + nc) = y;
+          } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) add_float(o + nc + v, (col_scale != nullptr ? col_scale[nc + v] : 1.f) * y[v]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    return has_next;
+  }
+};
+
+template <int FORM>
+__global__ __launch_bounds__(kWideThreads, 1) void moe_wide_kernel(
+    const bf16_t* __restrict__ a, const float* __restrict__ pair_weight, const bf16_t* __restrict__ w,
+    const int32_t* __restrict__ sorted, const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_first,
+    const int32_t* __restrict__ tile_count, const int32_t* __restrict__ n_tiles, bf16_t* __restrict__ out_act,
+    float* __restrict__ out_f32, int64_t tokens, int K, int N, int top, float gate_alpha, float limit, float up_shift,
+    int into_stream, const float* __restrict__ col_scale, int identity_to, const bf16_t* __restrict__ x,
+    const float* __restrict__ weight, int column_tiles) {
+  extern __shared__ __align__(16) unsigned char wide_smem[];
+  const int64_t work = static_cast<int64_t>(*n_tiles) * column_tiles;
+  const int die = static_cast<int>(blockIdx.x & 7);
+  ExpertTiles<FORM> tiles;
+  tiles.pair_weight = pair_weight, tiles.matrices = w, tiles.sorted = sorted, tiles.tile_expert = tile_expert, tiles.tile_first = tile_first;
+  tiles.tile_count = tile_count, tiles.out_act = out_act, tiles.out_f32 = out_f32, tiles.col_scale = col_scale, tiles.tokens = tokens;
+  tiles.K = K, tiles.N = N, tiles.top = top, tiles.into_stream = into_stream, tiles.column_tiles = column_tiles;
+  tiles.from = static_cast<int>(work * die / 8), tiles.to = static_cast<int>(work * (die + 1) / 8), tiles.at_once = static_cast<int>(gridDim.x >> 3);
+  tiles.gate_alpha = gate_alpha, tiles.limit = limit, tiles.up_shift = up_shift;
+  tiles.start();
+  wide_tiles(tiles, reinterpret_cast<const char*>(a), wide_smem, K / 64);
+  if (FORM == kFormDown && identity_to != 0)
+    copy_identity(sorted, tile_first[*n_tiles], identity_to, x, weight, out_f32, tokens, N, top, into_stream, col_scale);
 }
 
 // What the experts' two products have in common.
@@ -1157,10 +1310,10 @@ static int launch_stream(hipStream_t s, const ExpertCall& c, const int32_t* ints
   return launch_stream_form<kFormDown>(s, c, ints, max_tiles);
 }
 
-template <int TM, int TN, int WM, int WN, int FORM>
+template <int FORM>
 static int run_tiles(hipStream_t s, const ExpertCall& c, const int32_t* ints, int max_tiles) {
-  constexpr size_t kSmem = tile_smem_steps(TM, TN) + TM * sizeof(int32_t);
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(moe_tile_kernel<TM, TN, WM, WN, FORM>), hipFuncAttributeMaxDynamicSharedMemorySize,
+  constexpr size_t kSmem = kSmallSmem + kSmallTile * sizeof(int32_t);
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(moe_tile_kernel<FORM>), hipFuncAttributeMaxDynamicSharedMemorySize,
                           static_cast<int>(kSmem)) != hipSuccess)
     return fail("psamd_moe_experts_grouped: " + std::to_string(kSmem) + " bytes of LDS were refused");
   const int32_t* sorted = ints;
@@ -1169,11 +1322,9 @@ static int run_tiles(hipStream_t s, const ExpertCall& c, const int32_t* ints, in
   const int32_t* t_c = t_f + max_tiles;
   constexpr bool down = FORM == kFormDown;
   const int N = down ? c.K : c.F, K = down ? c.F : c.K;
-  const int column_tiles = static_cast<int>(ceil_div(N, FORM == kFormGated ? TN / 2 : TN));
-  // Of the large tiles one workgroup fills a compute unit: as many as there are units walk the tiles. The small ones come one each.
-  const int64_t most = 8 * ceil_div(static_cast<int64_t>(max_tiles) * column_tiles, 8);
-  const dim3 grid(static_cast<unsigned>(TM == 256 ? std::min<int64_t>(most, 256) : most));
-  moe_tile_kernel<TM, TN, WM, WN, FORM><<<grid, dim3(64 * WM * WN), kSmem, s>>>(
+  const int column_tiles = static_cast<int>(ceil_div(N, FORM == kFormGated ? kSmallTile / 2 : kSmallTile));
+  const dim3 grid(static_cast<unsigned>(8 * ceil_div(static_cast<int64_t>(max_tiles) * column_tiles, 8)));
+  moe_tile_kernel<FORM><<<grid, dim3(256), kSmem, s>>>(
       static_cast<const bf16_t*>(down ? c.act : c.x), (c.weight_on_output != 0) == down ? c.weight : nullptr,
       static_cast<const bf16_t*>(down ? c.w_down : c.w_in), sorted, t_e, t_f, t_c, t_c + max_tiles,
       down ? nullptr : static_cast<bf16_t*>(c.act), down ? c.out : nullptr, c.tokens, K, N, c.top, c.gate_alpha, c.limit,
@@ -1182,12 +1333,32 @@ static int run_tiles(hipStream_t s, const ExpertCall& c, const int32_t* ints, in
   return check_launch("psamd_moe_experts_grouped (tiles)");
 }
 
-template <int TM, int TN, int WM, int WN>
 static int launch_tiles(hipStream_t s, const ExpertCall& c, const int32_t* ints, int max_tiles) {
-  if (c.kind == kExpertGated ? run_tiles<TM, TN, WM, WN, kFormGated>(s, c, ints, max_tiles)
-                             : run_tiles<TM, TN, WM, WN, kFormSquaredRelu>(s, c, ints, max_tiles))
-    return 1;
-  return run_tiles<TM, TN, WM, WN, kFormDown>(s, c, ints, max_tiles);
+  if (c.kind == kExpertGated ? run_tiles<kFormGated>(s, c, ints, max_tiles) : run_tiles<kFormSquaredRelu>(s, c, ints, max_tiles)) return 1;
+  return run_tiles<kFormDown>(s, c, ints, max_tiles);
+}
+
+template <int FORM>
+static int run_wide(hipStream_t s, const ExpertCall& c, const int32_t* ints, int max_tiles) {
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(moe_wide_kernel<FORM>), hipFuncAttributeMaxDynamicSharedMemorySize, kWideSmem) != hipSuccess)
+    return fail("psamd_moe_experts_grouped: " + std::to_string(kWideSmem) + " bytes of LDS were refused");
+  const int32_t* t_e = ints + c.tokens * c.top;
+  constexpr bool down = FORM == kFormDown;
+  const int N = down ? c.K : c.F, K = down ? c.F : c.K;
+  const int column_tiles = static_cast<int>(ceil_div(N, FORM == kFormGated ? kWideTile / 2 : kWideTile));
+  const dim3 grid(static_cast<unsigned>(std::min<int64_t>(8 * ceil_div(static_cast<int64_t>(max_tiles) * column_tiles, 8), 256)));
+  moe_wide_kernel<FORM><<<grid, dim3(kWideThreads), kWideSmem, s>>>(
+      static_cast<const bf16_t*>(down ? c.act : c.x), (c.weight_on_output != 0) == down ? c.weight : nullptr,
+      static_cast<const bf16_t*>(down ? c.w_down : c.w_in), ints, t_e, t_e + max_tiles, t_e + 2 * max_tiles, t_e + 3 * max_tiles,
+      down ? nullptr : static_cast<bf16_t*>(c.act), down ? c.out : nullptr, c.tokens, K, N, c.top, c.gate_alpha, c.limit,
+      c.up_shift, c.into_stream, c.col_scale, c.identity > 0 ? static_cast<int>(c.tokens * c.top) : 0,
+      static_cast<const bf16_t*>(c.x), c.weight, column_tiles);
+  return check_launch("psamd_moe_experts_grouped (large tiles)");
+}
+
+static int launch_wide(hipStream_t s, const ExpertCall& c, const int32_t* ints, int max_tiles) {
+  if (c.kind == kExpertGated ? run_wide<kFormGated>(s, c, ints, max_tiles) : run_wide<kFormSquaredRelu>(s, c, ints, max_tiles)) return 1;
+  return run_wide<kFormDown>(s, c, ints, max_tiles);
 }
 
 // Whether the tiles of the kernel for many pairs take these experts: whole steps of 64 k in both products, and offsets inside
@@ -1235,6 +1406,7 @@ static int wide_tile_rows(int64_t pairs, int experts, int K, int F, int kind) {
     };
     return of(ceil_div(F, kind == kExpertGated ? rows / 2 : rows)) * (K + beside) + of(ceil_div(K, rows)) * (F + beside);
   };
+  if (std::min(K, F) < 64 * kWideMinSteps) return 128;
   return 1.2 * rounds(256, 256, 300) < rounds(128, 512, 0) ? 256 : 128;
 }
 
@@ -1408,8 +1580,8 @@ int psamd_moe_experts_grouped(void* stream, const void* x, const int32_t* chosen
   }
   const ExpertCall c{x, chosen, weight, w_in, w_down, act, out, tokens, K, F, experts, identity, top, kind,
                      gate_alpha, limit, up_shift, weight_on_output, into_stream, col_scale};
-  if (wide == 256) return launch_tiles<256, 256, 2, 4>(s, c, ints, max_tiles);
-  if (wide == 128) return launch_tiles<128, 128, 2, 2>(s, c, ints, max_tiles);
+  if (wide == 256) return launch_wide(s, c, ints, max_tiles);
+  if (wide == 128) return launch_tiles(s, c, ints, max_tiles);
   if (rows == 128) return launch_grouped<8, 2>(s, c, ints, max_tiles);
   if (rows == 64) return launch_grouped<4, 2>(s, c, ints, max_tiles);
   if (tiles_take(tokens, pairs, K, F)) return launch_stream(s, c, ints, max_tiles);
