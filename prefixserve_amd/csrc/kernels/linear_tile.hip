@@ -2,10 +2,13 @@
 // activation of a gated feed-forward, the rotation and the pages of a q/k/v projection, the sum into the float32 residual stream,
 // or K-slices that the norm behind it adds up. tile_product.h has the loop.
 
+#include <algorithm>
+
 #include "api.h"
 #include "common.h"
 #include "linear_stream.h"
 #include "tile_product.h"
+#include "wide_tile.h"
 
 namespace psamd {
 namespace {
@@ -125,6 +128,115 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void linear_tile_kernel(const bf
   }
 }
 
+// The largest tiles (256 x 256; wide_tile.h has the loop): workgroups of four waves that walk their die's stretch of the tiles.
+// ACT: the activation of the gated form (asked for number by number, it took 12 us a tile).
+template <int FORM, int ACT>
+struct DenseTiles {
+  void* __restrict__ out;
+  int M, N, K, row_tiles, to, at_once;
+  const char* w;
+  int cur, next_a, next_w, lane, wave;                 // tiles: multiplied, copied next
+
+  static constexpr int WROWS = kWideTile / 2, WCOLS = FORM == kTileGated ? WROWS / 2 : WROWS, COLS = 2 * WCOLS;
+  // (What follows from the lane alone would be computed in front of all tiles and held through them, where no register is free.)
+  __device__ __forceinline__ int own_lane() const {
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    return l;
+  }
+  __device__ __forceinline__ bool a_rows(uint32_t (&off)[8]) {
+    if (next_a >= to) return false;
+    const int lane = own_lane(), m0 = next_a % row_tiles * kWideTile;
+    next_a += at_once;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      off[i] = wide_row(min(m0 + 64 * wave + 8 * i + (lane >> 3), M - 1), K) + wide_piece(8 * i + (lane >> 3), lane);
+    return true;
+  }
+  // GATED: a lane's four columns of two neighbouring tiles of 16 stand side by side, 16 bytes of the output.
+  __device__ __forceinline__ bool w_rows(uint32_t (&off)[8]) {
+    if (next_w >= to) return false;
+    const int lane = own_lane(), n0 = next_w / row_tiles * COLS;
+    next_w += at_once;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int row = (wave * 8 + i) * 8 + (lane >> 3), in = row % WCOLS;
+      const int c = FORM == kTileGated ? (in & ~31) + (in >> 2 & 3) * 8 + (in >> 4 & 1) * 4 + (in & 3) : in;
+      const int col = min(n0 + row / WROWS * WCOLS + c, N - 1);
+      off[i] = wide_row(FORM == kTileGated && row % WROWS >= WCOLS ? N + col : col, K) + wide_piece(8 * i + (lane >> 3), lane);
+    }
+    return true;
+  }
+  __device__ __forceinline__ int rows() const { return min(kWideTile, M - cur % row_tiles * kWideTile); }
+  __device__ __forceinline__ void ahead() {}
+  template <int RM>
+  __device__ __forceinline__ bool finish(tile_f32x4 (&acc)[8][RM]) {
+    const int lane = own_lane(), r = lane & 15, g = lane >> 4;
+    const int c0 = cur / row_tiles * COLS + (wave & 1) * WCOLS, m0 = cur % row_tiles * kWideTile + (wave >> 1) * (16 * RM) + r;
+#pragma unroll
+    for (int j = 0; j < RM; ++j) {
+      const int m = m0 + 16 * j;
+      if (m >= M) continue;
+#pragma unroll
+      for (int i = 0; i < WCOLS / 16; i += FORM == kTileGated ? 2 : 1) {
+        const int n = c0 + 16 * i + (FORM == kTileGated ? 8 : 4) * g;
+        if (n >= N) continue;                          // N is a multiple of 16
+        if constexpr (FORM == kTileGated) {
+          union {
+            bf16_t h[8];
+            uint4 v;
+          } res;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float gate = bf16_to_float(float_to_bf16(acc[i + e / 4][j][e % 4])), up = bf16_to_float(float_to_bf16(acc[(i + e / 4 + 4) % 8][j][e % 4]));
+            res.h[e] = float_to_bf16(gate_act(gate, ACT) * up);
+          }
+          *reinterpret_cast<uint4*>(static_cast<bf16_t*>(out) + static_cast<int64_t>(m) * N + n) = res.v;
+        } else {
+          *reinterpret_cast<tile_f32x4*>(static_cast<float*>(out) + (static_cast<int64_t>(blockIdx.y) * M + m) * N + n) = acc[i][j];
+        }
+        __builtin_amdgcn_sched_barrier(0);             // a few sums at a time leave the accumulator registers
+      }
+    }
+    cur += at_once;
+    return cur < to;
+  }
+};
+
+template <int FORM, int ACT>
+__global__ __launch_bounds__(kWideThreads, 1) void linear_wide_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                                      void* __restrict__ out, int M, int N, int K, int slice_steps,
+                                                                      int row_tiles, int col_tiles) {
+  extern __shared__ __align__(16) unsigned char linear_wide_smem[];
+  const int tiles = row_tiles * col_tiles, per_die = (tiles + 7) / 8, die = static_cast<int>(blockIdx.x & 7);
+  const int64_t first = static_cast<int64_t>(blockIdx.y) * slice_steps;
+  DenseTiles<FORM, ACT> work;
+  work.out = out, work.M = M, work.N = N, work.K = K, work.row_tiles = row_tiles;
+  work.to = min((die + 1) * per_die, tiles), work.at_once = static_cast<int>(gridDim.x >> 3);
+  work.cur = work.next_a = work.next_w = die * per_die + static_cast<int>(blockIdx.x >> 3);
+  work.lane = threadIdx.x & 63, work.wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  work.w = reinterpret_cast<const char*>(w) + first * 128;
+  wide_tiles(work, reinterpret_cast<const char*>(x) + first * 128, linear_wide_smem, min(slice_steps, K / 64 - static_cast<int>(first)));
+}
+
+template <int FORM, int ACT>
+int launch_wide(hipStream_t s, const void* x, const void* w, void* out, int M, int N, int K, int ksplit) {
+  auto kernel = linear_wide_kernel<FORM, ACT>;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kWideSmem) != hipSuccess)
+    return fail("linear_tile: " + std::to_string(kWideSmem) + " bytes of LDS were refused");
+  const int row_tiles = static_cast<int>(ceil_div(M, kWideTile)), col_tiles = static_cast<int>(ceil_div(N, FORM == kTileGated ? kWideTile / 2 : kWideTile));
+  const int64_t most = 8 * ceil_div(static_cast<int64_t>(row_tiles) * col_tiles, 8), stay = std::max<int64_t>(8, 256 / ksplit / 8 * 8);
+  kernel<<<dim3(static_cast<unsigned>(std::min(most, stay)), static_cast<unsigned>(ksplit)), dim3(kWideThreads), kWideSmem, s>>>(
+      static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), out, M, N, K, static_cast<int>(ceil_div(K / 64, ksplit)), row_tiles, col_tiles);
+  return check_launch("linear_tile");
+}
+
+// The largest tiles come with two steps of k or more in every slice.
+bool wide_takes(int K, int ksplit) {
+  const int64_t steps = ceil_div(K / 64, ksplit);
+  return K / 64 - (ksplit - 1) * steps >= 2;
+}
+
 template <int TM, int TN, int WM, int WN, int STAGES, int OCC, int FORM>
 int launch_tile(hipStream_t s, const void* x, const void* w, void* out, int M, int N, int K, int ksplit, int act, const QkvOut& q) {
   constexpr size_t smem = static_cast<size_t>(STAGES) * (TM + TN) * 128;
@@ -150,7 +262,14 @@ template <int FORM>
 int launch_form(hipStream_t s, int shape, const void* x, const void* w, void* out, int M, int N, int K, int ksplit, int act,
                 const QkvOut& q = {}) {
   if constexpr (tile_shape_built(FORM, 0)) {
-    if (shape == 0) return launch_tile<256, 256, 2, 4, 2, 2, FORM>(s, x, w, out, M, N, K, ksplit, act, q);
+    if (shape == 0 && !wide_takes(K, ksplit)) shape = 3;       // the same sums
+    if (shape == 0) {
+      if constexpr (FORM == kTileGated) {
+        if (act == 1) return launch_wide<FORM, 1>(s, x, w, out, M, N, K, ksplit);
+        if (act == 2) return launch_wide<FORM, 2>(s, x, w, out, M, N, K, ksplit);
+      }
+      return launch_wide<FORM, 0>(s, x, w, out, M, N, K, ksplit);
+    }
     if (shape == 1) return launch_tile<192, 128, 2, 2, 2, 2, FORM>(s, x, w, out, M, N, K, ksplit, act, q);
     if (shape == 2) return launch_tile<192, 128, 2, 4, 3, 2, FORM>(s, x, w, out, M, N, K, ksplit, act, q);
   }
@@ -169,7 +288,7 @@ struct TileShape {
   double step, half_step, round, weights, reads, start;
 };
 constexpr TileShape kTileShapes[kTileShapeCount] = {
-    {256, 256, 1, 1.323, 0.0, 6.47, 0.003, 0.027, 0.73},      // asks for the fewest bytes a product
+    {256, 256, 1, 0.956, 0.0, 4.21, 0.0, 0.0355, 3.66},       // asks for the fewest bytes a product; four waves that walk its tiles
     {192, 128, 2, 1.127, 0.841, 0.27, 0.032, 0.023, 5.06},    // two on a unit: one's loop beside the other's beginning and end
     {192, 128, 1, 0.627, 0.0, 2.71, 0.023, 0.027, 2.78},      // three steps under way, for one round
     {128, 128, 1, 0.469, 0.0, 2.24, 0.011, 0.028, 2.91},      // four
@@ -205,13 +324,16 @@ struct TilePlan {
 //   q/k/v 3,072 x 2,048           16.4 (18.9)  17.5 (19.6)  19.3 (20.1)  21.7 > 20.3  22.4 > 21.1  28.4 (24.7)  30.8 (26.9)  33.4 (43.2)   38.6 (51.3)
 //   q/k/v 6,144 x 4,096           43.3 (33.3)  46.6 > 35.1  42.7 (38.8)  47.7 (44.6)  49.4 > 45.8  59.9 (81.0)  63.7 (86.2)  91.3 (127)    99.6 (138)
 //   gated 2 x 1,024 x 2,048       14.9 (17.3)  15.0 (17.9)  16.0 (17.9)  18.4 (17.5)  18.7 (18.0)  20.1 > 17.9  21.2 > 18.7  26.4 (23.1)   28.6 > 24.4
-//   gated 2 x 8,192 x 2,048       30.4 > 23.5  33.8 > 26.2  36.5 > 32.5  47.3 (50.8)  48.5 (52.3)  63.7 > 62.1  66.3 > 63.2  107 (109)     128 (133)
+//   gated 2 x 8,192 x 2,048       30.4 > 23.5  33.8 > 26.2  36.5 > 32.5  46.9 > 44.6  48.2 > 46.9  63.4 > 55.1  66.7 > 57.0  103 > 99.6    121 > 110
 //   gated 2 x 14,336 x 4,096      63.0 (61.2)  76.4 (92.3)  93.1 (105)   157 (155)    162 (187)    216 (227)    224 (229)    315 (336)     406 (436)
 //   with the norm 2,048 x 2,048   15.2 > 12.4  15.5 > 14.7  16.9 (17.2)  19.1 (19.6)  20.1 (20.2)  22.7 (22.7)  24.0 (23.7)
 //   2,048 x 8,192                 30.4 > 20.0  31.7 > 23.5  38.3 > 28.6  49.0 > 37.1  49.9 > 39.0  55.5 > 48.8  59.6 > 53.6  69.2 (82.9)   83.3 (93.6)
 //   4,096 x 4,096                 26.8 > 21.6  27.9 > 24.5  31.7 > 29.9  43.6 (40.9)  44.4 > 41.7  48.9 (50.0)  53.3 > 51.4  65.3 (67.1)   78.1 (102)
 //   4,096 x 14,336                62.5 > 38.5  68.4 > 51.2  86.5 > 61.6  122 > 98.6   127 > 102    140 > 124    152 > 130    192 (197)     236 (301)
-// (From 1,024 tokens on the tiles add into the stream.) In bfloat16 for the other norms the tiles had no lead: 2,048 x 2,048 15.1 / 19.0 at
+// (From 1,024 tokens on the tiles add into the stream.) With four waves of 128 x 128 in the largest shape instead of eight of 128 x 64 that began each tile
+// anew (both sides on one card): gated 2 x 8,192 x 2,048 at 2,048 tokens 122 by the library and the activation -> 110, 2 x 4,096 x 2,048 63 -> 56 (at 1,531
+// 52 -> 48), 2 x 2,816 x 1,024 43 -> 29, 2 x 8,192 x 3,072 172 -> 153; with the norm 4,096 x 14,336 at 767 tokens 105 -> 97, 4,096 x 11,008 at 640 81 -> 73. 2 x 14,336 x
+// 4,096 would gain 5 to 10% from 900 tokens on (385 -> 363 at 2,048) and lose as much at 535 and 640: left to the library. In bfloat16 for the other norms the tiles had no lead: 2,048 x 2,048 15.1 / 19.0 at
 // 130 tokens, 19.3 / 21.1 at 535, 34.8 / 34.9 at 2,048; such products are the library's.
 TilePlan tile_plan(int form, int M, int N, int K) {
   const bool stream = form == kTileSlices || form == kTileAdd;
@@ -229,6 +351,7 @@ TilePlan tile_plan(int form, int M, int N, int K) {
       if (slices > 1 && (!stream || K / 64 < 2 * slices || static_cast<int64_t>(slices) * M > kMostSliceRows)) break;
       const int64_t steps = ceil_div(K / 64, slices);
       if (ceil_div(K / 64, steps) != slices || !tile_shape_built(stream && slices == 1 ? kTileAdd : form, shape)) continue;
+      if (shape == 0 && !wide_takes(K, slices)) continue;
       const int64_t row_tiles = ceil_div(M, t.rows), groups = row_tiles * ceil_div(rows, t.cols) * slices, at_once = 256 * t.at_once;
       const int64_t left = groups % at_once;
       const bool half = t.at_once == 2 && left > 0 && left <= 256;

@@ -1,5 +1,6 @@
 // The loop of the bfloat16 products whose operands both pass through LDS in large tiles: a workgroup's tile of A [rows, K] times
-// its tile of W [rows, K]^T, 64 k at a time, for the experts with many pairs (moe.hip) and the dense products (linear_tile.hip).
+// its tile of W [rows, K]^T, 64 k at a time, for the experts with many pairs (moe.hip) and the dense products (linear_tile.hip). (Tiles of
+// 256 x 256: wide_tile.h.)
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -28,7 +29,7 @@ __device__ __forceinline__ int tile_copy_piece(int row, int lane) { return (lane
 // a_off[i] bytes behind `a` in k step 0 and goes to row 8 (wave LA + i) (w likewise). Every wave of the workgroup comes here with
 // the same `steps` (>= 1); where `works` is false (uniform for the wave) it only copies. What bounds it and what it does about it:
 //  * the latency of memory: STAGES - 1 steps are under way behind the one that is multiplied;
-//  * LDS, whose reads and writes take as long as the matrix instructions at 256 x 256 a workgroup and 128 x 64 a wave: the operands
+//  * LDS, whose reads and writes take as long as the matrix instructions at 192 x 128 a workgroup: the operands
 //    of half a step are read between the matrix instructions of the half before, and the one barrier of a step stands
 //    between its halves, where the matrix cores still have work; waves in their matrix instructions go first.
 // On return nothing is under way and LDS may still be read by other waves.
