@@ -22,6 +22,7 @@
 
 #include "api.h"
 #include "common.h"
+#include "tile_product.h"
 
 namespace psamd {
 
@@ -707,6 +708,7 @@ __global__ __launch_bounds__(256) void attn_masked_mfma_kernel(
 
 // ------------------------------------------------------------------ prefill, query heads of a kv head together
 
+// (Head sizes 64, 128 and 256 have the kernel behind this one.)
 // The same 32 queries for up to 4 query heads that share a kv head: one head per wave, all
 // keys, no merge. The 32-key tile of K and of V^T is brought into LDS ONCE per workgroup
 // (16-byte loads, whole contiguous pages) and read from there by the 4 waves: the texture
@@ -1019,6 +1021,392 @@ __global__ __launch_bounds__(256 * KP, NS <= 4 ? 4 : 2) void attn_prefill_groupe
       iteration(ra);
       iteration(rb);
     } while (k0 <= k_last);
+  }
+
+  if (KP > 1) {
+    // Merge the KP runs of keys by log-sum-exp; the K/V stages are free now.
+    constexpr int O_FLOATS = DT * 16 * 64;
+    float* mg = reinterpret_cast<float*>(smem_raw);
+    __syncthreads();
+    if (part > 0) {
+      float* dst = mg + ((part - 1) * 4 + (wave & 3)) * (O_FLOATS + 64);
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) dst[(dt * 16 + v) * 64 + lane] = o[dt][v];
+      if (hi == 0) {
+        dst[O_FLOATS + col] = m;
+        dst[O_FLOATS + 32 + col] = l;
+      }
+    }
+    __syncthreads();
+    if (part == 0) {
+    float mm = m;
+#pragma unroll
+    for (int p = 1; p < KP; ++p) mm = fmaxf(mm, mg[((p - 1) * 4 + wave) * (O_FLOATS + 64) + O_FLOATS + col]);
+    const float f0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mm);
+    l *= f0;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) o[dt][v] *= f0;
+#pragma unroll
+    for (int p = 1; p < KP; ++p) {
+      const float* src = mg + ((p - 1) * 4 + wave) * (O_FLOATS + 64);
+      const float mp = src[O_FLOATS + col];
+      const float f = mp == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mp - mm);
+      l += f * src[O_FLOATS + 32 + col];
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[dt][v] += f * src[(dt * 16 + v) * 64 + lane];
+    }
+    m = mm;
+    }
+  }
+  if (part != 0 || !head_valid || !q_valid) return;
+  if (nsplit > 1) {
+    // m is in units of the base-2 exponent; a query with no key in this run has m = -inf, l = 0.
+    if (hi == 0) {
+      part_ml[2 * part_slot] = m;
+      part_ml[2 * part_slot + 1] = l;
+    }
+    float* po = part_o + part_slot * D;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int v4 = 0; v4 < 4; ++v4) {
+        const int d = 32 * dt + 8 * v4 + 4 * hi;
+        if (d < D)
+          *reinterpret_cast<float4*>(po + d) =
+              float4{o[dt][4 * v4 + 0], o[dt][4 * v4 + 1], o[dt][4 * v4 + 2], o[dt][4 * v4 + 3]};
+      }
+    return;
+  }
+  if (ex.sink != nullptr) l += __builtin_amdgcn_exp2f(ex.sink[h] * kLog2e - m);
+  const float inv = 1.f / l;
+  bf16_t* op = out + static_cast<int64_t>(t0 + qi) * (static_cast<int64_t>(hq) * D) + h * D;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int v4 = 0; v4 < 4; ++v4) {
+      const int d = 32 * dt + 8 * v4 + 4 * hi;
+      if (d < D) {
+        float4 f = {inv, inv, inv, inv};
+        if (ex.gate != nullptr) {
+          const float4 gt = gate4(ex, t0 + qi, h * D + d);
+          f = float4{inv * gt.x, inv * gt.y, inv * gt.z, inv * gt.w};
+        }
+        ushort4 pk;
+        pk.x = float_to_bf16(o[dt][4 * v4 + 0] * f.x);
+        pk.y = float_to_bf16(o[dt][4 * v4 + 1] * f.y);
+        pk.z = float_to_bf16(o[dt][4 * v4 + 2] * f.z);
+        pk.w = float_to_bf16(o[dt][4 * v4 + 3] * f.w);
+        *reinterpret_cast<ushort4*>(op + d) = pk;
+      }
+    }
+}
+
+// The same with the keys and values copied to LDS past the registers, for head sizes 64, 128 and 256 (whole copies of 1,024 bytes a wave, a
+// power of two of pieces a key row). The kernel above had registers for one operand at a time there (a wait for LDS in front of every score
+// product), spilled others (with three-term weights a reload from scratch in every iteration, and with it a wait for all loads
+// under way) and stood in front of each barrier for a page lookup. Here no piece passes through registers, up to four stages are under
+// way, a page's number is asked for an iteration ahead by the scalar unit, and the two halves of a wave exchange maxima and sums by an
+// instruction of their own. The order of all sums is that of the kernel above, and so are the bits.
+// us a layer, above -> here: 2,048 tokens of 32 heads on 8 at head size 64 43 -> 38, with three-term weights 69 -> 54, 1,531 with a window of 1,024 57 -> 46;
+// at head size 128 2,048 tokens 67 -> 57, as many behind 2,048 156 -> 126; 1,500 tokens of 16 heads on one at 256, three terms, 204 -> 124.
+// What bounds it at head size 64: the vector unit is at work 37 of 91 thousand cycles, the matrix cores 17; a unit holds 2.2 waves a SIMD on the
+// average, as the longest tile's workgroup, 32 iterations, is alone in the end, its waves all in the same phase between two barriers. No gain: a barrier
+// for two iterations (37.7 / 36.9), sixteen waves a workgroup (42), other pairs of tiles (39 to 45).
+constexpr int copied_stage_bytes(int D, int kp) { return 2 * 32 * kp * 2 * D; }
+constexpr int copied_stages(int D, int kp) { return std::min(4, (D <= 64 || kp == 1 ? 65536 : 131072) / copied_stage_bytes(D, kp)); }
+// Which piece of a key row lies in its first 16 bytes: the rows that a read touches then lie on all banks.
+__device__ __forceinline__ int copied_swap(int D, int row) { return D == 64 ? (row >> 1) & 7 : row & 15; }
+__device__ __forceinline__ float other_half_max(float v) {
+  const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+}
+__device__ __forceinline__ float other_half_sum(float v) {
+  const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(both[0]) + __uint_as_float(both[1]);
+}
+
+template <int NS, int KP, bool P3>
+__global__ __launch_bounds__(256 * KP, NS <= 4 ? 4 : 2) void attn_prefill_copied_kernel(
+    const bf16_t* __restrict__ qkv, int q_stride, bf16_t* __restrict__ out, const bf16_t* __restrict__ kv,
+    const int32_t* __restrict__ pf_tiles, const int32_t* __restrict__ item_start,
+    const int32_t* __restrict__ item_pos0, const int32_t* __restrict__ table_off,
+    const int32_t* __restrict__ block_ids, int n_tiles, int hq, int hkv, float scale,
+    int window, float* __restrict__ part_o, float* __restrict__ part_ml, int pair_tiles, int tiles_per_wg,
+    const int32_t* __restrict__ pf_blocks, int n_blocks, Extras ex) {
+  constexpr int D = 16 * NS;
+  constexpr int DT = (D + 31) / 32;
+  constexpr int KEYS = 32 * KP;                  // keys per iteration
+  constexpr int STAGES = copied_stages(D, KP), STAGE = copied_stage_bytes(D, KP), V_AT = STAGE / 2;
+  constexpr int COPIES = D / 64;                 // of 1,024 bytes a wave brings per iteration, of the keys and of the values each
+  constexpr int ROW = 2 * D, PAGE_BYTES = kPage * ROW, PIECES = ROW / 16;
+  static_assert(NS == 4 || NS == 8 || NS == 16, "whole copies, and a power of two of pieces per key row");
+  extern __shared__ __align__(1024) unsigned char smem_raw[];
+
+  // A workgroup's four head slots (wave & 3) are four query heads of the kv head on one tile of
+  // queries, or, with fewer query heads per kv head, two heads on two consecutive tiles or one
+  // head on four (tiles_per_wg = 1, 2, 4): the keys and values a workgroup stages are then still
+  // used by four waves. Its tiles are those of one item: pf_blocks lists the first tile of every
+  // run of up to four consecutive tiles of an item, and gridDim.y is the number of those runs
+  // times the workgroups that share one (two with two tiles each).
+  const int group = hq / hkv;
+  const int heads_per_wg = 4 / tiles_per_wg;
+  const int wg_per_kv = (group + heads_per_wg - 1) / heads_per_wg;
+  // Grid: x = (kv head, block of 4 query heads), y = tile, the late tiles (which see the most
+  // keys) first. Workgroups are handed out in the order x + gridDim.x * y and go round robin over
+  // the dies: the heaviest tiles of every head start first, so no head's long tiles are left
+  // running alone at the end, and with a multiple of 8 workgroups in x a kv head's tiles all run
+  // on one die, whose L2 then holds that head's keys and values for all of them (a 2,048-token
+  // prompt at head size 64 fetched 20 MB from memory with the tile in x and 7 MB this way).
+  const int kvh = blockIdx.x / wg_per_kv;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int part = wave >> 2;                           // which of the iteration's KP runs of keys
+  const int slot = wave & 3;
+  const int head_in_group = (blockIdx.x - kvh * wg_per_kv) * heads_per_wg + slot % heads_per_wg;
+  const int tile_in_wg = slot / heads_per_wg;
+  bool head_valid = head_in_group < group;             // a spare wave repeats the last head and writes nothing
+  const int h = kvh * group + min(head_in_group, group - 1);
+  // pair_tiles (the whole grid runs at once, two workgroups to a compute unit): the second half
+  // of the workgroups, which join the first half's on their compute units, take the early tiles in
+  // ascending order, so that the longest tile shares its compute unit with the shortest and every
+  // compute unit has about the same number of keys to go through.
+  const int by = static_cast<int>(blockIdx.y), first_half = (n_tiles + 1) >> 1;
+  int wg_tile = (pair_tiles && by >= first_half) ? by - first_half : n_tiles - 1 - by;
+  int wg_q_off_more = 0;
+  if (tiles_per_wg > 1) {
+    const int sub = 4 / tiles_per_wg;                  // workgroups per run of four tiles
+    const int at = n_blocks * sub - 1 - by;            // late tiles first
+    wg_tile = pf_blocks[at / sub] + tiles_per_wg * (at % sub);
+    wg_q_off_more = 32 * tiles_per_wg * (at % sub);
+  }
+  const int item = pf_tiles[2 * (wg_tile - (wg_q_off_more >> 5))];
+  const int wg_q_off = pf_tiles[2 * (wg_tile - (wg_q_off_more >> 5)) + 1] + wg_q_off_more;
+  const int t0 = item_start[item];
+  const int n = item_start[item + 1] - t0;
+  if (wg_q_off >= n) return;                           // the run ends before this workgroup's tiles
+  const int pos0 = item_pos0[item];
+  const int col = lane & 31, hi = lane >> 5;
+
+  // This wave's tile: a block's tiles past the end of the item do not exist, the wave then
+  // repeats the block's first tile and writes nothing.
+  int tile = wg_tile, q_off = wg_q_off;
+  if (tile_in_wg > 0) {
+    if (wg_q_off + 32 * tile_in_wg < n) {
+      tile = wg_tile + tile_in_wg;
+      q_off = wg_q_off + 32 * tile_in_wg;
+    } else {
+      head_valid = false;
+    }
+  }
+  const int qi = min(q_off + col, n - 1);          // lanes past the end repeat the last query
+  const bool q_valid = q_off + col < n;
+  const int q_pos = pos0 + qi;
+  const int first_pos = pos0 + q_off;                          // of this wave's tile
+  const int last_pos = pos0 + min(q_off + 31, n - 1);
+  const int wg_last_pos = pos0 + min(wg_q_off + 32 * tiles_per_wg - 1, n - 1);   // of the block
+  const int k_lo_q = window > 0 ? max(0, q_pos - window + 1) : 0;
+  const int max_key = pos0 + n - 1;
+  const int k_begin_vis = window > 0 ? max(0, pos0 + wg_q_off - window + 1) : 0;   // the first key any query of the block sees
+  const int k_begin = k_begin_vis & ~(KEYS - 1);
+  const float c = scale * 1.44269504088896340736f;  // scores are exponentiated in base 2
+  // With gridDim.z > 1 the tile's keys are dealt out to that many workgroups in runs of whole
+  // pairs of iterations, at least kMinSplitKeys each; every workgroup leaves its sum, its
+  // maximum and its unnormalized output in part_ml / part_o for the merge kernel. A tile with
+  // too few keys for all of them leaves the last ones nothing: they write an empty sum.
+  const int nsplit = gridDim.z;
+  int k_first = k_begin, k_last = wg_last_pos;
+  int64_t part_slot = 0;
+  if (nsplit > 1) {
+    constexpr int PAIR = 2 * KEYS;
+    const int pairs = (wg_last_pos - k_begin) / PAIR + 1;
+    const int per = max((pairs + nsplit - 1) / nsplit, kMinSplitKeys / PAIR);
+    k_first = k_begin + static_cast<int>(blockIdx.z) * per * PAIR;
+    k_last = min(wg_last_pos, k_first + per * PAIR - 1);
+    part_slot = (static_cast<int64_t>(tile * 32 + col) * hq + h) * nsplit + blockIdx.z;
+    if (k_first > wg_last_pos) {
+      if (part == 0 && head_valid && q_valid && hi == 0) {
+        part_ml[2 * part_slot] = -INFINITY;
+        part_ml[2 * part_slot + 1] = 0.f;
+      }
+      return;
+    }
+  }
+  bf16x8 qf[NS];
+  f32x16 o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o[dt][v] = 0.f;
+  float m = -INFINITY, l = 0.f;       // m in base-2 units (score * c)
+
+  const int64_t page_bytes = 2LL * hkv * PAGE_BYTES;
+  const char* kv_head = reinterpret_cast<const char*>(kv) + static_cast<int64_t>(kvh) * PAGE_BYTES;
+  const int64_t to_values = static_cast<int64_t>(hkv) * PAGE_BYTES;
+  const auto* pages = (__attribute__((address_space(4))) const int32_t*)(block_ids + table_off[item]);
+  const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)smem_raw));
+  // This wave's copies lie in page wave / 2 of an iteration. What a lane brings to its 16 bytes of a copy: of a key's pieces
+  // the one that the key's number exchanges with it, of 32 value rows first all halves with keys 0 to 7, then the others.
+  uint32_t k_from[COPIES], v_from[COPIES];
+#pragma unroll
+  for (int i = 0; i < COPIES; ++i) {
+    const int at = ((wave & 1) * COPIES + i) * 1024 + lane * 16;       // in the page's keys, and in its values
+    const int row = at / ROW;
+    k_from[i] = row * ROW + ((at % ROW / 16) ^ copied_swap(D, row)) * 16;
+    v_from[i] = ((wave & 1) * COPIES + i) * 1024 + (lane & 31) * 32 + (lane >> 5) * 16;
+  }
+  auto page_of = [&](int k0) { return pages[min(k0 + kPage * (wave >> 1), wg_last_pos) >> 4]; };
+  auto copy = [&](int page, int stage) {
+    const char* from = kv_head + page * page_bytes;
+    const uint32_t to = base + stage * STAGE + wave * (COPIES * 1024);
+#pragma unroll
+    for (int i = 0; i < COPIES; ++i) copy_to_lds(to + i * 1024, k_from[i], from);
+#pragma unroll
+    for (int i = 0; i < COPIES; ++i) copy_to_lds(to + V_AT + i * 1024, v_from[i], from + to_values);
+  };
+  const uint32_t k_at = base + (32 * part + col) * ROW, k_piece = (hi ^ copied_swap(D, col & 15)) * 16;
+  const uint32_t v_at = base + V_AT + 2 * part * PAGE_BYTES + col * 16 + hi * 8;
+  typedef __attribute__((address_space(3))) const bf16x8 lds_piece;
+  typedef __attribute__((address_space(3))) const bf16x4 lds_half;
+  auto compute = [&](int stage, int k_iter) {
+    const int k0 = k_iter + 32 * part;               // this wave's keys of the iteration
+    if (k0 > last_pos) return;                       // all after the last query (the page lookups were clamped)
+    const uint32_t k_now = k_at + stage * STAGE, v_now = v_at + stage * STAGE;
+    const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    f32x16 s = zero;
+    constexpr int AT_ONCE = NS < 8 ? NS : 8;
+#pragma unroll
+    for (int i0 = 0; i0 < NS; i0 += AT_ONCE) {
+      bf16x8 kf[AT_ONCE];
+#pragma unroll
+      for (int i = 0; i < AT_ONCE; ++i) kf[i] = *reinterpret_cast<lds_piece*>(k_now + (k_piece ^ (32 * (i0 + i))));
+      __builtin_amdgcn_sched_barrier(0);             // all under way at once
+#pragma unroll
+      for (int i = 0; i < AT_ONCE; ++i) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i0 + i], s, 0, 0, 0);
+    }
+    const int key0 = k0 + 4 * hi;                    // register v's key: key0 + 8 (v / 4) + v % 4
+    const bool edge = k0 + 31 > max_key || k0 < k_begin_vis;           // slots nobody of this request wrote
+    auto values = [&](bf16x8 (&vv)[DT], int cpage) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const uint32_t at = v_now + cpage * PAGE_BYTES + dt * 1024;
+        vv[dt] = join(*reinterpret_cast<lds_half*>(at), *reinterpret_cast<lds_half*>(at + 512));
+      }
+    };
+    auto written = [&](bf16x8 (&vv)[DT], int cpage) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        u32x4 words = __builtin_bit_cast(u32x4, vv[dt]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int key = key0 + 16 * cpage + 8 * (e >> 2) + (e & 3);
+          if (key > max_key || key < k_begin_vis) words[e >> 1] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
+        }
+        vv[dt] = __builtin_bit_cast(bf16x8, words);
+      }
+    };
+    constexpr bool BOTH = NS <= 8;                   // both pages' values are asked for ahead of the softmax; no registers for that at 256
+    bf16x8 vv[BOTH ? 2 : 1][DT];
+    if constexpr (BOTH) {
+      values(vv[0], 0);
+      values(vv[1], 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (edge) {
+        written(vv[0], 0);
+        written(vv[1], 1);
+      }
+    }
+    if (ex.bias != nullptr) {
+      const float* bt = ex.bias + static_cast<int64_t>(h) * ex.n_dist;
+      const float unscale = 1.f / scale;
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        s[v] = fmaf(bt[min(max(q_pos - key0 - (8 * (v >> 2) + (v & 3)), 0), ex.n_dist - 1)], unscale, s[v]);
+    }
+    // Keys that are not after the first query, with no window, need no mask.
+    if (window > 0 || k0 + 31 > first_pos) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int key = key0 + 8 * (v >> 2) + (v & 3);
+        s[v] = (key <= q_pos && key >= k_lo_q) ? s[v] : -INFINITY;
+      }
+    }
+    float mx = s[0];
+#pragma unroll
+    for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
+    mx = other_half_max(mx) * c;
+    // The running maximum is only raised (and the accumulators rescaled) when some query's
+    // scores outgrow it by more than 2^8 (see the per-head kernel).
+    if (__any(mx > m + 8.f)) {
+      const float m_new = fmaxf(m, mx);
+      const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[dt][v] *= alpha;
+      m = m_new;
+    }
+    const float m_use = m == -INFINITY ? 0.f : m;
+    float rowsum = 0.f;
+#pragma unroll
+    for (int cpage = 0; cpage < 2; ++cpage) {
+      float p[8];
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        p[v] = __builtin_amdgcn_exp2f(fmaf(s[8 * cpage + v], c, -m_use));
+        rowsum += p[v];
+      }
+      const Weights w = split_weights<P3>(p);
+      if constexpr (!BOTH) {
+        values(vv[0], cpage);
+        if (edge) written(vv[0], cpage);
+      }
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv[BOTH ? cpage : 0][dt], w.hi, o[dt], 0, 0, 0);
+      if (P3) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv[BOTH ? cpage : 0][dt], w.mid, o[dt], 0, 0, 0);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv[BOTH ? cpage : 0][dt], w.lo, o[dt], 0, 0, 0);
+      }
+    }
+    l += other_half_sum(rowsum);
+  };
+
+  {
+    // Every wave brings its copies of every iteration, and of STAGES - 1 behind the last (of clamped pages), so that each wait counts the
+    // same. The page of the copies after the next is looked up an iteration ahead.
+#pragma unroll
+    for (int i = 0; i < STAGES - 1; ++i) copy(page_of(k_first + i * KEYS), i);
+    {
+      const bf16_t* qp = qkv + static_cast<int64_t>(t0 + qi) * q_stride + h * D + 8 * hi;
+#pragma unroll
+      for (int i = 0; i < NS; ++i) qf[i] = ld8(qp + 16 * i);
+    }
+    // Waited for here: the compiler does not count the copies and would wait for all of them in every iteration.
+#pragma unroll
+    for (int i = 0; i < NS; ++i) asm volatile("" : "+v"(qf[i]));
+    int page = page_of(k_first + (STAGES - 1) * KEYS), stage = 0, free_stage = STAGES - 1;
+    for (int k0 = k_first; k0 <= k_last; k0 += KEYS) {
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(wait_for_copies((STAGES - 2) * 2 * COPIES));    // this wave's part of the iteration has arrived,
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();                                              // everybody's; and nobody reads the one before
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      copy(page, free_stage);
+      page = page_of(k0 + STAGES * KEYS);
+      compute(stage, k0);
+      free_stage = stage;
+      stage = stage + 1 == STAGES ? 0 : stage + 1;
+    }
+    __builtin_amdgcn_s_waitcnt(wait_for_copies(0));                              // LDS is not used again, or given back, under a copy
+    asm volatile("" ::: "memory");
   }
 
   if (KP > 1) {
@@ -1730,13 +2118,35 @@ static int launch_prefill(hipStream_t s, const void* qkv, int q_stride, void* ou
       return launch_prefill_merge(s, part_o, part_ml, out, pf_tiles, item_start, n_tiles, hq, 16 * NS, nsplit);   \
     }                                                                                                             \
   }
+#define PSAMD_COPIED(KP_)                                                                                          \
+  {                                                                                                               \
+    constexpr int D = 16 * NS;                                                                                    \
+    const size_t merge = sizeof(float) * (KP_ - 1) * 4 * (((D + 31) / 32) * 16 * 64 + 64);                        \
+    const size_t smem = std::max<size_t>(copied_stages(D, KP_) * copied_stage_bytes(D, KP_), merge);              \
+    if (lds_allowed(attn_prefill_copied_kernel<NS, KP_, P3>, smem)) {                                             \
+      attn_prefill_copied_kernel<NS, KP_, P3><<<grid, dim3(256 * KP_), smem, s>>>(                                \
+          static_cast<const bf16_t*>(qkv), q_stride, static_cast<bf16_t*>(out), static_cast<const bf16_t*>(kv),   \
+          pf_tiles, item_start, item_pos0, table_off, block_ids, n_tiles, hq, hkv, scale, window, part_o,         \
+          part_ml, pair, tiles_per_wg, pf_blocks, n_blocks, g_extras);                                            \
+      const int rc = check_launch("psamd_attention_prefill");                                                     \
+      if (rc != 0 || nsplit == 1) return rc;                                                                      \
+      return launch_prefill_merge(s, part_o, part_ml, out, pf_tiles, item_start, n_tiles, hq, 16 * NS, nsplit);   \
+    }                                                                                                             \
+  }
     // From head size 96 on, where a compute unit holds one workgroup of eight waves, four
     // workgroups per compute unit's worth of tiles run 5% faster as two workgroups of four waves
     // (one wave per head): two barriers' worth of waves that do not wait for each other
     // (head size 128: 4,096 tokens 181 -> 171 us, 8,192 tokens 657 -> 623 us; 2,048 tokens 56 -> 67).
-    if (NS < 6 || wgs * grid.z < 1024) PSAMD_GROUPED(2)
-    PSAMD_GROUPED(1)
+    const bool two_waves = NS < 6 || wgs * grid.z < 1024;
+    if constexpr (NS == 4 || NS == 8 || NS == 16) {
+      if (two_waves) PSAMD_COPIED(2)
+      PSAMD_COPIED(1)
+    } else {
+      if (two_waves) PSAMD_GROUPED(2)
+      PSAMD_GROUPED(1)
+    }
 #undef PSAMD_GROUPED
+#undef PSAMD_COPIED
   }
   attn_prefill_mfma_kernel<NS, P3><<<dim3(hq, n_tiles, nsplit), dim3(256), sizeof(int32_t) * static_cast<size_t>(table_pages), s>>>(
       static_cast<const bf16_t*>(qkv), q_stride, static_cast<bf16_t*>(out), static_cast<const bf16_t*>(kv), pf_tiles,
