@@ -322,9 +322,11 @@ int psamd_qkv_rope_append(void* stream, const void* x, const void* w, void* qkv_
 // M (at most 4,608; 0: never any). The others return 2
 // where the library is to be taken: w of _gated is [gate; up] and activation 0 (silu), 1 (relu) or 2 (gelu, tanh form); _qkv
 // takes what psamd_qkv_rope_append does. _shaped runs one shape of tile whatever the rule says, for tests and measurements:
-// form 0 (K-slices), 1 (added), 2 (gated), 3 (q/k/v), shape 0 to 4 as in the file's table (1 and 3: 3 and 4 alone).
+// form 0 (K-slices), 1 (added), 2 (gated), 3 (q/k/v), shape 0 to 4 as in the file's table (1 and 3: 3 and 4 alone). _plan: what the rule
+// says of a product of that form, 16 x shape + slices, or -1 (the library).
 int psamd_linear_tile_slices(const void* x, const void* w, int M, int n_out, int K);
 int psamd_linear_tile_slice_rows(int n_out, int K);
+int psamd_linear_tile_plan(int form, int M, int n_out, int K, int activation);
 int psamd_linear_tile_stream(void* stream, const void* x, const void* w, float* out, int M, int n_out, int K);
 int psamd_linear_tile_gated(void* stream, const void* x, const void* w, void* out, int M, int n_out, int K, int activation);
 int psamd_linear_tile_qkv(void* stream, const void* x, const void* w, void* qkv_out, int M, int K, int hq, int hkv, int head_dim,

@@ -303,6 +303,13 @@ constexpr TileForm kStreamForm{2.83, 1.517, 6.99, 0.787, 0.145, 2.709, 0.090};  
 constexpr TileForm kGatedForm{0.0, 0.703, 6.27, 0.398, 0.104, 2.620, 0.194};
 constexpr TileForm kQkvForm{0.0, 1.504, 7.37, 0.524, 0.206, 2.026, 0.132};
 
+// What a round of the largest tiles takes longer with GELU than with SiLU, for which the table holds: its activations run with no matrix
+// instruction beside them (7.3 to 10.5 us over 48 products; ReLU takes 3 less than SiLU), less what the activation kernel behind the library's
+// product takes longer too. Anything from 5.5 to 7.5 decides alike over those products. Without it, gated products with GELU ran in these tiles where
+// something else is the faster (us, the largest tiles / what runs now): 2 x 8,192 x 2,048 at 640 tokens 54.9 / 47.0, 2 x 6,144 x 1,024 at 640 37.2 /
+// 26.8, 2 x 2,816 x 1,024 at 2,048 35.6 / 31.4, 2 x 8,192 x 2,048 at 4,096 235 / 223; 2 x 8,192 x 3,072 at 900 keeps them, 81 / 97.
+constexpr double kWideGelu = 6.5;
+
 constexpr int kTileMinTokens = 129;         // fewer: linear_stream.hip
 constexpr int kStreamMaxTokens = 1023;      // above, the library's product adds into the stream itself: tiles 0.97 to 1.32 of its time
 constexpr int64_t kStreamMaxNumbers = 4200000;   // tokens x columns, and columns: above, the library has work for the whole chip without
@@ -335,7 +342,7 @@ struct TilePlan {
 // 52 -> 48), 2 x 2,816 x 1,024 43 -> 29, 2 x 8,192 x 3,072 172 -> 153; with the norm 4,096 x 14,336 at 767 tokens 105 -> 97, 4,096 x 11,008 at 640 81 -> 73. 2 x 14,336 x
 // 4,096 would gain 5 to 10% from 900 tokens on (385 -> 363 at 2,048) and lose as much at 535 and 640: left to the library. In bfloat16 for the other norms the tiles had no lead: 2,048 x 2,048 15.1 / 19.0 at
 // 130 tokens, 19.3 / 21.1 at 535, 34.8 / 34.9 at 2,048; such products are the library's.
-TilePlan tile_plan(int form, int M, int N, int K) {
+TilePlan tile_plan(int form, int M, int N, int K, int act = 0) {
   const bool stream = form == kTileSlices || form == kTileAdd;
   const int64_t rows = form == kTileGated ? 2LL * N : N;
   if (stream && (M > kStreamMaxTokens || N > kStreamMaxColumns || static_cast<int64_t>(M) * N > kStreamMaxNumbers)) return TilePlan{};
@@ -357,7 +364,8 @@ TilePlan tile_plan(int form, int M, int N, int K) {
       const bool half = t.at_once == 2 && left > 0 && left <= 256;
       const double full = static_cast<double>(groups / at_once + (left > 0 && !half ? 1 : 0));
       const double time = t.start + f.start + full * (steps * t.step + t.round) + (half ? steps * t.half_step : 0.0) +
-                          mb * (t.weights + t.reads * row_tiles) + f.numbers * numbers * slices;
+                          mb * (t.weights + t.reads * row_tiles) + f.numbers * numbers * slices +
+                          (form == kTileGated && shape == 0 && act == 2 ? full * kWideGelu : 0.0);
       if (time < least) {
         least = time;
         plan = TilePlan{shape, slices};
@@ -393,6 +401,14 @@ int psamd_linear_tile_slice_rows(int n_out, int K) {
   return most;
 }
 
+int psamd_linear_tile_plan(int form, int M, int n_out, int K, int activation) {
+  if (form < kTileSlices || form > kTileQkv || n_out > INT32_MAX / 2 ||
+      !tile_takes(nullptr, nullptr, nullptr, M, n_out, form == kTileGated ? 2 * n_out : n_out, K))
+    return -1;
+  const TilePlan plan = tile_plan(form, M, n_out, K, activation);
+  return plan.shape < 0 ? -1 : 16 * plan.shape + plan.ksplit;
+}
+
 int psamd_linear_tile_stream(void* stream, const void* x, const void* w, float* out, int M, int n_out, int K) {
   PSAMD_REQUIRE(tile_takes(x, w, out, M, n_out, n_out, K), "operands that psamd_linear_tile_slices does not take");
   const TilePlan plan = tile_plan(kTileSlices, M, n_out, K);
@@ -405,7 +421,7 @@ int psamd_linear_tile_stream(void* stream, const void* x, const void* w, float* 
 int psamd_linear_tile_gated(void* stream, const void* x, const void* w, void* out, int M, int n_out, int K, int activation) {
   PSAMD_REQUIRE(activation >= 0 && activation <= 2, "activation 0 (silu), 1 (relu) or 2 (gelu)");
   if (!tile_takes(x, w, out, M, n_out, 2 * n_out, K)) return 2;
-  const TilePlan plan = tile_plan(kTileGated, M, n_out, K);
+  const TilePlan plan = tile_plan(kTileGated, M, n_out, K, activation);
   if (plan.shape < 0) return 2;
   return launch_form<kTileGated>(static_cast<hipStream_t>(stream), plan.shape, x, w, out, M, n_out, K, 1, activation);
 }

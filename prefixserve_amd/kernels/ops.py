@@ -53,6 +53,7 @@ _SIGNATURES = {
     "psamd_linear": [_vp, _vp, _i32, _vp, _i32, _vp, _i32, _i64, _i32, _i32],
     "psamd_linear_tile_slices": [_vp, _vp, _i32, _i32, _i32],
     "psamd_linear_tile_slice_rows": [_i32, _i32],
+    "psamd_linear_tile_plan": [_i32] * 5,
     "psamd_linear_tile_stream": [_vp, _vp, _vp, _vp, _i32, _i32, _i32],
     "psamd_linear_tile_gated": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32],
     "psamd_linear_tile_qkv": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp],

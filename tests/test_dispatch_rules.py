@@ -85,7 +85,7 @@ def test_one_and_two_tokens_among_any_number_of_experts(ops, t, experts, want):
 def planner():
     made = object.__new__(HipOps)
     made.lib, made._plans = ensure_kernels(), {}
-    for name in ("psamd_attention_decode_plan", "psamd_linear_skinny_takes", "psamd_linear_skinny_ksplit"):
+    for name in ("psamd_attention_decode_plan", "psamd_linear_skinny_takes", "psamd_linear_skinny_ksplit", "psamd_linear_tile_plan"):
         getattr(made.lib, name).argtypes = _SIGNATURES[name]
     made.lib.psamd_last_error.restype = ctypes.c_char_p
     return made
@@ -131,3 +131,21 @@ def test_a_step_left_to_the_library_asks_for_the_slices_of_a_shorter_one(ops, n,
     asked = dict(ops.ws.asked)
     assert ops.linear_to_residual(x[:40], w, "o").shape == (4, 40, n)
     assert ops.ws.asked == asked
+
+
+LIBRARY, GATED = -1, 2
+
+
+def plan_of(shape: int, slices: int = 1) -> int:
+    return 16 * shape + slices
+
+
+@pytest.mark.parametrize("m,n,k,silu,gelu", [
+    (640, 8192, 2048, plan_of(0), LIBRARY), (1531, 4096, 2048, plan_of(0), LIBRARY), (4096, 8192, 2048, plan_of(0), LIBRARY),   # the library is faster
+    (2048, 2816, 1024, plan_of(0), plan_of(1)), (900, 6144, 1024, plan_of(0), plan_of(1)),       # smaller tiles are
+    (900, 8192, 3072, plan_of(0), plan_of(0)), (1023, 8192, 2048, plan_of(0), plan_of(0)),       # faster there all the same
+    (256, 8192, 2048, plan_of(3), plan_of(3)), (535, 8192, 2048, LIBRARY, LIBRARY),
+])
+def test_the_largest_tiles_count_what_gelu_takes(planner, m, n, k, silu, gelu):
+    """Their activations run with no matrix instruction beside them: GELU takes longer than the SiLU that the table was made for."""
+    assert [planner.lib.psamd_linear_tile_plan(GATED, m, n, k, act) for act in (0, 1, 2)] == [silu, silu, gelu]
