@@ -219,14 +219,19 @@ __global__ __launch_bounds__(kWideThreads, 1) void linear_wide_kernel(const bf16
   wide_tiles(work, reinterpret_cast<const char*>(x) + first * 128, linear_wide_smem, min(slice_steps, K / 64 - static_cast<int>(first)));
 }
 
+// How many workgroups of the largest tiles a slice of K has, one a compute unit: each die's eighth of them walks the die's eighth of the
+// slice's tiles. (What they take is counted in these rounds: 252 tiles of three slices, 33 of them on a die, are two, 516 tokens x 6,960 x 5,440 97 us where
+// tiles of 192 x 128 take 65.)
+int64_t wide_workgroups(int ksplit) { return std::max<int64_t>(8, 256 / ksplit / 8 * 8); }
+
 template <int FORM, int ACT>
 int launch_wide(hipStream_t s, const void* x, const void* w, void* out, int M, int N, int K, int ksplit) {
   auto kernel = linear_wide_kernel<FORM, ACT>;
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kWideSmem) != hipSuccess)
     return fail("linear_tile: " + std::to_string(kWideSmem) + " bytes of LDS were refused");
   const int row_tiles = static_cast<int>(ceil_div(M, kWideTile)), col_tiles = static_cast<int>(ceil_div(N, FORM == kTileGated ? kWideTile / 2 : kWideTile));
-  const int64_t most = 8 * ceil_div(static_cast<int64_t>(row_tiles) * col_tiles, 8), stay = std::max<int64_t>(8, 256 / ksplit / 8 * 8);
-  kernel<<<dim3(static_cast<unsigned>(std::min(most, stay)), static_cast<unsigned>(ksplit)), dim3(kWideThreads), kWideSmem, s>>>(
+  const int64_t most = 8 * ceil_div(static_cast<int64_t>(row_tiles) * col_tiles, 8);
+  kernel<<<dim3(static_cast<unsigned>(std::min(most, wide_workgroups(ksplit))), static_cast<unsigned>(ksplit)), dim3(kWideThreads), kWideSmem, s>>>(
       static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), out, M, N, K, static_cast<int>(ceil_div(K / 64, ksplit)), row_tiles, col_tiles);
   return check_launch("linear_tile");
 }
@@ -362,7 +367,9 @@ TilePlan tile_plan(int form, int M, int N, int K, int act = 0) {
       const int64_t row_tiles = ceil_div(M, t.rows), groups = row_tiles * ceil_div(rows, t.cols) * slices, at_once = 256 * t.at_once;
       const int64_t left = groups % at_once;
       const bool half = t.at_once == 2 && left > 0 && left <= 256;
-      const double full = static_cast<double>(groups / at_once + (left > 0 && !half ? 1 : 0));
+      const int64_t rounds = shape == 0 ? ceil_div(ceil_div(groups / slices, 8), wide_workgroups(slices) / 8)
+                                        : groups / at_once + (left > 0 && !half ? 1 : 0);
+      const double full = static_cast<double>(rounds);
       const double time = t.start + f.start + full * (steps * t.step + t.round) + (half ? steps * t.half_step : 0.0) +
                           mb * (t.weights + t.reads * row_tiles) + f.numbers * numbers * slices +
                           (form == kTileGated && shape == 0 && act == 2 ? full * kWideGelu : 0.0);

@@ -133,7 +133,7 @@ def test_a_step_left_to_the_library_asks_for_the_slices_of_a_shorter_one(ops, n,
     assert ops.ws.asked == asked
 
 
-LIBRARY, GATED = -1, 2
+LIBRARY, SLICES, GATED = -1, 0, 2
 
 
 def plan_of(shape: int, slices: int = 1) -> int:
@@ -149,3 +149,17 @@ def plan_of(shape: int, slices: int = 1) -> int:
 def test_the_largest_tiles_count_what_gelu_takes(planner, m, n, k, silu, gelu):
     """Their activations run with no matrix instruction beside them: GELU takes longer than the SiLU that the table was made for."""
     assert [planner.lib.psamd_linear_tile_plan(GATED, m, n, k, act) for act in (0, 1, 2)] == [silu, silu, gelu]
+
+
+@pytest.mark.parametrize("m,n,k,want", [
+    (516, 6960, 5440, plan_of(1, 3)), (786, 5232, 6656, LIBRARY), (711, 3376, 8320, plan_of(0, 4)),    # 252 tiles, 33 of them on a die of 32 units
+    (413, 4992, 7744, plan_of(0, 6)), (422, 3344, 10880, plan_of(0, 8)), (471, 3888, 9536, plan_of(0, 8)),    # one round, up to 256 tiles
+])
+def test_the_largest_tiles_count_the_rounds_that_are_launched(planner, m, n, k, want):
+    """Products for the stream: three and six slices have 80 and 40 workgroups each, a die's eighth of a slice's tiles walked by an eighth of those.
+    Where all the tiles together are one round of the chip, a die's may be two."""
+    assert planner.lib.psamd_linear_tile_plan(SLICES, m, n, k, 0) == want
+    shape, slices = divmod(want, 16)
+    if want != LIBRARY and shape == 0:
+        tiles = -(-m // 256) * -(-n // 256)
+        assert -(-tiles // 8) <= 256 // slices // 8
