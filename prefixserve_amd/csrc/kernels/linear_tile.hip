@@ -314,6 +314,11 @@ constexpr TileForm kQkvForm{0.0, 1.504, 7.37, 0.524, 0.206, 2.026, 0.132};
 // something else is the faster (us, the largest tiles / what runs now): 2 x 8,192 x 2,048 at 640 tokens 54.9 / 47.0, 2 x 6,144 x 1,024 at 640 37.2 /
 // 26.8, 2 x 2,816 x 1,024 at 2,048 35.6 / 31.4, 2 x 8,192 x 2,048 at 4,096 235 / 223; 2 x 8,192 x 3,072 at 900 keeps them, 81 / 97.
 constexpr double kWideGelu = 6.5;
+// By what part products for the stream must be faster in the largest tiles than in smaller ones by the table, whose figures are good to that: of
+// 129 products that it would have do otherwise by any lead, 38 were slower by more than 2% (262 tokens x 6,944 x 7,552 54.0 -> 60.7 us) and 44 faster; with this
+// one 3 are slower (at most 9%) and the sum of the times is the same. Two slices of them, which are only ever chosen close to the library, lost to it by 3 to 8% in
+// all of four products (555 x 7,552 x 5,696 71.4 / 77.1) and are not taken.
+constexpr double kWideLead = 1.06;
 
 constexpr int kTileMinTokens = 129;         // fewer: linear_stream.hip
 constexpr int kStreamMaxTokens = 1023;      // above, the library's product adds into the stream itself: tiles 0.97 to 1.32 of its time
@@ -356,14 +361,14 @@ TilePlan tile_plan(int form, int M, int N, int K, int act = 0) {
   const double mb = 2e-6 * rows * K, numbers = 1e-6 * M * N;
   double least = f.library + f.library_gflop * 1e-3 * M * mb + f.library_mb * mb + f.library_numbers * numbers + f.library_step * (K / 64);
   TilePlan plan;
-  for (int shape = 0; shape < kTileShapeCount; ++shape) {
+  for (int shape : {1, 2, 3, 4, 0}) {
     const TileShape& t = kTileShapes[shape];
     for (int slices : {1, 2, 3, 4, 6, 8}) {
       if (slices % 3 == 0 && K > kThirdsMaxK) continue;
       if (slices > 1 && (!stream || K / 64 < 2 * slices || static_cast<int64_t>(slices) * M > kMostSliceRows)) break;
       const int64_t steps = ceil_div(K / 64, slices);
       if (ceil_div(K / 64, steps) != slices || !tile_shape_built(stream && slices == 1 ? kTileAdd : form, shape)) continue;
-      if (shape == 0 && !wide_takes(K, slices)) continue;
+      if (shape == 0 && (!wide_takes(K, slices) || (stream && slices == 2))) continue;
       const int64_t row_tiles = ceil_div(M, t.rows), groups = row_tiles * ceil_div(rows, t.cols) * slices, at_once = 256 * t.at_once;
       const int64_t left = groups % at_once;
       const bool half = t.at_once == 2 && left > 0 && left <= 256;
@@ -373,7 +378,7 @@ TilePlan tile_plan(int form, int M, int N, int K, int act = 0) {
       const double time = t.start + f.start + full * (steps * t.step + t.round) + (half ? steps * t.half_step : 0.0) +
                           mb * (t.weights + t.reads * row_tiles) + f.numbers * numbers * slices +
                           (form == kTileGated && shape == 0 && act == 2 ? full * kWideGelu : 0.0);
-      if (time < least) {
+      if ((shape == 0 && stream && plan.shape > 0 ? kWideLead * time : time) < least) {
         least = time;
         plan = TilePlan{shape, slices};
       }

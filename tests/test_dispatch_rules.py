@@ -152,8 +152,8 @@ def test_the_largest_tiles_count_what_gelu_takes(planner, m, n, k, silu, gelu):
 
 
 @pytest.mark.parametrize("m,n,k,want", [
-    (516, 6960, 5440, plan_of(1, 3)), (786, 5232, 6656, LIBRARY), (711, 3376, 8320, plan_of(0, 4)),    # 252 tiles, 33 of them on a die of 32 units
-    (413, 4992, 7744, plan_of(0, 6)), (422, 3344, 10880, plan_of(0, 8)), (471, 3888, 9536, plan_of(0, 8)),    # one round, up to 256 tiles
+    (516, 6960, 5440, plan_of(1, 3)), (786, 5232, 6656, LIBRARY), (711, 3376, 8320, plan_of(2, 2)),    # 252 tiles, 33 of them on a die of 32 units
+    (413, 4992, 7744, plan_of(0, 6)), (422, 3344, 10880, plan_of(0, 8)), (796, 4016, 5696, plan_of(0, 4)),    # one round, up to 256 tiles
 ])
 def test_the_largest_tiles_count_the_rounds_that_are_launched(planner, m, n, k, want):
     """Products for the stream: three and six slices have 80 and 40 workgroups each, a die's eighth of a slice's tiles walked by an eighth of those.
@@ -163,3 +163,14 @@ def test_the_largest_tiles_count_the_rounds_that_are_launched(planner, m, n, k, 
     if want != LIBRARY and shape == 0:
         tiles = -(-m // 256) * -(-n // 256)
         assert -(-tiles // 8) <= 256 // slices // 8
+
+
+@pytest.mark.parametrize("m,n,k,want", [
+    (262, 6944, 7552, plan_of(2, 2)), (281, 6880, 7168, plan_of(2, 2)), (285, 4496, 15424, plan_of(2, 3)), (253, 4544, 14464, plan_of(3, 3)),   # slower in the largest
+    (555, 7552, 5696, LIBRARY), (518, 7792, 6784, LIBRARY),                  # and in two slices of them
+    (1009, 2528, 7616, plan_of(0, 4)), (301, 5520, 9280, plan_of(0, 4)),     # close to the library by the table, but faster
+    (422, 3344, 10880, plan_of(0, 8)), (1023, 4096, 14336, plan_of(0, 4)),
+])
+def test_the_largest_tiles_replace_smaller_ones_by_a_lead(planner, m, n, k, want):
+    """Products for the stream: where the table has the largest tiles and smaller ones within its own error, the smaller ones stay."""
+    assert planner.lib.psamd_linear_tile_plan(SLICES, m, n, k, 0) == want
