@@ -156,6 +156,13 @@ int psamd_moe_experts_grouped(void* stream, const void* x, const int32_t* chosen
                               int64_t tokens, int K, int F, int experts, int identity, int top, float gate_alpha, float limit,
                               float up_shift, int grouped_already, int weight_on_output, int kind, int into_stream,
                               const float* col_scale);
+// Which large tiles psamd_moe_experts_grouped takes for pairs that it sorts itself: 256 (tiles of up to so many pairs, cut by the step's counts), 128 or
+// 0 (small ones). psamd_moe_experts_tiled takes 256 or 128 whatever that says, for tests and measurements, with as many `ints` for the same sizes.
+int psamd_moe_expert_tile_rows(int64_t tokens, int K, int F, int experts, int identity, int top, int kind);
+int psamd_moe_experts_tiled(void* stream, const void* x, const int32_t* chosen, const float* weight,
+                            const void* w_in, const void* w_down, void* act, float* out, int32_t* ints,
+                            int64_t tokens, int K, int F, int experts, int identity, int top, float gate_alpha, float limit,
+                            float up_shift, int weight_on_output, int kind, int into_stream, const float* col_scale, int tile_rows);
 // psamd_moe_topk and the sorting of the pairs into `ints` in one workgroup, for up to 64 tokens (buckets: the experts with
 // matrices, plus one if there are identity experts; psamd_moe_grouped_max_tiles then takes buckets for experts);
 // psamd_moe_experts_grouped is then called with grouped_already = 1 and the same `ints`.

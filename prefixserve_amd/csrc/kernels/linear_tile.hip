@@ -137,6 +137,7 @@ struct DenseTiles {
   const char* w;
   int cur, next_a, next_w, lane, wave;                 // tiles: multiplied, copied next
 
+  static constexpr int kMinSteps = 2;                  // the tiles that are copied are counted apart from the one that is multiplied
   static constexpr int WROWS = kWideTile / 2, WCOLS = FORM == kTileGated ? WROWS / 2 : WROWS, COLS = 2 * WCOLS;
   // (What follows from the lane alone would be computed in front of all tiles and held through them, where no register is free.)
   __device__ __forceinline__ int own_lane() const {
@@ -219,6 +220,12 @@ __global__ __launch_bounds__(kWideThreads, 1) void linear_wide_kernel(const bf16
   wide_tiles(work, reinterpret_cast<const char*>(x) + first * 128, linear_wide_smem, min(slice_steps, K / 64 - static_cast<int>(first)));
 }
 
+// Whether every slice of K has the steps that the largest tiles work with.
+bool wide_takes(int K, int ksplit) {
+  const int64_t steps = ceil_div(K / 64, ksplit);
+  return K / 64 - (ksplit - 1) * steps >= DenseTiles<kTileSlices, 0>::kMinSteps;
+}
+
 // How many workgroups of the largest tiles a slice of K has, one a compute unit: each die's eighth of them walks the die's eighth of the
 // slice's tiles. (What they take is counted in these rounds: 252 tiles of three slices, 33 of them on a die, are two, 516 tokens x 6,960 x 5,440 97 us where
 // tiles of 192 x 128 take 65.)
@@ -226,6 +233,7 @@ int64_t wide_workgroups(int ksplit) { return std::max<int64_t>(8, 256 / ksplit /
 
 template <int FORM, int ACT>
 int launch_wide(hipStream_t s, const void* x, const void* w, void* out, int M, int N, int K, int ksplit) {
+  if (!wide_takes(K, ksplit)) return fail("linear_tile: too few steps of k for the largest tiles");
   auto kernel = linear_wide_kernel<FORM, ACT>;
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kWideSmem) != hipSuccess)
     return fail("linear_tile: " + std::to_string(kWideSmem) + " bytes of LDS were refused");
@@ -234,12 +242,6 @@ int launch_wide(hipStream_t s, const void* x, const void* w, void* out, int M, i
   kernel<<<dim3(static_cast<unsigned>(std::min(most, wide_workgroups(ksplit))), static_cast<unsigned>(ksplit)), dim3(kWideThreads), kWideSmem, s>>>(
       static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), out, M, N, K, static_cast<int>(ceil_div(K / 64, ksplit)), row_tiles, col_tiles);
   return check_launch("linear_tile");
-}
-
-// The largest tiles come with two steps of k or more in every slice.
-bool wide_takes(int K, int ksplit) {
-  const int64_t steps = ceil_div(K / 64, ksplit);
-  return K / 64 - (ksplit - 1) * steps >= 2;
 }
 
 template <int TM, int TN, int WM, int WN, int STAGES, int OCC, int FORM>

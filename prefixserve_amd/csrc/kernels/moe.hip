@@ -1079,6 +1079,7 @@ struct ExpertTiles {
   float gate_alpha, limit, up_shift;
 
   static constexpr bool GATED = FORM == kFormGated;
+  static constexpr int kMinSteps = 4;           // a_rows takes the pairs that ahead() asked for
   static constexpr int WROWS = kWideTile / 2, WCOLS = GATED ? WROWS / 2 : WROWS, COLS = 2 * WCOLS;
   struct Item {
     int expert, first, count, n0;
@@ -1340,6 +1341,8 @@ static int launch_tiles(hipStream_t s, const ExpertCall& c, const int32_t* ints,
 
 template <int FORM>
 static int run_wide(hipStream_t s, const ExpertCall& c, const int32_t* ints, int max_tiles) {
+  if ((FORM == kFormDown ? c.F : c.K) < 64 * ExpertTiles<FORM>::kMinSteps)
+    return fail("psamd_moe_experts_grouped: too few steps of k for tiles of 256 pairs");
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(moe_wide_kernel<FORM>), hipFuncAttributeMaxDynamicSharedMemorySize, kWideSmem) != hipSuccess)
     return fail("psamd_moe_experts_grouped: " + std::to_string(kWideSmem) + " bytes of LDS were refused");
   const int32_t* t_e = ints + c.tokens * c.top;
@@ -1406,7 +1409,7 @@ static int wide_tile_rows(int64_t pairs, int experts, int K, int F, int kind) {
     };
     return of(ceil_div(F, kind == kExpertGated ? rows / 2 : rows)) * (K + beside) + of(ceil_div(K, rows)) * (F + beside);
   };
-  if (std::min(K, F) < 64 * kWideMinSteps) return 128;
+  if (std::min(K, F) < 64 * ExpertTiles<kFormGated>::kMinSteps) return 128;
   return 1.2 * rounds(256, 256, 300) < rounds(128, 512, 0) ? 256 : 128;
 }
 
@@ -1450,14 +1453,50 @@ __global__ __launch_bounds__(256) void row_gate_kernel(float* __restrict__ out, 
   for (int i = threadIdx.x; i < out_hidden; i += 256) o[i] *= g;
 }
 
+// What the grouped form refuses, on the host.
+static const char* bad_experts(const ExpertCall& c, const int32_t* ints) {
+  if (c.kind != kExpertGated && c.kind != kExpertSquaredRelu) return "experts are gated (0) or squared ReLU without a gate (1)";
+  if (c.tokens < 0 || c.K <= 0 || c.F <= 0 || c.experts <= 0 || c.identity < 0 || c.top < 1 || c.top > c.experts + c.identity) return "bad sizes";
+  if (c.K % 8 != 0 || c.F % 8 != 0) return "K and F must be multiples of 8";
+  if (c.experts > 4096 || c.tokens * c.top > (1 << 24)) return "too many experts or pairs";
+  return ints == nullptr ? "the grouping needs its integer scratch" : nullptr;
+}
+
+// `wide`: the pairs of a large tile, 256 (at most) or 128, or 0 for the kernels of small ones.
+static int run_experts(hipStream_t s, const ExpertCall& c, int32_t* ints, int grouped_already, int wide) {
+  if (c.tokens == 0) return 0;
+  const int64_t pairs = c.tokens * c.top;
+  const int buckets = c.experts + (c.identity > 0 ? 1 : 0);  // all identity pairs lie in one, behind the experts'
+  const int rows = wide != 0 ? wide : psamd_moe_grouped_tile_rows(pairs, buckets);
+  const int least = rows == 256 ? 128 : rows;                // the device may cut into tiles of 128
+  const int max_tiles = static_cast<int>(std::min<int64_t>(ceil_div(pairs, least) + buckets, pairs));
+  if (wide == 0 && max_tiles > 65535) return fail("psamd_moe_experts_grouped: too many tiles for one launch");   // they are gridDim.y of moe_grouped_kernel alone
+  if (grouped_already == 0) {
+    const TileRule rule{rows == 256 ? 0 : rows,
+                        {static_cast<int>(ceil_div(c.F, c.kind == kExpertGated ? 128 : 256)), static_cast<int>(ceil_div(c.K, 256))}, {c.K, c.F}};
+    const bool staged = group_staged(pairs, buckets);
+    const size_t smem = sizeof(int32_t) * (group_smem_ints(buckets) + (staged ? pairs : 0));
+    if (smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(moe_group_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                static_cast<int>(smem)) != hipSuccess)
+      return fail("psamd_moe_experts_grouped: " + std::to_string(smem) + " bytes of LDS were refused");
+    moe_group_kernel<<<dim3(1), dim3(1024), smem, s>>>(
+        c.chosen, static_cast<int>(pairs), buckets, rule, c.identity > 0 && wide != 0, max_tiles, staged, ints, ints + pairs,
+        ints + pairs + max_tiles, ints + pairs + 2 * max_tiles);
+    if (check_launch("psamd_moe_experts_grouped (grouping)")) return 1;
+  }
+  if (wide == 256) return launch_wide(s, c, ints, max_tiles);
+  if (wide == 128) return launch_tiles(s, c, ints, max_tiles);
+  if (rows == 128) return launch_grouped<8, 2>(s, c, ints, max_tiles);
+  if (rows == 64) return launch_grouped<4, 2>(s, c, ints, max_tiles);
+  if (tiles_take(c.tokens, pairs, c.K, c.F)) return launch_stream(s, c, ints, max_tiles);
+  return launch_grouped<1, 1>(s, c, ints, max_tiles);
+}
+
 }  // namespace psamd
 
 using namespace psamd;
 
 extern "C" {
-
-int psamd_moe_grouped_tile_rows(int64_t pairs, int experts);
-int psamd_moe_grouped_max_tiles(int64_t pairs, int experts);
 
 int psamd_moe_route(void* stream, const void* x, int x_dtype, const float* w_router, int32_t* chosen, float* weight,
                     int64_t tokens, int K, int experts, int top, const float* bias, int mode,
@@ -1545,47 +1584,34 @@ int psamd_moe_grouped_max_tiles(int64_t pairs, int experts) {
   return static_cast<int>(std::min<int64_t>(ceil_div(pairs, rows) + experts, pairs));
 }
 
+int psamd_moe_expert_tile_rows(int64_t tokens, int K, int F, int experts, int identity, int top, int kind) {
+  const int64_t pairs = tokens * top;
+  return tiles_take(tokens, pairs, K, F) ? wide_tile_rows(pairs, experts + (identity > 0 ? 1 : 0), K, F, kind) : 0;
+}
+
 int psamd_moe_experts_grouped(void* stream, const void* x, const int32_t* chosen, const float* weight,
                               const void* w_in, const void* w_down, void* act, float* out, int32_t* ints,
                               int64_t tokens, int K, int F, int experts, int identity, int top, float gate_alpha, float limit,
                               float up_shift, int grouped_already, int weight_on_output, int kind, int into_stream,
                               const float* col_scale) {
-  PSAMD_REQUIRE(kind == kExpertGated || kind == kExpertSquaredRelu, "experts are gated (0) or squared ReLU without a gate (1)");
-  PSAMD_REQUIRE(tokens >= 0 && K > 0 && F > 0 && experts > 0 && identity >= 0 && top >= 1 && top <= experts + identity, "bad sizes");
-  PSAMD_REQUIRE(K % 8 == 0 && F % 8 == 0, "K and F must be multiples of 8");
-  PSAMD_REQUIRE(experts <= 4096 && tokens * top <= (1 << 24), "too many experts or pairs");
-  PSAMD_REQUIRE(ints != nullptr, "the grouping needs its integer scratch");
-  if (tokens == 0) return 0;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const int64_t pairs = tokens * top;
-  const int buckets = experts + (identity > 0 ? 1 : 0);      // all identity pairs lie in one, behind the experts'
-  // Pairs that the router's kernel has sorted lie in the tiles of a small step.
-  const int wide = grouped_already == 0 && tiles_take(tokens, pairs, K, F) ? wide_tile_rows(pairs, buckets, K, F, kind) : 0;
-  const int rows = wide != 0 ? wide : psamd_moe_grouped_tile_rows(pairs, buckets);
-  const int least = rows == 256 ? 128 : rows;                // the device may cut into tiles of 128
-  const int max_tiles = static_cast<int>(std::min<int64_t>(ceil_div(pairs, least) + buckets, pairs));
-  PSAMD_REQUIRE(wide != 0 || max_tiles <= 65535, "too many tiles for one launch");       // they are gridDim.y of moe_grouped_kernel alone
-  if (grouped_already == 0) {
-    const TileRule rule{rows == 256 ? 0 : rows,
-                        {static_cast<int>(ceil_div(F, kind == kExpertGated ? 128 : 256)), static_cast<int>(ceil_div(K, 256))}, {K, F}};
-    const bool staged = group_staged(pairs, buckets);
-    const size_t smem = sizeof(int32_t) * (group_smem_ints(buckets) + (staged ? pairs : 0));
-    if (smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(moe_group_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                static_cast<int>(smem)) != hipSuccess)
-      return fail("psamd_moe_experts_grouped: " + std::to_string(smem) + " bytes of LDS were refused");
-    moe_group_kernel<<<dim3(1), dim3(1024), smem, s>>>(
-        chosen, static_cast<int>(pairs), buckets, rule, identity > 0 && wide != 0, max_tiles, staged, ints, ints + pairs,
-        ints + pairs + max_tiles, ints + pairs + 2 * max_tiles);
-    if (check_launch("psamd_moe_experts_grouped (grouping)")) return 1;
-  }
   const ExpertCall c{x, chosen, weight, w_in, w_down, act, out, tokens, K, F, experts, identity, top, kind,
                      gate_alpha, limit, up_shift, weight_on_output, into_stream, col_scale};
-  if (wide == 256) return launch_wide(s, c, ints, max_tiles);
-  if (wide == 128) return launch_tiles(s, c, ints, max_tiles);
-  if (rows == 128) return launch_grouped<8, 2>(s, c, ints, max_tiles);
-  if (rows == 64) return launch_grouped<4, 2>(s, c, ints, max_tiles);
-  if (tiles_take(tokens, pairs, K, F)) return launch_stream(s, c, ints, max_tiles);
-  return launch_grouped<1, 1>(s, c, ints, max_tiles);
+  if (const char* bad = bad_experts(c, ints)) return fail(std::string(__func__) + ": " + bad);
+  // Pairs that the router's kernel has sorted lie in the tiles of a small step.
+  return run_experts(static_cast<hipStream_t>(stream), c, ints, grouped_already,
+                     grouped_already == 0 ? psamd_moe_expert_tile_rows(tokens, K, F, experts, identity, top, kind) : 0);
+}
+
+int psamd_moe_experts_tiled(void* stream, const void* x, const int32_t* chosen, const float* weight,
+                            const void* w_in, const void* w_down, void* act, float* out, int32_t* ints,
+                            int64_t tokens, int K, int F, int experts, int identity, int top, float gate_alpha, float limit,
+                            float up_shift, int weight_on_output, int kind, int into_stream, const float* col_scale, int tile_rows) {
+  const ExpertCall c{x, chosen, weight, w_in, w_down, act, out, tokens, K, F, experts, identity, top, kind,
+                     gate_alpha, limit, up_shift, weight_on_output, into_stream, col_scale};
+  if (const char* bad = bad_experts(c, ints)) return fail(std::string(__func__) + ": " + bad);
+  PSAMD_REQUIRE(tiles_take(tokens, tokens * top, K, F) && (tile_rows == 128 || tile_rows == 256), "operands and tiles that these kernels take");
+  PSAMD_REQUIRE(tile_rows == 128 || std::min(K, F) >= 64 * ExpertTiles<kFormGated>::kMinSteps, "too few steps of k for tiles of 256 pairs");
+  return run_experts(static_cast<hipStream_t>(stream), c, ints, 0, tile_rows);
 }
 
 int psamd_row_gate(void* stream, float* out, const void* x, int act_dtype, const float* w, int64_t tokens, int out_hidden,

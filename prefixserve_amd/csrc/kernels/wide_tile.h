@@ -12,9 +12,9 @@ constexpr int kWideTile = 256;                         // rows of A and of W a t
 constexpr int kWideUnit = kWideTile * 128;             // one operand's 64 k of a tile in LDS
 constexpr int kWideSmem = 5 * kWideUnit;               // all of a compute unit's
 constexpr int kWideThreads = 256;
-constexpr int kWideMinSteps = 4;                       // of 64 k
 
-// A workgroup's tiles, one after the other; `Work` says what they are:
+// A workgroup's tiles of `steps` times 64 k, one after the other; `Work` says what they are:
+//   int kMinSteps                        the fewest steps that it works with, 2 or more; whoever launches it refuses fewer
 //   bool a_rows(uint32_t (&off)[8])      the next tile's rows of A for the copies of this wave (copy i: rows 64 wave + 8 i + lane / 8), as
 //                                        byte offsets from `a` of 16 bytes each (wide_piece); false: there is no next tile
 //   bool w_rows(uint32_t (&off)[8])      likewise of W, behind work.w
@@ -22,7 +22,8 @@ constexpr int kWideMinSteps = 4;                       // of 64 k
 //   void ahead()                         called behind that tile's first step: what may be loaded for the tiles to come
 //   void finish<RM>(acc)                 acc[i][j]: lane (r, g) holds, of row 128 / 8 RM (wave / 2) + 16 j + r of A, rows 128 (wave % 2) + 16 i
 //                                        + 4 g .. + 3 of W
-// a_rows and w_rows are called once more than there are tiles, each at most one tile ahead of finish. `steps`: K / 64, at least kWideMinSteps.
+// a_rows and w_rows are called once more than there are tiles. Copies run two steps ahead, so both are asked for the tile behind this one three steps in front
+// of this one's end: from four steps on behind ahead(), with three in front of it, with two in front of this tile's rows() and two tiles ahead of finish.
 //
 // What bounds it: the matrix instructions' power at long K (256 x 256 tiles of 2,048 x 16,384 x 8,192: matrix cores busy 73% of the time at 1.93
 // GHz; the library's kernel 84% at 1.75), beginnings and ends of tiles at short K. Why so:
@@ -34,6 +35,7 @@ constexpr int kWideMinSteps = 4;                       // of 64 k
 //  * one barrier a step, between its halves: each half's operands are read while the half before is multiplied.
 template <class Work>
 __device__ __forceinline__ void wide_tiles(Work& work, const char* a, unsigned char* smem, int steps) {
+  static_assert(Work::kMinSteps >= 2, "two steps are under way in front of the first");
   constexpr int RN = 8, RING = 5 * kWideUnit, COPIES = 8;
   const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)smem));
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));

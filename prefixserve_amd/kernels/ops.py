@@ -106,6 +106,9 @@ _SIGNATURES = {
     "psamd_moe_grouped_max_tiles": [_i64, _i32],
     "psamd_moe_experts_grouped": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _f32, _f32, _f32, _i32, _i32,
                                   _i32, _i32, _vp],
+    "psamd_moe_expert_tile_rows": [_i64, _i32, _i32, _i32, _i32, _i32, _i32],
+    "psamd_moe_experts_tiled": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _f32, _f32, _f32, _i32, _i32,
+                                _i32, _vp, _i32],
     "psamd_moe_topk_group": [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, _i32, _i32, _i32, _f32, _i32, _vp],
     "psamd_moe_experts_rows": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _i32, _i32, _i32, _i32, _i32, _f32, _f32, _f32, _i32,
                                _i32, _i32, _vp],

@@ -85,7 +85,8 @@ def test_one_and_two_tokens_among_any_number_of_experts(ops, t, experts, want):
 def planner():
     made = object.__new__(HipOps)
     made.lib, made._plans = ensure_kernels(), {}
-    for name in ("psamd_attention_decode_plan", "psamd_linear_skinny_takes", "psamd_linear_skinny_ksplit", "psamd_linear_tile_plan"):
+    for name in ("psamd_attention_decode_plan", "psamd_linear_skinny_takes", "psamd_linear_skinny_ksplit", "psamd_linear_tile_plan",
+                 "psamd_moe_expert_tile_rows", "psamd_moe_experts_tiled"):
         getattr(made.lib, name).argtypes = _SIGNATURES[name]
     made.lib.psamd_last_error.restype = ctypes.c_char_p
     return made
@@ -174,3 +175,16 @@ def test_the_largest_tiles_count_the_rounds_that_are_launched(planner, m, n, k, 
 def test_the_largest_tiles_replace_smaller_ones_by_a_lead(planner, m, n, k, want):
     """Products for the stream: where the table has the largest tiles and smaller ones within its own error, the smaller ones stay."""
     assert planner.lib.psamd_linear_tile_plan(SLICES, m, n, k, 0) == want
+
+
+@pytest.mark.parametrize("tokens,k,f,experts,rows", [
+    (24000, 3264, 256, 5, 256), (24000, 3264, 192, 5, 128), (100000, 192, 3264, 8, 128), (16384, 2048, 1024, 32, 256),
+    (24000, 256, 72, 5, 0), (512, 2048, 1024, 32, 0),
+])
+def test_tiles_of_256_pairs_come_with_four_steps_of_k_or_more(planner, tokens, k, f, experts, rows):
+    """Their next tile's pairs are asked for behind a tile's first step and used three steps in front of its end: with fewer steps than four the next
+    tile's copies would take this one's pairs. Asked for all the same, they are refused on the host."""
+    assert planner.lib.psamd_moe_expert_tile_rows(tokens, k, f, experts, 0, 1, 0) == rows
+    for short_k, short_f in ((192, 256), (256, 192), (64, 64)):
+        assert planner.lib.psamd_moe_experts_tiled(*[None] * 8, 1, 100, short_k, short_f, 2, 0, 1, 1.0, 7.0, 0.0, 1, 0, 0, None, 256) == 1
+        assert b"too few steps" in planner.lib.psamd_last_error()
