@@ -380,6 +380,8 @@ int psamd_attention_mfma_supports(int hq, int hkv, int head_dim);
 // part_o [32 * n_tiles * hq * nsplit * head_dim] and part_ml [32 * n_tiles * hq * nsplit * 2] carry
 // to a merge kernel.
 int psamd_attention_prefill_nsplit(int n_tiles, int max_kv_len, int hq, int hkv, int head_dim);
+// The waves a query head has in the kernel that takes the heads of a kv head together (0: the per-head kernel runs), for tests.
+int psamd_attention_prefill_waves(int n_tiles, int n_blocks, int max_kv_len, int hq, int hkv, int head_dim, int nsplit);
 // exact_weights (here and in psamd_attention_decode): the softmax weights enter the second product
 // as three bfloat16 terms whose sum is the float32 weight exactly, instead of rounded to bfloat16.
 // pf_tiles: (item, first query) of every tile of 32 queries; pf_blocks: the first tile of every run

@@ -1999,8 +1999,6 @@ static bool lds_allowed(Kernel kernel, size_t bytes) {
 // to even out the triangle) were measured against the order of workgroups described in the kernel
 // and dropped: within 3% at best, 12% slower at 3,072 tokens, up to 15% slower on top of a cached
 // prefix.
-enum class PrefillForm { kPerHead, kGrouped };
-
 // With one or two query heads per kv head a workgroup of the grouped kernel takes four or two
 // consecutive tiles of queries, so that four waves still share the keys and values it stages.
 static int prefill_tiles_per_wg(int group) { return group == 1 ? 4 : (group == 2 ? 2 : 1); }
@@ -2016,10 +2014,6 @@ static int64_t grouped_workgroups(int n_tiles, int hq, int hkv) {
 // Few enough of them that the per-head kernel, with four times as many, does better.
 static bool few_grouped_workgroups(int n_tiles, int hq, int hkv, int head_dim) {
   return grouped_workgroups(n_tiles, hq, hkv) <= (head_dim <= 64 ? 128 : 80);
-}
-
-static PrefillForm prefill_form(int n_tiles, int hq, int hkv, int head_dim) {
-  return few_grouped_workgroups(n_tiles, hq, hkv, head_dim) ? PrefillForm::kPerHead : PrefillForm::kGrouped;
 }
 
 static int launch_prefill_merge(hipStream_t s, const float* part_o, const float* part_ml, void* out,
@@ -2080,6 +2074,28 @@ static int prefill_nsplit(int n_tiles, int max_kv_len, int hq, int hkv, int head
   return per_head_nsplit(n_tiles, max_kv_len, hq);
 }
 
+// One or two query heads per kv head: the per-head kernel without the list of runs of tiles, and
+// where the keys are cut by its rule and not by the grouped kernel's.
+static bool prefill_per_head(int n_tiles, int n_blocks, int max_kv_len, int hq, int hkv, int head_dim, int nsplit) {
+  if (hq / hkv <= 2 && (n_blocks == 0 || (nsplit > 1 && grouped_nsplit(n_tiles, max_kv_len, hq, hkv, head_dim) == 1))) return true;
+  return nsplit == 1 && few_grouped_workgroups(n_tiles, hq, hkv, head_dim);
+}
+
+// The grid of the kernels that take the query heads of a kv head together.
+static dim3 grouped_grid(int n_tiles, int n_blocks, int hq, int hkv, int nsplit) {
+  const int group = hq / hkv, tiles_per_wg = prefill_tiles_per_wg(group), heads_per_wg = 4 / tiles_per_wg;
+  return dim3(hkv * ((group + heads_per_wg - 1) / heads_per_wg), tiles_per_wg == 1 ? n_tiles : n_blocks * heads_per_wg, nsplit);
+}
+
+// How many waves a query head has there, each its own run of keys.
+// From head size 96 on, where a compute unit holds one workgroup of eight waves, four
+// workgroups per compute unit's worth of tiles run 5% faster as two workgroups of four waves
+// (one wave per head): two barriers' worth of waves that do not wait for each other
+// (head size 128: 4,096 tokens 181 -> 171 us, 8,192 tokens 657 -> 623 us; 2,048 tokens 56 -> 67).
+static int grouped_waves(const dim3& grid, int head_dim) {
+  return head_dim < 96 || static_cast<int64_t>(grid.x) * grid.y * grid.z < 1024 ? 2 : 1;
+}
+
 template <int NS, bool P3>
 static int launch_prefill(hipStream_t s, const void* qkv, int q_stride, void* out, const void* kv,
                           const int32_t* pf_tiles, int n_tiles, const int32_t* pf_blocks, int n_blocks, int max_kv_len,
@@ -2088,18 +2104,11 @@ static int launch_prefill(hipStream_t s, const void* qkv, int q_stride, void* ou
                           float* part_o, float* part_ml, int nsplit) {
   const int group = hq / hkv;
   const int table_pages = static_cast<int>(ceil_div(max_kv_len, kPage));
-  // One or two query heads per kv head: the per-head kernel without the list of runs of tiles, and
-  // where the keys are cut by its rule and not by the grouped kernel's.
-  const bool small_per_head =
-      group <= 2 && (n_blocks == 0 || (nsplit > 1 && grouped_nsplit(n_tiles, max_kv_len, hq, hkv, 16 * NS) == 1));
-  const PrefillForm form = nsplit > 1 || small_per_head ? (small_per_head ? PrefillForm::kPerHead : PrefillForm::kGrouped)
-                                                        : prefill_form(n_tiles, hq, hkv, 16 * NS);
   // The heads of a kv head share its keys and values through LDS, two waves per head (each its
   // own run of keys) if the stages fit, else one.
-  if (form != PrefillForm::kPerHead) {
-    const int tiles_per_wg = prefill_tiles_per_wg(group), heads_per_wg = 4 / tiles_per_wg;
-    const dim3 grid(hkv * ((group + heads_per_wg - 1) / heads_per_wg), tiles_per_wg == 1 ? n_tiles : n_blocks * heads_per_wg,
-                    nsplit);
+  if (!prefill_per_head(n_tiles, n_blocks, max_kv_len, hq, hkv, 16 * NS, nsplit)) {
+    const int tiles_per_wg = prefill_tiles_per_wg(group);
+    const dim3 grid = grouped_grid(n_tiles, n_blocks, hq, hkv, nsplit);
     // More than one workgroup per compute unit but no more than run at once (two of eight waves
     // up to head size 64): see pair_tiles in the kernel.
     const int64_t wgs = static_cast<int64_t>(grid.x) * grid.y;
@@ -2133,12 +2142,10 @@ static int launch_prefill(hipStream_t s, const void* qkv, int q_stride, void* ou
       return launch_prefill_merge(s, part_o, part_ml, out, pf_tiles, item_start, n_tiles, hq, 16 * NS, nsplit);   \
     }                                                                                                             \
   }
-    // From head size 96 on, where a compute unit holds one workgroup of eight waves, four
-    // workgroups per compute unit's worth of tiles run 5% faster as two workgroups of four waves
-    // (one wave per head): two barriers' worth of waves that do not wait for each other
-    // (head size 128: 4,096 tokens 181 -> 171 us, 8,192 tokens 657 -> 623 us; 2,048 tokens 56 -> 67).
-    const bool two_waves = NS < 6 || wgs * grid.z < 1024;
-    if constexpr (NS == 4 || NS == 8 || NS == 16) {
+    const bool two_waves = grouped_waves(grid, 16 * NS) == 2;
+    if constexpr (NS == 4) {
+      PSAMD_COPIED(2)
+    } else if constexpr (NS == 8 || NS == 16) {
       if (two_waves) PSAMD_COPIED(2)
       PSAMD_COPIED(1)
     } else {
@@ -2248,6 +2255,15 @@ int psamd_attention_mfma_supports(int hq, int hkv, int head_dim) {
 int psamd_attention_prefill_nsplit(int n_tiles, int max_kv_len, int hq, int hkv, int head_dim) {
   if (!psamd_attention_mfma_supports(hq, hkv, head_dim) || n_tiles <= 0) return 1;
   return prefill_nsplit(n_tiles, max_kv_len, hq, hkv, head_dim);
+}
+
+// How many waves a query head has in the kernel that takes the heads of a kv head together, for a step that psamd_attention_prefill runs with
+// these sizes; 0: the step goes to the per-head kernel.
+int psamd_attention_prefill_waves(int n_tiles, int n_blocks, int max_kv_len, int hq, int hkv, int head_dim, int nsplit) {
+  if (!psamd_attention_mfma_supports(hq, hkv, head_dim) || n_tiles <= 0 ||
+      prefill_per_head(n_tiles, n_blocks, max_kv_len, hq, hkv, head_dim, nsplit))
+    return 0;
+  return grouped_waves(grouped_grid(n_tiles, n_blocks, hq, hkv, nsplit), head_dim);
 }
 
 // Rows of part_o / part_ml (32 * n_tiles * nsplit) that no step of this shape exceeds while

@@ -74,6 +74,7 @@ _SIGNATURES = {
                             _vp, _vp, _i32, _vp, _i64],
     "psamd_attention_mfma_supports": [_i32, _i32, _i32],
     "psamd_attention_prefill_nsplit": [_i32, _i32, _i32, _i32, _i32],
+    "psamd_attention_prefill_waves": [_i32] * 7,
     "psamd_attention_prefill_part_rows": [_i32, _i32, _i32],
     "psamd_attention_decode_skewed": [_i32, _i32, _i64],
     "psamd_attention_decode_plan": [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp],
