@@ -1114,7 +1114,11 @@ __global__ __launch_bounds__(256 * KP, NS <= 4 ? 4 : 2) void attn_prefill_groupe
 // way, a page's number is asked for an iteration ahead by the scalar unit, and the two halves of a wave exchange maxima and sums by an
 // instruction of their own. The order of all sums is that of the kernel above, and so are the bits.
 // us a layer, above -> here: 2,048 tokens of 32 heads on 8 at head size 64 43 -> 38, with three-term weights 69 -> 54, 1,531 with a window of 1,024 57 -> 46;
-// at head size 128 2,048 tokens 67 -> 57, as many behind 2,048 156 -> 126; 1,500 tokens of 16 heads on one at 256, three terms, 204 -> 124.
+// at head size 128 2,048 tokens 67 -> 57, as many behind 2,048 156 -> 126; 1,500 tokens of 16 heads on one at 256, three terms, 204 -> 124. Over 819 steps of nine
+// geometries (windows, cached prefixes, uneven portions) 0.75 to 0.98 of the time at head size 64, 0.91 to 0.98 at 128, 0.45 to 0.68 at 256.
+// At head size 256 queries, sums and operands are more than the registers here too: 28 to 33 of them are spilled, and six loads (with three-term weights eight) from
+// scratch in front of every iteration's score products, and a wait, behind the copies just asked for: with the two stages there are there, nothing is
+// under way behind the products. (64 and 128 have no scratch.)
 // What bounds it at head size 64: the vector unit is at work 37 of 91 thousand cycles, the matrix cores 17; a unit holds 2.2 waves a SIMD on the
 // average, as the longest tile's workgroup, 32 iterations, is alone in the end, its waves all in the same phase between two barriers. No gain: a barrier
 // for two iterations (37.7 / 36.9), sixteen waves a workgroup (42), other pairs of tiles (39 to 45).
@@ -1987,18 +1991,21 @@ static bool lds_allowed(Kernel kernel, size_t bytes) {
 
 // Which kernel a step's portions go to, when two or more query heads share a kv head
 // (measured on 256 compute units with 32 query heads on 8 kv heads; us per layer, per-head /
-// grouped, at head size 64 and at head size 128):
-//   256 on 1,792 cached     18 / 30      31 / 43       384 on 3,712 cached     48 / 53      94 / 78
-//   512 from position 0     11 / 12      21 / 18       512 on 7,680 cached     91 / 101    180 / 148
-//   768 on 2,304 cached     50 / 42     104 / 63       1,024 on 3,072 cached   84 / 56     176 / 88
-//   2,048 from position 0   57 / 36     142 / 58       8,192 from 0             - / 355      - / 655
+// grouped with copied keys and one run of them, at head sizes 64, 128 and 256):
+//   256 on 1,792 cached     17 / 29    30 / 42    202 / 110      384 on 3,712 cached     47 / 52    91 / 76    623 / 215
+//   384 on 1,027 cached     21 / 23    39 / 33    230 / 83       512 on 7,680 cached     90 / 100  177 / 144  1,453 / 420
+//   512 on 1,027 cached     22 / 25    42 / 35    280 / 92       640 on 1,000 cached     28 / 26    60 / 37    379 / 97
+//   768 on 2,304 cached     50 / 41   102 / 60    770 / 169      1,024 on 3,072 cached   81 / 54   170 / 80  1,335 / 227
+//   2,048 from position 0   55 / 33   134 / 55    881 / 140      8,192 from 0           776 / 345 1,628 / 610
 // The per-head kernel, whose grid is four times as large, fills the chip better while the grouped
 // one has few workgroups: up to 128 of them at head sizes up to 64, up to 80 above (the grouped
-// kernel's advantage, every key and value read once for four heads, grows with the head size).
+// kernel's advantage, every key and value read once for four heads, grows with the head size; at 256,
+// where the line was drawn with the kernel without copies, it would lie below 64).
 // Two tiles per workgroup (the b-th from the end and the b-th from the start of a causal prompt,
 // to even out the triangle) were measured against the order of workgroups described in the kernel
 // and dropped: within 3% at best, 12% slower at 3,072 tokens, up to 15% slower on top of a cached
 // prefix.
+
 // With one or two query heads per kv head a workgroup of the grouped kernel takes four or two
 // consecutive tiles of queries, so that four waves still share the keys and values it stages.
 static int prefill_tiles_per_wg(int group) { return group == 1 ? 4 : (group == 2 ? 2 : 1); }
@@ -2031,20 +2038,20 @@ static int launch_prefill_merge(hipStream_t s, const float* part_o, const float*
 // workgroups for 256 compute units: their keys are then dealt out to more of them, up to as many
 // workgroups as run at once (two per compute unit up to head size 64, one above), each run no
 // shorter than 512 keys, and a merge kernel puts the runs together. Measured with 32 query heads
-// on 8 kv heads, us per layer at head size 64 / 128, no cut -> cut: 512 tokens on 7,680 cached
-// 92 -> 60 / 148 -> 94; 512 on 60,000 625 -> 332 / 1,045 -> 590; 128 on 8,064 48 -> 27 / 92 -> 37;
-// 20 on 16,000 88 -> 23 / 170 -> 32. Where the per-head kernel would run (few workgroups), fewer
+// on 8 kv heads, us per layer at head size 64 / 128 with copied keys, no cut -> cut: 512 tokens on 7,680
+// cached 99 -> 56 / 144 -> 88; 512 on 60,000 707 -> 321 / 1,040 -> 587; 128 on 8,064 99 -> 29 / 146 -> 37;
+// 20 on 16,000 193 -> 23 / 275 -> 31 (the per-head kernel, whole: 90, 625, 48, 88 / 177, -, 92, 170). Where that would run (few workgroups), fewer
 // than four runs lose to it, and so do runs of under 1,024 keys once it has a workgroup per
 // compute unit itself (256 on 1,792: 17 -> 20 with four); where the grouped kernel would run
-// without a cut, two runs pay from 4,096 keys on (512 on 3,584 at head size 128: 78 -> 58) and,
-// above 128 workgroups, from 8,192 on (1,024 on 3,072: 56 -> 60; on 15,000: 199 -> 183).
+// without a cut, two runs pay from 4,096 keys on (512 on 3,584 at head size 128: 76 -> 55) and,
+// above 128 workgroups, from 8,192 on (1,024 on 3,072: 54 -> 58; on 15,000: 196 -> 174).
 static int grouped_nsplit(int n_tiles, int max_kv_len, int hq, int hkv, int head_dim) {
   const int64_t workgroups = grouped_workgroups(n_tiles, hq, hkv);
   const int at_once = head_dim <= 64 ? 512 : 256;
   if (2 * workgroups > at_once) return 1;
   if (grouped_smem(head_dim, 1, 1, static_cast<int>(ceil_div(max_kv_len, kPage))) > 160 * 1024) return 1;
   // 65 to 128 workgroups on 2,048 to 4,095 keys: two runs (512 tokens on 2,560 cached at head size
-  // 64 / 128: 43 -> 36 / 70 -> 54 us; on 1,536 cached 30 -> 28 / 44 -> 41).
+  // 64 / 128: 41 -> 31 / 59 -> 48 us; on 1,536 cached 29 -> 26 / 42 -> 39).
   if (workgroups > 64 && workgroups <= 128 && max_kv_len >= 2048 && max_kv_len < 4096) return 2;
   const int nsplit = static_cast<int>(std::min<int64_t>({at_once / workgroups, max_kv_len / kMinSplitKeys, kMaxPrefillSplit}));
   const bool per_head_else = few_grouped_workgroups(n_tiles, hq, hkv, head_dim);
@@ -2089,9 +2096,11 @@ static dim3 grouped_grid(int n_tiles, int n_blocks, int hq, int hkv, int nsplit)
 
 // How many waves a query head has there, each its own run of keys.
 // From head size 96 on, where a compute unit holds one workgroup of eight waves, four
-// workgroups per compute unit's worth of tiles run 5% faster as two workgroups of four waves
-// (one wave per head): two barriers' worth of waves that do not wait for each other
-// (head size 128: 4,096 tokens 181 -> 171 us, 8,192 tokens 657 -> 623 us; 2,048 tokens 56 -> 67).
+// workgroups per compute unit's worth of tiles run up to 15% faster as two workgroups of four waves
+// (one wave per head): two barriers' worth of waves that do not wait for each other (head
+// size 128, with copied keys: 4,096 tokens 175 -> 167 us, 5,000 267 -> 233, 8,192 670 -> 585, with three-term
+// weights 254 -> 253 and 955 -> 903; 2,048 tokens 54 -> 60, but 3,072, 768 workgroups, 113 -> 96; head size 256: 4,096 tokens
+// 467 -> 395, 8,192 1,724 -> 1,498; 2,048 135 -> 159).
 static int grouped_waves(const dim3& grid, int head_dim) {
   return head_dim < 96 || static_cast<int64_t>(grid.x) * grid.y * grid.z < 1024 ? 2 : 1;
 }

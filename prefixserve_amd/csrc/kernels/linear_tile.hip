@@ -289,7 +289,8 @@ int launch_form(hipStream_t s, int shape, const void* x, const void* w, void* ou
 // `half_step` where two share a unit and the round has only one for each, `round` beside the steps; a million bytes of w on their way
 // from memory, and each time another row of tiles asks for them; `start` once. Fitted, as the forms below, to the device's time
 // of 15,000 kernels, with weights that lay in no cache, as in a step: 130 to 8,192 tokens, 56 products from 64 x 64 to 2 x 28,672 x
-// 8,192. One in ten is off by 12% or more, and one in ten of those near the library's time by 9% or more.
+// 8,192. One in ten is off by 12% or more, and one in ten of those near the library's time by 9% or more. The largest shape's were fitted again to its loop of
+// four waves, with SiLU: over 260 gated products 0.92 to 1.12 of the measured time but for one in ten at either end, over 163 for the stream 0.98 on average.
 struct TileShape {
   int rows, cols, at_once;
   double step, half_step, round, weights, reads, start;
@@ -314,7 +315,8 @@ constexpr TileForm kQkvForm{0.0, 1.504, 7.37, 0.524, 0.206, 2.026, 0.132};
 // instruction beside them (7.3 to 10.5 us over 48 products; ReLU takes 3 less than SiLU), less what the activation kernel behind the library's
 // product takes longer too. Anything from 5.5 to 7.5 decides alike over those products. Without it, gated products with GELU ran in these tiles where
 // something else is the faster (us, the largest tiles / what runs now): 2 x 8,192 x 2,048 at 640 tokens 54.9 / 47.0, 2 x 6,144 x 1,024 at 640 37.2 /
-// 26.8, 2 x 2,816 x 1,024 at 2,048 35.6 / 31.4, 2 x 8,192 x 2,048 at 4,096 235 / 223; 2 x 8,192 x 3,072 at 900 keeps them, 81 / 97.
+// 26.8, 2 x 2,816 x 1,024 at 2,048 35.6 / 31.4, 2 x 8,192 x 2,048 at 4,096 235 / 223; 2 x 8,192 x 3,072 at 900 keeps them, 81 / 97, and 2 x 8,192 x 2,048 at 2,048,
+// which takes 118 / 118 one after the other and 136 to 141 / 130 to 137 among a step's other kernels.
 constexpr double kWideGelu = 6.5;
 // By what part products for the stream must be faster in the largest tiles than in smaller ones by the table, whose figures are good to that: of
 // 129 products that it would have do otherwise by any lead, 38 were slower by more than 2% (262 tokens x 6,944 x 7,552 54.0 -> 60.7 us) and 44 faster; with this
@@ -336,23 +338,24 @@ struct TilePlan {
 
 // The shape (and K-slices) of the least time by the table, if that is less than what the library takes by it. The library's figures are
 // fitted with errors towards more counted up to twice and lowered by up to 3%: its times of neighbouring sizes differ by a tenth and more, and no
-// product that it does faster should be taken from it. Of the 1,175 measured products 496 run in tiles, at 0.78 of the library's time
-// (stream), 0.76 (gated) and 0.83 (q/k/v); two are slower, by 5 and 11%. Of 1,980 others, drawn at random, 860 do, at 0.77, 0.69 and 0.78; 14
-// are slower by more than 2%, at most by 17% (915 tokens x 256 x 3,840, 13.5 / 15.8). us, the library and what follows > the tiles, or (the best tiles) where it stays with the library:
+// product that it does faster should be taken from it. Of 220 products for the stream, 220 gated ones with SiLU and 220 with GELU, drawn at random (129 to 1,023
+// and 4,096 tokens), 120, 113 and 92 run in tiles; those of them that take the library 30 us or more (36, 27, 23) at 0.73, 0.67 and 0.77 of its time; three,
+// none and two are slower by more than 2%, at most by 16% (387 tokens x 2,640 x 10,880 59.5 / 69.1). Of q/k/v products, whose shapes are older, 0.78 to 0.83. us,
+// the library and what follows > the tiles, or (the best tiles) where it stays with the library:
 //   tokens                        150          256          384          535          640          900          1,023        1,531         2,048
 //   q/k/v 3,072 x 2,048           16.4 (18.9)  17.5 (19.6)  19.3 (20.1)  21.7 > 20.3  22.4 > 21.1  28.4 (24.7)  30.8 (26.9)  33.4 (43.2)   38.6 (51.3)
 //   q/k/v 6,144 x 4,096           43.3 (33.3)  46.6 > 35.1  42.7 (38.8)  47.7 (44.6)  49.4 > 45.8  59.9 (81.0)  63.7 (86.2)  91.3 (127)    99.6 (138)
 //   gated 2 x 1,024 x 2,048       14.9 (17.3)  15.0 (17.9)  16.0 (17.9)  18.4 (17.5)  18.7 (18.0)  20.1 > 17.9  21.2 > 18.7  26.4 (23.1)   28.6 > 24.4
-//   gated 2 x 8,192 x 2,048       30.4 > 23.5  33.8 > 26.2  36.5 > 32.5  46.9 > 44.6  48.2 > 46.9  63.4 > 55.1  66.7 > 57.0  103 > 99.6    121 > 110
-//   gated 2 x 14,336 x 4,096      63.0 (61.2)  76.4 (92.3)  93.1 (105)   157 (155)    162 (187)    216 (227)    224 (229)    315 (336)     406 (436)
+//   gated 2 x 8,192 x 2,048       29.8 > 22.1  33.2 > 25.6  35.4 > 30.2  45.2 (43.8)  46.7 > 45.0  62.8 > 52.4  65.0 > 54.0  98.0 (96.2)   118 > 104
+//   gated 2 x 14,336 x 4,096      59.7 (57.0)  71.5 (83.3)  84.7 (89.7)  133 (144)    139 (159)    190 (174)    197 (179)    280 (274)     364 (371)
 //   with the norm 2,048 x 2,048   15.2 > 12.4  15.5 > 14.7  16.9 (17.2)  19.1 (19.6)  20.1 (20.2)  22.7 (22.7)  24.0 (23.7)
-//   2,048 x 8,192                 30.4 > 20.0  31.7 > 23.5  38.3 > 28.6  49.0 > 37.1  49.9 > 39.0  55.5 > 48.8  59.6 > 53.6  69.2 (82.9)   83.3 (93.6)
-//   4,096 x 4,096                 26.8 > 21.6  27.9 > 24.5  31.7 > 29.9  43.6 (40.9)  44.4 > 41.7  48.9 (50.0)  53.3 > 51.4  65.3 (67.1)   78.1 (102)
-//   4,096 x 14,336                62.5 > 38.5  68.4 > 51.2  86.5 > 61.6  122 > 98.6   127 > 102    140 > 124    152 > 130    192 (197)     236 (301)
+//   2,048 x 8,192                 29.5 > 19.3  30.4 > 22.9  36.6 > 27.5  46.7 > 34.0  47.3 > 36.6  50.5 > 45.0  54.8 > 50.3  69.2 (82.9)   83.3 (93.6)
+//   4,096 x 4,096                 26.0 > 20.1  27.2 > 23.5  30.7 > 28.5  41.5 (37.9)  41.6 > 38.6  46.6 (44.7)  49.7 > 47.9  65.3 (67.1)   78.1 (102)
+//   4,096 x 14,336                62.4 > 38.3  66.8 > 50.9  85.4 > 61.4  114 > 88.2   117 > 88.5   125 > 103    138 > 108    192 (197)     236 (301)
 // (From 1,024 tokens on the tiles add into the stream.) With four waves of 128 x 128 in the largest shape instead of eight of 128 x 64 that began each tile
 // anew (both sides on one card): gated 2 x 8,192 x 2,048 at 2,048 tokens 122 by the library and the activation -> 110, 2 x 4,096 x 2,048 63 -> 56 (at 1,531
 // 52 -> 48), 2 x 2,816 x 1,024 43 -> 29, 2 x 8,192 x 3,072 172 -> 153; with the norm 4,096 x 14,336 at 767 tokens 105 -> 97, 4,096 x 11,008 at 640 81 -> 73. 2 x 14,336 x
-// 4,096 would gain 5 to 10% from 900 tokens on (385 -> 363 at 2,048) and lose as much at 535 and 640: left to the library. In bfloat16 for the other norms the tiles had no lead: 2,048 x 2,048 15.1 / 19.0 at
+// 4,096 would gain 9% at 900 and 1,023 tokens and 2% at 1,531, and lose 2% at 2,048 and 15% at 640: left to the library. In bfloat16 for the other norms the tiles had no lead: 2,048 x 2,048 15.1 / 19.0 at
 // 130 tokens, 19.3 / 21.1 at 535, 34.8 / 34.9 at 2,048; such products are the library's.
 TilePlan tile_plan(int form, int M, int N, int K, int act = 0) {
   const bool stream = form == kTileSlices || form == kTileAdd;

@@ -414,7 +414,10 @@ struct TileCut {
   __device__ __forceinline__ int first(int tile) const { return 64 * (tile * units + min(tile, larger)); }
 };
 
-// The time of a large tile by its 64s of pairs, in 1/64 of a full one's (measured there).
+// The time of a large tile by its 64s of pairs, in 1/64 of a full one's, as measured of the loop of eight waves that stood in wide_tile.h's place. There 128
+// experts of 2,048 x 1,024 with 64, 128, 192 and 256 pairs each take 338, 388, 449 and 514 us (42, 48, 56, 64; before 342, 398, 485, 582); over 480
+// steps (ten shapes, 64 to 2,000 pairs an expert, even to uneven) the limit that these numbers choose takes 0.3% more than the best of the three, 9% at most, and those of
+// the new loop choose no better.
 __device__ __forceinline__ int tile_cost(int units) { return units <= 2 ? 42 : units == 3 ? 54 : 64; }
 
 // The time of the step's tiles under a limit of pairs, computed by one wave: every die runs an eighth of the tiles, 32 at once, and a
@@ -947,7 +950,9 @@ __global__ __launch_bounds__(64 * (TN / 16) * KG) void moe_stream_kernel(
 //    uneven) 0.91 of the time of tiles of 256 and a rest, 0.97 of that of the even cut (all of them with the loop before wide_tile.h's);
 //  * as many workgroups as there are units stay and walk the large tiles, the copies of one under the end of the one before: that and waves of 128
 //    x 128 against eight of 128 x 64 that began each tile anew, us of sorting and both products, 32 experts of 2,048 x 1,024: 448 pairs an expert
-//    225 -> 204, 512 273 -> 249 (all even 242 -> 227), 1,024 525 -> 455; 8 of 4,096 x 3,584 at 512 526 -> 469; 64 of 2,048 x 1,408 at 192 345 -> 314.
+//    225 -> 204, 512 273 -> 249 (all even 242 -> 227), 1,024 525 -> 455; 8 of 4,096 x 3,584 at 512 526 -> 469; 64 of 2,048 x 1,408 at 192 345 -> 314. Over 480 steps
+//    0.88 of the time, and 1.02 to 1.05 in twelve of them, mostly of 90 to 128 pairs an expert (32 of 2,048 x 1,024 at 90 116 -> 118, at 128 123 -> 127, 32 of 4,096 x
+//    2,048 at 90 349 -> 357): every tile's copies are those of 256 rows, and eight waves asked for a step more of the matrices where a tile had fewer.
 //    What is left of 249: gate and up 136 (one tile after the other 1.6 us a step of 64 k where the dense product takes 1.4: 268 MB of matrices come from
 //    memory meanwhile; 4 us of activations behind each tile, under which no matrix core works), down 90 (134 MB of float32 leave, 134 MB of matrices come).
 // GATED: a wave's rows of the matrix are gate rows and then the up rows of the same columns.
@@ -1391,14 +1396,14 @@ static int64_t tiles_from_pairs(int experts, int K, int F, int kind) {
 // in the second, and 300 more for what a large tile does in front of and behind its loop, which the two small ones on a unit do beside
 // each other's. An expert's last tile is half empty on average. us of both products and the sorting, 256 / 128 (E experts of K x F,
 // choices at random):
-//   32 of 2,048 x 1,024:  50 pairs an expert 109 / 109, 140 126 / 146, 260 163 / 194, 448 232 / 261, 1,000 580 / 594
-//    8 of 2,048 x 1,024:  64 59 / 58, 260 70 / 66, 512 92 / 107, 1,000 166 / 156, 2,000 262 / 279
-//    8 of 4,096 x 3,584:  64 156 / 159, 260 301 / 397, 448 377 / 547, 1,000 848 / 1,128
-//   24 of 1,024 x 320:    64 38 / 33, 512 75 / 72, 2,000 247 / 204
-//    4 of 1,024 x 512:    64 36 / 29, 512 43 / 34, 2,000 54 / 50
-//   64 of 2,048 x 1,408:  64 266 / 277, 448 639 / 750, 1,000 1,303 / 1,527
-// Over eight shapes at 17 sizes, choices even and uneven, the choice is on average 1.0% over the faster (always 256: 2.9%, always
-// 128: 7.8%), at worst 17%.
+//   32 of 2,048 x 1,024:  50 pairs an expert 111 / 108, 140 129 / 151, 260 161 / 208, 448 204 / 253, 1,000 467 / 586
+//    8 of 2,048 x 1,024:  64 63 / 57, 260 67 / 63, 512 77 / 100, 1,000 138 / 155, 2,000 224 / 272
+//    8 of 4,096 x 3,584:  64 170 / 165, 260 271 / 395, 448 324 / 540, 1,000 709 / 1,123
+//   24 of 1,024 x 320:    64 42 / 35, 512 65 / 70, 2,000 207 / 200
+//    4 of 1,024 x 512:    64 35 / 29, 512 41 / 33, 2,000 56 / 65
+//   64 of 2,048 x 1,408:  140 284 / 378, 448 530 / 721, 1,000 1,093 / 1,497
+// The 1.2 and the 300 were fitted to the loop of eight waves, whose tiles did not begin under the end of the one before: over 724 steps (ten shapes, 64 to 2,000
+// pairs an expert, even to uneven) the choice is 1.5% over the faster on average (always 256: 0.7%, always 128: 21%), 30% at worst, all of them left to 128.
 static int wide_tile_rows(int64_t pairs, int experts, int K, int F, int kind) {
   if (pairs < tiles_from_pairs(experts, K, F, kind) * experts) return 0;
   auto rounds = [&](int rows, int at_once, int beside) {
