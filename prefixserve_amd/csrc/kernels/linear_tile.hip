@@ -316,11 +316,12 @@ constexpr TileForm kQkvForm{0.0, 1.504, 7.37, 0.524, 0.206, 2.026, 0.132};
 // product takes longer too. Anything from 5.5 to 7.5 decides alike over those products. Without it, gated products with GELU ran in these tiles where
 // something else is the faster (us, the largest tiles / what runs now): 2 x 8,192 x 2,048 at 640 tokens 54.9 / 47.0, 2 x 6,144 x 1,024 at 640 37.2 /
 // 26.8, 2 x 2,816 x 1,024 at 2,048 35.6 / 31.4, 2 x 8,192 x 2,048 at 4,096 235 / 223; 2 x 8,192 x 3,072 at 900 keeps them, 81 / 97, and 2 x 8,192 x 2,048 at 2,048,
-// which takes 118 / 118 one after the other and 136 to 141 / 130 to 137 among a step's other kernels.
+// which takes 118 / 118 one after the other and 136 to 141 / 130 to 137 among a step's other kernels. Over 36 products with GELU 0.98 of the time that it is without this;
+// the library's fit, on its fast side, keeps some that these tiles do faster (2 x 11,008 x 1,536 at 2,048 tokens 143 / 165, at 4,096 290 / 300).
 constexpr double kWideGelu = 6.5;
 // By what part products for the stream must be faster in the largest tiles than in smaller ones by the table, whose figures are good to that: of
 // 129 products that it would have do otherwise by any lead, 38 were slower by more than 2% (262 tokens x 6,944 x 7,552 54.0 -> 60.7 us) and 44 faster; with this
-// one 3 are slower (at most 9%) and the sum of the times is the same. Two slices of them, which are only ever chosen close to the library, lost to it by 3 to 8% in
+// one 3 are slower (at most 9%) and the sum of the times is the same; of 110 others that run in the largest tiles by it, at 0.88 of the time, 6 are slower, by 2 to 7%. Two slices of them, which are only ever chosen close to the library, lost to it by 3 to 8% in
 // all of four products (555 x 7,552 x 5,696 71.4 / 77.1) and are not taken.
 constexpr double kWideLead = 1.06;
 
